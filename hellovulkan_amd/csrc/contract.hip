@@ -1,20 +1,43 @@
 // contract.hip — the dense-contraction cube filter on FP16 MFMA
 // (hvx_ibl_contract_* and hvx_ibl_filter_contract of include/hvx.h).
 //
-// The operator is defined in hvx_contract.h. A plan holds, per output mip,
-// the precomputed weight matrices of the canonical face (shared by all six
-// faces), built on the GPU in FP64: the row normalisation sums are FP64
-// reductions, and each row is stored in FP16 scaled by a power of two that
-// puts its largest weight just under 2^15. A filter call stages the input
-// radiance as FP16 scaled per face by a power of two (largest value under
-// 2^15), then runs one MFMA GEMM per weight matrix:
+// The operator is defined in hvx_contract.h: per output mip a weight matrix
+// W(o, k) of the canonical face, shared by all six faces. The geometry is
+// also symmetric under the eight maps g of the square onto itself (u -> -u,
+// v -> -v, u <-> v, acting on the output face's plane and, as rotations and
+// reflections about its axis, on the whole sphere): W(g o, g k) = W(o, k). So
+// a plan holds only the rows of one octant of the face (0 <= x <= y < So / 2)
+// and a filter call multiplies each row into 6 faces x 8 maps x 3 channels:
 //
-//   C[rows, 6 faces x 4] = W[rows, K] * R[K, 6 faces x 4]    (FP32 accumulate)
+//   C[rows, 144] = W[rows, K] * R[K, 144]    (FP16 MFMA, FP32 accumulate)
 //
-// where column block f of R holds the input texels seen from output face f
-// (a permutation of the level for full-sphere sums; face f's padded plane
-// window for the near field). Rows are canonical output texels, so one
-// weight matrix serves the six faces as six column blocks.
+// where column (g, f, c) of R holds channel c of the input texel that output
+// face f sees as g k: C's column (g, f, c) is the output at g o of face f. A
+// row of weights (the matrices do not fit the caches) is thus read once for
+// 48 output texels instead of 6; 144 columns are nine 16-wide MFMA column
+// tiles without padding.
+//
+// K runs over units of eight texels along a row of the summed level (of the
+// padded face plane for the near field). Rows are ordered along a Morton
+// curve, so 128 consecutive ones (a block) lie close together on the face,
+// and a block keeps only the units in which any of its rows has weight: half
+// of the sphere lies behind a row, and a near window is a disk, not its
+// bounding box.
+//
+// The weights are built on the GPU in FP64: the row normalisation sums are
+// FP64 reductions, and each row is stored in FP16 scaled by a power of two
+// that puts its largest weight just under 2^15. A filter call stages the
+// input radiance as FP16 scaled per face by a power of two (largest value
+// under 2^15).
+//
+// Measured (MI355X, whole calls, before: one row per output texel of the
+// canonical face, 6 faces x 4 padded columns, windows as bounding boxes):
+//   1024^2 -> 512^2 x 10, FP16           444 -> 129 us (weights 1606 -> 108 MB)
+//   512^2 -> 256^2 x 9, split BF16       353 -> 100 us
+//   24 probes 256^2 -> 128^2 x 8, FP16   855 -> 340 us
+// The 129 us are 45 us of GEMM, 36 us of staging with the roughness-0 mip
+// (100 MB of level 0 read, 25 MB written), 22 us for the near rows' epilogue
+// and 22 us for the four small launches.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -45,18 +68,13 @@ using hvx::texel_dir;
 
 enum Piece { PIECE_WHOLE = 0, PIECE_NEAR = 1, PIECE_FAR = 2 };
 
-// Dense (full-sphere) weight matrix: rows are the canonical texels of an
-// So x So face, columns every texel of a 6 x Sin x Sin level.
-struct DenseGeom {
-    int type, piece;
-    double alpha2, t0, t1;
-    uint32_t So, Sin;
-    uint32_t rows, rt, ks;  // rows = So^2, row tiles of 16, k-steps of 32
-};
+constexpr int kMaxJobs = 2 * hvx::kContractMaxMips;  // weight matrices (and staged inputs) of a plan
+constexpr uint32_t kImages = 48;                     // output texels of a row: 8 maps x 6 faces
+constexpr uint32_t kCols = 3 * kImages;              // columns of the contraction
+constexpr uint32_t kBlockRows = 128;                 // rows that share a unit list
+constexpr uint32_t kFaceMaxBlocks = 32;
+constexpr uint32_t kMaxProbes = 4096;  // probes of one multi-probe call (grid dimension y)
 
-// Near-field window of one 16 x 16 output tile, in (unpadded) texel indices
-// of the face plane at the near level; woff = weight offset in half8 units.
-// The tile's weights are [k-step][row tile (16)][lane (64)][8].
 // The probes of one filter call: input chains and output chains (one probe:
 // the by-value pointers; several: device arrays of pointers), and where probe
 // p's copy of the per-call scratch lives: a scratch pointer of the plan moves
@@ -67,32 +85,132 @@ struct Probes {
     const float4* const* chains;
     float4* const* outs;
     uint64_t delta, pstride;
-    uint32_t probe_fast;  // GEMMs: grid x = probe group, y = workgroup (groups sharing weights dispatch together)
-    uint32_t n;           // probes in the call
+    uint32_t n;  // probes in the call
 };
-// (workgroup, probe) of a GEMM launch
-__device__ __forceinline__ uint2 gemm_block(const Probes& Q) {
-    return Q.probe_fast ? make_uint2(blockIdx.y, blockIdx.x) : make_uint2(blockIdx.x, blockIdx.y);
-}
 __device__ __forceinline__ const float4* probe_chain(const Probes& Q, uint32_t p) { return Q.chains ? Q.chains[p] : Q.chain0; }
 __device__ __forceinline__ float4* probe_out(const Probes& Q, uint32_t p) { return Q.outs ? Q.outs[p] : Q.out0; }
 template <class T> __device__ __forceinline__ T* scr(const Probes& Q, T* ptr, uint32_t p) {
     return reinterpret_cast<T*>(reinterpret_cast<uintptr_t>(ptr) + Q.delta + (uint64_t)p * Q.pstride);
 }
 
-struct NearTile {
-    int32_t x0, y0;
-    uint32_t w, h;
-    uint64_t woff;
+// One weight matrix: the whole sum of a mip, or its near or far piece.
+struct Job {
+    int type, piece;
+    double alpha2, t0, t1;
+    uint32_t So;     // output face of the rows (far: the far grid's face)
+    uint32_t Sf;     // near: the far map's face
+    float4* map;     // far: the far map written; near: the far map added (scratch)
+    float4* zmap;    // far: the far normaliser at the far grid, written at plan creation; near: read there
+    size_t out_off;  // whole and near: the mip in the output chain, float4 units
 };
 
-struct NearGeom {
-    int type;
-    double alpha2, t0, t1;
-    uint32_t So, Si, te;  // output face, near level face, tiles per edge
+// A row: canonical output texel (x, y) of its job's face, x <= y < So / 2.
+struct Row {
+    uint16_t x, y, job, block;
+};
+
+// A staged input: a level of the chain (pad 0: unit u holds texels 8u .. 8u+7
+// of the 6 x S x S canonical level) or the face planes continued past the
+// edges (pad 1: unit u holds texels 8 (u % Pw8) .. of row u / Pw8 of the
+// Pw x Pw plane, Pw = S + 2B, whose texel (B, B) is the face's first).
+struct Source {
+    uint32_t pad, S, B, Pw8;
+};
+
+// 128 rows (fewer at a source's end) and the units they sum: nsteps K steps
+// of four units, the weights as [step][row tile (nrt)][lane (64)][8], cut
+// into K slices whose partial sums are added in slice order.
+struct Block {
+    uint32_t row0, nrows, nrt, nunits, nsteps;
+    uint32_t unit0;  // first entry in the unit list (staged unit indices)
+    uint32_t src, split, item0, nslices;
+    uint64_t woff, w_lo;  // 16-byte units; w_lo: split BF16, from hi to lo
+};
+
+// K slice of a block: steps [s0, s0 + n); slot: its partial sums.
+struct Item {
+    uint32_t block, s0, n, slot;
 };
 
 // ---------------------------------------------------------- device helpers
+// Map g of the square of n texels per edge onto itself: swap for g >= 4, then
+// mirror x (bit 0) and y (bit 1).
+__device__ __forceinline__ void image_of(uint32_t g, uint32_t n, uint32_t& x, uint32_t& y) {
+    if (g & 4u) {
+        const uint32_t t = x;
+        x = y;
+        y = t;
+    }
+    if (g & 1u) x = n - 1 - x;
+    if (g & 2u) y = n - 1 - y;
+}
+// Whether map g writes its own image of row (x, y): a row on the diagonal
+// (or on a 1 x 1 face) is its own mirror image and written once.
+__device__ __forceinline__ bool image_written(uint32_t g, uint32_t n, uint32_t x, uint32_t y) {
+    return n == 1 ? g == 0 : (g < 4 || x != y);
+}
+
+// Plane point (a, b) of face f at distance w from the centre (texel_dir's
+// convention, as contract_face_point).
+__host__ __device__ inline void face_ipoint(uint32_t f, int a, int b, int w, int p[3]) {
+    switch (f) {
+        case 0: p[0] = w; p[1] = -b; p[2] = -a; break;
+        case 1: p[0] = -w; p[1] = -b; p[2] = a; break;
+        case 2: p[0] = a; p[1] = w; p[2] = b; break;
+        case 3: p[0] = a; p[1] = -w; p[2] = -b; break;
+        case 4: p[0] = a; p[1] = -b; p[2] = w; break;
+        default: p[0] = -a; p[1] = -b; p[2] = -w; break;
+    }
+}
+
+// Texel (face, i, j) of a level of face s that output face f sees as g k, k the
+// canonical input texel (x, y) of face t: exact integer arithmetic in doubled
+// texel units (a texel centre of face t is the plane point (a, b), odd, at
+// distance s; the canonical output face is (u, v, 1), so g acts on the first
+// two components).
+inline void dense_source(uint32_t f, uint32_t g, uint32_t t, int x, int y, int s, int out[3]) {
+    int p[3], q[3];
+    face_ipoint(t, 2 * x + 1 - s, 2 * y + 1 - s, s, p);
+    if (g & 4u) std::swap(p[0], p[1]);
+    if (g & 1u) p[0] = -p[0];
+    if (g & 2u) p[1] = -p[1];
+    face_ipoint(f, p[0], p[1], p[2], q);
+    const int ax = std::abs(q[0]), ay = std::abs(q[1]), az = std::abs(q[2]);
+    int nf, na, nb;
+    if (ax >= ay && ax >= az) {
+        nf = q[0] > 0 ? 0 : 1;
+        na = q[0] > 0 ? -q[2] : q[2];
+        nb = -q[1];
+    } else if (ay >= az) {
+        nf = q[1] > 0 ? 2 : 3;
+        na = q[0];
+        nb = q[1] > 0 ? q[2] : -q[2];
+    } else {
+        nf = q[2] > 0 ? 4 : 5;
+        na = q[2] > 0 ? q[0] : -q[0];
+        nb = -q[1];
+    }
+    out[0] = nf;
+    out[1] = (na + s - 1) / 2;
+    out[2] = (nb + s - 1) / 2;
+}
+
+// dense_source as data, entry [t][6 g + f]: the face (3 bits), then whether x
+// and y swap (8), and then whether i (16) and j (32) run backwards.
+std::vector<uint8_t> source_table() {
+    std::vector<uint8_t> tab(6 * kImages);
+    for (uint32_t t = 0; t < 6; ++t)
+        for (uint32_t g = 0; g < 8; ++g)
+            for (uint32_t f = 0; f < 6; ++f) {
+                int o[3], a[3];
+                dense_source(f, g, t, 0, 0, 2, o);
+                dense_source(f, g, t, 1, 0, 2, a);
+                tab[t * kImages + 6 * g + f] =
+                    (uint8_t)(o[0] | (a[1] == o[1] ? 8 : 0) | (o[1] ? 16 : 0) | (o[2] ? 32 : 0));
+            }
+    return tab;
+}
+
 __device__ __forceinline__ void local_dir(double u, double v, double d[3]) {
     const double r = 1.0 / sqrt(1.0 + u * u + v * v);
     d[0] = u * r;
@@ -100,47 +218,38 @@ __device__ __forceinline__ void local_dir(double u, double v, double d[3]) {
     d[2] = r;
 }
 
-// Canonical input texel k of a 6 x S x S level: direction and solid angle.
-__device__ __forceinline__ void canon_input(uint32_t k, uint32_t S, double l[3], double* dw) {
-    const uint32_t S2 = S * S, g = k / S2, rem = k - g * S2, y = rem / S, x = rem - y * S;
-    const double u = hvx::contract_coord((int)x, S), v = hvx::contract_coord((int)y, S);
+// Direction and solid angle of texel q of unit u of a source.
+__device__ __forceinline__ void unit_texel(const Source& G, uint32_t unit, uint32_t q, double l[3], double* dw) {
+    if (G.pad) {
+        const uint32_t py = unit / G.Pw8, px = (unit - py * G.Pw8) * 8 + q;
+        const double u = hvx::contract_coord((int)px - (int)G.B, G.S), v = hvx::contract_coord((int)py - (int)G.B, G.S);
+        local_dir(u, v, l);
+        *dw = hvx::contract_dw(u, v, G.S);
+        return;
+    }
+    const uint32_t k = unit * 8 + q, S2 = G.S * G.S, t = k / S2, rem = k - t * S2, y = rem / G.S, x = rem - y * G.S;
+    const double u = hvx::contract_coord((int)x, G.S), v = hvx::contract_coord((int)y, G.S);
     double p[3];
-    hvx::contract_face_point((int)g, u, v, p);
+    hvx::contract_face_point((int)t, u, v, p);
     const double r = 1.0 / sqrt(1.0 + u * u + v * v);
     l[0] = p[0] * r;
     l[1] = p[1] * r;
     l[2] = p[2] * r;
-    *dw = hvx::contract_dw(u, v, S);
+    *dw = hvx::contract_dw(u, v, G.S);
 }
 
-__device__ __forceinline__ double piece_weight(int type, int piece, double alpha2, double t0, double t1, double c,
-                                               double dw) {
-    double w = hvx::contract_weight(type, alpha2, c);
+__device__ __forceinline__ void row_dir(const Row& R, uint32_t So, double n[3]) {
+    local_dir(hvx::contract_coord((int)R.x, So), hvx::contract_coord((int)R.y, So), n);
+}
+
+__device__ __forceinline__ double row_weight(const Job& J, const double n[3], const double l[3], double dw) {
+    const double c = (n[0] * l[0] + n[1] * l[1]) + n[2] * l[2];
+    double w = hvx::contract_weight(J.type, J.alpha2, c);
     if (w == 0.0) return 0.0;
     w *= dw;
-    if (piece == PIECE_NEAR) w *= hvx::contract_phi(t0, t1, c);
-    else if (piece == PIECE_FAR) w *= 1.0 - hvx::contract_phi(t0, t1, c);
+    if (J.piece == PIECE_NEAR) w *= hvx::contract_phi(J.t0, J.t1, c);
+    else if (J.piece == PIECE_FAR) w *= 1.0 - hvx::contract_phi(J.t0, J.t1, c);
     return w;
-}
-
-__device__ __forceinline__ void dense_row_dir(const DenseGeom& G, uint32_t row, double n[3]) {
-    const uint32_t y = row / G.So, x = row - y * G.So;
-    local_dir(hvx::contract_coord((int)x, G.So), hvx::contract_coord((int)y, G.So), n);
-}
-
-__device__ __forceinline__ double dense_w(const DenseGeom& G, const double n[3], uint32_t k) {
-    double l[3], dw;
-    canon_input(k, G.Sin, l, &dw);
-    const double c = (n[0] * l[0] + n[1] * l[1]) + n[2] * l[2];
-    return piece_weight(G.type, G.piece, G.alpha2, G.t0, G.t1, c, dw);
-}
-
-__device__ __forceinline__ double near_w(const NearGeom& G, const double n[3], int px, int py) {
-    const double u = hvx::contract_coord(px, G.Si), v = hvx::contract_coord(py, G.Si);
-    double l[3];
-    local_dir(u, v, l);
-    const double c = (n[0] * l[0] + n[1] * l[1]) + n[2] * l[2];
-    return piece_weight(G.type, PIECE_NEAR, G.alpha2, G.t0, G.t1, c, hvx::contract_dw(u, v, G.Si));
 }
 
 // Power-of-two exponent s with w_max * 2^s in (2^14, 2^15].
@@ -170,157 +279,145 @@ __device__ void block_sum_max(double s, double m, double* sh_s, double* sh_m, do
     }
 }
 
-// ------------------------------------------------------ plan: dense weights
-__global__ __launch_bounds__(256) void dense_row_kernel(DenseGeom G, double* __restrict__ Z,
-                                                        double* __restrict__ wmax) {
+// ------------------------------------------------------------ plan: weights
+// flags[b][u] = 1 when any row of block block0 + b may have weight in unit u:
+// the texel lies in front of the row and, for the near piece, inside the
+// window (each bound relaxed by more than the cosine's rounding).
+__global__ __launch_bounds__(256) void unit_flag_kernel(Source G, const Job* __restrict__ jobs,
+                                                        const Row* __restrict__ rows, const Block* __restrict__ blocks,
+                                                        uint32_t block0, uint32_t raw, uint8_t* __restrict__ flags) {
+    __shared__ double sd[kBlockRows][3], sc[kBlockRows];
+    const Block B = blocks[block0 + blockIdx.y];
+    for (uint32_t r = threadIdx.x; r < B.nrows; r += 256) {
+        const Row R = rows[B.row0 + r];
+        const Job& J = jobs[R.job];
+        row_dir(R, J.So, sd[r]);
+        sc[r] = (J.piece == PIECE_NEAR ? cos(J.t1) : 0.0) - 1e-9;
+    }
+    __syncthreads();
+    const uint32_t u = blockIdx.x * 256 + threadIdx.x;
+    if (u >= raw) return;
+    bool any = false;
+    for (uint32_t q = 0; q < 8 && !any; ++q) {
+        double l[3], dw;
+        unit_texel(G, u, q, l, &dw);
+        for (uint32_t r = 0; r < B.nrows && !any; ++r)
+            any = (sd[r][0] * l[0] + sd[r][1] * l[1]) + sd[r][2] * l[2] > sc[r];
+    }
+    flags[(size_t)blockIdx.y * raw + u] = any ? 1 : 0;
+}
+
+// Sum and largest weight of every row of a source (one workgroup per row).
+// units: the source's staged units; ulist: the blocks' lists of them.
+__global__ __launch_bounds__(256) void row_sum_kernel(Source G, const Job* __restrict__ jobs,
+                                                      const Row* __restrict__ rows, const Block* __restrict__ blocks,
+                                                      const uint32_t* __restrict__ ulist,
+                                                      const uint32_t* __restrict__ units, uint32_t row0,
+                                                      double* __restrict__ Z, double* __restrict__ wmax) {
     __shared__ double sh_s[256], sh_m[256];
-    const uint32_t row = blockIdx.x;
+    const uint32_t row = row0 + blockIdx.x;
+    const Row R = rows[row];
+    const Job J = jobs[R.job];
+    const Block B = blocks[R.block];
     double n[3];
-    dense_row_dir(G, row, n);
-    const uint32_t K = 6 * G.Sin * G.Sin;
+    row_dir(R, J.So, n);
     double s = 0.0, m = 0.0;
-    for (uint32_t k = threadIdx.x; k < K; k += 256) {
-        const double w = dense_w(G, n, k);
+    for (uint32_t k = threadIdx.x; k < B.nunits * 8; k += 256) {
+        double l[3], dw;
+        unit_texel(G, units[ulist[B.unit0 + k / 8]], k & 7, l, &dw);
+        const double w = row_weight(J, n, l, dw);
         s += w;
         m = m < w ? w : m;
     }
     block_sum_max(s, m, sh_s, sh_m, &Z[row], &wmax[row]);
 }
 
-// SPLIT: BF16 hi at W, lo = bf16(v - hi) at W + lo_off (16-byte units)
+// The MFMA A operands of a source's blocks (grid y: block; padding rows and
+// units hold zeros). SPLIT: the scaled weight v as BF16 hi = bf16(v) and, at
+// w_lo, lo = bf16(v - hi) (hi + lo carries ~16 significant bits).
 template <bool SPLIT>
-__global__ __launch_bounds__(256) void dense_fill_kernel(DenseGeom G, const double* __restrict__ wmax,
-                                                         half8* __restrict__ W, uint64_t lo_off) {
-    const uint64_t id = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-    if (id >= (uint64_t)G.rt * G.ks * 64) return;
-    const uint32_t lane = (uint32_t)(id & 63);
-    const uint64_t t = id >> 6;
-    const uint32_t ks = (uint32_t)(t % G.ks), rt = (uint32_t)(t / G.ks);
-    const uint32_t row = rt * 16 + (lane & 15), k0 = ks * 32 + 8 * (lane >> 4);
-    double v[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    if (row < G.rows) {
-        double n[3];
-        dense_row_dir(G, row, n);
-        const double sc = ldexp(1.0, row_exponent(wmax[row]));
-#pragma unroll
-        for (int q = 0; q < 8; ++q) v[q] = dense_w(G, n, k0 + q) * sc;
-    }
-    if constexpr (SPLIT) {
-        bf16x8 hi, lo;
-#pragma unroll
-        for (int q = 0; q < 8; ++q) {
-            hi[q] = (__bf16)(float)v[q];
-            lo[q] = (__bf16)(float)(v[q] - (double)(float)hi[q]);
+__global__ __launch_bounds__(256) void weight_fill_kernel(Source G, const Job* __restrict__ jobs,
+                                                          const Row* __restrict__ rows,
+                                                          const Block* __restrict__ blocks, uint32_t block0,
+                                                          const uint32_t* __restrict__ ulist,
+                                                          const uint32_t* __restrict__ units,
+                                                          const double* __restrict__ wmax, half8* __restrict__ W) {
+    const Block B = blocks[block0 + blockIdx.y];
+    const uint32_t total = B.nsteps * B.nrt * 64;
+    for (uint32_t id = blockIdx.x * 256 + threadIdx.x; id < total; id += gridDim.x * 256) {
+        const uint32_t lane = id & 63, rt = (id >> 6) % B.nrt, step = (id >> 6) / B.nrt;
+        const uint32_t r = rt * 16 + (lane & 15), u = step * 4 + (lane >> 4);
+        double v[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+        if (r < B.nrows && u < B.nunits) {
+            const Row R = rows[B.row0 + r];
+            const Job& J = jobs[R.job];
+            double n[3];
+            row_dir(R, J.So, n);
+            const double sc = ldexp(1.0, row_exponent(wmax[B.row0 + r]));
+            const uint32_t unit = units[ulist[B.unit0 + u]];
+            for (uint32_t q = 0; q < 8; ++q) {
+                double l[3], dw;
+                unit_texel(G, unit, q, l, &dw);
+                v[q] = row_weight(J, n, l, dw) * sc;
+            }
         }
-        reinterpret_cast<bf16x8*>(W)[id] = hi;
-        reinterpret_cast<bf16x8*>(W)[id + lo_off] = lo;
-    } else {
-        half8 out;
-#pragma unroll
-        for (int q = 0; q < 8; ++q) out[q] = (_Float16)(float)v[q];
-        W[id] = out;
-    }
-}
-
-// rowscale = 2^-s / Z (normalised rows) or 2^-s (raw far rows; then the
-// far normaliser goes to a six-face map, identical on every face).
-__global__ __launch_bounds__(256) void dense_scale_kernel(uint32_t rows, const double* __restrict__ Z,
-                                                          const double* __restrict__ wmax, int raw,
-                                                          float* __restrict__ rowscale, float4* __restrict__ zmap) {
-    const uint32_t r = blockIdx.x * 256 + threadIdx.x;
-    if (r >= rows) return;
-    const double p = ldexp(1.0, -row_exponent(wmax[r]));
-    rowscale[r] = raw ? (float)p : (float)(p / Z[r]);
-    if (raw)
-        for (uint32_t f = 0; f < 6; ++f) zmap[f * rows + r] = make_float4((float)Z[r], 0.0f, 0.0f, 0.0f);
-}
-
-// -------------------------------------------------------- plan: near weights
-__global__ __launch_bounds__(256) void near_row_kernel(NearGeom G, const NearTile* __restrict__ tiles,
-                                                       double* __restrict__ Z, double* __restrict__ wmax) {
-    __shared__ double sh_s[256], sh_m[256];
-    const uint32_t o = blockIdx.x, Y = o / G.So, X = o - Y * G.So;
-    const NearTile T = tiles[(Y / 16) * G.te + X / 16];
-    double n[3];
-    local_dir(hvx::contract_coord((int)X, G.So), hvx::contract_coord((int)Y, G.So), n);
-    const uint32_t K = T.w * T.h;
-    double s = 0.0, m = 0.0;
-    for (uint32_t k = threadIdx.x; k < K; k += 256) {
-        const uint32_t r = k / T.w, c = k - r * T.w;
-        const double w = near_w(G, n, T.x0 + (int)c, T.y0 + (int)r);
-        s += w;
-        m = m < w ? w : m;
-    }
-    block_sum_max(s, m, sh_s, sh_m, &Z[o], &wmax[o]);
-}
-
-// grid: tiles x 16 row tiles; each block writes one row tile's k-steps.
-// SPLIT: the scaled weight v is stored as BF16 hi = bf16(v) at W and
-// lo = bf16(v - hi) at W + lo_off (hi + lo carries ~16 significant bits).
-template <bool SPLIT>
-__global__ __launch_bounds__(256) void near_fill_kernel(NearGeom G, const NearTile* __restrict__ tiles,
-                                                        const double* __restrict__ wmax, half8* __restrict__ W,
-                                                        uint64_t lo_off) {
-    const uint32_t tile = blockIdx.x / 16, rt = blockIdx.x % 16;
-    const NearTile T = tiles[tile];
-    const uint32_t KS = T.h * (T.w / 32);
-    const uint32_t X0 = (tile % G.te) * 16, Y = (tile / G.te) * 16 + rt;
-    for (uint32_t idx = threadIdx.x; idx < KS * 64; idx += 256) {
-        const uint32_t ks = idx >> 6, lane = idx & 63;
-        const uint32_t X = X0 + (lane & 15), o = Y * G.So + X;
-        double n[3];
-        local_dir(hvx::contract_coord((int)X, G.So), hvx::contract_coord((int)Y, G.So), n);
-        const double sc = ldexp(1.0, row_exponent(wmax[o]));
-        const uint32_t k0 = ks * 32 + 8 * (lane >> 4), r = k0 / T.w, c0 = k0 - r * T.w;
-        const uint64_t at = T.woff + ((uint64_t)ks * 16 + rt) * 64 + lane;  // K-step major
         if constexpr (SPLIT) {
             bf16x8 hi, lo;
 #pragma unroll
             for (int q = 0; q < 8; ++q) {
-                const double v = near_w(G, n, T.x0 + (int)(c0 + q), T.y0 + (int)r) * sc;
-                hi[q] = (__bf16)(float)v;
-                lo[q] = (__bf16)(float)(v - (double)(float)hi[q]);
+                hi[q] = (__bf16)(float)v[q];
+                lo[q] = (__bf16)(float)(v[q] - (double)(float)hi[q]);
             }
-            reinterpret_cast<bf16x8*>(W)[at] = hi;
-            reinterpret_cast<bf16x8*>(W)[at + lo_off] = lo;
+            reinterpret_cast<bf16x8*>(W)[B.woff + id] = hi;
+            reinterpret_cast<bf16x8*>(W)[B.woff + id + B.w_lo] = lo;
         } else {
             half8 out;
 #pragma unroll
-            for (int q = 0; q < 8; ++q)
-                out[q] = (_Float16)(float)(near_w(G, n, T.x0 + (int)(c0 + q), T.y0 + (int)r) * sc);
-            W[at] = out;
+            for (int q = 0; q < 8; ++q) out[q] = (_Float16)(float)v[q];
+            W[B.woff + id] = out;
         }
     }
 }
 
-// Z(o) = Z_near(o) + far normaliser interpolated at o (any face: the far
-// normaliser map is the same on every face).
-__global__ __launch_bounds__(256) void near_scale_kernel(NearGeom G, uint32_t Sf, const double* __restrict__ Z,
-                                                         const double* __restrict__ wmax,
-                                                         const float4* __restrict__ zmap,
-                                                         float* __restrict__ rowscale, float* __restrict__ invZ) {
-    const uint32_t o = blockIdx.x * 256 + threadIdx.x;
-    if (o >= G.So * G.So) return;
-    const uint32_t Y = o / G.So, X = o - Y * G.So;
-    const f3 zf = sample_cube(zmap, (int)Sf, texel_dir(0, (int)X, (int)Y, (int)G.So));
-    const double Zt = Z[o] + (double)zf.x;
-    rowscale[o] = (float)(ldexp(1.0, -row_exponent(wmax[o])) / Zt);
-    invZ[o] = (float)(1.0 / Zt);
+// Far rows: the normaliser at every image of the row (the same on all faces).
+__global__ __launch_bounds__(256) void far_norm_kernel(const Job* __restrict__ jobs, const Row* __restrict__ rows,
+                                                       uint32_t row0, uint32_t n, const double* __restrict__ Z) {
+    const uint32_t id = blockIdx.x * 256 + threadIdx.x;
+    if (id >= n * kImages) return;
+    const uint32_t r = row0 + id / kImages, gf = id % kImages;
+    const Row R = rows[r];
+    const Job& J = jobs[R.job];
+    if (J.piece != PIECE_FAR) return;
+    uint32_t x = R.x, y = R.y;
+    if (!image_written(gf / 6, J.So, x, y)) return;
+    image_of(gf / 6, J.So, x, y);
+    J.zmap[((gf % 6) * J.So + y) * J.So + x] = make_float4((float)Z[r], 0.0f, 0.0f, 0.0f);
+}
+
+// rowscale = 2^-s / Z (whole rows), 2^-s (far rows), 2^-s / (Z + far
+// normaliser interpolated at the row's direction) (near rows, with the
+// reciprocal of that sum in invZ).
+__global__ __launch_bounds__(256) void row_scale_kernel(const Job* __restrict__ jobs, const Row* __restrict__ rows,
+                                                        uint32_t n, const double* __restrict__ Z,
+                                                        const double* __restrict__ wmax, float* __restrict__ rowscale,
+                                                        float* __restrict__ invZ) {
+    const uint32_t r = blockIdx.x * 256 + threadIdx.x;
+    if (r >= n) return;
+    const Row R = rows[r];
+    const Job& J = jobs[R.job];
+    double z = J.piece == PIECE_FAR ? 1.0 : Z[r];
+    if (J.piece == PIECE_NEAR) {
+        const f3 zf = sample_cube(J.zmap, (int)J.Sf, texel_dir(0, (int)R.x, (int)R.y, (int)J.So));
+        z += (double)zf.x;
+    }
+    rowscale[r] = (float)(ldexp(1.0, -row_exponent(wmax[r])) / z);
+    invZ[r] = (float)(1.0 / z);
 }
 
 // ------------------------------------------------------ per-call staging
-// A filter call is eight launches: face maxima, exponent scales, all staging
-// (every dense level and padded plane), all dense GEMMs, all their
-// epilogues, all near-field tiles, all far-field additions, and the
-// roughness-0 mip. Each fused launch finds its job by running offsets in a
-// table passed by value.
-constexpr int kMaxJobs = 2 * hvx::kContractMaxMips;
-constexpr uint32_t kFaceMaxBlocks = 32;
-constexpr uint32_t kMaxProbes = 4096;  // probes of one multi-probe call (grid dimension y)
-#ifndef HVX_PROBE_GROUP
-#define HVX_PROBE_GROUP 4
-#endif
-constexpr int kProbeGroup = HVX_PROBE_GROUP;  // probes per wave in multi-probe GEMMs
+// A filter call is at most seven launches: face maxima, staging (with the
+// roughness-0 mip), the maps of the staged planes, the GEMM over every weight
+// matrix, the epilogue of the whole and far rows, that of the near rows.
 
 // partial[f][b]: largest RGB magnitude of block b's share of face f
 __global__ __launch_bounds__(256) void facemax_kernel(Probes Q, size_t level_off, uint32_t S, float* partial) {
@@ -343,1176 +440,474 @@ __global__ __launch_bounds__(256) void facemax_kernel(Probes Q, size_t level_off
     if (threadIdx.x == 0) partial[f * gridDim.x + blockIdx.x] = sh[0];
 }
 
-// sc[f] = 2^-e_f, sc[6+f] = 2^e_f for the padded plane of face f (bounded by
-// face f and its four neighbours); sc[12] = 2^-e, sc[13] = 2^e over all faces.
-__global__ __launch_bounds__(64) void scales_kernel(Probes Q, const float* partial, uint32_t nb, float* sc) {
-    __shared__ float fm[6];
-    const uint32_t t = threadIdx.x;
-    partial = scr(Q, partial, blockIdx.x);
-    sc = scr(Q, sc, blockIdx.x);
-    if (t < 6) {
-        float m = 0.0f;
-        for (uint32_t b = 0; b < nb; ++b) m = fmaxf(m, partial[t * nb + b]);
-        fm[t] = m;
-    }
-    __syncthreads();
-    if (t > 6) return;
-    float m = 0.0f;
-    for (uint32_t g = 0; g < 6; ++g)
-        if (t == 6 || g != (t ^ 1u)) m = fmaxf(m, fm[g]);
+// Power-of-two exponent that brings m under 2^15 (0 for 0 and non-finite m).
+__device__ __forceinline__ int scale_exponent(float m) {
     int e = 0;
     if (m > 0.0f && m <= 3.0e38f) {
         int ex;
         (void)frexpf(m, &ex);
         e = ex - 15;
     }
-    if (t < 6) {
-        sc[t] = ldexpf(1.0f, -e);
-        sc[6 + t] = ldexpf(1.0f, e);
-    } else {
-        sc[12] = ldexpf(1.0f, -e);
-        sc[13] = ldexpf(1.0f, e);
-    }
+    return e;
 }
 
+// A workgroup's exponents from the face maxima (nb <= 32 partials a face):
+// se[f] for the padded plane of face f (bounded by face f and its four
+// neighbours), se[6] over all faces. Each staging workgroup forms them itself:
+// a launch of their own costs more.
+__device__ void block_exponents(const float* __restrict__ partial, uint32_t nb, int* se) {
+    __shared__ float fm[6];
+    const uint32_t t = threadIdx.x, f = t >> 5, b = t & 31;
+    float m = f < 6 && b < nb ? partial[f * nb + b] : 0.0f;
+    for (int d = 16; d > 0; d >>= 1) m = fmaxf(m, __shfl_xor(m, d, 64));
+    if (f < 6 && b == 0) fm[f] = m;
+    __syncthreads();
+    if (t < 7) {
+        float v = 0.0f;
+        for (uint32_t g = 0; g < 6; ++g)
+            if (t == 6 || g != (t ^ 1u)) v = fmaxf(v, fm[g]);
+        se[t] = scale_exponent(v);
+    }
+    __syncthreads();
+}
+
+typedef _Float16 half4v __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x4v __attribute__((ext_vector_type(4)));
+
+enum StageKind { STAGE_DENSE = 0, STAGE_PLANE = 1, STAGE_DELTA = 2 };
 struct StageItem {
-    int kind;  // 0: a dense level (permuted), 1: padded face planes; 3, 2: the same as BF16 hi + lo
+    int kind, split;
     uint32_t S, B, Pw;
-    size_t level_off;  // float4 offset of the level in the input chain
-    const int32_t* perm;
-    half8* dst;
-    uint32_t begin;  // first thread of the item (kind 2: lo parts at dst + the item's thread count)
+    uint32_t n;              // units, plane texels or output texels (one face)
+    uint32_t block_begin;    // first workgroup of the item
+    size_t level_off;        // float4 offset of the level in the input chain (STAGE_DELTA: in the output chain)
+    const uint32_t* list;    // dense: the staged units; planes: the texels needed (index in the Pw x Pw plane)
+    half8* dst;              // dense: R[unit][144][8]
+    uint64_t lo_off;         // split: offset of the lo parts (16-byte units; planes: in the texel's own record)
 };
 struct StageTable {
     StageItem it[kMaxJobs];
-    uint32_t n, total;
+    uint32_t n, blocks;
+    const uint32_t* map;  // source_table
 };
 
-// Writes channel values v[3] of element q of a staged 8-element operand at
-// unit `at` (and the next two units) as FP16, or as BF16 hi + lo with the lo
-// parts `lo_off` units further.
+// Writes the staged operand R[unit][col][8] of a few consecutive units (eight;
+// four split-BF16): column 3 (6 g + f) + c, element q holds channel c of what
+// face f sees as g (texel q of the unit). A wave takes one image (g, f) of all
+// of the units' texels per pass (split: two), so that its loads cover a small
+// patch of one face - consecutive units are stacked in y - and the values go
+// through LDS to be stored unit by unit, each 2304 contiguous bytes. With a
+// thread per (unit, image) instead, loading eight texels of its own, every
+// load touched 64 cache lines: 24 probes 256^2 -> 128^2 x 8 took 220 us to
+// stage and 80 us to map.
+// fetch(unit, q, image): the texel; V::hi(c), V::lo(c) its staged channels.
+constexpr uint32_t kColsPad = kCols + 1;  // LDS units: the eight rows of a pass fall into different banks
+constexpr uint32_t kTileUnits = 8;
 template <bool SPLIT>
-__device__ __forceinline__ void stage_store3(half8* __restrict__ D, size_t at, uint32_t q, const float v[3],
-                                             size_t lo_off) {
+constexpr uint32_t tile_units() { return SPLIT ? kTileUnits / 2 : kTileUnits; }
+template <bool SPLIT, class V, class Fetch>
+__device__ __forceinline__ void stage_tile(half8* sT, uint32_t u0, uint32_t nu, half8* __restrict__ R, uint64_t lo_off,
+                                           Fetch fetch) {
+    constexpr uint32_t UT = tile_units<SPLIT>(), kWide = 64 / (8 * UT), kPasses = kImages / (4 * kWide);
+    const uint32_t t = threadIdx.x, lane = t & 63, q = lane & 7, u = (lane >> 3) % UT, sub = lane / (8 * UT);
+    const uint32_t m = min(UT, nu - u0);
+    const uint32_t image0 = (t >> 6) * kPasses * kWide + sub;
+    V v[kPasses];
 #pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        const size_t e = (at + c) * 8 + q;
-        if constexpr (SPLIT) {
-            const __bf16 hi = (__bf16)v[c];
-            reinterpret_cast<__bf16*>(D)[e] = hi;
-            reinterpret_cast<__bf16*>(D)[lo_off * 8 + e] = (__bf16)(v[c] - (float)hi);
-        } else {
-            reinterpret_cast<_Float16*>(D)[e] = (_Float16)v[c];
+    for (uint32_t k = 0; k < kPasses; ++k) v[k] = fetch(min(u, m - 1), q, image0 + k * kWide);
+#pragma unroll
+    for (uint32_t k = 0; k < kPasses; ++k) {
+        const size_t e = (u * kColsPad + 3 * (image0 + k * kWide)) * 8 + q;
+#pragma unroll
+        for (uint32_t c = 0; c < 3; ++c) {
+            if constexpr (SPLIT) {
+                reinterpret_cast<__bf16*>(sT)[e + 8 * c] = v[k].hi(c);
+                reinterpret_cast<__bf16*>(sT + UT * kColsPad)[e + 8 * c] = v[k].lo(c);
+            } else {
+                reinterpret_cast<_Float16*>(sT)[e + 8 * c] = v[k].hi(c);
+            }
         }
+    }
+    __syncthreads();
+    for (uint32_t e = t; e < m * kCols; e += 256) {
+        const uint32_t at = e / kCols * kColsPad + e % kCols;
+        R[(size_t)u0 * kCols + e] = sT[at];
+        if constexpr (SPLIT) R[lo_off + (size_t)u0 * kCols + e] = sT[UT * kColsPad + at];
     }
 }
 
-// R[k/8][col][8]: col = 4 f + c holds channel c (< 3) of the level texel
-// that output face f sees as canonical input k; other columns are zero (from
-// plan creation). One thread per (k, f); lanes 8 apart share k / 8.
+// Texel of a level, scaled, as the staged formats.
 template <bool SPLIT>
-__device__ __forceinline__ void stage_dense_body(const float4* __restrict__ level, uint32_t Sin,
-                                                 const int32_t* __restrict__ perm, float s, half8* __restrict__ R,
-                                                 uint32_t id) {
-    const uint32_t K = 6 * Sin * Sin;
-    const uint32_t q = id & 7, rest = id >> 3, f = rest % 6, k8 = rest / 6;
-    const float4 t = level[perm[(size_t)f * K + k8 * 8 + q]];
-    const float v[3] = {t.x * s, t.y * s, t.z * s};
-    stage_store3<SPLIT>(R, (size_t)k8 * 32 + 4 * f, q, v, (size_t)K / 8 * 32);
+struct LevelTexel {
+    float4 t;
+    float s;
+    __device__ float at(uint32_t c) const { return (c == 0 ? t.x : c == 1 ? t.y : t.z) * s; }
+    __device__ auto hi(uint32_t c) const {
+        if constexpr (SPLIT) return (__bf16)at(c);
+        else return (_Float16)at(c);
+    }
+    __device__ __bf16 lo(uint32_t c) const { return (__bf16)(at(c) - (float)(__bf16)at(c)); }
+};
+// Texel of a staged plane.
+template <bool SPLIT>
+struct PlaneTexel {
+    std::conditional_t<SPLIT, bf16x8, half4v> t;
+    __device__ auto hi(uint32_t c) const { return t[c]; }
+    __device__ __bf16 lo(uint32_t c) const { return (__bf16)t[4 + c]; }
+};
+
+// A level's units: face f sees canonical texel (x, y) of face t as g k where
+// source_table says.
+template <bool SPLIT>
+__device__ __forceinline__ void stage_dense(const float4* __restrict__ level, const StageItem& I, float s,
+                                            half8* __restrict__ R, uint32_t blk, half8* sT, const uint8_t* sMap) {
+    constexpr uint32_t UT = tile_units<SPLIT>();
+    const uint32_t u0 = blk * UT, m = min(UT, I.n - u0), lane = threadIdx.x & 63, S = I.S;
+    const uint32_t k = I.list[u0 + min((lane >> 3) % UT, m - 1)] * 8 + (lane & 7);
+    const uint32_t S2 = S * S, t = k / S2, rem = k - t * S2, y = rem / S, x = rem - y * S;
+    stage_tile<SPLIT, LevelTexel<SPLIT>>(sT, u0, I.n, R, I.lo_off, [&](uint32_t, uint32_t, uint32_t image) {
+        const uint32_t b = sMap[t * kImages + image];
+        uint32_t i = b & 8u ? y : x, j = b & 8u ? x : y;
+        i = b & 16u ? S - 1 - i : i;
+        j = b & 32u ? S - 1 - j : j;
+        return LevelTexel<SPLIT>{level[((b & 7u) * S + j) * S + i], s};
+    });
 }
 
-// P[py][px/8][col][8] over the padded plane (Pw x Pw, texel index -B .. Si+B)
-// of each face: inside the face the texel itself, outside the bilinear
-// seamless sample of the level at the plane point's direction. One thread
-// per (texel, face); columns 4 f + 3 and 24..31 are zero from plan creation.
+// T[f][py][px]: the scaled texel of face f's plane continued past its edges:
+// inside the face the texel itself, outside the bilinear seamless sample of
+// the level at the plane point's direction; four FP16 values (RGB, 0), or
+// four BF16 hi then four lo. One thread per needed (texel, face).
 template <bool SPLIT>
-__device__ __forceinline__ void stage_pad_body(const float4* __restrict__ level, uint32_t Si, uint32_t B, uint32_t Pw,
-                                               const float* __restrict__ sc, half8* __restrict__ P, uint32_t id) {
-    const uint32_t Pw8 = Pw / 8;
-    const uint32_t q = id & 7, rest = id >> 3, f = rest % 6, cell = rest / 6, px8 = cell % Pw8, py = cell / Pw8;
-    const int x = (int)(px8 * 8 + q) - (int)B, y = (int)py - (int)B;
+__device__ __forceinline__ void stage_plane(const float4* __restrict__ level, const StageItem& I, const int* se,
+                                            half8* __restrict__ dst, uint32_t id) {
+    const uint32_t f = id / I.n, p = I.list[id - f * I.n], py = p / I.Pw, px = p - py * I.Pw;
+    const int x = (int)px - (int)I.B, y = (int)py - (int)I.B;
     f3 t;
-    if (x >= 0 && y >= 0 && x < (int)Si && y < (int)Si) {
-        const float4 v = level[((size_t)f * Si + y) * Si + x];
+    if (x >= 0 && y >= 0 && x < (int)I.S && y < (int)I.S) {
+        const float4 v = level[((size_t)f * I.S + y) * I.S + x];
         t = f3{v.x, v.y, v.z};
     } else {
-        double p[3];
-        hvx::contract_face_point((int)f, hvx::contract_coord(x, Si), hvx::contract_coord(y, Si), p);
-        t = sample_cube(level, (int)Si, normalize3(f3{(float)p[0], (float)p[1], (float)p[2]}));
+        // plane points in doubled texel units: exact in FP32, and the sample
+        // needs no unit direction
+        int q[3];
+        face_ipoint(f, 2 * x + 1 - (int)I.S, 2 * y + 1 - (int)I.S, (int)I.S, q);
+        const f3 d = {(float)q[0], (float)q[1], (float)q[2]};
+        // taps first, so that their loads run together also at the face edges
+        const hvx::CubeTaps c = hvx::cube_taps((int)I.S, d);
+        const float4 w[4] = {level[c.idx[0]], level[c.idx[1]], level[c.idx[2]], level[c.idx[3]]};
+        t = hvx::cube_combine(level, (int)I.S, d, c, w);
     }
-    const float sf = sc[f];
-    const float v[3] = {t.x * sf, t.y * sf, t.z * sf};
-    stage_store3<SPLIT>(P, (size_t)cell * 32 + 4 * f, q, v, (size_t)Pw * Pw8 * 32);
+    const float s = ldexpf(1.0f, -se[f]), v[3] = {t.x * s, t.y * s, t.z * s};
+    const size_t at = (size_t)f * I.Pw * I.Pw + p;
+    if constexpr (SPLIT) {
+        bf16x8 h;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            h[c] = (__bf16)v[c];
+            h[4 + c] = (__bf16)(v[c] - (float)h[c]);
+        }
+        h[3] = h[7] = (__bf16)0.0f;
+        reinterpret_cast<bf16x8*>(dst)[at] = h;
+    } else {
+        reinterpret_cast<half4v*>(dst)[at] = half4v{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)0.0f};
+    }
 }
 
-__global__ __launch_bounds__(256) void stage_all_kernel(Probes Q, StageTable T, const float* sc) {
-    const uint32_t id = blockIdx.x * 256 + threadIdx.x, pr = blockIdx.y;
-    if (id >= T.total) return;
+// sc[f] = 2^e_f of face f's plane, sc[6] = 2^e of the whole levels: what the
+// epilogues multiply by. delta0 (nullable): the chain the roughness-0 mip
+// samples instead of the probe's.
+__global__ __launch_bounds__(256) void stage_kernel(Probes Q, StageTable T, const float* partial, uint32_t nb,
+                                                    float* sc, const float4* delta0, uint32_t S0) {
+    __shared__ half8 sT[kTileUnits * kColsPad];
+    __shared__ uint32_t sMap[6 * kImages / 4];
+    const uint32_t pr = blockIdx.y, blk = blockIdx.x;
     uint32_t j = 0;
-    while (j + 1 < T.n && id >= T.it[j + 1].begin) ++j;
+    while (j + 1 < T.n && blk >= T.it[j + 1].block_begin) ++j;  // uniform over the workgroup
     const StageItem& I = T.it[j];
+    const uint32_t id = (blk - I.block_begin) * 256 + threadIdx.x;
+    if (I.kind == STAGE_DELTA) {
+        // roughness 0: the bilinear seamless sample of level 0 at the texel direction
+        const uint32_t So = I.S, So2 = So * So;
+        if (id >= 6 * So2) return;
+        const uint32_t f = id / So2, o = id - f * So2, Y = o / So, X = o - Y * So;
+        const f3 c = sample_cube(delta0 ? delta0 : probe_chain(Q, pr), (int)S0, texel_dir((int)f, (int)X, (int)Y, (int)So));
+        probe_out(Q, pr)[I.level_off + id] = make_float4(c.x, c.y, c.z, 1.0f);
+        return;
+    }
+    __shared__ int se[7];
+    if (threadIdx.x < 6 * kImages / 4) sMap[threadIdx.x] = T.map[threadIdx.x];
+    block_exponents(scr(Q, partial, pr), nb, se);
+    if (blk == 0 && threadIdx.x < 7) scr(Q, sc, pr)[threadIdx.x] = ldexpf(1.0f, se[threadIdx.x]);
     const float4* level = probe_chain(Q, pr) + I.level_off;
-    sc = scr(Q, sc, pr);
     half8* dst = scr(Q, I.dst, pr);
-    if (I.kind == 0) stage_dense_body<false>(level, I.S, I.perm, sc[12], dst, id - I.begin);
-    else if (I.kind == 3) stage_dense_body<true>(level, I.S, I.perm, sc[12], dst, id - I.begin);
-    else if (I.kind == 1) stage_pad_body<false>(level, I.S, I.B, I.Pw, sc, dst, id - I.begin);
-    else stage_pad_body<true>(level, I.S, I.B, I.Pw, sc, dst, id - I.begin);
-}
-
-// ----------------------------------------------------------- MFMA GEMMs
-struct DenseJob {
-    const half8* W;
-    const half8* R;
-    uint32_t rt, ks, splitk, rows;
-    float* part;            // [splitk][rt * 16][32]
-    const float* rowscale;
-    float4* out;            // plan-owned far map, or nullptr: the output chain at out_off
-    size_t out_off;
-    float alpha;
-    uint32_t wave_begin, epi_begin;
-    uint64_t w_lo, r_lo;  // split BF16 (w_lo != 0): offsets (16-byte units) of the lo parts of W and R
-};
-struct DenseTable {
-    DenseJob j[kMaxJobs];
-    uint32_t n, waves, epi;
-};
-
-// One K step of a wave's RT (1 or 2) row tiles x 32 columns: the weight
-// fragments of the row tiles (x[0..RT-1]; split: hi, then lo in
-// x[RT..2RT-1]) and PG probes' two 16-column B fragments (b[q][0..1]; split:
-// hi, then lo in b[q][2..3]).
-template <bool SPLIT, int PG, int RT = 2>
-struct KStep {
-    using V = std::conditional_t<SPLIT, bf16x8, half8>;
-    static constexpr int kW = SPLIT ? 2 * RT : RT, kB = SPLIT ? 4 : 2;
-    V x[kW];
-    V b[PG][kB];
-};
-
-// acc[q][2 * h + nb] += row tile h x column block nb; split: hi*hi + hi*lo +
-// lo*hi (the lo*lo term is below the FP32 accumulation's resolution)
-template <bool SPLIT, int PG, int RT>
-__device__ __forceinline__ void kstep_mac(f32x4 (&acc)[PG][2 * RT], const KStep<SPLIT, PG, RT>& o) {
-#pragma unroll
-    for (int q = 0; q < PG; ++q) {
-#pragma unroll
-        for (int h = 0; h < RT; ++h)
-#pragma unroll
-            for (int nb = 0; nb < 2; ++nb) {
-                f32x4& a = acc[q][2 * h + nb];
-                a = hvx::mfma16x16x32(o.x[h], o.b[q][nb], a);
-                if constexpr (SPLIT) {
-                    a = hvx::mfma16x16x32(o.x[h], o.b[q][2 + nb], a);
-                    a = hvx::mfma16x16x32(o.x[RT + h], o.b[q][nb], a);
-                }
-            }
+    if (I.kind == STAGE_DENSE) {
+        const float s = ldexpf(1.0f, -se[6]);
+        const uint8_t* map = reinterpret_cast<const uint8_t*>(sMap);
+        if (I.split) stage_dense<true>(level, I, s, dst, blk - I.block_begin, sT, map);
+        else stage_dense<false>(level, I, s, dst, blk - I.block_begin, sT, map);
+    } else {
+        if (id >= I.n * 6) return;
+        if (I.split) stage_plane<true>(level, I, se, dst, id);
+        else stage_plane<false>(level, I, se, dst, id);
     }
 }
 
-// Runs n >= 1 K steps as a software pipeline over groups of U steps: a
-// group's loads are issued before the MFMAs of the group loaded before it.
-// load_next(KStep&) loads the next step and advances a cursor that stops at
-// the last step (the group loaded ahead of the final one repeats it, unused).
-// The accumulation order is that of a plain loop over the steps.
-template <uint32_t U, bool SPLIT, int PG, int RT, class LoadNext>
-__device__ __forceinline__ void kstep_pipeline(f32x4 (&acc)[PG][2 * RT], uint32_t n, LoadNext load_next) {
-    KStep<SPLIT, PG, RT> cur[U];
-#pragma unroll
-    for (uint32_t u = 0; u < U; ++u) load_next(cur[u]);
-    uint32_t s = 0;
-    for (; s + U <= n; s += U) {
-        KStep<SPLIT, PG, RT> nx[U];
-#pragma unroll
-        for (uint32_t u = 0; u < U; ++u) load_next(nx[u]);
-#pragma unroll
-        for (uint32_t u = 0; u < U; ++u) kstep_mac<SPLIT, PG, RT>(acc, cur[u]);
-#pragma unroll
-        for (uint32_t u = 0; u < U; ++u) cur[u] = nx[u];
-    }
-#pragma unroll
-    for (uint32_t u = 0; u < U; ++u)
-        if (s + u < n) kstep_mac<SPLIT, PG, RT>(acc, cur[u]);
-}
+struct MapItem {
+    uint32_t Pw, n, block_begin;
+    const uint32_t* list;  // the staged units
+    const half8* T;        // stage_plane's texels
+    half8* dst;            // R[unit][144][8]
+    uint64_t lo_off;       // 0: FP16
+};
+struct MapTable {
+    MapItem it[kMaxJobs];
+    uint32_t n, blocks;
+};
 
-#ifndef HVX_KSTEP_UNROLL
-#define HVX_KSTEP_UNROLL 8
-#endif
-// FP16 K steps whose loads are in flight together (half as many split-BF16
-// steps, which load twice the fragments): the near field's largest mip runs
-// about two waves per SIMD, too few to stream the weights otherwise
-constexpr uint32_t kStepUnroll = HVX_KSTEP_UNROLL;
+// The staged operand of the padded planes: texel (px, py) of the plane maps to
+// g (px, py) of face f's plane.
 template <bool SPLIT>
-constexpr uint32_t kstep_unroll() { return SPLIT ? (kStepUnroll + 1) / 2 : kStepUnroll; }
-// The single-probe near GEMM's own depths (FP16, split BF16). Its waves
-// (one row tile each) outnumber what the chip holds, so it gains more from
-// loads in flight per wave than from waves per SIMD. Whole FP16 call on the
-// 512^2 GGX chain: 4 steps (6 waves per SIMD) 0.605 ms, 8 (4 waves) 0.58,
-// 10 0.552, 12 (3 waves) 0.536 - 0.546, 14 0.541, 16 (2 waves) 0.549, 20
-// spills; split BF16: 4 steps 0.943 - 0.999, 5 0.913 - 0.927, 6 0.93, 8 0.908.
-#ifndef HVX_NEAR_UNROLL
-#define HVX_NEAR_UNROLL 12
-#endif
-#ifndef HVX_NEAR_UNROLL_SPLIT
-#define HVX_NEAR_UNROLL_SPLIT 5
-#endif
-template <bool SPLIT>
-constexpr uint32_t near_unroll() { return SPLIT ? HVX_NEAR_UNROLL_SPLIT : HVX_NEAR_UNROLL; }
-
-// Dense: a wave owns two row tiles (32 rows) x 32 columns over one K slice;
-// partial sums go to part[slice][row][32] and are reduced in slice order.
-// PG probes per wave (grid dimension: probe group): each weight fragment is
-// loaded once and multiplied into every probe of the group; each probe's
-// accumulation is the same sequence as with PG = 1.
-// Wave w of a job: four consecutive waves take four row-tile pairs of one K
-// slice (a job's pairs are padded to a multiple of four), so a workgroup's
-// waves share the slice's B operand.
-__device__ __forceinline__ void dense_wave(const DenseJob& J, uint32_t w, uint32_t& pair, uint32_t& slice) {
-    const uint32_t per = 4 * J.splitk, grp = w / per, r = w - grp * per;
-    slice = r / 4;
-    pair = grp * 4 + (r & 3);
+__device__ __forceinline__ void map_plane(const MapItem& I, const half8* T, half8* R, uint32_t blk, half8* sT) {
+    constexpr uint32_t UT = tile_units<SPLIT>();
+    using V = PlaneTexel<SPLIT>;
+    const V* P = reinterpret_cast<const V*>(T);
+    const uint32_t u0 = blk * UT, m = min(UT, I.n - u0), lane = threadIdx.x & 63, Pw = I.Pw;
+    const uint32_t unit = I.list[u0 + min((lane >> 3) % UT, m - 1)], py = unit / (Pw / 8);
+    const uint32_t px = (unit - py * (Pw / 8)) * 8 + (lane & 7);
+    stage_tile<SPLIT, V>(sT, u0, I.n, R, I.lo_off, [&](uint32_t, uint32_t, uint32_t image) {
+        const uint32_t g = image / 6, f = image - 6 * g;
+        uint32_t x = px, y = py;
+        image_of(g, Pw, x, y);
+        return P[(f * Pw + y) * Pw + x];
+    });
 }
 
-template <int PG>
-__global__ __launch_bounds__(256) void dense_gemm_kernel(Probes Q, DenseTable T) {
-    const uint2 wb = gemm_block(Q);
-    const uint32_t gw = wb.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63, p0 = wb.y * PG;
-    if (gw >= T.waves) return;  // uniform per wave; the kernel has no barriers
-    const uint32_t np = min((uint32_t)PG, Q.n - p0);
-    uint32_t jj = 0;
-    while (jj + 1 < T.n && gw >= T.j[jj + 1].wave_begin) ++jj;
-    const DenseJob& J = T.j[jj];
-    const uint32_t rt = J.rt, ks = J.ks, splitk = J.splitk;
-    uint32_t pair, slice;
-    dense_wave(J, gw - J.wave_begin, pair, slice);
-    const uint32_t rt0 = 2 * pair;
-    if (rt0 >= rt) return;  // padding wave (uniform per wave)
-    const bool has1 = rt0 + 1 < rt;
-    const uint32_t kb = (uint32_t)((uint64_t)slice * ks / splitk), ke = (uint32_t)((uint64_t)(slice + 1) * ks / splitk);
-    const uint32_t i = lane & 15, g = lane >> 4;
-    const half8* w0 = J.W + (size_t)rt0 * ks * 64 + lane;
-    const half8* w1 = has1 ? w0 + (size_t)ks * 64 : w0;
-    const half8* rb[PG];
-#pragma unroll
-    for (int q = 0; q < PG; ++q) rb[q] = scr(Q, J.R, p0 + ((uint32_t)q < np ? q : 0)) + g * 32 + i;
-    f32x4 acc[PG][4];
-#pragma unroll
-    for (int q = 0; q < PG; ++q)
-#pragma unroll
-        for (int k = 0; k < 4; ++k) acc[q][k] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    // steps [kb, ke) of the slice; an empty slice (ke == kb) loads step kb,
-    // which exists (kb < ks), and accumulates nothing
-    auto run = [&](auto split_tag) {
-        constexpr bool SPLIT = decltype(split_tag)::value;
-        using Op = KStep<SPLIT, PG>;
-        using V = typename Op::V;
-        using GV = const __attribute__((address_space(1))) V*;
-        const GV v0 = (GV)reinterpret_cast<const V*>(w0), v1 = (GV)reinterpret_cast<const V*>(w1);
-        GV rv[PG];
-#pragma unroll
-        for (int q = 0; q < PG; ++q) rv[q] = (GV)reinterpret_cast<const V*>(rb[q]);
-        uint32_t ls = kb;
-        kstep_pipeline<kstep_unroll<SPLIT>(), SPLIT, PG, 2>(acc, ke - kb, [&](Op& o) {
-            const size_t wo = (size_t)ls * 64, qo = (size_t)ls * 128;
-            o.x[0] = v0[wo];
-            o.x[1] = v1[wo];
-            if constexpr (SPLIT) {
-                o.x[2] = v0[wo + J.w_lo];
-                o.x[3] = v1[wo + J.w_lo];
-            }
-#pragma unroll
-            for (int q = 0; q < PG; ++q) {
-                o.b[q][0] = rv[q][qo];
-                o.b[q][1] = rv[q][qo + 16];
-                if constexpr (SPLIT) {
-                    o.b[q][2] = rv[q][qo + J.r_lo];
-                    o.b[q][3] = rv[q][qo + 16 + J.r_lo];
-                }
-            }
-            ls += ls + 1 < ke ? 1u : 0u;
-        });
-    };
-    if (J.w_lo)  // split BF16
-        run(std::true_type{});
-    else
-        run(std::false_type{});
-#pragma unroll
-    for (int q = 0; q < PG; ++q) {
-        if ((uint32_t)q >= np) break;
-        float* p = scr(Q, J.part, p0 + q) + (size_t)slice * rt * 16 * 32;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const uint32_t row0 = rt0 * 16 + 4 * g + r;
-            p[(size_t)row0 * 32 + i] = acc[q][0][r];
-            p[(size_t)row0 * 32 + 16 + i] = acc[q][1][r];
-            if (has1) {
-                p[(size_t)(row0 + 16) * 32 + i] = acc[q][2][r];
-                p[(size_t)(row0 + 16) * 32 + 16 + i] = acc[q][3][r];
-            }
-        }
-    }
+__global__ __launch_bounds__(256) void plane_map_kernel(Probes Q, MapTable M) {
+    __shared__ half8 sT[kTileUnits * kColsPad];
+    const uint32_t pr = blockIdx.y;
+    uint32_t j = 0;
+    while (j + 1 < M.n && blockIdx.x >= M.it[j + 1].block_begin) ++j;  // uniform over the workgroup
+    const MapItem& I = M.it[j];
+    const half8* T = scr(Q, I.T, pr);
+    half8* R = scr(Q, I.dst, pr);
+    if (I.lo_off) map_plane<true>(I, T, R, blockIdx.x - I.block_begin, sT);
+    else map_plane<false>(I, T, R, blockIdx.x - I.block_begin, sT);
 }
 
-// The grouped dense GEMM with each K step's B operand (PG probes' 4 x 32
-// half8, plus the lo parts when split) staged once per workgroup in LDS,
-// double buffered, as near_gemm_staged_kernel does: the workgroup's four
-// waves share the K slice. Padding waves stage and synchronise but compute
-// nothing.
-template <int PG>
-__global__ __launch_bounds__(256) void dense_gemm_staged_kernel(Probes Q, DenseTable T) {
-    const uint2 wb = gemm_block(Q);
-    const uint32_t gw0 = wb.x * 4;
-    if (gw0 >= T.waves) return;  // uniform per workgroup: jobs hold multiples of four waves
-    const uint32_t t = threadIdx.x, gw = gw0 + (t >> 6), lane = t & 63, p0 = wb.y * PG;
-    const uint32_t np = min((uint32_t)PG, Q.n - p0);
-    uint32_t jj = 0;
-    while (jj + 1 < T.n && gw0 >= T.j[jj + 1].wave_begin) ++jj;
-    const DenseJob& J = T.j[jj];
-    const uint32_t rt = J.rt, ks = J.ks, splitk = J.splitk;
-    uint32_t pair, slice;
-    dense_wave(J, gw - J.wave_begin, pair, slice);
-    const uint32_t rt0 = 2 * pair;
-    const bool active = rt0 < rt, has1 = rt0 + 1 < rt;
-    const uint32_t kb = (uint32_t)((uint64_t)slice * ks / splitk), ke = (uint32_t)((uint64_t)(slice + 1) * ks / splitk);
-    const uint32_t i = lane & 15, g = lane >> 4;
-    const half8* w0 = J.W + (active ? (size_t)rt0 * ks * 64 + lane : 0);
-    const half8* w1 = has1 ? w0 + (size_t)ks * 64 : w0;
-    const half8* Rp[PG];
-#pragma unroll
-    for (int q = 0; q < PG; ++q) Rp[q] = scr(Q, J.R, p0 + ((uint32_t)q < np ? q : 0));
-    constexpr uint32_t kMaxB = PG * 128 * 2;  // half8 per step, split
-    __shared__ half8 sB[2][kMaxB];
-    // the B operand is read through global (not generic) pointers: generic
-    // loads count against the LDS counter too, so each step's LDS reads
-    // would wait for the next step's B loads
-    using GH = const __attribute__((address_space(1))) half8*;
-    GH Rg[PG];
-#pragma unroll
-    for (int q = 0; q < PG; ++q) Rg[q] = (GH)Rp[q];
-    f32x4 acc[PG][4];
-#pragma unroll
-    for (int q = 0; q < PG; ++q)
-#pragma unroll
-        for (int k = 0; k < 4; ++k) acc[q][k] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    // the job's precision is uniform per workgroup; each variant has its own
-    // loop so that its loads are unconditional (conditional loads make the
-    // waits conservative)
-    auto run = [&](auto split_tag) {
-        constexpr bool SPLIT = decltype(split_tag)::value;
-        constexpr uint32_t nB = PG * 128 * (SPLIT ? 2u : 1u), kPer = (nB + 255) / 256;
-        // element e = t + 256 k of a step's block: lo part e / (PG * 128),
-        // probe (e / 128) % PG, unit e % 128; with whole 256-element passes
-        // and an even PG the part is the same for the whole pass
-        constexpr bool kWhole = nB % 256 == 0 && (PG * 128) % 256 == 0;
-        auto b_load = [&](uint32_t s, half8 (&v)[kPer]) {
-#pragma unroll
-            for (uint32_t k = 0; k < kPer; ++k) {
-                const uint32_t e = t + 256u * k, q = (e / 128) % PG, o = e % 128;
-                if constexpr (kWhole) {
-                    const uint32_t lo = (256u * k) / (PG * 128);
-                    v[k] = Rg[q][(size_t)s * 128 + o + (lo ? J.r_lo : 0)];
-                } else {
-                    const uint32_t lo = e / (PG * 128);
-                    if (e < nB) v[k] = Rg[q][(size_t)s * 128 + o + (lo ? J.r_lo : 0)];
-                }
-            }
-        };
-        auto b_store = [&](uint32_t buf, const half8 (&v)[kPer]) {
-#pragma unroll
-            for (uint32_t k = 0; k < kPer; ++k)
-                if (kWhole || t + 256u * k < nB) sB[buf][t + 256u * k] = v[k];
-        };
-        half8 nx[kPer];
-        if (kb < ke) {
-            b_load(kb, nx);
-            b_store(0, nx);
-        }
-        __syncthreads();
-        for (uint32_t s = kb; s < ke; ++s) {
-            const bool more = s + 1 < ke;
-            // this step's weights are loaded (every wave; an inactive wave's
-            // pointers are the job's first row) before the next step's B
-            // operand: the load counter completes in order, so the MFMAs'
-            // wait for the weights leaves the B loads in flight
-            const size_t o = (size_t)s * 64;
-            half8 xw[SPLIT ? 4 : 2];
-            xw[0] = w0[o];
-            xw[1] = w1[o];
-            if constexpr (SPLIT) {
-                xw[2] = w0[o + J.w_lo];
-                xw[3] = w1[o + J.w_lo];
-            }
-            b_load(more ? s + 1 : s, nx);       // the last step reloads itself
-            __asm__ volatile("" ::: "memory");  // keeps the B loads ahead of the MFMAs
-            const half8* sb = sB[(s - kb) & 1];
-            if (active) {
-                if constexpr (SPLIT) {
-                    const bf16x8 x0 = __builtin_bit_cast(bf16x8, xw[0]), x1 = __builtin_bit_cast(bf16x8, xw[1]);
-                    const bf16x8 y0 = __builtin_bit_cast(bf16x8, xw[2]), y1 = __builtin_bit_cast(bf16x8, xw[3]);
-#pragma unroll
-                    for (int q = 0; q < PG; ++q) {
-                        const bf16x8* rv = reinterpret_cast<const bf16x8*>(sb + q * 128 + g * 32 + i);
-                        const bf16x8 b0 = rv[0], b1 = rv[16], c0 = rv[PG * 128], c1 = rv[PG * 128 + 16];
-                        acc[q][0] = hvx::mfma16x16x32(x0, b0, acc[q][0]);
-                        acc[q][0] = hvx::mfma16x16x32(x0, c0, acc[q][0]);
-                        acc[q][0] = hvx::mfma16x16x32(y0, b0, acc[q][0]);
-                        acc[q][1] = hvx::mfma16x16x32(x0, b1, acc[q][1]);
-                        acc[q][1] = hvx::mfma16x16x32(x0, c1, acc[q][1]);
-                        acc[q][1] = hvx::mfma16x16x32(y0, b1, acc[q][1]);
-                        acc[q][2] = hvx::mfma16x16x32(x1, b0, acc[q][2]);
-                        acc[q][2] = hvx::mfma16x16x32(x1, c0, acc[q][2]);
-                        acc[q][2] = hvx::mfma16x16x32(y1, b0, acc[q][2]);
-                        acc[q][3] = hvx::mfma16x16x32(x1, b1, acc[q][3]);
-                        acc[q][3] = hvx::mfma16x16x32(x1, c1, acc[q][3]);
-                        acc[q][3] = hvx::mfma16x16x32(y1, b1, acc[q][3]);
-                    }
-                } else {
-                    const half8 x0 = xw[0], x1 = xw[1];
-#pragma unroll
-                    for (int q = 0; q < PG; ++q) {
-                        const half8* rv = sb + q * 128 + g * 32 + i;
-                        const half8 b0 = rv[0], b1 = rv[16];
-                        acc[q][0] = hvx::mfma16x16x32(x0, b0, acc[q][0]);
-                        acc[q][1] = hvx::mfma16x16x32(x0, b1, acc[q][1]);
-                        acc[q][2] = hvx::mfma16x16x32(x1, b0, acc[q][2]);
-                        acc[q][3] = hvx::mfma16x16x32(x1, b1, acc[q][3]);
-                    }
-                }
-            }
-            // stored unconditionally: after the last step the buffer is no
-            // longer read (its readers passed the previous barrier), and a
-            // store under a branch would draw the B loads into the branch,
-            // after the MFMAs
-            b_store((s + 1 - kb) & 1, nx);
-            __syncthreads();
-        }
-    };
-    if (J.w_lo != 0)  // split BF16
-        run(std::true_type{});
-    else
-        run(std::false_type{});
-    if (!active) return;
-#pragma unroll
-    for (int q = 0; q < PG; ++q) {
-        if ((uint32_t)q >= np) break;
-        float* p = scr(Q, J.part, p0 + q) + (size_t)slice * rt * 16 * 32;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const uint32_t row0 = rt0 * 16 + 4 * g + r;
-            p[(size_t)row0 * 32 + i] = acc[q][0][r];
-            p[(size_t)row0 * 32 + 16 + i] = acc[q][1][r];
-            if (has1) {
-                p[(size_t)(row0 + 16) * 32 + i] = acc[q][2][r];
-                p[(size_t)(row0 + 16) * 32 + 16 + i] = acc[q][3][r];
-            }
-        }
-    }
-}
-
-// The dense GEMM with the K slice's B blocks staged in LDS: the four waves
-// of a workgroup (four row-tile pairs of one K slice) share each step's B
-// block (128 half8 per probe, twice that split), loaded once per workgroup,
-// GS steps at a time (GS / 2 split), double buffered, one barrier per group;
-// weights a group ahead. PG probes per wave (grouped multi-probe calls):
-// each weight fragment is loaded once for the group. Each output's
-// accumulation is the same sequence of MFMAs as in dense_gemm_kernel, so the
-// partial sums are identical. Single probe: its B block is a third of a
-// step's loads, not two thirds as in the near field, so the gain is small:
-// whole FP16 call on the 512^2 GGX chain 0.469 ms with dense_gemm_kernel,
-// GS = 4: 0.466, 8: 0.461 (split BF16 0.767, 0.758, 0.759). Four probes per
-// wave (54 probes 512^2 -> 256^2 x 9, FP16 / split): dense_gemm_staged_kernel
-// (a barrier per step) 4.36 / 6.16 ms; GS = 2: 3.96 / 6.00; 4: 4.56 / 6.50
-// (one wave per SIMD).
-#ifndef HVX_DENSE_LDS_GROUP
-#define HVX_DENSE_LDS_GROUP 8
-#endif
-#ifndef HVX_DENSE_LDS_GROUP_MULTI
-#define HVX_DENSE_LDS_GROUP_MULTI 2
-#endif
-// non-temporal weight loads in the dense GEMM: no gain for one probe (0.451
-// -> 0.449 ms), and a loss when probe groups share each weight block through
-// the caches (54 probes 512^2: 3.98 -> 4.27 ms)
-#ifndef HVX_DENSE_NT
-#define HVX_DENSE_NT 0
-#endif
-constexpr int kDenseLdsGroup = HVX_DENSE_LDS_GROUP;             // 0: dense_gemm_kernel
-constexpr int kDenseLdsGroupMulti = HVX_DENSE_LDS_GROUP_MULTI;  // 0: dense_gemm_staged_kernel
-template <int PG, int GS>
-__global__ __launch_bounds__(256) void dense_gemm_lds_kernel(Probes Q, DenseTable T) {
-    static_assert(GS % 4 == 0 || (GS % 2 == 0 && PG % 2 == 0), "whole B passes per group, split groups of GS / 2");
-    const uint2 wb = gemm_block(Q);
-    const uint32_t gw0 = wb.x * 4;
-    if (gw0 >= T.waves) return;  // whole workgroups (T.waves is a multiple of 4)
-    const uint32_t t = threadIdx.x, gw = gw0 + (t >> 6), lane = t & 63, p0 = wb.y * PG;
-    const uint32_t np = min((uint32_t)PG, Q.n - p0);
-    uint32_t jj = 0;
-    while (jj + 1 < T.n && gw0 >= T.j[jj + 1].wave_begin) ++jj;  // wave_begin: multiples of 4
-    const DenseJob& J = T.j[jj];
-    const uint32_t rt = J.rt, ks = J.ks, splitk = J.splitk;
-    uint32_t pair, slice;
-    dense_wave(J, gw - J.wave_begin, pair, slice);  // slice: the same for the workgroup's waves
-    const uint32_t rt0 = 2 * pair;
-    const bool live = rt0 < rt;  // padding waves load and wait with the others
-    const bool has1 = rt0 + 1 < rt;
-    const uint32_t kb = (uint32_t)((uint64_t)slice * ks / splitk), ke = (uint32_t)((uint64_t)(slice + 1) * ks / splitk);
-    const uint32_t i = lane & 15, g = lane >> 4;
-    using GH = const __attribute__((address_space(1))) half8*;
-    const GH w0 = (GH)(J.W + (size_t)(live ? rt0 : 0) * ks * 64 + lane);
-    const GH w1 = has1 ? w0 + (size_t)ks * 64 : w0;
-    __shared__ half8 sB[2][GS * PG * 128];  // a group's B blocks: [step][probe][unit (hi, then lo split)]
-    f32x4 acc[PG][4];
-#pragma unroll
-    for (int q = 0; q < PG; ++q)
-#pragma unroll
-        for (int k = 0; k < 4; ++k) acc[q][k] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    auto run = [&](auto split_tag) {
-        constexpr bool SPLIT = decltype(split_tag)::value;
-        constexpr uint32_t G = SPLIT ? GS / 2 : GS;  // steps per group
-        constexpr uint32_t kBw = SPLIT ? 256 : 128;  // half8 per probe and step
-        constexpr int kWs = SPLIT ? 4 : 2;            // weight fragments per step
-        constexpr int kPer = G * PG * kBw / 256;
-        static_assert(G * PG * kBw % 256 == 0, "whole 256-lane passes");
-        const size_t r_lo = J.r_lo, w_lo = J.w_lo;
-        const uint32_t n = ke - kb, groups = (n + G - 1) / G;
-        if (groups == 0) return;  // uniform over the workgroup
-        auto step_of = [&](uint32_t s) { return kb + (s < n ? s : n - 1); };  // steps past the last repeat it
-        auto b_load = [&](uint32_t s0, half8 (&v)[kPer]) {
-#pragma unroll
-            for (int k = 0; k < kPer; ++k) {
-                const uint32_t e = t + 256u * k, st = e / (PG * kBw), rem = e % (PG * kBw), q = rem / kBw,
-                               o = rem % kBw;
-                const GH rq = (GH)scr(Q, J.R, p0 + (q < np ? q : 0));
-                v[k] = rq[(size_t)step_of(s0 + st) * 128 + o % 128 + (o >= 128 ? r_lo : 0)];
-            }
-        };
-        auto b_store = [&](uint32_t buf, const half8 (&v)[kPer]) {
-#pragma unroll
-            for (int k = 0; k < kPer; ++k) sB[buf][t + 256u * k] = v[k];
-        };
-        auto w_load = [&](uint32_t s0, half8 (&x)[G][kWs]) {
-#pragma unroll
-            for (uint32_t k = 0; k < G; ++k) {
-                const size_t o = (size_t)step_of(s0 + k) * 64;
-#if HVX_DENSE_NT
-                x[k][0] = __builtin_nontemporal_load(&w0[o]);
-                x[k][1] = __builtin_nontemporal_load(&w1[o]);
-                if constexpr (SPLIT) {
-                    x[k][2] = __builtin_nontemporal_load(&w0[o + w_lo]);
-                    x[k][3] = __builtin_nontemporal_load(&w1[o + w_lo]);
-                }
-#else
-                x[k][0] = w0[o];
-                x[k][1] = w1[o];
-                if constexpr (SPLIT) {
-                    x[k][2] = w0[o + w_lo];
-                    x[k][3] = w1[o + w_lo];
-                }
-#endif
-            }
-        };
-        half8 nb[kPer], xw[G][kWs], xn[G][kWs];
-        b_load(0, nb);
-        w_load(0, xw);
-        b_store(0, nb);
-        __syncthreads();
-        for (uint32_t gi = 0; gi < groups; ++gi) {
-            const uint32_t s0 = gi * G, sn = gi + 1 < groups ? s0 + G : s0;
-            w_load(sn, xn);
-            b_load(sn, nb);
-            __asm__ volatile("" ::: "memory");
-            const half8* sb = sB[gi & 1];
-#pragma unroll
-            for (uint32_t k = 0; k < G; ++k) {
-                if (live && s0 + k < n) {
-#pragma unroll
-                    for (int q = 0; q < PG; ++q) {
-                        const half8* bk = sb + (k * PG + q) * kBw + g * 32 + i;
-#pragma unroll
-                        for (int h = 0; h < 2; ++h)
-#pragma unroll
-                            for (int nbk = 0; nbk < 2; ++nbk) {
-                                f32x4& a = acc[q][2 * h + nbk];
-                                if constexpr (SPLIT) {
-                                    const bf16x8 x = __builtin_bit_cast(bf16x8, xw[k][h]);
-                                    const bf16x8 y = __builtin_bit_cast(bf16x8, xw[k][2 + h]);
-                                    const bf16x8 b = __builtin_bit_cast(bf16x8, bk[16 * nbk]);
-                                    const bf16x8 c = __builtin_bit_cast(bf16x8, bk[128 + 16 * nbk]);
-                                    a = hvx::mfma16x16x32(x, b, a);
-                                    a = hvx::mfma16x16x32(x, c, a);
-                                    a = hvx::mfma16x16x32(y, b, a);
-                                } else {
-                                    a = hvx::mfma16x16x32(xw[k][h], bk[16 * nbk], a);
-                                }
-                            }
-                    }
-                }
-            }
-            b_store((gi & 1) ^ 1, nb);
-#pragma unroll
-            for (uint32_t k = 0; k < G; ++k)
-#pragma unroll
-                for (int u = 0; u < kWs; ++u) xw[k][u] = xn[k][u];
-            __syncthreads();
-        }
-    };
-    if (J.w_lo)  // split BF16 (uniform over the workgroup: one job per workgroup)
-        run(std::true_type{});
-    else
-        run(std::false_type{});
-    if (!live) return;
-#pragma unroll
-    for (int q = 0; q < PG; ++q) {
-        if ((uint32_t)q >= np) break;
-        float* p = scr(Q, J.part, p0 + q) + (size_t)slice * rt * 16 * 32;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const uint32_t row0 = rt0 * 16 + 4 * g + r;
-            p[(size_t)row0 * 32 + i] = acc[q][0][r];
-            p[(size_t)row0 * 32 + 16 + i] = acc[q][1][r];
-            if (has1) {
-                p[(size_t)(row0 + 16) * 32 + i] = acc[q][2][r];
-                p[(size_t)(row0 + 16) * 32 + 16 + i] = acc[q][3][r];
-            }
-        }
-    }
-}
-
-// out[f][row] = (sum over slices) * rowscale[row] * 2^e  (alpha 1 in the
-// chain, 0 in a far map)
-__global__ __launch_bounds__(256) void dense_epilogue_kernel(Probes Q, DenseTable T, const float* sc) {
-    const uint32_t id = blockIdx.x * 256 + threadIdx.x, pr = blockIdx.y;
-    if (id >= T.epi) return;
-    sc = scr(Q, sc, pr);
-    uint32_t jj = 0;
-    while (jj + 1 < T.n && id >= T.j[jj + 1].epi_begin) ++jj;
-    const DenseJob& J = T.j[jj];
-    const uint32_t local = id - J.epi_begin, rows = J.rows, f = local / rows, row = local - f * rows;
-    const uint32_t rows_pad = J.rt * 16;
-    float v[3] = {0.0f, 0.0f, 0.0f};
-    for (uint32_t s = 0; s < J.splitk; ++s) {
-        const float* p = scr(Q, J.part, pr) + ((size_t)s * rows_pad + row) * 32 + f * 4;
-        v[0] += p[0];
-        v[1] += p[1];
-        v[2] += p[2];
-    }
-    const float k = J.rowscale[row] * sc[13];
-    float4* out = J.out ? scr(Q, J.out, pr) : probe_out(Q, pr) + J.out_off;
-    out[(size_t)f * rows + row] = make_float4(v[0] * k, v[1] * k, v[2] * k, J.alpha);
-}
-
-struct NearJob {
+// ------------------------------------------------------------- MFMA GEMM
+struct GemmArgs {
     const half8* W;
-    const NearTile* tiles;
-    const half8* P;
-    uint32_t Pw8, B, te, So, Sf;
-    const float* rowscale;
-    const float* invZ;
-    const float4* far;
-    size_t out_off;  // float4 offset of the mip in the output chain
-    uint32_t tile_begin, texel_begin;
-    uint64_t w_lo, p_lo;  // split BF16: offsets (16-byte units) of the lo parts of W and P
+    const Block* blocks;
+    const Item* items;
+    const uint32_t* ulist;
+    float* part;  // [slot][kBlockRows][kCols]
+    uint32_t nitems;
+    const half8* R[kMaxJobs];
+    uint64_t r_lo[kMaxJobs];
 };
-struct NearTable {
-    NearJob j[kMaxJobs];
-    uint32_t n, tiles, texels;
-};
-
-// the tables travel as kernel arguments (at most 4 KB)
-static_assert(sizeof(StageTable) < 4000 && sizeof(DenseTable) < 4000 && sizeof(NearTable) < 4000,
+static_assert(sizeof(StageTable) < 4000 && sizeof(MapTable) < 4000 && sizeof(GemmArgs) < 4000,
               "launch tables must fit the kernel argument space");
 
-// Near field: one workgroup per 16 x 16 output tile, eight waves of two
-// output rows each; B rows come from the face planes' window. SPLIT:
-// weights and radiance are BF16 hi + lo pairs and each product is
-// hi*hi + hi*lo + lo*hi (the lo*lo term is below the FP32 accumulation's
-// resolution), three MFMAs per FP16 one.
-constexpr uint32_t kNearWaves = 8;  // waves per 16x16 output tile (two row tiles each)
-constexpr uint32_t kNearParts = 2;  // workgroups per tile (fixed by the 256-lane LDS staging below)
-static_assert(kNearWaves % kNearParts == 0, "a tile splits into whole waves");
-static_assert(64 * kNearWaves / kNearParts == 256, "the near GEMM's LDS staging assumes 256-lane workgroups");
-#ifndef HVX_NEAR_ROWS
-#define HVX_NEAR_ROWS 1
-#endif
-// The single-probe near GEMM: row tiles per wave (a tile's 16 row tiles take
-// 16 / kNearRows waves, in 256-lane workgroups). One row tile per wave
-// doubles the waves that stream the weights but loads each B fragment twice
-// as often (from L2); four row tiles per wave halve the B loads and the
-// waves. Measured on the 512^2 GGX chain, whole FP16 call: one 0.595 ms, two
-// 0.625 ms (the smaller work units balance mip 2, whose corner tiles have
-// windows 3.4x the mean). Each output's accumulation order is the same for all.
-constexpr uint32_t kNearRows = HVX_NEAR_ROWS;
-constexpr uint32_t kNearSingleParts = 16 / kNearRows / 4;
-static_assert(kNearRows == 1 || kNearRows == 2 || kNearRows == 4, "1, 2 or 4 row tiles per wave");
-// XCD-aware order of the single-probe near GEMM: workgroups are dealt to the
-// 8 XCDs round-robin, so consecutive workgroups (the parts of one tile)
-// would each fetch the tile's radiance window into a different L2. Instead
-// hardware workgroup b (XCD b % 8, its k = b / 8-th workgroup there) takes
-// part k % P of tile ((k / (P G)) * 8 + b % 8) * G + (k % (P G)) / P: all
-// parts of a tile, and runs of G neighbouring tiles, share one XCD, and the
-// tiles still start in the order of the table (largest windows first).
-// Measured on the 512^2 GGX chain (whole call, FP16 / split BF16): hardware
-// order 0.597 / 0.998 ms; G = 1: 0.585 / 0.974; 4: 0.581 / 0.932; 8: 0.590 /
-// 0.965; 16: 0.625 / 1.151 (too few XCD turns to balance the mips).
-#ifndef HVX_NEAR_XCD_GROUP
-#define HVX_NEAR_XCD_GROUP 4
-#endif
-constexpr uint32_t kNearXcdGroup = HVX_NEAR_XCD_GROUP;  // 0: hardware order
-constexpr uint32_t kXcdCount = 8;
-// workgroups of the single-probe near GEMM over `tiles` tiles (padding
-// workgroups of the XCD-aware order return at once)
-__host__ __device__ constexpr uint32_t near_single_wgs(uint32_t tiles) {
-    return kNearXcdGroup ? (tiles + kXcdCount * kNearXcdGroup - 1) / (kXcdCount * kNearXcdGroup) * kXcdCount *
-                               kNearXcdGroup * kNearSingleParts
-                         : tiles * kNearSingleParts;
-}
-// logical workgroup (tile * P + part) of hardware workgroup b
-__device__ __forceinline__ uint32_t near_single_block(uint32_t b) {
-    if constexpr (kNearXcdGroup == 0) return b;
-    constexpr uint32_t P = kNearSingleParts, PG = P * kNearXcdGroup;
-    const uint32_t x = b % kXcdCount, k = b / kXcdCount;
-    const uint32_t tile = ((k / PG) * kXcdCount + x) * kNearXcdGroup + (k % PG) / P;
-    return tile * P + k % P;
-}
+constexpr uint32_t kGroup = 4;        // K steps staged per barrier (half as many split-BF16 ones)
+constexpr uint32_t kMinSlice = 8;     // and at least
+constexpr uint32_t kGoodSlice = 32;   // and at least in plans that fill the chip
+constexpr uint32_t kMaxSlice = 64;    // K steps of an item, at most
+constexpr uint32_t kXcds = 8;
+constexpr uint32_t kNt = kCols / 16;  // MFMA column tiles
 
-template <bool SPLIT, int PG>
-__global__ __launch_bounds__(512) void near_gemm_kernel(Probes Q, NearTable T, const float* sc) {
-    const uint2 wb = gemm_block(Q);
-    const uint32_t p0 = wb.y * PG, np = min((uint32_t)PG, Q.n - p0);
-    uint32_t jj = 0;
-    // logical workgroup lb owns part lb % kNearSingleParts (four waves' row
-    // tiles) of tile lb / kNearSingleParts: finer work units than whole tiles
-    // balance the unequal mips across the CUs
-    const uint32_t lb = near_single_block(wb.x);
-    const uint32_t gt = lb / kNearSingleParts;
-    if (gt >= T.tiles) return;  // padding of the XCD-aware order (uniform; no barriers below)
-    while (jj + 1 < T.n && gt >= T.j[jj + 1].tile_begin) ++jj;
-    const NearJob& J = T.j[jj];
-    const uint32_t tile = gt - J.tile_begin, lane = threadIdx.x & 63;
-    const uint32_t wave = (threadIdx.x >> 6) + (lb % kNearSingleParts) * 4;
-    const NearTile Tl = J.tiles[tile];
-    // PG probes per wave: each weight fragment is loaded once for the group;
-    // each probe's accumulation is the same sequence as with PG = 1
-    const half8* Pp[PG];
-#pragma unroll
-    for (int q = 0; q < PG; ++q) Pp[q] = scr(Q, J.P, p0 + ((uint32_t)q < np ? q : 0));
-    const uint32_t wc = Tl.w / 32, KS = Tl.h * wc;
-    const uint32_t i = lane & 15, g = lane >> 4, rt0 = kNearRows * wave;
-    // weights of a tile stored K-step major: step s of all 16 row tiles is one
-    // contiguous 16 KB block
-    constexpr size_t kStep = 16 * 64, kRow = 64;
-    const half8* w0 = J.W + Tl.woff + (size_t)rt0 * kRow + lane;
-    const uint32_t xb = (uint32_t)(Tl.x0 + (int)J.B) / 8 + g;
-    f32x4 acc[PG][2 * kNearRows];
-#pragma unroll
-    for (int q = 0; q < PG; ++q)
-#pragma unroll
-        for (uint32_t k = 0; k < 2 * kNearRows; ++k) acc[q][k] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    // operands read through global (not generic) pointers, so each MFMA
-    // waits only for its own loads
-    using Op = KStep<SPLIT, PG, kNearRows>;
-    using V = typename Op::V;
-    using GV = const __attribute__((address_space(1))) V*;
-    const GV wv = (GV)reinterpret_cast<const V*>(w0);
-    GV pv[PG];
-#pragma unroll
-    for (int q = 0; q < PG; ++q) pv[q] = (GV)reinterpret_cast<const V*>(Pp[q]);
-    // load cursor: step ls at window row lr, 32-column block lcc. A tile's
-    // window spans at least 3 rows and 32 columns (the host pads the
-    // footprint by a texel on each side), so KS >= 3.
-    uint32_t ls = 0, lr = 0, lcc = 0;
-    kstep_pipeline<near_unroll<SPLIT>(), SPLIT, PG, kNearRows>(acc, KS, [&](Op& o) {
-        const size_t pidx = (((size_t)(Tl.y0 + (int)J.B + (int)lr) * J.Pw8 + xb + lcc * 4) * 32) + i;
-        const size_t o0 = (size_t)ls * kStep;
-#pragma unroll
-        for (uint32_t h = 0; h < kNearRows; ++h) {
-            o.x[h] = wv[o0 + h * kRow];
-            if constexpr (SPLIT) o.x[kNearRows + h] = wv[o0 + h * kRow + J.w_lo];
-        }
-#pragma unroll
-        for (int q = 0; q < PG; ++q) {
-            o.b[q][0] = pv[q][pidx];
-            o.b[q][1] = pv[q][pidx + 16];
-            if constexpr (SPLIT) {
-                o.b[q][2] = pv[q][pidx + J.p_lo];
-                o.b[q][3] = pv[q][pidx + 16 + J.p_lo];
-            }
-        }
-        const uint32_t step = ls + 1 < KS ? 1u : 0u;  // selects, not branches, between the loads
-        ls += step;
-        lcc += step;
-        const bool wrap = lcc == wc;
-        lr += wrap ? 1u : 0u;
-        lcc = wrap ? 0u : lcc;
-    });
-    const uint32_t So = J.So, X0 = (tile % J.te) * 16, Y0 = (tile / J.te) * 16;
-    const size_t So2 = (size_t)So * So;
-#pragma unroll
-    for (int q = 0; q < PG; ++q) {
-        if ((uint32_t)q >= np) break;
-        float* out = reinterpret_cast<float*>(probe_out(Q, p0 + q) + J.out_off);
-        const float* sq = scr(Q, sc, p0 + q);
-#pragma unroll
-        for (uint32_t h = 0; h < kNearRows; ++h) {
-            const uint32_t Y = Y0 + rt0 + h;
-#pragma unroll
-            for (int nb = 0; nb < 2; ++nb) {
-                const f32x4 a = acc[q][2 * h + nb];
-                const uint32_t col = nb * 16 + i, f = col >> 2, c = col & 3;
-                if (col >= 24) continue;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const uint32_t X = X0 + 4 * g + e, o = Y * So + X;
-                    out[((size_t)f * So2 + o) * 4 + c] = c < 3 ? a[e] * J.rowscale[o] * sq[6 + f] : 1.0f;
-                }
-            }
-        }
-    }
-}
-
-// The single-probe near GEMM with the radiance window staged in LDS: a
-// workgroup's four waves (four row tiles of one tile) share each K step's B
-// block (128 half8, twice that split), so the workgroup loads it once into
-// LDS, GS steps at a time, double buffered, with one barrier per GS steps;
-// each wave then issues one global load per step for its weights (two
-// split) instead of also loading the block itself. Weights are loaded a
-// group ahead. Each output's accumulation is the same sequence of MFMAs as
-// in near_gemm_kernel, so the outputs are identical. Measured on the 512^2
-// GGX chain (whole call): FP16 with near_gemm_kernel 0.54 ms; GS = 4: 0.555,
-// 8: 0.496, 12: 0.476, 16: 0.464 (2 waves per SIMD), 20: 0.475, 24 spills;
-// split BF16 with near_gemm_kernel 0.915 ms; GS = 4: 0.837, 6: 0.794, 8:
-// 0.762 (2 waves per SIMD).
-#ifndef HVX_NEAR_LDS_GROUP
-#define HVX_NEAR_LDS_GROUP 16
-#endif
-// weights are read once per call: non-temporal loads (whole FP16 / split
-// call on the 512^2 GGX chain: 0.460 / 0.754 ms -> 0.449 / 0.723)
-#ifndef HVX_NEAR_NT
-#define HVX_NEAR_NT 1
-#endif
-#ifndef HVX_NEAR_LDS_GROUP_SPLIT
-#define HVX_NEAR_LDS_GROUP_SPLIT 8
-#endif
-constexpr int kNearLdsGroup = HVX_NEAR_LDS_GROUP;             // 0: near_gemm_kernel
-constexpr int kNearLdsGroupSplit = HVX_NEAR_LDS_GROUP_SPLIT;  // 0: near_gemm_kernel
-template <bool SPLIT, int GS>
-__global__ __launch_bounds__(256) void near_gemm_lds_kernel(Probes Q, NearTable T, const float* sc) {
-    static_assert(kNearRows == 1 && GS % 2 == 0, "one row tile per wave, whole B passes per group");
-    const uint32_t lb = near_single_block(blockIdx.x);
-    const uint32_t gt = lb / kNearSingleParts;
-    if (gt >= T.tiles) return;  // padding of the XCD-aware order (uniform, before any barrier)
-    uint32_t jj = 0;
-    while (jj + 1 < T.n && gt >= T.j[jj + 1].tile_begin) ++jj;
-    const NearJob& J = T.j[jj];
-    const uint32_t tile = gt - J.tile_begin, t = threadIdx.x, lane = t & 63;
-    const uint32_t wave = (t >> 6) + (lb % kNearSingleParts) * 4;
-    const NearTile Tl = J.tiles[tile];
-    const uint32_t wc = Tl.w / 32, KS = Tl.h * wc;
-    const uint32_t i = lane & 15, g = lane >> 4, rt0 = wave;
-    constexpr size_t kStep = 16 * 64;
-    constexpr uint32_t kBw = SPLIT ? 256 : 128;  // half8 of a step's B block (hi, then lo)
-    constexpr int kWs = SPLIT ? 2 : 1;            // weight fragments per step (hi, lo)
+// Bound by what reaches the CUs: at 512^2 x 10 about 110 MB of weights and
+// 125 MB of staged units (each read by the blocks whose windows hold it) in
+// 45 us, while its MFMAs need 6 us and its LDS reads 7 us.
+// One workgroup per (item, probe): four waves of two 16-row tiles each over
+// the item's K steps, all 144 columns, so a wave's 18 accumulators reuse each
+// weight fragment nine times and each B fragment twice. The B operand of a
+// step (four units of 144 half8, contiguous) is shared by the waves and
+// staged in LDS, kGroup steps per barrier, double buffered, a group ahead;
+// weights go straight to registers, a group ahead.
+template <bool SPLIT>
+__device__ __forceinline__ void gemm_item(const GemmArgs& A, const Block& B, const Item& I, const half8* Rp,
+                                          half8 (*sB)[kGroup * 4 * kCols], const uint32_t* sU, f32x4 (&acc)[2][kNt]) {
+    constexpr uint32_t G = SPLIT ? kGroup / 2 : kGroup;  // steps per group
+    constexpr uint32_t kStepB = 4 * kCols * (SPLIT ? 2 : 1);
+    constexpr uint32_t kPer = G * kStepB / 256;
+    constexpr int kWs = SPLIT ? 4 : 2;
+    static_assert(G * kStepB % 256 == 0, "whole passes of the workgroup");
     using GH = const __attribute__((address_space(1))) half8*;
-    const GH wv = (GH)(J.W + Tl.woff + (size_t)rt0 * 64 + lane);
-    const GH pv = (GH)scr(Q, J.P, 0);
-    const uint32_t xb0 = (uint32_t)(Tl.x0 + (int)J.B) / 8;
-    const size_t p_lo = J.p_lo, w_lo = J.w_lo;
-    // B block of step s: 128 consecutive half8 at ((row * Pw8 + xb0 + col * 4) * 32)
-    // (its lo part p_lo further), row = s / wc, col = s % wc; steps past the
-    // last repeat it
-    auto b_base = [&](uint32_t s) {
-        s = s < KS ? s : KS - 1;
-        const uint32_t r = s / wc, c = s - r * wc;
-        return ((size_t)(Tl.y0 + (int)J.B + (int)r) * J.Pw8 + xb0 + c * 4) * 32;
-    };
-    constexpr int kPer = GS * kBw / 256;  // half8 of a group's B per thread
-    __shared__ half8 sB[2][GS][kBw];
-    auto b_load = [&](uint32_t s0, half8 (&v)[kPer]) {
+    const uint32_t t = threadIdx.x, lane = t & 63, wave = t >> 6, i = lane & 15, g = lane >> 4;
+    const uint32_t nrt = B.nrt, rt0 = 2 * wave, n = I.n;
+    const bool live = rt0 < nrt, has1 = rt0 + 1 < nrt;  // uniform per wave
+    const GH w0 = (GH)(A.W + B.woff + ((size_t)I.s0 * nrt + (live ? rt0 : 0)) * 64 + lane);
+    const GH w1 = has1 ? w0 + 64 : w0;
+    const size_t wstep = (size_t)nrt * 64, w_lo = B.w_lo, r_lo = A.r_lo[B.src];
+    const GH R = (GH)Rp;
+    // steps past the slice's last repeat it (loaded, not used)
+    auto w_load = [&](uint32_t s, half8 (&x)[G][kWs]) {
 #pragma unroll
-        for (int k = 0; k < kPer; ++k) {
-            const uint32_t e = t + 256u * k, o = e % kBw;
-            v[k] = pv[b_base(s0 + e / kBw) + o % 128 + (o >= 128 ? p_lo : 0)];
+        for (uint32_t k = 0; k < G; ++k) {
+            const size_t o = (size_t)(s + k < n ? s + k : n - 1) * wstep;
+            x[k][0] = w0[o];
+            x[k][1] = w1[o];
+            if constexpr (SPLIT) {
+                x[k][2] = w0[o + w_lo];
+                x[k][3] = w1[o + w_lo];
+            }
+        }
+    };
+    // sU holds the slice's units, padded to whole groups
+    auto b_load = [&](uint32_t s, half8 (&v)[kPer]) {
+#pragma unroll
+        for (uint32_t k = 0; k < kPer; ++k) {
+            const uint32_t e = t + 256u * k, st = e / kStepB, r = e % kStepB, lo = r / (4 * kCols), rr = r % (4 * kCols);
+            v[k] = R[(size_t)sU[(s + st) * 4 + rr / kCols] * kCols + rr % kCols + (lo ? r_lo : 0)];
         }
     };
     auto b_store = [&](uint32_t buf, const half8 (&v)[kPer]) {
 #pragma unroll
-        for (int k = 0; k < kPer; ++k) {
-            const uint32_t e = t + 256u * k;
-            sB[buf][e / kBw][e % kBw] = v[k];
-        }
+        for (uint32_t k = 0; k < kPer; ++k) sB[buf][t + 256u * k] = v[k];
     };
-    auto w_load = [&](uint32_t s0, half8 (&x)[GS][kWs]) {
-#pragma unroll
-        for (int k = 0; k < GS; ++k) {
-            const size_t o = (size_t)(s0 + k < KS ? s0 + k : KS - 1) * kStep;
-#if HVX_NEAR_NT
-            x[k][0] = __builtin_nontemporal_load(&wv[o]);
-            if constexpr (SPLIT) x[k][1] = __builtin_nontemporal_load(&wv[o + w_lo]);
-#else
-            x[k][0] = wv[o];
-            if constexpr (SPLIT) x[k][1] = wv[o + w_lo];
-#endif
-        }
-    };
-    f32x4 acc[2] = {f32x4{0.0f, 0.0f, 0.0f, 0.0f}, f32x4{0.0f, 0.0f, 0.0f, 0.0f}};
-    half8 nb[kPer], xw[GS][kWs], xn[GS][kWs];
+    half8 nb[kPer], xw[G][kWs], xn[G][kWs];
     b_load(0, nb);
     w_load(0, xw);
     b_store(0, nb);
     __syncthreads();
-    const uint32_t groups = (KS + GS - 1) / GS;
+    const uint32_t groups = (n + G - 1) / G;
     for (uint32_t gi = 0; gi < groups; ++gi) {
-        const uint32_t s0 = gi * GS;
-        // the next group's weights, then its B block, are in flight during
-        // this group's MFMAs (the last group reloads itself, unused)
-        const uint32_t sn = gi + 1 < groups ? s0 + GS : s0;
+        const uint32_t s = gi * G, sn = gi + 1 < groups ? s + G : s;
         w_load(sn, xn);
         b_load(sn, nb);
         __asm__ volatile("" ::: "memory");
-        const uint32_t buf = gi & 1;
+        const half8* sb = sB[gi & 1];
 #pragma unroll
-        for (int k = 0; k < GS; ++k) {
-            if (s0 + k < KS) {  // uniform over the workgroup
-                const half8* sb = sB[buf][k];
-                if constexpr (SPLIT) {
-                    const bf16x8 x = __builtin_bit_cast(bf16x8, xw[k][0]), y = __builtin_bit_cast(bf16x8, xw[k][1]);
-                    const bf16x8 b0 = __builtin_bit_cast(bf16x8, sb[g * 32 + i]);
-                    const bf16x8 b1 = __builtin_bit_cast(bf16x8, sb[g * 32 + 16 + i]);
-                    const bf16x8 c0 = __builtin_bit_cast(bf16x8, sb[128 + g * 32 + i]);
-                    const bf16x8 c1 = __builtin_bit_cast(bf16x8, sb[128 + g * 32 + 16 + i]);
-                    acc[0] = hvx::mfma16x16x32(x, b0, acc[0]);
-                    acc[0] = hvx::mfma16x16x32(x, c0, acc[0]);
-                    acc[0] = hvx::mfma16x16x32(y, b0, acc[0]);
-                    acc[1] = hvx::mfma16x16x32(x, b1, acc[1]);
-                    acc[1] = hvx::mfma16x16x32(x, c1, acc[1]);
-                    acc[1] = hvx::mfma16x16x32(y, b1, acc[1]);
-                } else {
-                    const half8 b0 = sb[g * 32 + i], b1 = sb[g * 32 + 16 + i];
-                    acc[0] = hvx::mfma16x16x32(xw[k][0], b0, acc[0]);
-                    acc[1] = hvx::mfma16x16x32(xw[k][0], b1, acc[1]);
+        for (uint32_t k = 0; k < G; ++k) {
+            if (live && s + k < n) {
+#pragma unroll
+                for (uint32_t nt = 0; nt < kNt; ++nt) {
+                    const half8* bk = sb + k * kStepB + g * kCols + nt * 16 + i;
+                    if constexpr (SPLIT) {
+                        const bf16x8 b = __builtin_bit_cast(bf16x8, bk[0]), c = __builtin_bit_cast(bf16x8, bk[4 * kCols]);
+#pragma unroll
+                        for (int h = 0; h < 2; ++h) {
+                            const bf16x8 x = __builtin_bit_cast(bf16x8, xw[k][h]);
+                            const bf16x8 y = __builtin_bit_cast(bf16x8, xw[k][2 + h]);
+                            // hi*hi + hi*lo + lo*hi (lo*lo is below the FP32 accumulation's resolution)
+                            acc[h][nt] = hvx::mfma16x16x32(x, b, acc[h][nt]);
+                            acc[h][nt] = hvx::mfma16x16x32(x, c, acc[h][nt]);
+                            acc[h][nt] = hvx::mfma16x16x32(y, b, acc[h][nt]);
+                        }
+                    } else {
+                        const half8 b = bk[0];
+                        acc[0][nt] = hvx::mfma16x16x32(xw[k][0], b, acc[0][nt]);
+                        acc[1][nt] = hvx::mfma16x16x32(xw[k][1], b, acc[1][nt]);
+                    }
                 }
             }
         }
-        // the other buffer's readers passed the previous barrier
-        b_store(buf ^ 1, nb);
+        b_store((gi & 1) ^ 1, nb);  // its readers passed the previous barrier
 #pragma unroll
-        for (int k = 0; k < GS; ++k)
+        for (uint32_t k = 0; k < G; ++k)
 #pragma unroll
             for (int u = 0; u < kWs; ++u) xw[k][u] = xn[k][u];
         __syncthreads();
     }
-    const uint32_t So = J.So, X0 = (tile % J.te) * 16, Y0 = (tile / J.te) * 16;
-    const size_t So2 = (size_t)So * So;
-    float* out = reinterpret_cast<float*>(probe_out(Q, 0) + J.out_off);
-    const float* sq = scr(Q, sc, 0);
-    const uint32_t Y = Y0 + rt0;
-#pragma unroll
-    for (int n = 0; n < 2; ++n) {
-        const f32x4 a = acc[n];
-        const uint32_t col = n * 16 + i, f = col >> 2, c = col & 3;
-        if (col >= 24) continue;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const uint32_t X = X0 + 4 * g + e, o = Y * So + X;
-            out[((size_t)f * So2 + o) * 4 + c] = c < 3 ? a[e] * J.rowscale[o] * sq[6 + f] : 1.0f;
-        }
-    }
 }
 
-template <bool SPLIT, int PG>
-__global__ __launch_bounds__(256) void near_gemm_staged_kernel(Probes Q, NearTable T, const float* sc) {
-    const uint2 wb = gemm_block(Q);
-    const uint32_t p0 = wb.y * PG, np = min((uint32_t)PG, Q.n - p0);
-    uint32_t jj = 0;
-    // workgroup b owns half b & 1 (eight row tiles) of tile b >> 1: finer
-    // work units than whole tiles balance the unequal mips across the CUs
-    const uint32_t gt = wb.x / kNearParts;
-    while (jj + 1 < T.n && gt >= T.j[jj + 1].tile_begin) ++jj;
-    const NearJob& J = T.j[jj];
-    const uint32_t tile = gt - J.tile_begin, lane = threadIdx.x & 63;
-    const uint32_t wave = (threadIdx.x >> 6) + (wb.x % kNearParts) * (kNearWaves / kNearParts);
-    const NearTile Tl = J.tiles[tile];
-    // PG probes per wave: each weight fragment is loaded once for the group;
-    // each probe's accumulation is the same sequence as with PG = 1
-    const half8* Pp[PG];
-#pragma unroll
-    for (int q = 0; q < PG; ++q) Pp[q] = scr(Q, J.P, p0 + ((uint32_t)q < np ? q : 0));
-    const uint32_t wc = Tl.w / 32, KS = Tl.h * wc;
-    const uint32_t i = lane & 15, g = lane >> 4, rt0 = 2 * wave;
-    // weights of a tile stored K-step major: step s of all 16 row tiles is one
-    // contiguous 16 KB block
-    constexpr size_t kStep = 16 * 64, kRow = 64;
-    const half8* w0 = J.W + Tl.woff + (size_t)rt0 * kRow + lane;
-    const uint32_t xb0 = (uint32_t)(Tl.x0 + (int)J.B) / 8;
-    // The B operand of a K step (for each probe: 4 x 32 consecutive half8 of
-    // the staged plane, plus as many lo parts when split) is the same for
-    // every wave of the workgroup: it is staged once per step in LDS, double
-    // buffered, the next step's copy loaded while this step's MFMAs run. With
-    // PG probes per wave this cuts the workgroup's operand reads PG-fold per
-    // step, which pays for the barrier (256-probe batch, contraction mode: 8.8 -> 8.4 ms).
-    // Single-probe calls stage several steps per barrier instead
-    // (near_gemm_lds_kernel): with a barrier per step one probe lost (512^2 x 10
-    // GGX chain: 0.366 -> 0.392 ms).
-    constexpr int kB = PG * 128 * (SPLIT ? 2 : 1);  // half8 per step
-    constexpr int kPer = (kB + 255) / 256;           // per thread (256 lanes)
-    static_assert(kB % 256 == 0 || kB < 256, "the B block splits evenly over the workgroup");
-    __shared__ half8 sB[2][kB];
-    const uint32_t t = threadIdx.x;
-    // the B operand is read through global (not generic) pointers: generic
-    // loads count against the LDS counter too, so each step's LDS reads
-    // would wait for the next step's B loads
-    using GH = const __attribute__((address_space(1))) half8*;
-    GH Pg[PG];
-#pragma unroll
-    for (int q = 0; q < PG; ++q) Pg[q] = (GH)Pp[q];
-    // element e = t + 256 k of the step's block: lo part e / (PG * 128),
-    // probe (e / 128) % PG, unit e % 128. With whole 256-element passes and
-    // an even PG the part is the same for the whole pass, so every lane
-    // loads unconditionally (conditional loads make the waits conservative).
-    const uint32_t p_lo = J.p_lo;
-    auto b_load = [&](uint32_t r, uint32_t cc, half8 (&v)[kPer]) {
-        const size_t base = ((size_t)(Tl.y0 + (int)J.B + (int)r) * J.Pw8 + xb0 + cc * 4) * 32;
-#pragma unroll
-        for (int k = 0; k < kPer; ++k) {
-            const uint32_t e = t + 256u * k, q = (e / 128) % PG, o = e % 128;
-            if constexpr (kB % 256 == 0 && (PG * 128) % 256 == 0) {
-                const uint32_t lo = (256u * k) / (PG * 128);
-                v[k] = Pg[q][base + o + (lo ? p_lo : 0)];
-            } else {
-                const uint32_t lo = e / (PG * 128);
-                if (e < (uint32_t)kB) v[k] = Pg[q][base + o + (lo ? p_lo : 0)];
-            }
-        }
-    };
-    half8 nx[kPer];
-    b_load(0, 0, nx);
-#pragma unroll
-    for (int k = 0; k < kPer; ++k)
-        if (t + 256u * k < (uint32_t)kB) sB[0][t + 256u * k] = nx[k];
+__global__ __launch_bounds__(256, 2) void contract_gemm_kernel(Probes Q, GemmArgs A) {
+    __shared__ half8 sB[2][kGroup * 4 * kCols];
+    __shared__ uint32_t sU[(kMaxSlice + kGroup) * 4];
+    // hardware workgroup b runs on XCD b % 8: each XCD takes one run of the
+    // items, whose neighbours share staged units, and of an item's probes,
+    // which share its weights
+    const uint32_t run = (A.nitems * Q.n + kXcds - 1) / kXcds;
+    const uint32_t id = blockIdx.x % kXcds * run + blockIdx.x / kXcds;
+    if (id >= A.nitems * Q.n) return;  // uniform; padding of the last run
+    const uint32_t item = id / Q.n, pr = id - item * Q.n, t = threadIdx.x;
+    const Item I = A.items[item];
+    const Block B = A.blocks[I.block];
+    const uint32_t left = B.nunits - I.s0 * 4;  // units from the slice's first on (its last step may be short of four)
+    for (uint32_t k = t; k < (kMaxSlice + kGroup) * 4; k += 256)
+        sU[k] = A.ulist[B.unit0 + I.s0 * 4 + min(k, min(I.n * 4, left) - 1)];
     __syncthreads();
-    f32x4 acc[PG][4];
+    const half8* R = scr(Q, A.R[B.src], pr);
+    f32x4 acc[2][kNt];
 #pragma unroll
-    for (int q = 0; q < PG; ++q)
+    for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int k = 0; k < 4; ++k) acc[q][k] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    uint32_t r = 0, cc = 0;
-    for (uint32_t s = 0; s < KS; ++s) {
-        uint32_t rn = r, cn = cc + 1;
-        if (cn == wc) {
-            cn = 0;
-            ++rn;
-        }
-        const bool more = s + 1 < KS;
-        // this step's weights are loaded before the next step's B operand:
-        // the load counter completes in order, so the MFMAs' wait for the
-        // weights leaves the B loads in flight
-        using V = std::conditional_t<SPLIT, bf16x8, half8>;
-        const V* wv = reinterpret_cast<const V*>(w0);
-        const size_t o0 = (size_t)s * kStep, o1 = o0 + kRow;
-        V xw[SPLIT ? 4 : 2];
-        xw[0] = wv[o0];
-        xw[1] = wv[o1];
-        if constexpr (SPLIT) {
-            xw[2] = wv[o0 + J.w_lo];
-            xw[3] = wv[o1 + J.w_lo];
-        }
-        b_load(more ? rn : r, more ? cn : cc, nx);  // the last step reloads itself
-        __asm__ volatile("" ::: "memory");          // keeps the B loads ahead of the MFMAs
-        const half8* sb = sB[s & 1];
-        if constexpr (SPLIT) {
-            const bf16x8 x0 = xw[0], x1 = xw[1], y0 = xw[2], y1 = xw[3];
+        for (uint32_t nt = 0; nt < kNt; ++nt) acc[h][nt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    if (B.split) gemm_item<true>(A, B, I, R, sB, sU, acc);
+    else gemm_item<false>(A, B, I, R, sB, sU, acc);
+    const uint32_t lane = t & 63, i = lane & 15, g = lane >> 4, rt0 = 2 * (t >> 6);
+    float* p = scr(Q, A.part, pr) + (size_t)I.slot * kBlockRows * kCols;
 #pragma unroll
-            for (int q = 0; q < PG; ++q) {
-                const bf16x8* pv = reinterpret_cast<const bf16x8*>(sb + q * 128 + g * 32 + i);
-                const bf16x8 b0 = pv[0], b1 = pv[16], c0 = pv[PG * 128], c1 = pv[PG * 128 + 16];
-                acc[q][0] = hvx::mfma16x16x32(x0, b0, acc[q][0]);
-                acc[q][0] = hvx::mfma16x16x32(x0, c0, acc[q][0]);
-                acc[q][0] = hvx::mfma16x16x32(y0, b0, acc[q][0]);
-                acc[q][1] = hvx::mfma16x16x32(x0, b1, acc[q][1]);
-                acc[q][1] = hvx::mfma16x16x32(x0, c1, acc[q][1]);
-                acc[q][1] = hvx::mfma16x16x32(y0, b1, acc[q][1]);
-                acc[q][2] = hvx::mfma16x16x32(x1, b0, acc[q][2]);
-                acc[q][2] = hvx::mfma16x16x32(x1, c0, acc[q][2]);
-                acc[q][2] = hvx::mfma16x16x32(y1, b0, acc[q][2]);
-                acc[q][3] = hvx::mfma16x16x32(x1, b1, acc[q][3]);
-                acc[q][3] = hvx::mfma16x16x32(x1, c1, acc[q][3]);
-                acc[q][3] = hvx::mfma16x16x32(y1, b1, acc[q][3]);
-            }
-        } else {
-            const half8 x0 = xw[0], x1 = xw[1];
+    for (uint32_t h = 0; h < 2; ++h) {
+        if (rt0 + h >= B.nrt) break;
 #pragma unroll
-            for (int q = 0; q < PG; ++q) {
-                const half8* pv = sb + q * 128 + g * 32 + i;
-                const half8 b0 = pv[0], b1 = pv[16];
-                acc[q][0] = hvx::mfma16x16x32(x0, b0, acc[q][0]);
-                acc[q][1] = hvx::mfma16x16x32(x0, b1, acc[q][1]);
-                acc[q][2] = hvx::mfma16x16x32(x1, b0, acc[q][2]);
-                acc[q][3] = hvx::mfma16x16x32(x1, b1, acc[q][3]);
-            }
-        }
-        // stored unconditionally: after the last step the buffer is no longer
-        // read (its readers passed the previous barrier), and a store under a
-        // branch would draw the B loads into the branch, after the MFMAs
+        for (uint32_t nt = 0; nt < kNt; ++nt)
 #pragma unroll
-        for (int k = 0; k < kPer; ++k)
-            if (t + 256u * k < (uint32_t)kB) sB[(s + 1) & 1][t + 256u * k] = nx[k];
-        __syncthreads();
-        r = rn;
-        cc = cn;
-    }
-    const uint32_t So = J.So, X0 = (tile % J.te) * 16, Y0 = (tile / J.te) * 16;
-    const size_t So2 = (size_t)So * So;
-#pragma unroll
-    for (int q = 0; q < PG; ++q) {
-        if ((uint32_t)q >= np) break;
-        float* out = reinterpret_cast<float*>(probe_out(Q, p0 + q) + J.out_off);
-        const float* sq = scr(Q, sc, p0 + q);
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const uint32_t Y = Y0 + rt0 + h;
-#pragma unroll
-            for (int nb = 0; nb < 2; ++nb) {
-                const f32x4 a = acc[q][2 * h + nb];
-                const uint32_t col = nb * 16 + i, f = col >> 2, c = col & 3;
-                if (col >= 24) continue;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const uint32_t X = X0 + 4 * g + e, o = Y * So + X;
-                    out[((size_t)f * So2 + o) * 4 + c] = c < 3 ? a[e] * J.rowscale[o] * sq[6 + f] : 1.0f;
-                }
-            }
-        }
+            for (uint32_t r = 0; r < 4; ++r)
+                p[((rt0 + h) * 16 + 4 * g + r) * kCols + nt * 16 + i] = acc[h][nt][r];
     }
 }
 
-// out(o) += far field interpolated at o / Z(o)
-__global__ __launch_bounds__(256) void far_add_kernel(Probes Q, NearTable T) {
-    const uint32_t id = blockIdx.x * 256 + threadIdx.x, pr = blockIdx.y;
-    if (id >= T.texels) return;
-    uint32_t jj = 0;
-    while (jj + 1 < T.n && id >= T.j[jj + 1].texel_begin) ++jj;
-    const NearJob& J = T.j[jj];
-    const uint32_t So = J.So, So2 = So * So, local = id - J.texel_begin;
-    const uint32_t f = local / So2, o = local - f * So2, Y = o / So, X = o - Y * So;
-    const f3 F = sample_cube(scr(Q, J.far, pr), (int)J.Sf, texel_dir((int)f, (int)X, (int)Y, (int)So));
-    const float z = J.invZ[o];
-    float4* out = probe_out(Q, pr) + J.out_off;
-    float4 v = out[local];
-    v.x += F.x * z;
-    v.y += F.y * z;
-    v.z += F.z * z;
-    out[local] = v;
+// The far map (face Sf) at the centre of output texel (x, y) of face f: the
+// texel's plane coordinates are exact in FP32 (sizes are powers of two), so
+// inside the face the four taps need no direction.
+__device__ __forceinline__ f3 far_sample(const float4* __restrict__ map, uint32_t Sf, uint32_t f, uint32_t x,
+                                         uint32_t y, uint32_t So) {
+    const float r = (float)Sf / (float)So;
+    const float u = ((float)x + 0.5f) * r - 0.5f, v = ((float)y + 0.5f) * r - 0.5f;
+    const float fu = floorf(u), fv = floorf(v), a = u - fu, b = v - fv;
+    const int i = (int)fu, j = (int)fv;
+    if (i < 0 || j < 0 || i + 1 >= (int)Sf || j + 1 >= (int)Sf)
+        return sample_cube(map, (int)Sf, texel_dir((int)f, (int)x, (int)y, (int)So));
+    const float4* p = map + ((size_t)f * Sf + j) * Sf + i;
+    const float4 q00 = p[0], q10 = p[1], q01 = p[Sf], q11 = p[Sf + 1];
+    const float w00 = (1.0f - a) * (1.0f - b), w10 = a * (1.0f - b), w01 = (1.0f - a) * b, w11 = a * b;
+    return {((w00 * q00.x + w10 * q10.x) + w01 * q01.x) + w11 * q11.x,
+            ((w00 * q00.y + w10 * q10.y) + w01 * q01.y) + w11 * q11.y,
+            ((w00 * q00.z + w10 * q10.z) + w01 * q01.z) + w11 * q11.z};
 }
 
-// Roughness 0: the bilinear seamless sample of level 0 at the texel direction.
-__global__ __launch_bounds__(256) void delta_kernel(Probes Q, uint32_t S, uint32_t So, size_t out_off) {
+// Output texel (g o, f) of each row from the slices' sums, in slice order. NEAR
+// false: whole rows into the chain, far rows into their map (not normalised);
+// true: near rows plus the far field interpolated at the texel, over Z.
+template <bool NEAR>
+__global__ __launch_bounds__(256) void epilogue_kernel(Probes Q, const Job* __restrict__ jobs,
+                                                       const Row* __restrict__ rows, const Block* __restrict__ blocks,
+                                                       const float* part, const float* __restrict__ rowscale,
+                                                       const float* __restrict__ invZ, const float* sc, uint32_t row0,
+                                                       uint32_t n) {
     const uint32_t id = blockIdx.x * 256 + threadIdx.x, pr = blockIdx.y;
-    const float4* level0 = probe_chain(Q, pr);
-    float4* out = probe_out(Q, pr) + out_off;
-    const uint32_t So2 = So * So;
-    if (id >= 6 * So2) return;
-    const uint32_t f = id / So2, o = id - f * So2, Y = o / So, X = o - Y * So;
-    const f3 c = sample_cube(level0, (int)S, texel_dir((int)f, (int)X, (int)Y, (int)So));
-    out[id] = make_float4(c.x, c.y, c.z, 1.0f);
+    if (id >= n * kImages) return;
+    const uint32_t r = row0 + id / kImages, gf = id % kImages, g = gf / 6, f = gf - 6 * g;
+    const Row R = rows[r];
+    const Job& J = jobs[R.job];
+    uint32_t x = R.x, y = R.y;
+    if (!image_written(g, J.So, x, y)) return;
+    image_of(g, J.So, x, y);
+    const Block& B = blocks[R.block];
+    const uint32_t ns = B.nslices;
+    const float* p = scr(Q, part, pr) + ((size_t)B.item0 * kBlockRows + (r - B.row0)) * kCols + 3 * gf;
+    float v[3] = {0.0f, 0.0f, 0.0f};
+#pragma unroll 4
+    for (uint32_t s = 0; s < ns; ++s, p += kBlockRows * kCols) {
+        v[0] += p[0];
+        v[1] += p[1];
+        v[2] += p[2];
+    }
+    const size_t o = ((size_t)f * J.So + y) * J.So + x;
+    const float* q = scr(Q, sc, pr);
+    if constexpr (NEAR) {
+        const float k = rowscale[r], sf = q[f], z = invZ[r];
+        const f3 F = far_sample(scr(Q, J.map, pr), J.Sf, f, x, y, J.So);
+        probe_out(Q, pr)[J.out_off + o] =
+            make_float4(v[0] * k * sf + F.x * z, v[1] * k * sf + F.y * z, v[2] * k * sf + F.z * z, 1.0f);
+    } else {
+        const float k = rowscale[r] * q[6];
+        const bool far = J.piece == PIECE_FAR;
+        float4* out = far ? scr(Q, J.map, pr) : probe_out(Q, pr) + J.out_off;
+        out[o] = make_float4(v[0] * k, v[1] * k, v[2] * k, far ? 0.0f : 1.0f);
+    }
 }
 
 // --------------------------------------------------- bright-texel split
@@ -1883,6 +1278,7 @@ __global__ __launch_bounds__(256) void hot_add_kernel(HotAdd A) {
     r.z = __builtin_fmaf(az, M.scale, r.z);
 }
 
+
 // -------------------------------------------------------------- host side
 uint32_t ilog2(uint32_t v) {
     uint32_t l = 0;
@@ -1890,128 +1286,49 @@ uint32_t ilog2(uint32_t v) {
     return l;
 }
 
-// Integer frame of face f: world point of face-plane (u, v) = u E0 + v E1 + E2.
-void face_frame(int f, int E[3][3]) {
-    double z[3], a[3], b[3];
-    hvx::contract_face_point(f, 0.0, 0.0, z);
-    hvx::contract_face_point(f, 1.0, 0.0, a);
-    hvx::contract_face_point(f, 0.0, 1.0, b);
-    for (int j = 0; j < 3; ++j) {
-        E[0][j] = (int)(a[j] - z[j]);
-        E[1][j] = (int)(b[j] - z[j]);
-        E[2][j] = (int)z[j];
-    }
-}
-
-// World texel index (face-major) of the texel whose direction is output
-// face f's frame applied to canonical input k: exact integer arithmetic in
-// doubled texel units (a texel centre of face g is a E0 + b E1 + S E2 with
-// odd a, b in (-S, S)).
-int32_t perm_index(int f, uint32_t k, uint32_t S) {
-    const uint32_t S2 = S * S, g = k / S2, rem = k % S2, y = rem / S, x = rem % S;
-    const int s = (int)S, a = 2 * (int)x + 1 - s, b = 2 * (int)y + 1 - s;
-    int Eg[3][3], Ef[3][3], p[3], q[3];
-    face_frame((int)g, Eg);
-    face_frame(f, Ef);
-    for (int j = 0; j < 3; ++j) p[j] = a * Eg[0][j] + b * Eg[1][j] + s * Eg[2][j];
-    for (int j = 0; j < 3; ++j) q[j] = p[0] * Ef[0][j] + p[1] * Ef[1][j] + p[2] * Ef[2][j];
-    const int ax = std::abs(q[0]), ay = std::abs(q[1]), az = std::abs(q[2]);
-    int nf, na, nb;
-    if (ax >= ay && ax >= az) {
-        if (q[0] > 0) { nf = 0; na = -q[2]; nb = -q[1]; }
-        else { nf = 1; na = q[2]; nb = -q[1]; }
-    } else if (ay >= az) {
-        if (q[1] > 0) { nf = 2; na = q[0]; nb = q[2]; }
-        else { nf = 3; na = q[0]; nb = -q[2]; }
-    } else {
-        if (q[2] > 0) { nf = 4; na = q[0]; nb = -q[1]; }
-        else { nf = 5; na = -q[0]; nb = -q[1]; }
-    }
-    const int ni = (na + s - 1) / 2, nj = (nb + s - 1) / 2;
-    return (int32_t)(((size_t)nf * S + nj) * S + ni);
-}
-
-void orthonormal(const double n[3], double e1[3], double e2[3]) {
-    const double a[3] = {std::fabs(n[0]) < 0.9 ? 1.0 : 0.0, std::fabs(n[0]) < 0.9 ? 0.0 : 1.0, 0.0};
-    e1[0] = a[1] * n[2] - a[2] * n[1];
-    e1[1] = a[2] * n[0] - a[0] * n[2];
-    e1[2] = a[0] * n[1] - a[1] * n[0];
-    const double l = std::sqrt(e1[0] * e1[0] + e1[1] * e1[1] + e1[2] * e1[2]);
-    for (int j = 0; j < 3; ++j) e1[j] /= l;
-    e2[0] = n[1] * e1[2] - n[2] * e1[1];
-    e2[1] = n[2] * e1[0] - n[0] * e1[2];
-    e2[2] = n[0] * e1[1] - n[1] * e1[0];
-}
-
-// Windows (bounding boxes of the angular caps of radius t1 around every
-// output of a tile, on the face plane at the near level), aligned for the
-// GEMM's B loads: x0 to 8 texels, width to 32.
-std::vector<NearTile> near_tiles(uint32_t So, uint32_t Si, double t1, uint32_t* B_out) {
-    const uint32_t te = So / 16;
-    std::vector<NearTile> tiles(te * te);
-    int B = 0;
-    uint64_t woff = 0;
-    const double ct = std::cos(t1), st = std::sin(t1);
-    for (uint32_t ty = 0; ty < te; ++ty)
-        for (uint32_t tx = 0; tx < te; ++tx) {
-            double xmin = 1e30, xmax = -1e30, ymin = 1e30, ymax = -1e30;
-            for (uint32_t yy = 0; yy < 16; ++yy)
-                for (uint32_t xx = 0; xx < 16; ++xx) {
-                    const double u = hvx::contract_coord((int)(tx * 16 + xx), So);
-                    const double v = hvx::contract_coord((int)(ty * 16 + yy), So);
-                    const double r = 1.0 / std::sqrt(1.0 + u * u + v * v);
-                    const double n[3] = {u * r, v * r, r};
-                    double e1[3], e2[3];
-                    orthonormal(n, e1, e2);
-                    for (int j = 0; j < 64; ++j) {
-                        const double a = 2.0 * hvx::kContractPi * j / 64.0, ca = std::cos(a), sa = std::sin(a);
-                        double l[3];
-                        for (int q = 0; q < 3; ++q) l[q] = ct * n[q] + st * (ca * e1[q] + sa * e2[q]);
-                        const double pu = l[0] / l[2], pv = l[1] / l[2];
-                        const double px = ((pu + 1.0) * Si - 1.0) / 2.0, py = ((pv + 1.0) * Si - 1.0) / 2.0;
-                        xmin = std::min(xmin, px);
-                        xmax = std::max(xmax, px);
-                        ymin = std::min(ymin, py);
-                        ymax = std::max(ymax, py);
-                    }
-                }
-            const int x_lo = (int)std::floor(xmin) - 1, x_hi = (int)std::ceil(xmax) + 1;
-            const int y_lo = (int)std::floor(ymin) - 1, y_hi = (int)std::ceil(ymax) + 1;
-            NearTile& T = tiles[ty * te + tx];
-            T.x0 = x_lo >= 0 ? (x_lo / 8) * 8 : -(((-x_lo) + 7) / 8) * 8;
-            T.w = (uint32_t)(((x_hi + 1 - T.x0) + 31) / 32 * 32);
-            T.y0 = y_lo;
-            T.h = (uint32_t)(y_hi + 1 - y_lo);
-            T.woff = woff;
-            woff += (uint64_t)16 * T.h * (T.w / 32) * 64;
-            B = std::max({B, -T.x0, T.x0 + (int)T.w - (int)Si, -T.y0, T.y0 + (int)T.h - (int)Si});
+// Rows of an So x So face: the octant 0 <= x <= y < So / 2 (the one texel of a
+// 1 x 1 face) along a Morton curve, so that runs of rows are compact patches.
+std::vector<Row> octant_rows(uint32_t So, uint16_t job) {
+    const uint32_t h = std::max(So / 2, 1u);
+    std::vector<Row> rows;
+    rows.reserve((size_t)h * (h + 1) / 2);
+    for (uint64_t m = 0; m < (uint64_t)h * h; ++m) {  // h is a power of two
+        uint32_t x = 0, y = 0;
+        for (uint32_t b = 0; (1u << b) < h; ++b) {
+            x |= (uint32_t)((m >> (2 * b)) & 1) << b;
+            y |= (uint32_t)((m >> (2 * b + 1)) & 1) << b;
         }
-    *B_out = (uint32_t)((B + 7) / 8 * 8);
-    return tiles;
+        if (x <= y) rows.push_back(Row{(uint16_t)x, (uint16_t)y, job, 0});
+    }
+    return rows;
 }
 
-struct DenseMat {
-    DenseGeom G;
-    int stage;  // index into the staged dense levels
-    bool split = false;  // split-BF16 weights (hi, then lo after rt * ks * 64 units)
-    uint32_t splitk;
-    half8* W = nullptr;
-    float* rowscale = nullptr;
-};
-
-struct StageDense {
-    uint32_t Sin, level;
-    bool split = false;  // BF16 hi + lo (lo after K / 8 * 32 units)
-    int32_t* perm = nullptr;
-    half8* R = nullptr;  // in the per-call scratch, at off
-    size_t off = 0;
-};
-
-struct StagePad {
-    uint32_t Si, level, B, Pw;
-    half8* P = nullptr;  // in the per-call scratch, at off
-    size_t off = 0;
-};
+// Texels by which the angular caps of radius t1 around the output texels of a
+// face reach past the near level's face on its plane, and four more, rounded
+// up to whole units. By symmetry the octant's rows reach the furthest, and of
+// those the ones along the face's edge (y = 0).
+uint32_t plane_border(uint32_t So, uint32_t Si, double t1) {
+    const double ct = std::cos(t1), st = std::sin(t1);
+    double reach = 1.0;
+    for (uint32_t x = 0; x < std::max(So / 2, 1u); ++x) {
+        const double u = hvx::contract_coord((int)x, So), v = hvx::contract_coord(0, So);
+        const double r = 1.0 / std::sqrt(1.0 + u * u + v * v), n[3] = {u * r, v * r, r};
+        // e1, e2: any two directions orthogonal to n and to each other
+        const double a[3] = {std::fabs(n[0]) < 0.9 ? 1.0 : 0.0, std::fabs(n[0]) < 0.9 ? 0.0 : 1.0, 0.0};
+        double e1[3] = {a[1] * n[2] - a[2] * n[1], a[2] * n[0] - a[0] * n[2], a[0] * n[1] - a[1] * n[0]};
+        const double l = std::sqrt(e1[0] * e1[0] + e1[1] * e1[1] + e1[2] * e1[2]);
+        for (double& e : e1) e /= l;
+        const double e2[3] = {n[1] * e1[2] - n[2] * e1[1], n[2] * e1[0] - n[0] * e1[2], n[0] * e1[1] - n[1] * e1[0]};
+        for (int j = 0; j < 256; ++j) {
+            const double w = 2.0 * hvx::kContractPi * j / 256.0, ca = std::cos(w), sa = std::sin(w);
+            double p[3];
+            for (int q = 0; q < 3; ++q) p[q] = ct * n[q] + st * (ca * e1[q] + sa * e2[q]);
+            reach = std::max({reach, std::fabs(p[0] / p[2]), std::fabs(p[1] / p[2])});
+        }
+    }
+    const uint32_t B = (uint32_t)std::ceil((reach - 1.0) * 0.5 * Si) + 4;
+    return (B + 7) / 8 * 8;
+}
 
 // Reserves `bytes` (256-byte aligned) at the end of a scratch layout.
 size_t scratch_take(size_t* total, size_t bytes) {
@@ -2020,21 +1337,22 @@ size_t scratch_take(size_t* total, size_t bytes) {
     return at;
 }
 
+// A source while the plan is built: its geometry, the jobs that sum it, and
+// the staged units (those any row has weight in).
+struct SourcePlan {
+    Source G{};
+    uint32_t level = 0;  // of the input chain
+    bool split = false;
+    uint32_t raw = 0;    // units of the whole level or plane
+    uint32_t row0 = 0, rows = 0, block0 = 0, nblocks = 0;
+    std::vector<uint32_t> units, need;  // need (planes): the texels the staged units' images read
+    size_t units_off = 0, need_off = 0;  // in the plan's tables
+    size_t r_off = 0, t_off = 0;  // staged operand in the per-call scratch, plane texels in its last part
+};
+
 struct MipPlan {
     ContractLevel L{};
-    int dense = -1;  // FULL: the mip's matrix; SPLIT: the far matrix
-    int pad = -1;    // SPLIT: staged padded planes
-    NearGeom NG{};
-    std::vector<NearTile> tiles;
-    NearTile* d_tiles = nullptr;
-    half8* Wn = nullptr;
-    float* rowscale_n = nullptr;
-    float* invZ = nullptr;
-    float4* far_map = nullptr;  // in the per-call scratch, at far_off
-    size_t far_off = 0;
-    float4* zfar_map = nullptr;
     uint64_t weight_bytes = 0;
-    uint64_t w_lo = 0;  // split BF16: offset of the lo weights in Wn (16-byte units)
 };
 
 }  // namespace
@@ -2044,25 +1362,26 @@ struct hvx_contract_plan {
     int type = 0, precision = 0;
     uint32_t S = 0, So = 0, mips = 0;
     std::vector<MipPlan> mp;
-    std::vector<DenseMat> dm;
-    std::vector<StageDense> sd;
-    std::vector<StagePad> sp;
     // Per-call scratch, carved from one block of scratch_bytes: far maps,
     // staged levels and planes, face maxima, scales, K-slice partial sums.
-    // Multi-probe calls use mcap further copies of the block (mscratch).
+    // Multi-probe calls of up to mcap probes use mcopies further copies of the
+    // block (mscratch), that many probes at a time.
     char* scratch = nullptr;
     size_t scratch_bytes = 0;
     char* mscratch = nullptr;
-    uint32_t mcap = 0;
+    uint32_t mcap = 0, mcopies = 0;
     float* fmax = nullptr;  // per-face partial maxima [6][kFaceMaxBlocks]
     float* sc = nullptr;
-    float* part = nullptr;   // every dense job's K-slice partial sums
     uint32_t min_level = 0;  // deepest input chain level read
     uint32_t scale_level = ~0u;  // finest staged level: its maxima bound every staged value
-    uint32_t delta_mip = ~0u;
     StageTable stage{};
-    DenseTable dense{};
-    NearTable near{};
+    MapTable maps{};
+    GemmArgs gemm{};
+    uint32_t items = 0;
+    uint32_t dense_rows = 0, near_rows = 0;  // rows [0, dense_rows) whole and far, then the near ones
+    const Job* d_jobs = nullptr;
+    const Row* d_rows = nullptr;
+    const float *rowscale = nullptr, *invZ = nullptr;
     // bright-texel split (hvx_ibl_contract_plan_set_hot): off while hot_k == 0
     uint32_t hot_k = 0;
     float* hot_chain = nullptr;  // the clamped chain, min_level + 1 levels
@@ -2096,89 +1415,379 @@ int pfail(hvx_ctx* ctx, int st, const char* fmt, ...) {
     return st;
 }
 
-int stage_dense_index(hvx_contract_plan* P, uint32_t Sin, bool split) {
-    for (size_t i = 0; i < P->sd.size(); ++i)
-        if (P->sd[i].Sin == Sin && P->sd[i].split == split) return (int)i;
-    StageDense s;
-    s.Sin = Sin;
+// Memory used while a plan is built, released with it.
+struct Scratch {
+    void* p = nullptr;
+    ~Scratch() {
+        if (p) (void)hipFree(p);
+    }
+    template <class T> hipError_t get(T** q, size_t n) {
+        const hipError_t e = hipMalloc(&p, std::max<size_t>(n, 1) * sizeof(T));
+        *q = static_cast<T*>(p);
+        return e;
+    }
+};
+
+// A plan's tables, put together on the host and uploaded as one allocation:
+// a call on a new plan then misses in few pages.
+struct Tables {
+    std::vector<char> bytes;
+    template <class T> size_t add(const T* v, size_t n) {
+        const size_t at = (bytes.size() + 255) / 256 * 256;
+        bytes.resize(at + n * sizeof(T));
+        if (v && n) std::memcpy(bytes.data() + at, v, n * sizeof(T));
+        return at;
+    }
+    template <class T> size_t add(const std::vector<T>& v) { return add(v.data(), v.size()); }
+};
+
+// Index of the source (added if new) for a level of face S.
+uint32_t source_index(std::vector<SourcePlan>& src, uint32_t face, uint32_t S, bool split) {
+    for (size_t i = 0; i < src.size(); ++i)
+        if (!src[i].G.pad && src[i].G.S == S && src[i].split == split) return (uint32_t)i;
+    SourcePlan s;
+    s.G.S = S;
     s.split = split;
-    s.level = ilog2(P->S / Sin);
-    P->sd.push_back(s);
-    return (int)P->sd.size() - 1;
+    s.level = ilog2(face / S);
+    s.raw = 6 * S * S / 8;
+    src.push_back(s);
+    return (uint32_t)src.size() - 1;
 }
 
-hipError_t build_dense(hvx_contract_plan* P, DenseMat& D, int num_cus, float4* zmap) {
-    const DenseGeom& G = D.G;
+// Rows, blocks, unit lists, weights, slices and launch tables of a plan whose
+// levels are chosen. Sources are ordered levels first, planes after, so that
+// the far normalisers exist when the near rows need them.
+hipError_t build_plan(hvx_contract_plan* P, int ctype, bool split) {
     hipError_t e;
-    double *Z = nullptr, *wm = nullptr;
-    if ((e = hipMalloc(&Z, G.rows * sizeof(double))) != hipSuccess) return e;
-    if ((e = hipMalloc(&wm, G.rows * sizeof(double))) != hipSuccess) {
-        (void)hipFree(Z);
+    std::vector<Job> jobs;
+    std::vector<uint32_t> job_src, job_mip;
+    std::vector<SourcePlan> src;
+    size_t sbytes = 0, tbytes = 0;  // the scratch and, in it, the planes' texels
+    std::vector<std::pair<uint32_t, size_t>> map_at;  // (far job, offset of its map in the scratch)
+    uint32_t delta_mip = ~0u;
+    size_t ztotal = 0;  // far normaliser maps, needed only here
+    for (uint32_t m = 0; m < P->mips; ++m) {
+        const ContractLevel& L = P->mp[m].L;
+        if (L.kind == hvx::CONTRACT_DELTA) {
+            delta_mip = m;
+            continue;
+        }
+        Job J{};
+        J.type = ctype;
+        J.alpha2 = L.alpha2;
+        J.t0 = L.t0;
+        J.t1 = L.t1;
+        J.out_off = hvx::cube_level_offset_floats(P->So, m) / 4;
+        if (L.kind == hvx::CONTRACT_FULL) {
+            J.piece = PIECE_WHOLE;
+            J.So = L.So;
+            job_src.push_back(source_index(src, P->S, L.Si, false));
+        } else {
+            J.piece = PIECE_FAR;
+            J.So = L.Sf;
+            job_src.push_back(source_index(src, P->S, L.Sf, split));  // low-roughness mips: near and far
+            map_at.emplace_back((uint32_t)jobs.size(), scratch_take(&sbytes, 6 * (size_t)L.Sf * L.Sf * sizeof(float4)));
+            J.zmap = (float4*)(ztotal * sizeof(float4));  // offset, until the maps are allocated
+            ztotal += 6 * (size_t)L.Sf * L.Sf;
+        }
+        jobs.push_back(J);
+        job_mip.push_back(m);
+    }
+    const uint32_t far_jobs = (uint32_t)map_at.size();
+    for (uint32_t k = 0; k < far_jobs; ++k) {  // the near job of each far job, with a plane of its own
+        const uint32_t m = job_mip[map_at[k].first];
+        const ContractLevel& L = P->mp[m].L;
+        Job J = jobs[map_at[k].first];
+        J.piece = PIECE_NEAR;
+        J.So = L.So;
+        J.Sf = L.Sf;
+        SourcePlan s;
+        s.G.pad = 1;
+        s.G.S = L.Si;
+        s.G.B = plane_border(L.So, L.Si, L.t1);
+        s.G.Pw8 = (L.Si + 2 * s.G.B) / 8;
+        s.split = split;
+        s.level = ilog2(P->S / L.Si);
+        s.raw = (L.Si + 2 * s.G.B) * s.G.Pw8;
+        job_src.push_back((uint32_t)src.size());
+        src.push_back(s);
+        map_at.emplace_back((uint32_t)jobs.size(), map_at[k].second);
+        jobs.push_back(J);
+        job_mip.push_back(m);
+    }
+    // rows and blocks by source
+    std::vector<Row> rows;
+    std::vector<Block> blocks;
+    for (uint32_t s = 0; s < src.size(); ++s) {
+        SourcePlan& S = src[s];
+        S.row0 = (uint32_t)rows.size();
+        S.block0 = (uint32_t)blocks.size();
+        for (uint32_t j = 0; j < jobs.size(); ++j)
+            if (job_src[j] == s) {
+                const std::vector<Row> r = octant_rows(jobs[j].So, (uint16_t)j);
+                rows.insert(rows.end(), r.begin(), r.end());
+            }
+        S.rows = (uint32_t)rows.size() - S.row0;
+        for (uint32_t r = 0; r < S.rows; r += kBlockRows) {
+            Block B{};
+            B.row0 = S.row0 + r;
+            B.nrows = std::min(kBlockRows, S.rows - r);
+            B.nrt = (B.nrows + 15) / 16;
+            B.src = s;
+            B.split = S.split;
+            for (uint32_t k = 0; k < B.nrows; ++k) rows[B.row0 + k].block = (uint16_t)blocks.size();
+            blocks.push_back(B);
+        }
+        S.nblocks = (uint32_t)blocks.size() - S.block0;
+        (S.G.pad ? P->near_rows : P->dense_rows) += S.rows;
+        P->min_level = std::max(P->min_level, S.level);
+        P->scale_level = std::min(P->scale_level, S.level);
+    }
+    Scratch zmaps;
+    float4* d_zmaps = nullptr;
+    if ((e = zmaps.get(&d_zmaps, ztotal)) != hipSuccess) return e;
+    for (Job& J : jobs)
+        if (J.piece != PIECE_WHOLE) J.zmap = d_zmaps + (size_t)J.zmap / sizeof(float4);
+    // unit lists: the blocks' units with weight, as indices into the source's staged units
+    std::vector<uint32_t> ulist;
+    Tables first;
+    const size_t fj = first.add(jobs), fr = first.add(rows), fb = first.add(blocks);
+    Scratch first_mem;
+    char* d_first = nullptr;
+    if ((e = first_mem.get(&d_first, first.bytes.size())) != hipSuccess ||
+        (!first.bytes.empty() &&
+         (e = hipMemcpy(d_first, first.bytes.data(), first.bytes.size(), hipMemcpyHostToDevice)) != hipSuccess))
         return e;
+    for (SourcePlan& S : src) {
+        Scratch mem;
+        uint8_t* d_flags = nullptr;
+        const size_t nf = (size_t)S.nblocks * S.raw;
+        std::vector<uint8_t> flags(nf);
+        if ((e = mem.get(&d_flags, nf)) != hipSuccess) return e;
+        hipLaunchKernelGGL(unit_flag_kernel, dim3((S.raw + 255) / 256, S.nblocks), dim3(256), 0, nullptr, S.G,
+                           (const Job*)(d_first + fj), (const Row*)(d_first + fr), (const Block*)(d_first + fb),
+                           S.block0, S.raw, d_flags);
+        if ((e = hipGetLastError()) != hipSuccess ||
+            (e = hipMemcpy(flags.data(), d_flags, nf, hipMemcpyDeviceToHost)) != hipSuccess)
+            return e;
+        std::vector<uint8_t> any(S.raw, 0);
+        std::vector<uint32_t> index(S.raw, ~0u);
+        for (uint32_t b = 0; b < S.nblocks; ++b)
+            for (uint32_t u = 0; u < S.raw; ++u) any[u] |= flags[(size_t)b * S.raw + u];
+        for (uint32_t u = 0; u < S.raw; ++u)
+            if (any[u]) S.units.push_back(u);
+        // stacked in y, eight rows at a time, so that staging works on square patches
+        const uint32_t w = S.G.pad ? S.G.Pw8 : std::max(S.G.S / 8, 1u);
+        auto key = [&](uint32_t u) { return ((uint64_t)(u / w / 8) * w + u % w) * 8 + u / w % 8; };
+        std::sort(S.units.begin(), S.units.end(), [&](uint32_t a, uint32_t b) { return key(a) < key(b); });
+        for (uint32_t k = 0; k < S.units.size(); ++k) index[S.units[k]] = k;
+        for (uint32_t b = 0; b < S.nblocks; ++b) {
+            Block& B = blocks[S.block0 + b];
+            B.unit0 = (uint32_t)ulist.size();
+            for (uint32_t u : S.units)
+                if (flags[(size_t)b * S.raw + u]) ulist.push_back(index[u]);
+            B.nunits = (uint32_t)ulist.size() - B.unit0;
+            B.nsteps = (B.nunits + 3) / 4;
+        }
+        if (S.G.pad) {  // the texels that the staged units' eight images read
+            const uint32_t Pw = 8 * S.G.Pw8;
+            std::vector<uint8_t> seen((size_t)Pw * Pw, 0);
+            for (uint32_t u : S.units)
+                for (uint32_t q = 0; q < 8; ++q) {
+                    const uint32_t x = (u % S.G.Pw8) * 8 + q, y = u / S.G.Pw8, xr = Pw - 1 - x, yr = Pw - 1 - y;
+                    for (const auto& p : {std::pair{x, y}, {xr, y}, {x, yr}, {xr, yr}}) {
+                        seen[(size_t)p.second * Pw + p.first] = 1;
+                        seen[(size_t)p.first * Pw + p.second] = 1;
+                    }
+                }
+            // texels of the face itself, then those sampled inside another
+            // face, then those whose taps meet an edge: the last kind takes
+            // several times the instructions and would hold up most waves
+            // (a row of the plane crosses two edges)
+            auto kind = [&](uint32_t p) {
+                const int s1 = (int)S.G.S, a = std::abs(2 * ((int)(p % Pw) - (int)S.G.B) + 1 - s1),
+                          b = std::abs(2 * ((int)(p / Pw) - (int)S.G.B) + 1 - s1), m = std::max(a, b);
+                if (m < s1) return 0;
+                // the sample's coordinates off the other face's centre: S and min(a, b), over m
+                const double hi = 0.5 * s1 * (1.0 + (double)std::max(s1, std::min(a, b)) / m) - 0.5;
+                return hi + 1.0 < s1 - 1e-3 ? 1 : 2;
+            };
+            for (int k = 0; k < 3; ++k)
+                for (uint32_t p = 0; p < Pw * Pw; ++p)
+                    if (seen[p] && kind(p) == k) S.need.push_back(p);
+            S.t_off = scratch_take(&tbytes, 6 * (size_t)Pw * Pw * (S.split ? 16 : 8));
+        }
+        S.r_off = scratch_take(&sbytes, S.units.size() * kCols * sizeof(half8) * (S.split ? 2 : 1));
     }
-    const uint64_t n = (uint64_t)G.rt * G.ks * 64;
-    if ((e = P->alloc(&D.W, D.split ? 2 * n : n)) == hipSuccess && (e = P->alloc(&D.rowscale, G.rows)) == hipSuccess) {
-        hipLaunchKernelGGL(dense_row_kernel, dim3(G.rows), dim3(256), 0, nullptr, G, Z, wm);
-        if (D.split)
-            hipLaunchKernelGGL(dense_fill_kernel<true>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, nullptr, G,
-                               wm, D.W, n);
-        else
-            hipLaunchKernelGGL(dense_fill_kernel<false>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, nullptr, G,
-                               wm, D.W, (uint64_t)0);
-        hipLaunchKernelGGL(dense_scale_kernel, dim3((G.rows + 255) / 256), dim3(256), 0, nullptr, G.rows, Z, wm,
-                           G.piece == PIECE_FAR ? 1 : 0, D.rowscale, zmap);
-        e = hipDeviceSynchronize();
+    // K slices: at most two workgroups per CU (what fits: one round, without a
+    // tail) of kGoodSlice to kMaxSlice steps, a split step counting as two;
+    // plans too small to fill the chip that way have shorter ones, for the
+    // latency of a single probe (irradiance 32^2: 19.6 us against 25.4 with slices of 32). A
+    // slice costs its 74 KB of partial sums, written and read once: 24 probes
+    // 256^2 -> 128^2 x 8 took 384 us with slices of at least 16 steps, 361 us
+    // with 24, 349 us with 32, 347 us with 40 (one probe 512^2 -> 256^2 x 9 in
+    // split BF16 100 us up to 32, 103 us with 40); the 512^2 x 10 chain 139 us
+    // with 541 slices, in two rounds, 129 us with 440 in one.
+    uint64_t wunits = 0;
+    const uint32_t slots = 2u * (uint32_t)std::max(P->ctx->num_cus, 1);
+    auto slices = [&](const Block& B, uint32_t len) {
+        const uint32_t groups = (B.nsteps + kGroup - 1) / kGroup, per = (B.split ? len / 2 : len) / kGroup;
+        return (groups + per - 1) / per;
+    };
+    uint32_t len = kMinSlice;
+    for (; len < kMaxSlice; len += 2 * kGroup) {
+        uint32_t n = 0;
+        for (const Block& B : blocks) n += slices(B, len);
+        if (n <= (len < kGoodSlice ? slots / 8 : slots)) break;
     }
-    (void)hipFree(Z);
-    (void)hipFree(wm);
-    // K slices: enough waves to keep the weight stream in flight
-    const uint32_t pairs = (G.rt + 1) / 2;
-    const uint32_t want = (uint32_t)std::max(1, num_cus * 8) / std::max(pairs, 1u);
-    D.splitk = std::max(1u, std::min(want, std::max(1u, G.ks / 16)));
-    return e;
+    std::vector<Item> items;
+    for (uint32_t b = 0; b < blocks.size(); ++b) {
+        Block& B = blocks[b];
+        const uint64_t n = (uint64_t)B.nsteps * B.nrt * 64;
+        B.woff = wunits;
+        B.w_lo = B.split ? n : 0;
+        wunits += B.split ? 2 * n : n;
+        const uint32_t groups = (B.nsteps + kGroup - 1) / kGroup;
+        B.nslices = slices(B, len);
+        B.item0 = (uint32_t)items.size();
+        for (uint32_t s = 0; s < B.nslices; ++s) {
+            const uint32_t s0 = s * groups / B.nslices * kGroup, s1 = std::min((s + 1) * groups / B.nslices * kGroup, B.nsteps);
+            items.push_back(Item{b, s0, s1 - s0, (uint32_t)items.size()});
+        }
+        for (uint32_t r = 0; r < B.nrows; ++r)
+            P->mp[job_mip[rows[B.row0 + r].job]].weight_bytes += (uint64_t)B.nsteps * 32 * 2 * (B.split ? 2 : 1);
+    }
+    P->items = (uint32_t)items.size();
+    // a level's blocks sum much the same units: slices at the same place of
+    // their lists run side by side. Planes stay block by block: neighbouring
+    // blocks have neighbouring windows.
+    std::stable_sort(items.begin(), items.end(), [&](const Item& a, const Item& b) {
+        const Block &A = blocks[a.block], &B = blocks[b.block];
+        if (A.src != B.src) return A.src < B.src;
+        return !src[A.src].G.pad && a.s0 < b.s0;
+    });
+    // per-call scratch
+    const size_t fmax_off = scratch_take(&sbytes, 6 * kFaceMaxBlocks * sizeof(float));
+    const size_t sc_off = scratch_take(&sbytes, 8 * sizeof(float));
+    // the planes' texels are read for the last time before the first partial sum is written
+    const size_t part_off = scratch_take(&sbytes, std::max((size_t)P->items * kBlockRows * kCols * sizeof(float), tbytes));
+    P->scratch_bytes = (sbytes + 255) & ~(size_t)255;
+    if ((e = P->alloc(&P->scratch, P->scratch_bytes)) != hipSuccess) return e;
+    P->fmax = reinterpret_cast<float*>(P->scratch + fmax_off);
+    P->sc = reinterpret_cast<float*>(P->scratch + sc_off);
+    for (const auto& [j, off] : map_at) jobs[j].map = reinterpret_cast<float4*>(P->scratch + off);
+    // pages touched here are not first touched by a call
+    if ((e = hipMemset(P->scratch, 0, P->scratch_bytes)) != hipSuccess) return e;
+    Tables tab;
+    const size_t tj = tab.add(jobs), tr = tab.add(rows), tb = tab.add(blocks), ti = tab.add(items), tu = tab.add(ulist);
+    for (SourcePlan& S : src) {
+        S.units_off = tab.add(S.units);
+        S.need_off = tab.add(S.need);
+    }
+    const size_t tm = tab.add(source_table()), ts = tab.add<float>(nullptr, rows.size()),
+                 tz = tab.add<float>(nullptr, rows.size());
+    char* d_tab = nullptr;
+    half8* W = nullptr;
+    if ((e = P->alloc(&d_tab, tab.bytes.size())) != hipSuccess || (e = P->alloc(&W, wunits)) != hipSuccess ||
+        (e = hipMemcpy(d_tab, tab.bytes.data(), tab.bytes.size(), hipMemcpyHostToDevice)) != hipSuccess)
+        return e;
+    const Job* d_jobs = reinterpret_cast<const Job*>(d_tab + tj);
+    const Row* d_rows = reinterpret_cast<const Row*>(d_tab + tr);
+    const Block* d_blocks = reinterpret_cast<const Block*>(d_tab + tb);
+    const uint32_t* d_ulist = reinterpret_cast<const uint32_t*>(d_tab + tu);
+    float *rowscale = reinterpret_cast<float*>(d_tab + ts), *invZ = reinterpret_cast<float*>(d_tab + tz);
+    auto d_units = [&](const SourcePlan& S) { return reinterpret_cast<const uint32_t*>(d_tab + S.units_off); };
+    // weights
+    if (!rows.empty()) {
+        Scratch zmem, wmem;
+        double *Z = nullptr, *wm = nullptr;
+        if ((e = zmem.get(&Z, rows.size())) != hipSuccess || (e = wmem.get(&wm, rows.size())) != hipSuccess) return e;
+        for (const SourcePlan& S : src) {
+            hipLaunchKernelGGL(row_sum_kernel, dim3(S.rows), dim3(256), 0, nullptr, S.G, d_jobs, d_rows, d_blocks,
+                               d_ulist, d_units(S), S.row0, Z, wm);
+            uint32_t most = 0;
+            for (uint32_t b = 0; b < S.nblocks; ++b) {
+                const Block& B = blocks[S.block0 + b];
+                most = std::max(most, (B.nsteps * B.nrt * 64 + 255) / 256);
+            }
+            const dim3 grid(std::min(most, 4096u), S.nblocks);
+            if (S.split)
+                hipLaunchKernelGGL(weight_fill_kernel<true>, grid, dim3(256), 0, nullptr, S.G, d_jobs, d_rows,
+                                   d_blocks, S.block0, d_ulist, d_units(S), wm, W);
+            else
+                hipLaunchKernelGGL(weight_fill_kernel<false>, grid, dim3(256), 0, nullptr, S.G, d_jobs, d_rows,
+                                   d_blocks, S.block0, d_ulist, d_units(S), wm, W);
+            hipLaunchKernelGGL(far_norm_kernel, dim3((S.rows * kImages + 255) / 256), dim3(256), 0, nullptr, d_jobs,
+                               d_rows, S.row0, S.rows, Z);
+        }
+        hipLaunchKernelGGL(row_scale_kernel, dim3((uint32_t)(rows.size() + 255) / 256), dim3(256), 0, nullptr, d_jobs,
+                           d_rows, (uint32_t)rows.size(), Z, wm, rowscale, invZ);
+        if ((e = hipGetLastError()) != hipSuccess || (e = hipDeviceSynchronize()) != hipSuccess) return e;
+    }
+    P->d_jobs = d_jobs;
+    P->d_rows = d_rows;
+    P->rowscale = rowscale;
+    P->invZ = invZ;
+    // launch tables
+    GemmArgs& A = P->gemm;
+    A.W = W;
+    A.blocks = d_blocks;
+    A.items = reinterpret_cast<const Item*>(d_tab + ti);
+    A.ulist = d_ulist;
+    A.nitems = P->items;
+    A.part = reinterpret_cast<float*>(P->scratch + part_off);
+    StageTable& ST = P->stage;
+    MapTable& MT = P->maps;
+    auto stage_item = [&](StageItem I, uint32_t workgroups) {
+        I.block_begin = ST.blocks;
+        ST.blocks += workgroups;
+        ST.it[ST.n++] = I;
+    };
+    ST.map = reinterpret_cast<const uint32_t*>(d_tab + tm);
+    for (uint32_t s = 0; s < src.size(); ++s) {
+        const SourcePlan& S = src[s];
+        const uint32_t nu = (uint32_t)S.units.size();
+        const uint64_t lo = S.split ? (uint64_t)nu * kCols : 0;
+        const uint32_t ut = S.split ? tile_units<true>() : tile_units<false>(), tiles = (nu + ut - 1) / ut;
+        half8* R = reinterpret_cast<half8*>(P->scratch + S.r_off);
+        A.R[s] = R;
+        A.r_lo[s] = lo;
+        StageItem I{};
+        I.split = S.split;
+        I.S = S.G.S;
+        I.level_off = hvx::cube_level_offset_floats(P->S, S.level) / 4;
+        if (S.G.pad) {
+            I.kind = STAGE_PLANE;
+            I.B = S.G.B;
+            I.Pw = 8 * S.G.Pw8;
+            I.n = (uint32_t)S.need.size();
+            I.list = reinterpret_cast<const uint32_t*>(d_tab + S.need_off);
+            I.dst = reinterpret_cast<half8*>(P->scratch + part_off + S.t_off);
+            stage_item(I, (6 * I.n + 255) / 256);
+            MT.it[MT.n++] = MapItem{I.Pw, nu, MT.blocks, d_units(S), I.dst, R, lo};
+            MT.blocks += tiles;
+        } else {
+            I.kind = STAGE_DENSE;
+            I.n = nu;
+            I.list = d_units(S);
+            I.dst = R;
+            I.lo_off = lo;
+            stage_item(I, tiles);
+        }
+    }
+    if (delta_mip != ~0u) {
+        StageItem I{};
+        I.kind = STAGE_DELTA;
+        I.S = P->mp[delta_mip].L.So;
+        I.level_off = hvx::cube_level_offset_floats(P->So, delta_mip) / 4;
+        stage_item(I, (6 * I.S * I.S + 255) / 256);
+    }
+    return hipSuccess;
 }
 
-hipError_t build_near(hvx_contract_plan* P, MipPlan& M, bool split) {
-    hipError_t e;
-    const uint32_t So = M.L.So, rows = So * So;
-    uint64_t halfs8 = 0;
-    for (const NearTile& T : M.tiles) halfs8 += (uint64_t)16 * T.h * (T.w / 32) * 64;
-    M.w_lo = split ? halfs8 : 0;
-    double *Z = nullptr, *wm = nullptr;
-    if ((e = hipMalloc(&Z, rows * sizeof(double))) != hipSuccess) return e;
-    if ((e = hipMalloc(&wm, rows * sizeof(double))) != hipSuccess) {
-        (void)hipFree(Z);
-        return e;
-    }
-    if ((e = P->alloc(&M.d_tiles, M.tiles.size())) == hipSuccess &&
-        (e = hipMemcpy(M.d_tiles, M.tiles.data(), M.tiles.size() * sizeof(NearTile), hipMemcpyHostToDevice)) ==
-            hipSuccess &&
-        (e = P->alloc(&M.Wn, split ? 2 * halfs8 : halfs8)) == hipSuccess &&
-        (e = P->alloc(&M.rowscale_n, rows)) == hipSuccess && (e = P->alloc(&M.invZ, rows)) == hipSuccess) {
-        hipLaunchKernelGGL(near_row_kernel, dim3(rows), dim3(256), 0, nullptr, M.NG, M.d_tiles, Z, wm);
-        if (split)
-            hipLaunchKernelGGL(near_fill_kernel<true>, dim3((unsigned)M.tiles.size() * 16), dim3(256), 0, nullptr,
-                               M.NG, M.d_tiles, wm, M.Wn, halfs8);
-        else
-            hipLaunchKernelGGL(near_fill_kernel<false>, dim3((unsigned)M.tiles.size() * 16), dim3(256), 0, nullptr,
-                               M.NG, M.d_tiles, wm, M.Wn, (uint64_t)0);
-        hipLaunchKernelGGL(near_scale_kernel, dim3((rows + 255) / 256), dim3(256), 0, nullptr, M.NG, M.L.Sf, Z, wm,
-                           M.zfar_map, M.rowscale_n, M.invZ);
-        e = hipDeviceSynchronize();
-    }
-    M.weight_bytes += halfs8 * 16 * (split ? 2 : 1);
-    (void)hipFree(Z);
-    (void)hipFree(wm);
-    return e;
-}
-
-}  // namespace
-
-namespace {
-
-// The eight launches of a filter call over n probes (grid dimension y, z for
-// the face maxima: probe). delta_chain (single probe, nullable): the chain the
-// delta mip samples instead of the probe's chain.
+// The launches of a filter call over n probes (grid dimension y, z for the
+// face maxima, interleaved for the GEMM: probe). delta_chain (single probe,
+// nullable): the chain the delta mip samples instead of the probe's chain.
 int launch_call(hvx_contract_plan* P, const Probes& Q, uint32_t n, uint32_t chain_levels, hipStream_t s,
                 const char* what, const float4* delta_chain = nullptr) {
     hvx_ctx* ctx = P->ctx;
@@ -2190,72 +1799,42 @@ int launch_call(hvx_contract_plan* P, const Probes& Q, uint32_t n, uint32_t chai
         return pfail(ctx, HVX_ERR_HIP, "cannot bind device %d", ctx->device);
     // exponent scales from the finest staged level: coarser levels are its box
     // means and padded texels its bilinear samples, so its maxima bound them
-    if (P->stage.total) {
+    uint32_t nb = 0;
+    if (P->items) {
         const uint32_t Sl = std::max(P->S >> P->scale_level, 1u), S2 = Sl * Sl;
-        const uint32_t nb = std::min(kFaceMaxBlocks, (S2 + 255) / 256);
+        nb = std::min(kFaceMaxBlocks, (S2 + 255) / 256);
         hipLaunchKernelGGL(facemax_kernel, dim3(nb, 6, n), dim3(256), 0, s, Q,
                            hvx::cube_level_offset_floats(P->S, P->scale_level) / 4, Sl, P->fmax);
-        hipLaunchKernelGGL(scales_kernel, dim3(n), dim3(64), 0, s, Q, P->fmax, nb, P->sc);
-        hipLaunchKernelGGL(stage_all_kernel, dim3((P->stage.total + 255) / 256, n), dim3(256), 0, s, Q, P->stage,
-                           P->sc);
     }
-    // GEMMs with several probes: groups of kProbeGroup probes per wave share
-    // each weight fragment, and the group index is the fastest grid dimension,
-    // so groups reading one weight block run together and share it in the caches
-    Probes G = Q;
-    // single-probe calls stage the B operand in LDS several K steps per
-    // barrier (near_gemm_lds_kernel, dense_gemm_lds_kernel<1, ...>): with one
-    // barrier per step it paid only when several probes share it (512^2 x 10
-    // GGX chain: FP16 near GEMM 203 us unstaged, 246 us staged per step)
-    const bool grouped = n > 1;
-    const uint32_t dense_wgs = (P->dense.waves + 3) / 4,
-                   near_wgs = grouped ? P->near.tiles * kNearParts : near_single_wgs(P->near.tiles);
-    const uint32_t groups = grouped ? (n + kProbeGroup - 1) / kProbeGroup : 1;
-    G.probe_fast = grouped && std::max(dense_wgs, near_wgs) <= 65535u;
-    if (P->dense.n) {
-        const dim3 grid = G.probe_fast ? dim3(groups, dense_wgs) : dim3(dense_wgs, groups);
-        if (grouped && kDenseLdsGroupMulti > 0)
-            hipLaunchKernelGGL((dense_gemm_lds_kernel<kProbeGroup, (kDenseLdsGroupMulti > 0 ? kDenseLdsGroupMulti : 4)>),
-                               grid, dim3(256), 0, s, G, P->dense);
-        else if (grouped)
-            hipLaunchKernelGGL(dense_gemm_staged_kernel<kProbeGroup>, grid, dim3(256), 0, s, G, P->dense);
-        else if (kDenseLdsGroup > 0)
-            hipLaunchKernelGGL((dense_gemm_lds_kernel<1, (kDenseLdsGroup > 0 ? kDenseLdsGroup : 4)>), grid, dim3(256), 0,
-                               s, G, P->dense);
-        else
-            hipLaunchKernelGGL(dense_gemm_kernel<1>, grid, dim3(256), 0, s, G, P->dense);
-        hipLaunchKernelGGL(dense_epilogue_kernel, dim3((P->dense.epi + 255) / 256, n), dim3(256), 0, s, Q, P->dense,
-                           P->sc);
+    if (P->stage.blocks)
+        hipLaunchKernelGGL(stage_kernel, dim3(P->stage.blocks, n), dim3(256), 0, s, Q, P->stage, P->fmax, nb, P->sc,
+                           delta_chain, P->S);
+    if (P->maps.blocks)
+        hipLaunchKernelGGL(plane_map_kernel, dim3(P->maps.blocks, n), dim3(256), 0, s, Q, P->maps);
+    if (P->items) {
+        hipLaunchKernelGGL(contract_gemm_kernel, dim3((P->items * n + kXcds - 1) / kXcds * kXcds), dim3(256), 0,
+                           s, Q, P->gemm);
+        hipLaunchKernelGGL(epilogue_kernel<false>, dim3((P->dense_rows * kImages + 255) / 256, n), dim3(256), 0, s, Q,
+                           P->d_jobs, P->d_rows, P->gemm.blocks, P->gemm.part, P->rowscale, P->invZ, P->sc, 0u,
+                           P->dense_rows);
     }
-    if (P->near.n) {
-        const dim3 grid = G.probe_fast ? dim3(groups, near_wgs) : dim3(near_wgs, groups),
-                   block(64 * kNearWaves / kNearParts);
-        const bool split = P->precision == HVX_PRECISION_BF16_SPLIT;
-        if (grouped && split)
-            hipLaunchKernelGGL((near_gemm_staged_kernel<true, kProbeGroup>), grid, block, 0, s, G, P->near, P->sc);
-        else if (grouped)
-            hipLaunchKernelGGL((near_gemm_staged_kernel<false, kProbeGroup>), grid, block, 0, s, G, P->near, P->sc);
-        else if (split && kNearLdsGroupSplit > 0)
-            hipLaunchKernelGGL((near_gemm_lds_kernel<true, (kNearLdsGroupSplit > 0 ? kNearLdsGroupSplit : 2)>), grid,
-                               block, 0, s, G, P->near, P->sc);
-        else if (split)
-            hipLaunchKernelGGL((near_gemm_kernel<true, 1>), grid, block, 0, s, G, P->near, P->sc);
-        else if (kNearLdsGroup > 0)
-            hipLaunchKernelGGL((near_gemm_lds_kernel<false, (kNearLdsGroup > 0 ? kNearLdsGroup : 2)>), grid, block, 0,
-                               s, G, P->near, P->sc);
-        else
-            hipLaunchKernelGGL((near_gemm_kernel<false, 1>), grid, block, 0, s, G, P->near, P->sc);
-        hipLaunchKernelGGL(far_add_kernel, dim3((P->near.texels + 255) / 256, n), dim3(256), 0, s, Q, P->near);
-    }
-    if (P->delta_mip != ~0u) {
-        const uint32_t So = P->mp[P->delta_mip].L.So;
-        Probes D = Q;
-        if (delta_chain) D.chain0 = delta_chain;
-        hipLaunchKernelGGL(delta_kernel, dim3((6 * So * So + 255) / 256, n), dim3(256), 0, s, D, P->S, So,
-                           hvx::cube_level_offset_floats(P->So, P->delta_mip) / 4);
-    }
+    if (P->near_rows)
+        hipLaunchKernelGGL(epilogue_kernel<true>, dim3((P->near_rows * kImages + 255) / 256, n), dim3(256), 0, s, Q,
+                           P->d_jobs, P->d_rows, P->gemm.blocks, P->gemm.part, P->rowscale, P->invZ, P->sc,
+                           P->dense_rows, P->near_rows);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? HVX_OK : pfail(ctx, HVX_ERR_HIP, "%s: %s", what, hipGetErrorString(e));
+}
+
+// Copies of the per-call scratch that a multi-probe call over n probes runs
+// in: all of them up to 16 GiB, then the call is cut. Cutting it further, so
+// that what one launch stages stays in the caches for the next, does not pay:
+// 24 probes 256^2 -> 128^2 x 8 take 519 us at once, 563 us cut at 512 MiB,
+// 660 us at 128 MiB.
+constexpr size_t kMultiBytes = 16ull << 30;
+uint32_t multi_copies(size_t scratch_bytes, uint32_t n) {
+    const size_t fit = kMultiBytes / std::max<size_t>(scratch_bytes, 1);
+    return (uint32_t)std::min<size_t>(n, std::max<size_t>(fit, 4));
 }
 
 // Hot-texel blocks at least max(0.5, 300 level-0 texel widths) radians
@@ -2290,7 +1869,7 @@ int launch_hot_call(hvx_contract_plan* P, const float* d_chain, uint32_t chain_l
     if (P->min_level > 0 && (e = hvx::launch_cube_mips(P->hot_chain, P->S, P->min_level + 1, s)) != hipSuccess)
         return pfail(ctx, HVX_ERR_HIP, "clamped chain levels: %s", hipGetErrorString(e));
     const Probes Q{reinterpret_cast<const float4*>(P->hot_chain), reinterpret_cast<float4*>(d_out), nullptr, nullptr,
-                   0, 0, 0, 1};
+                   0, 0, 1};
     int st = launch_call(P, Q, 1, chain_levels, s, "hvx_ibl_filter_contract", reinterpret_cast<const float4*>(d_chain));
     if (st) return st;
     HotAdd A{};
@@ -2358,167 +1937,18 @@ int hvx_ibl_contract_plan_create(hvx_ctx* ctx, int type, uint32_t face, uint32_t
     ContractLevel lv[hvx::kContractMaxMips];
     const int ctype = type == HVX_FILTER_DIFFUSE ? hvx::CONTRACT_DIFFUSE : hvx::CONTRACT_SPECULAR;
     hvx::contract_levels(ctype, face, out_face, out_mips, lv);
-    auto fail_destroy = [&](hipError_t e, const char* where) {
-        hvx_ibl_contract_plan_destroy(P);
-        return pfail(ctx, HVX_ERR_HIP, "%s: %s", where, hipGetErrorString(e));
-    };
-    hipError_t e;
-    size_t part_floats = 0, sbytes = 0;
     P->mp.resize(out_mips);
-    for (uint32_t m = 0; m < out_mips; ++m) {
-        MipPlan& M = P->mp[m];
-        M.L = lv[m];
-        if (M.L.kind == hvx::CONTRACT_DELTA) continue;
-        DenseMat D;
-        D.G.type = ctype;
-        D.G.alpha2 = M.L.alpha2;
-        D.G.t0 = M.L.t0;
-        D.G.t1 = M.L.t1;
-        if (M.L.kind == hvx::CONTRACT_FULL) {
-            D.G.piece = PIECE_WHOLE;
-            D.G.So = M.L.So;
-            D.G.Sin = M.L.Si;
-        } else {
-            D.G.piece = PIECE_FAR;
-            D.G.So = M.L.Sf;
-            D.G.Sin = M.L.Sf;
-            M.far_off = scratch_take(&sbytes, 6 * (size_t)M.L.Sf * M.L.Sf * sizeof(float4));
-            if ((e = P->alloc(&M.zfar_map, 6 * (size_t)M.L.Sf * M.L.Sf)) != hipSuccess)
-                return fail_destroy(e, "far normaliser map");
-        }
-        D.G.rows = D.G.So * D.G.So;
-        D.G.rt = (D.G.rows + 15) / 16;
-        D.G.ks = 6 * D.G.Sin * D.G.Sin / 32;
-        D.split = split && M.L.kind == hvx::CONTRACT_SPLIT;  // low-roughness mips: near and far
-        D.stage = stage_dense_index(P, D.G.Sin, D.split);
-        if ((e = build_dense(P, D, ctx->num_cus, M.zfar_map)) != hipSuccess) return fail_destroy(e, "dense weights");
-        M.weight_bytes += (uint64_t)D.G.rt * D.G.ks * 64 * 16 * (D.split ? 2 : 1);
-        part_floats += (size_t)D.splitk * D.G.rt * 16 * 32;
-        P->dm.push_back(D);
-        M.dense = (int)P->dm.size() - 1;
-        if (M.L.kind == hvx::CONTRACT_SPLIT) {
-            M.NG = NearGeom{ctype, M.L.alpha2, M.L.t0, M.L.t1, M.L.So, M.L.Si, M.L.So / 16};
-            uint32_t B = 0;
-            M.tiles = near_tiles(M.L.So, M.L.Si, M.L.t1, &B);
-            StagePad sp;
-            sp.Si = M.L.Si;
-            sp.level = ilog2(face / M.L.Si);
-            sp.B = B;
-            sp.Pw = M.L.Si + 2 * B;
-            P->sp.push_back(sp);
-            M.pad = (int)P->sp.size() - 1;
-            if ((e = build_near(P, M, split)) != hipSuccess) return fail_destroy(e, "near weights");
-        }
+    for (uint32_t m = 0; m < out_mips; ++m) P->mp[m].L = lv[m];
+    hipError_t e;
+    try {
+        e = build_plan(P, ctype, split);
+    } catch (const std::bad_alloc&) {
+        e = hipErrorOutOfMemory;
     }
-    // staged inputs and shared scratch
-    for (StageDense& s : P->sd) {
-        const uint32_t K = 6 * s.Sin * s.Sin;
-        std::vector<int32_t> perm((size_t)6 * K);
-        for (int f = 0; f < 6; ++f)
-            for (uint32_t k = 0; k < K; ++k) perm[(size_t)f * K + k] = perm_index(f, k, s.Sin);
-        if ((e = P->alloc(&s.perm, perm.size())) != hipSuccess ||
-            (e = hipMemcpy(s.perm, perm.data(), perm.size() * 4, hipMemcpyHostToDevice)) != hipSuccess)
-            return fail_destroy(e, "dense staging");
-        s.off = scratch_take(&sbytes, (size_t)K / 8 * 32 * (s.split ? 2 : 1) * sizeof(half8));
-        P->min_level = std::max(P->min_level, s.level);
+    if (e != hipSuccess) {
+        hvx_ibl_contract_plan_destroy(P);
+        return pfail(ctx, HVX_ERR_HIP, "contraction plan: %s", hipGetErrorString(e));
     }
-    for (StagePad& s : P->sp) {
-        s.off = scratch_take(&sbytes, (size_t)s.Pw * (s.Pw / 8) * 32 * (split ? 2 : 1) * sizeof(half8));
-        P->min_level = std::max(P->min_level, s.level);
-    }
-    const size_t fmax_off = scratch_take(&sbytes, 6 * kFaceMaxBlocks * sizeof(float));
-    const size_t sc_off = scratch_take(&sbytes, 16 * sizeof(float));
-    const size_t part_off = scratch_take(&sbytes, part_floats * sizeof(float));
-    // one block; zeroed once (the pad columns of staged operands stay zero)
-    P->scratch_bytes = (sbytes + 255) & ~(size_t)255;
-    if ((e = P->alloc(&P->scratch, P->scratch_bytes)) != hipSuccess ||
-        (e = hipMemset(P->scratch, 0, P->scratch_bytes)) != hipSuccess)
-        return fail_destroy(e, "scratch");
-    for (MipPlan& M : P->mp)
-        if (M.L.kind == hvx::CONTRACT_SPLIT) M.far_map = reinterpret_cast<float4*>(P->scratch + M.far_off);
-    for (StageDense& s : P->sd) s.R = reinterpret_cast<half8*>(P->scratch + s.off);
-    for (StagePad& s : P->sp) s.P = reinterpret_cast<half8*>(P->scratch + s.off);
-    P->fmax = reinterpret_cast<float*>(P->scratch + fmax_off);
-    P->sc = reinterpret_cast<float*>(P->scratch + sc_off);
-    P->part = reinterpret_cast<float*>(P->scratch + part_off);
-    // launch tables of a filter call: every staged level, dense job and near job
-    StageTable& ST = P->stage;
-    for (const StageDense& sd : P->sd) P->scale_level = std::min(P->scale_level, sd.level);
-    for (const StagePad& sp : P->sp) P->scale_level = std::min(P->scale_level, sp.level);
-    for (const StageDense& sd : P->sd) {
-        StageItem& I = ST.it[ST.n++];
-        I = StageItem{sd.split ? 3 : 0, sd.Sin, 0, 0, hvx::cube_level_offset_floats(face, sd.level) / 4, sd.perm,
-                      sd.R, ST.total};
-        ST.total += 6 * sd.Sin * sd.Sin * 6;
-    }
-    for (const StagePad& sp : P->sp) {
-        StageItem& I = ST.it[ST.n++];
-        I = StageItem{split ? 2 : 1, sp.Si, sp.B, sp.Pw, hvx::cube_level_offset_floats(face, sp.level) / 4, nullptr,
-                      sp.P, ST.total};
-        ST.total += sp.Pw * sp.Pw * 6;
-    }
-    DenseTable& DT = P->dense;
-    NearTable& NT = P->near;
-    double near_k[kMaxJobs] = {};  // mean window (K) of each near job
-    float* part = P->part;
-    for (uint32_t m = 0; m < out_mips; ++m) {
-        const MipPlan& M = P->mp[m];
-        if (M.L.kind == hvx::CONTRACT_DELTA) {
-            P->delta_mip = m;
-            continue;
-        }
-        const DenseMat& D = P->dm[M.dense];
-        DenseJob& J = DT.j[DT.n++];
-        J.W = D.W;
-        J.R = P->sd[D.stage].R;
-        J.rt = D.G.rt;
-        J.ks = D.G.ks;
-        J.splitk = D.splitk;
-        J.rows = D.G.rows;
-        J.part = part;
-        part += (size_t)D.splitk * D.G.rt * 16 * 32;
-        J.rowscale = D.rowscale;
-        J.out = M.L.kind == hvx::CONTRACT_FULL ? nullptr : M.far_map;
-        J.out_off = hvx::cube_level_offset_floats(out_face, m) / 4;
-        J.alpha = M.L.kind == hvx::CONTRACT_FULL ? 1.0f : 0.0f;
-        J.wave_begin = DT.waves;
-        J.epi_begin = DT.epi;
-        J.w_lo = D.split ? (uint64_t)D.G.rt * D.G.ks * 64 : 0;
-        J.r_lo = D.split ? (uint64_t)6 * D.G.Sin * D.G.Sin / 8 * 32 : 0;
-        DT.waves += ((D.G.rt + 1) / 2 + 3) / 4 * 4 * D.splitk;  // pairs padded to a multiple of four
-        DT.epi += 6 * D.G.rows;
-        if (M.L.kind == hvx::CONTRACT_SPLIT) {
-            const StagePad& sp = P->sp[M.pad];
-            NearJob& N = NT.j[NT.n++];
-            N = NearJob{M.Wn, M.d_tiles, sp.P, sp.Pw / 8, sp.B, M.NG.te, M.L.So, M.L.Sf, M.rowscale_n, M.invZ,
-                        M.far_map, hvx::cube_level_offset_floats(out_face, m) / 4, NT.tiles, NT.texels, M.w_lo,
-                        split ? (uint64_t)sp.Pw * (sp.Pw / 8) * 32 : 0};
-            NT.tiles += (uint32_t)M.tiles.size();
-            NT.texels += 6 * M.L.So * M.L.So;
-            double k = 0.0;
-            for (const NearTile& t : M.tiles) k += (double)t.w * t.h;
-            near_k[NT.n - 1] = k / (double)M.tiles.size();
-        }
-    }
-    // near jobs in decreasing mean window size: the workgroups with the most
-    // K steps start first and the many shorter ones fill in behind them (the
-    // per-output accumulation does not depend on the order)
-    {
-        std::vector<uint32_t> ord(NT.n);
-        for (uint32_t k = 0; k < NT.n; ++k) ord[k] = k;
-        std::stable_sort(ord.begin(), ord.end(), [&](uint32_t a, uint32_t b) { return near_k[a] > near_k[b]; });
-        NearTable sorted = NT;
-        uint32_t tb = 0, xb = 0;
-        for (uint32_t k = 0; k < NT.n; ++k) {
-            sorted.j[k] = NT.j[ord[k]];
-            sorted.j[k].tile_begin = tb;
-            sorted.j[k].texel_begin = xb;
-            tb += sorted.j[k].te * sorted.j[k].te;
-            xb += 6 * sorted.j[k].So * sorted.j[k].So;
-        }
-        NT = sorted;
-    }
-    if ((e = hipDeviceSynchronize()) != hipSuccess) return fail_destroy(e, "plan set-up");
     *out = P;
     return HVX_OK;
 }
@@ -2554,7 +1984,7 @@ int hvx_ibl_filter_contract(hvx_contract_plan* P, const float* d_chain, uint32_t
     if (!d_chain || !d_out) return pfail(ctx, HVX_ERR_NULL, "NULL chain or output");
     if (((uintptr_t)d_chain | (uintptr_t)d_out) % 16) return pfail(ctx, HVX_ERR_ALIGN, "chains need 16-byte alignment");
     if (P->hot_k) return launch_hot_call(P, d_chain, chain_levels, d_out, (hipStream_t)stream);
-    const Probes Q{reinterpret_cast<const float4*>(d_chain), reinterpret_cast<float4*>(d_out), nullptr, nullptr, 0, 0, 0, 1};
+    const Probes Q{reinterpret_cast<const float4*>(d_chain), reinterpret_cast<float4*>(d_out), nullptr, nullptr, 0, 0, 1};
     return launch_call(P, Q, 1, chain_levels, (hipStream_t)stream, "hvx_ibl_filter_contract");
 }
 
@@ -2595,11 +2025,16 @@ int hvx_ibl_contract_plan_reserve(hvx_contract_plan* P, uint32_t max_probes) {
     if (max_probes == 0 || max_probes > kMaxProbes)
         return pfail(P->ctx, HVX_ERR_INVALID_ARG, "max_probes must be in [1, %u]", kMaxProbes);
     if (max_probes <= P->mcap) return HVX_OK;
+    const uint32_t copies = multi_copies(P->scratch_bytes, max_probes);
+    if (copies <= P->mcopies) {
+        P->mcap = max_probes;
+        return HVX_OK;
+    }
     (void)hipDeviceSynchronize();  // the old copies may be in use
     if (P->mscratch) (void)hipFree(P->mscratch);
     P->mscratch = nullptr;
-    P->mcap = 0;
-    const size_t bytes = P->scratch_bytes * max_probes;
+    P->mcap = P->mcopies = 0;
+    const size_t bytes = P->scratch_bytes * copies;
     hipError_t e;
     if ((e = hipMalloc(reinterpret_cast<void**>(&P->mscratch), bytes)) != hipSuccess ||
         (e = hipMemset(P->mscratch, 0, bytes)) != hipSuccess) {
@@ -2608,6 +2043,7 @@ int hvx_ibl_contract_plan_reserve(hvx_contract_plan* P, uint32_t max_probes) {
         return pfail(P->ctx, HVX_ERR_HIP, "multi-probe scratch (%zu bytes): %s", bytes, hipGetErrorString(e));
     }
     P->mcap = max_probes;
+    P->mcopies = copies;
     return HVX_OK;
 }
 
@@ -2621,11 +2057,16 @@ int hvx_ibl_filter_contract_multi(hvx_contract_plan* P, uint32_t n, const float*
                      n, P->mcap);
     if (P->hot_k)
         return pfail(P->ctx, HVX_ERR_UNSUPPORTED, "the bright-texel split serves single-probe calls only");
-    const Probes Q{nullptr, nullptr, reinterpret_cast<const float4* const*>(d_chains),
-                   reinterpret_cast<float4* const*>(d_outs),
-                   (uint64_t)(reinterpret_cast<uintptr_t>(P->mscratch) - reinterpret_cast<uintptr_t>(P->scratch)),
-                   (uint64_t)P->scratch_bytes, 0, n};
-    return launch_call(P, Q, n, chain_levels, (hipStream_t)stream, "hvx_ibl_filter_contract_multi");
+    for (uint32_t p = 0; p < n; p += P->mcopies) {
+        const uint32_t m = std::min(n - p, P->mcopies);
+        const Probes Q{nullptr, nullptr, reinterpret_cast<const float4* const*>(d_chains) + p,
+                       reinterpret_cast<float4* const*>(d_outs) + p,
+                       (uint64_t)(reinterpret_cast<uintptr_t>(P->mscratch) - reinterpret_cast<uintptr_t>(P->scratch)),
+                       (uint64_t)P->scratch_bytes, m};
+        const int st = launch_call(P, Q, m, chain_levels, (hipStream_t)stream, "hvx_ibl_filter_contract_multi");
+        if (st) return st;
+    }
+    return HVX_OK;
 }
 
 }  // extern "C"
