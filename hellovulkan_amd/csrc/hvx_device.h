@@ -74,6 +74,38 @@ __device__ __forceinline__ float rcp_rn_normal(float b) {
     return __builtin_fmaf(e, y, y);
 }
 
+// 1.0f / sqrtf(q) (both correctly rounded) of a squared length q within 2048
+// floats of 1, from its bit pattern alone. With q = 1 + d 2^-23, d >= 0, the
+// square root 1 + d/2 2^-23 - O(d^2) 2^-46 rounds to 1 + floor(d/2) 2^-23 (a
+// tie is broken downwards by the small term), whose reciprocal rounds to
+// 1 - floor(d/2) 2^-23, twice as many of the floats below 1; with q = 1 +
+// d 2^-24, d < 0, the root rounds to 1 - ceil(-d/2) 2^-24 and the reciprocal
+// to 1 + ceil(ceil(-d/2)/2) 2^-23. Holds for -8190 <= d <= 2897 (every float
+// checked, tests/test_gpu_unit_length.py). Eight integer operations for the 13 and
+// two transcendental ones of rcp_rn_normal(sqrt_rn_normal(q)), to which other
+// values fall back.
+__host__ __device__ __forceinline__ uint32_t inv_unit_length_bits(int d) {
+    const int one = 0x3f800000;
+    return (uint32_t)(d >= 0 ? one - (d & ~1) : one + ((3 - d) >> 2));
+}
+__device__ __forceinline__ float inv_unit_length(float q) {
+    const int d = (int)f2u(q) - 0x3f800000;
+    if (__builtin_expect((uint32_t)(d + 2048) > 4096u, 0)) return rcp_rn_normal(sqrt_rn_normal(q));
+    return u2f(inv_unit_length_bits(d));
+}
+
+// a / b correctly rounded where a, b, a / b and the residuals a - b q (down to
+// about |a| 2^-24) are normal: the correctly rounded reciprocal, then two
+// Newton steps of the quotient with fused residuals. The first leaves q within
+// an ulp, and from there the second rounds correctly (Markstein). Without the
+// scaling and special cases of the compiler's division.
+__device__ __forceinline__ float div_rn_normal(float a, float b) {
+    const float y = rcp_rn_normal(b);
+    float q = a * y;
+    q = __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
+    return __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
+}
+
 // normalize3 of a vector whose squared length is a float in [2^-102, FLT_MAX]
 // (every near-unit vector): the same correctly rounded square root and
 // reciprocal, by the fast paths above, so the result is bit-identical.

@@ -63,22 +63,32 @@ __device__ __forceinline__ f3 ggx_world(const Frame& fr, f3 N, float4 h) {
 // ---------------------------------------------------------------- BRDF LUT
 constexpr int kLutChunk = 1024;
 
-__global__ __launch_bounds__(256) void brdf_lut_kernel(uint32_t W, uint32_t H, uint32_t n, float2* __restrict__ lut) {
+// A workgroup per row (its roughness' half vectors staged in LDS), PER texels
+// per lane. Bound by VALU issue. The shader's N is (0, 0, 1) and V = (x, 0, z):
+// the products with their zeros only ever add a zero, and of the light vector
+// only its length and z count, so they are left out (signs of zero cannot
+// reach the sums: every factor they meet is a positive sum or a product with
+// N.L > 0); G's V half is the texel's, N.H the sample's. FAST (sample counts
+// up to 2^20, where no half vector is horizontal): the exact divisions without
+// scaling and the exact normalisation from the length's bit pattern (|L| = 1
+// up to rounding). 512^2 x 1024: 428 us (1,186 us with four texels per lane, half of them
+// past the row's end, and the general operations).
+template <int PER, bool FAST>
+__global__ __launch_bounds__(512) void brdf_lut_kernel(uint32_t W, uint32_t H, uint32_t n, float2* __restrict__ lut) {
     __shared__ float4 s_h[kLutChunk];
     const uint32_t y = blockIdx.x;
     const float rough = 1.0f - ((float)y + 0.5f) / (float)H;
     const f3 N = make3(0.0f, 0.0f, 1.0f);
     const Frame fr = ggx_frame(N);
     const float alpha = (rough * rough) / 2.0f;  // AlphaIBL
-    // each lane owns up to 4 texels of the row (W <= 1024)
-    constexpr int kPer = 4;
-    float lx[kPer], ly[kPer], nov[kPer];
-    f3 V[kPer];
+    const float oma = 1.0f - alpha;
+    float lx[PER], ly[PER], nov[PER], vx[PER], GV[PER];
 #pragma unroll
-    for (int q = 0; q < kPer; ++q) {
+    for (int q = 0; q < PER; ++q) {
         const uint32_t x = threadIdx.x + q * blockDim.x;
         nov[q] = ((float)min(x, W - 1) + 0.5f) / (float)W;
-        V[q] = make3(sqrtf_(1.0f - nov[q] * nov[q]), 0.0f, nov[q]);
+        vx[q] = sqrtf_(1.0f - nov[q] * nov[q]);
+        GV[q] = nov[q] / (nov[q] * oma + alpha);
         lx[q] = 0.0f;
         ly[q] = 0.0f;
     }
@@ -88,24 +98,23 @@ __global__ __launch_bounds__(256) void brdf_lut_kernel(uint32_t W, uint32_t H, u
         for (uint32_t i = threadIdx.x; i < cn; i += blockDim.x) {
             const float4 h = ggx_tangent_sample(c0 + i, n, rough);
             const f3 w = ggx_world(fr, N, h);
-            s_h[i] = make_float4(w.x, w.y, w.z, 0.0f);
+            s_h[i] = make_float4(w.x, w.y, w.z, gmax(w.z, 0.0f));
         }
         __syncthreads();
         for (uint32_t i = 0; i < cn; ++i) {
-            const float4 hh = s_h[i];
-            const f3 Hh = make3(hh.x, hh.y, hh.z);
+            const float4 h = s_h[i];
 #pragma unroll
-            for (int q = 0; q < kPer; ++q) {
-                const f3 L = normalize3(sub3(mul3(Hh, 2.0f * dot3(V[q], Hh)), V[q]));
-                const float dotNL = gmax(dot3(N, L), 0.0f);
+            for (int q = 0; q < PER; ++q) {
+                const float vh = vx[q] * h.x + nov[q] * h.z, k = 2.0f * vh;
+                const float Lx = h.x * k - vx[q], Ly = h.y * k, Lz = h.z * k - nov[q];
+                const float len2 = (Lx * Lx + Ly * Ly) + Lz * Lz;
+                const float dotNL = Lz * (FAST ? inv_unit_length(len2) : 1.0f / sqrtf_(len2));
                 if (dotNL > 0.0f) {
-                    const float dotNV = gmax(dot3(N, V[q]), 0.0f);
-                    const float dotVH = gmax(dot3(V[q], Hh), 0.0f);
-                    const float dotNH = gmax(dot3(Hh, N), 0.0f);
-                    const float GL = dotNL / (dotNL * (1.0f - alpha) + alpha);
-                    const float GV = dotNV / (dotNV * (1.0f - alpha) + alpha);
-                    const float G = GL * GV;
-                    const float G_Vis = (G * dotVH) / (dotNH * dotNV);
+                    const float dotVH = gmax(vh, 0.0f);
+                    const float gl = dotNL * oma + alpha, d = h.w * nov[q];
+                    const float GL = FAST ? div_rn_normal(dotNL, gl) : dotNL / gl;
+                    const float g = (GL * GV[q]) * dotVH;
+                    const float G_Vis = FAST ? div_rn_normal(g, d) : g / d;
                     const float Fc = pow5f(1.0f - dotVH);
                     lx[q] = lx[q] + (1.0f - Fc) * G_Vis;
                     ly[q] = ly[q] + Fc * G_Vis;
@@ -114,7 +123,7 @@ __global__ __launch_bounds__(256) void brdf_lut_kernel(uint32_t W, uint32_t H, u
         }
     }
 #pragma unroll
-    for (int q = 0; q < kPer; ++q) {
+    for (int q = 0; q < PER; ++q) {
         const uint32_t x = threadIdx.x + q * blockDim.x;
         if (x < W) lut[(size_t)y * W + x] = make_float2(lx[q] / (float)n, ly[q] / (float)n);
     }
@@ -630,7 +639,14 @@ probe_batch_kernel(const ProbeJob* __restrict__ jobs, const ProbeItem* __restric
 
 // ================================================================ launchers
 hipError_t launch_brdf_lut(uint32_t w, uint32_t h, uint32_t n, float* d_lut, hipStream_t s) {
-    hipLaunchKernelGGL(brdf_lut_kernel, dim3(h), dim3(256), 0, s, w, h, n, reinterpret_cast<float2*>(d_lut));
+    // one texel per lane up to 256 lanes (rounded to whole waves), then two:
+    // 512^2 takes the same time either way (429 and 430 us)
+    const bool one = w <= 256, fast = n <= (1u << 20);
+    const uint32_t lanes = (one ? w : (w + 1) / 2), threads = (lanes + 63) / 64 * 64;  // w <= 1024
+    float2* lut = reinterpret_cast<float2*>(d_lut);
+    const auto kernel = fast ? (one ? brdf_lut_kernel<1, true> : brdf_lut_kernel<2, true>)
+                             : (one ? brdf_lut_kernel<1, false> : brdf_lut_kernel<2, false>);
+    hipLaunchKernelGGL(kernel, dim3(h), dim3(threads), 0, s, w, h, n, lut);
     return hipGetLastError();
 }
 
