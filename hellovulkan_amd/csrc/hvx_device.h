@@ -99,17 +99,25 @@ __device__ __forceinline__ float inv_unit_length(float q) {
 // Newton steps of the quotient with fused residuals. The first leaves q within
 // an ulp, and from there the second rounds correctly (Markstein). Without the
 // scaling and special cases of the compiler's division.
-__device__ __forceinline__ float div_rn_normal(float a, float b) {
-    const float y = rcp_rn_normal(b);
+__device__ __forceinline__ float div_by_normal(float a, float b, float y) {  // y = rcp_rn_normal(b)
     float q = a * y;
     q = __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
     return __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
 }
+__device__ __forceinline__ float div_rn_normal(float a, float b) { return div_by_normal(a, b, rcp_rn_normal(b)); }
 
 // normalize3 of a vector whose squared length is a float in [2^-102, FLT_MAX]
 // (every near-unit vector): the same correctly rounded square root and
 // reciprocal, by the fast paths above, so the result is bit-identical.
 __device__ __forceinline__ f3 normalize3_rn(f3 a) { return mul3(a, rcp_rn_normal(sqrt_rn_normal(dot3(a, a)))); }
+
+// normalize3, bit-identical, of a vector whose squared length is known to be
+// within 2048 floats of 1 (a combination of an orthonormal frame with unit
+// coefficients, a reflection of one unit vector about another: both within a
+// few tens of floats).
+__device__ __forceinline__ f3 normalize3_unit(f3 a) {
+    return mul3(a, u2f(inv_unit_length_bits((int)f2u(dot3(a, a)) - 0x3f800000)));
+}
 
 // ------------------------------------------------------------ cube sampling
 struct CubeCoord {
@@ -117,25 +125,34 @@ struct CubeCoord {
     float s, t;
 };
 
+// Face and plane coordinates of direction r. Selects and sign flips instead of
+// a branch per face: the lanes of a wave look all ways. UNIT: r has unit
+// length up to rounding, so the divisions by the major component (at least
+// 0.57) need no scaling; they share its reciprocal. (A numerator near zero
+// whose residual is subnormal vanishes in the sum with 1.)
+template <bool UNIT = false>
 __device__ __forceinline__ CubeCoord cube_select(f3 r) {
     const float ax = absf(r.x), ay = absf(r.y), az = absf(r.z);
+    const bool X = ax >= ay && ax >= az, Y = !X && ay >= az;
+    const float ma = X ? ax : (Y ? ay : az);
+    const bool neg = !((X ? r.x : (Y ? r.y : r.z)) >= 0.0f);
+    const uint32_t flip = neg ? 0x80000000u : 0u;
+    // sc: -z, z, x, x, x, -x and tc: -y, -y, z, -z, -y, -y of faces 0 .. 5
+    const float sc = u2f(f2u(X ? -r.z : r.x) ^ (Y ? 0u : flip));
+    const float tc = u2f(f2u(Y ? r.z : -r.y) ^ (Y ? flip : 0u));
     CubeCoord c;
-    float sc, tc, ma;
-    if (ax >= ay && ax >= az) {
-        ma = ax;
-        if (r.x >= 0.0f) { c.face = 0; sc = -r.z; tc = -r.y; }
-        else { c.face = 1; sc = r.z; tc = -r.y; }
-    } else if (ay >= az) {
-        ma = ay;
-        if (r.y >= 0.0f) { c.face = 2; sc = r.x; tc = r.z; }
-        else { c.face = 3; sc = r.x; tc = -r.z; }
+    c.face = (X ? 0 : (Y ? 2 : 4)) + (neg ? 1 : 0);
+    float qs, qt;
+    if constexpr (UNIT) {
+        const float y = rcp_rn_normal(ma);
+        qs = div_by_normal(sc, ma, y);
+        qt = div_by_normal(tc, ma, y);
     } else {
-        ma = az;
-        if (r.z >= 0.0f) { c.face = 4; sc = r.x; tc = -r.y; }
-        else { c.face = 5; sc = -r.x; tc = -r.y; }
+        qs = sc / ma;
+        qt = tc / ma;
     }
-    c.s = 0.5f * (sc / ma + 1.0f);
-    c.t = 0.5f * (tc / ma + 1.0f);
+    c.s = 0.5f * (qs + 1.0f);
+    c.t = 0.5f * (qt + 1.0f);
     return c;
 }
 
@@ -261,8 +278,9 @@ __device__ __forceinline__ int cube_tap_index(int S, int f, int i, int j) {
     return -1;
 }
 
+template <bool UNIT = false>
 __device__ __forceinline__ CubeTaps cube_taps(int S, f3 dir) {
-    const CubeCoord cc = cube_select(dir);
+    const CubeCoord cc = cube_select<UNIT>(dir);
     const float u = cc.s * (float)S - 0.5f;
     const float v = cc.t * (float)S - 0.5f;
     const float fu = floorf_(u), fv = floorf_(v);
@@ -277,7 +295,7 @@ __device__ __forceinline__ CubeTaps cube_taps(int S, f3 dir) {
     t.face = cc.face;
     t.i0 = i0;
     t.j0 = j0;
-    t.interior = i0 >= 0 && j0 >= 0 && i0 + 1 < S && j0 + 1 < S;
+    t.interior = (uint32_t)i0 < (uint32_t)(S - 1) && (uint32_t)j0 < (uint32_t)(S - 1);
     if (t.interior) {
         const int base = (cc.face * S + j0) * S + i0;
         t.idx[0] = base;

@@ -305,7 +305,7 @@ diffuse_kernel(const float4* __restrict__ cube, uint32_t S, const float4* __rest
         p.ct = s_ct[it];
         const float tx = p.st * cp, ty = p.st * sp, tz = p.ct;
         p.L = add3(add3(mul3(right, tx), mul3(up, ty)), mul3(N, tz));
-        p.taps = cube_taps((int)S, p.L);
+        p.taps = cube_taps<true>((int)S, p.L);
         if constexpr (STAGED) {
             // i0, j0 lie in [-1, S - 1] (the face coordinates are in [0, 1]);
             // the clamp only keeps the index inside the table
@@ -436,8 +436,20 @@ __global__ __launch_bounds__(256) void specular_delta_kernel(const float4* __res
 // sample order, so every sum is the reference's sequential sum (bit-exact).
 // Few texels per wave keep the texels in flight per XCD few, so the GGX lobes
 // being read at any time share the XCD's L2: tiles are taken in 16x16-tile
-// supertiles, and the workgroups of one XCD (workgroup b runs on XCD b % 8)
-// get one contiguous run of tiles.
+// supertiles, and XCD x (workgroups b with b % 8 = x) gets run x of every
+// mip's tiles.
+// What bounds it (512^2 x 10 from 1024^2, 1024 samples): the texture
+// addresser, at about a lane per cycle for gathers of lanes in different lines,
+// then VALU issue (236 instructions per 64 samples). So the two lanes of a pair
+// load the two texels of a footprint row together, one sample of the pair per
+// load (cube_taps / pair_taps): lanes side by side in one line are one access.
+//   one run of all mips' tiles per XCD                   7.43 ms
+//   (two XCDs held the tiles of mip 2, which cost about
+//   twice those of mip 1; six waited for them)
+//   a run of every mip per XCD                           4.33 ms
+//   lengths from bit patterns, faces by selects          4.33 ms (still the addresser)
+//   footprint rows loaded by lane pairs                  3.78 ms (addresser 88 -> 70 % busy)
+//   no length checks, 32-bit offsets                     3.71 ms (VALU 81 % busy)
 #ifndef HVX_SPEC_TPW
 #define HVX_SPEC_TPW 4
 #endif
@@ -454,70 +466,112 @@ struct SpecSplitArgs {
     uint32_t S;
     float4* out;
     uint32_t So, mips, n, emulate;
-    uint32_t n_tiles, per_xcd;          // padded tiles of mips 1.. and tiles per XCD run
-    uint32_t tile_begin[kMaxMips + 1];  // first tile of mip m (mips 1..), tile_begin[1] = 0
+    uint32_t run_begin[kMaxMips + 1];  // first workgroup of mip m (mips 1..) in an XCD's sequence, run_begin[1] = 0
     const float4* table;
 };
 
 // One GGX sample of the specular loop, split so its texel loads overlap other
-// work: spec_begin forms L and NoL and issues the four tap loads (always, so
-// the loads are not under a branch; a rejected sample's taps are valid
-// texels whose values are not used), spec_term forms the sample's terms.
+// work: spec_begin forms L and NoL and issues the four tap loads of the pair's
+// samples (always, so the loads are not under a branch; a rejected sample's
+// taps are valid texels whose values are not used), spec_term forms the
+// sample's terms.
 struct SpecSample {
     f3 L;
     float nol;
     CubeTaps taps;
-    float4 q[4];
+    f3 q[4];  // [2 r + s]: row r, column (lane & 1) of the footprint of the pair's sample s
 };
 
+// The value of the other lane of a pair (2k, 2k + 1).
+__device__ __forceinline__ int pair_swap(int v) { return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xf, 0xf, true); }
+__device__ __forceinline__ float pair_swap(float v) {
+    return __builtin_bit_cast(float, pair_swap(__builtin_bit_cast(int, v)));
+}
+
+// Texel i of a cube level. WIDE false: the level is smaller than 4 GiB, so a
+// 32-bit byte offset from the uniform base will do.
+constexpr uint32_t kNarrowFace = 6688;  // largest face of such a level
+template <bool WIDE>
+__device__ __forceinline__ float4 cube_at(const float4* __restrict__ cube, int i) {
+    if constexpr (WIDE) return cube[i];
+    else return *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(cube) + ((uint32_t)i << 4));
+}
+
+template <bool WIDE>
 __device__ __forceinline__ void spec_begin(SpecSample& p, const float4* __restrict__ cube, int S, const Frame& fr,
                                            f3 N, float4 h) {
-    // both vectors are unit length up to rounding: normalize3_rn is exact here
-    const f3 Hh = normalize3_rn(add3(add3(mul3(fr.t, h.x), mul3(fr.b, h.y)), mul3(N, h.z)));  // ggx_world
-    p.L = normalize3_rn(sub3(mul3(Hh, 2.0f * dot3(N, Hh)), N));                            // V = N
+    // both vectors are unit length up to rounding
+    const f3 Hh = normalize3_unit(add3(add3(mul3(fr.t, h.x), mul3(fr.b, h.y)), mul3(N, h.z)));  // ggx_world
+    p.L = normalize3_unit(sub3(mul3(Hh, 2.0f * dot3(N, Hh)), N));                              // V = N
     p.nol = gmax(dot3(N, p.L), 0.0f);
-    p.taps = cube_taps(S, p.L);
+    p.taps = cube_taps<true>(S, p.L);
+    const bool odd = threadIdx.x & 1u;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) p.q[k] = cube[p.taps.idx[k]];
+    for (int r = 0; r < 2; ++r) {
+        const int i0 = p.taps.idx[2 * r], i1 = p.taps.idx[2 * r + 1];
+        const int s0 = pair_swap(i0), s1 = pair_swap(i1);
+        const int a0 = odd ? s1 : i0, a1 = odd ? i1 : s0;
+        const float4 v0 = cube_at<WIDE>(cube, a0), v1 = cube_at<WIDE>(cube, a1);
+        p.q[2 * r] = {v0.x, v0.y, v0.z};
+        p.q[2 * r + 1] = {v1.x, v1.y, v1.z};
+    }
+}
+
+// The two texels t0, t1 of this lane's sample: the even lane loaded texel 0 of
+// both samples (v0: the even lane's sample, v1: the odd one's), the odd lane
+// texel 1.
+__device__ __forceinline__ void pair_taps(float v0, float v1, bool odd, float& t0, float& t1) {
+    const float x0 = pair_swap(v0), x1 = pair_swap(v1);
+    t0 = odd ? x1 : v0;
+    t1 = odd ? v1 : x0;
 }
 
 // (c * NoL, NoL) of a sample that counts (NoL > 0); -0 in every term of one
 // that does not (a rejected or padding sample): x + (-0) == x for every x.
 __device__ __forceinline__ float4 spec_term(const SpecSample& p, bool live, const float4* __restrict__ cube, int S) {
+    const bool odd = threadIdx.x & 1u;
+    float4 q[4];
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+        pair_taps(p.q[2 * r].x, p.q[2 * r + 1].x, odd, q[2 * r].x, q[2 * r + 1].x);
+        pair_taps(p.q[2 * r].y, p.q[2 * r + 1].y, odd, q[2 * r].y, q[2 * r + 1].y);
+        pair_taps(p.q[2 * r].z, p.q[2 * r + 1].z, odd, q[2 * r].z, q[2 * r + 1].z);
+    }
     if (!(live && p.nol > 0.0f)) return make_float4(-0.0f, -0.0f, -0.0f, -0.0f);
-    const f3 c = cube_combine(cube, S, p.L, p.taps, p.q);
+    const f3 c = cube_combine(cube, S, p.L, p.taps, q);
     return make_float4(c.x * p.nol, c.y * p.nol, c.z * p.nol, p.nol);
 }
 
-// Tile geometry of one mip of size Sm: tiles of kSpecTW x kSpecTH texels,
-// taken in 16 x 16-tile supertiles (row-major supertiles, row-major tiles in
-// each); padded tile k of a face maps to (tx, ty), outside the face when the
-// supertile is partial.
+// Tiles of one mip of size Sm: kSpecTW x kSpecTH texels, taken face by face in
+// supertiles of 16 x 16 tiles (row-major supertiles, row-major tiles in each;
+// the last column and row of supertiles are as wide and high as is left).
 struct SpecTileGeom {
-    uint32_t tiles_x, tiles_y, super_x, per_face;  // per_face: padded tiles per face
+    uint32_t tiles_x, tiles_y, per_face;
 };
 __host__ __device__ inline SpecTileGeom spec_tile_geom(uint32_t Sm) {
     SpecTileGeom g;
     g.tiles_x = (Sm + kSpecTW - 1) / kSpecTW;
     g.tiles_y = (Sm + kSpecTH - 1) / kSpecTH;
-    g.super_x = (g.tiles_x + 15) / 16;
-    g.per_face = g.super_x * ((g.tiles_y + 15) / 16) * 256u;
+    g.per_face = g.tiles_x * g.tiles_y;
     return g;
 }
-// Padded tile index -> (face, tx, ty); false for a padding slot.
-__host__ __device__ inline bool spec_tile_at(const SpecTileGeom& g, uint32_t k, uint32_t& face, uint32_t& tx,
+// Tile index (< 6 per_face) -> (face, tx, ty).
+__host__ __device__ inline void spec_tile_at(const SpecTileGeom& g, uint32_t k, uint32_t& face, uint32_t& tx,
                                              uint32_t& ty) {
     face = k / g.per_face;
-    const uint32_t kk = k % g.per_face, ks = kk / 256u, kw = kk % 256u;
-    tx = (ks % g.super_x) * 16u + kw % 16u;
-    ty = (ks / g.super_x) * 16u + kw / 16u;
-    return tx < g.tiles_x && ty < g.tiles_y;
+    const uint32_t kk = k % g.per_face, row = kk / (16u * g.tiles_x), kr = kk % (16u * g.tiles_x);
+    const uint32_t high = g.tiles_y - 16u * row < 16u ? g.tiles_y - 16u * row : 16u;
+    const uint32_t col = kr / (16u * high), kc = kr % (16u * high);
+    const uint32_t wide = g.tiles_x - 16u * col < 16u ? g.tiles_x - 16u * col : 16u;
+    tx = 16u * col + kc % wide;
+    ty = 16u * row + kc / wide;
 }
 
 // One tile of the sample-split specular loop (four waves, each independent):
 // texels of face `face` of a mip of size Sm whose directions lie on a D x D
 // grid, out_level that mip's texels, tab its n tangent-space samples, s_buf
 // the workgroup's [4][2][kSpecTPW][kSpecRow] summation buffer.
+template <bool WIDE>
 __device__ __forceinline__ void specular_split_tile(const float4* __restrict__ cube, int S,
                                                     float4* __restrict__ out_level, uint32_t Sm, uint32_t D,
                                                     const float4* __restrict__ tab, uint32_t n, uint32_t face,
@@ -551,13 +605,13 @@ __device__ __forceinline__ void specular_split_tile(const float4* __restrict__ c
     };
     SpecSample A, B;
     float4 hA = tab_at(0), hB = tab_at(1);
-    spec_begin(A, cube, S, fr, N, hA);
+    spec_begin<WIDE>(A, cube, S, fr, N, hA);
     hA = tab_at(2);
     for (uint32_t r = 0; r < rounds; r += 2) {
-        spec_begin(B, cube, S, fr, N, hB);
+        spec_begin<WIDE>(B, cube, S, fr, N, hB);
         hB = tab_at(r + 3);
         sum_round(0, spec_term(A, r * kSpecSPR + s < n, cube, S));
-        spec_begin(A, cube, S, fr, N, hA);
+        spec_begin<WIDE>(A, cube, S, fr, N, hA);
         hA = tab_at(r + 4);
         sum_round(1, spec_term(B, (r + 1) * kSpecSPR + s < n, cube, S));
     }
@@ -575,18 +629,23 @@ __device__ __forceinline__ void specular_split_tile(const float4* __restrict__ c
 #ifndef HVX_SPEC_WAVES_PER_EU
 #define HVX_SPEC_WAVES_PER_EU 4
 #endif
+template <bool WIDE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HVX_SPEC_WAVES_PER_EU, 8))) void
 specular_split_kernel(SpecSplitArgs a) {
     __shared__ __align__(16) float s_buf[4][2][kSpecTPW][kSpecRow];
-    const uint32_t b = blockIdx.x;
-    const uint32_t tile = (b % 8u) * a.per_xcd + b / 8u;
-    if (tile >= a.n_tiles) return;
+    // XCD x (workgroups b with b % 8 = x) works through run x of every mip's
+    // tiles in turn: a mip's tiles cost about the same, but those of different
+    // mips up to several times each other (wider lobes miss the L2 more)
+    const uint32_t x = blockIdx.x % 8u, k = blockIdx.x / 8u;
     uint32_t m = 1;
-    while (tile >= a.tile_begin[m + 1]) ++m;
+    while (k >= a.run_begin[m + 1]) ++m;
     const uint32_t Sm = max(a.So >> m, 1u);
+    const SpecTileGeom g = spec_tile_geom(Sm);
+    const uint32_t tile = x * (a.run_begin[m + 1] - a.run_begin[m]) + k - a.run_begin[m];
+    if (tile >= 6u * g.per_face) return;  // the last run may be short
     uint32_t face, tx, ty;
-    if (!spec_tile_at(spec_tile_geom(Sm), tile - a.tile_begin[m], face, tx, ty)) return;  // padding
-    specular_split_tile(a.cube, (int)a.S, a.out + cube_level_offset_floats(a.So, m) / 4, Sm, a.emulate ? a.So : Sm,
+    spec_tile_at(g, tile, face, tx, ty);
+    specular_split_tile<WIDE>(a.cube, (int)a.S, a.out + cube_level_offset_floats(a.So, m) / 4, Sm, a.emulate ? a.So : Sm,
                         a.table + (size_t)m * a.n, a.n, face, tx, ty, &s_buf[0][0][0][0]);
 }
 
@@ -597,7 +656,7 @@ specular_split_kernel(SpecSplitArgs a) {
 // tile and cuts the runs at equal estimated cost, so each XCD works through
 // neighbouring tiles of a few probes and shares their texels in its L2.
 // Items of mip 0 are texel ranges (lane per texel, as specular_delta_kernel);
-// other items are runs of padded tiles (specular_split_tile).
+// other items are runs of tiles (specular_split_tile).
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HVX_SPEC_WAVES_PER_EU, 8))) void
 probe_batch_kernel(const ProbeJob* __restrict__ jobs, const ProbeItem* __restrict__ items,
                    const uint32_t* __restrict__ xcd_begin, const float4* __restrict__ tables,
@@ -628,8 +687,11 @@ probe_batch_kernel(const ProbeJob* __restrict__ jobs, const ProbeItem* __restric
             const SpecTileGeom g = spec_tile_geom(Sm);
             for (uint32_t k = it.first; k < it.first + it.count; ++k) {
                 uint32_t face, tx, ty;
-                if (spec_tile_at(g, k, face, tx, ty))
-                    specular_split_tile(j.cube, (int)j.S, out, Sm, Sm, tab, j.n, face, tx, ty, &s_buf[0][0][0][0]);
+                spec_tile_at(g, k, face, tx, ty);
+                if (j.S > kNarrowFace)
+                    specular_split_tile<true>(j.cube, (int)j.S, out, Sm, Sm, tab, j.n, face, tx, ty, &s_buf[0][0][0][0]);
+                else
+                    specular_split_tile<false>(j.cube, (int)j.S, out, Sm, Sm, tab, j.n, face, tx, ty, &s_buf[0][0][0][0]);
             }
         }
     }
@@ -733,12 +795,11 @@ hipError_t launch_specular(const float* d_cube, uint32_t S, float* d_out, uint32
         a.table = ggx_table;
         uint32_t t = 0;
         for (uint32_t m = 1; m <= (uint32_t)kMaxMips; ++m) {
-            a.tile_begin[m] = t;
-            if (m < mips) t += 6u * spec_tile_geom(std::max(So >> m, 1u)).per_face;
+            a.run_begin[m] = t;
+            if (m < mips) t += (6u * spec_tile_geom(std::max(So >> m, 1u)).per_face + 7) / 8;
         }
-        a.n_tiles = t;
-        a.per_xcd = (t + 7) / 8;
-        hipLaunchKernelGGL(specular_split_kernel, dim3(a.per_xcd * 8), dim3(256), 0, s, a);
+        hipLaunchKernelGGL(S > kNarrowFace ? specular_split_kernel<true> : specular_split_kernel<false>, dim3(t * 8),
+                           dim3(256), 0, s, a);
     }
     return hipGetLastError();
 }
@@ -758,7 +819,7 @@ hipError_t launch_probe_batch(const ProbeJob* d_jobs, const ProbeItem* d_items, 
 
 // Batch work items (probe, mip, range) for the probes of `jobs`, in probe,
 // mip, tile order: mip 0 as ranges of `texels` texels, other mips as runs of
-// padded tiles holding about texels / 16 tiles each; xcd_begin[0..8] cuts the
+// about texels / 16 tiles; xcd_begin[0..8] cuts the
 // list into eight runs of equal estimated cost.
 void make_probe_items(const ProbeJob* jobs, uint32_t n_probes, uint32_t texels, std::vector<ProbeItem>& items,
                       uint32_t xcd_begin[9]) {
@@ -779,18 +840,10 @@ void make_probe_items(const ProbeJob* jobs, uint32_t n_probes, uint32_t texels, 
                 continue;
             }
             const SpecTileGeom g = spec_tile_geom(Sm);
-            const uint32_t slots = 6u * g.per_face;
-            uint32_t k = 0;
-            while (k < slots) {
-                uint32_t first = k, valid = 0;
-                for (; k < slots && valid < per_item; ++k) {
-                    uint32_t f, tx, ty;
-                    if (spec_tile_at(g, k, f, tx, ty)) valid += 1;
-                }
-                if (valid) {
-                    items.push_back({p, m, first, k - first});
-                    cost.push_back((double)valid * kSpecTW * kSpecTH * j.n * 216.0);
-                }
+            for (uint32_t k = 0; k < 6u * g.per_face; k += per_item) {
+                const uint32_t c = std::min(per_item, 6u * g.per_face - k);
+                items.push_back({p, m, k, c});
+                cost.push_back((double)c * kSpecTW * kSpecTH * j.n * 216.0);
             }
         }
     }
