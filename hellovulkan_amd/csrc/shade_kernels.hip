@@ -279,7 +279,9 @@ __device__ __forceinline__ void shade_one(const ShadeArgs& a, uint32_t idx, uint
         const float omk = 1.0f - alphaRough;
         const float GV = NoV * rcp_fast(__builtin_fmaf(NoV, omk, alphaRough));
         const float a2m1 = alpha2 - 1.0f;
+        // (NoL omk + k) (4 NoV NoL + 1e-4), k = alphaRough, as a polynomial in NoL
         const float nov4 = 4.0f * NoV;
+        const float q2 = omk * nov4, q1 = __builtin_fmaf(omk, 0.0001f, alphaRough * nov4), q0 = alphaRough * 0.0001f;
         const float negf = -a.pc.light_falloff;
         const float aGVpi = (alpha2 * GV) * (1.0f / kPiF);
         // A light's BRDF term per channel, (1 - F) q + F DGr with
@@ -294,16 +296,21 @@ __device__ __forceinline__ void shade_one(const ShadeArgs& a, uint32_t idx, uint
         // one light's term, added to Lo
         auto light = [&](const float4 A, const float4 B) {
             const f3 d = {A.x - wp.x, A.y - wp.y, A.z - wp.z};
-            float s, NoH;
+            float s, r, NoH;
             f3 L, Hh;
-            // A light out of range of every lane (squared distance at least
-            // B.w = r^2 (1 + 2^-16)) has attenuation exactly 0 in each: its
-            // terms add nothing, so the wave skips it.
+            // |d| N.L, whose sign is N.L's
+            const float ndd = __builtin_fmaf(N.z, d.z, __builtin_fmaf(N.y, d.y, N.x * d.x));
+            // A light that is out of range (squared distance at least
+            // B.w = r^2 (1 + 2^-16), so attenuation exactly 0) or behind the
+            // surface (N.L = 0) in every lane adds nothing: the wave skips it.
+            // The waves of a surface face one way, so many of their lights are
+            // behind it (3840x2160, 65,536 lights, whole frame: 1.91 -> 1.56 ms
+            // on smooth surfaces; 1.90 ms either way with independent normals).
             if (fastH) {
                 // L and H from the hardware reciprocal square root (a few ulp)
                 const float dd = __builtin_fmaf(d.z, d.z, __builtin_fmaf(d.y, d.y, d.x * d.x));
-                if (HVX_SHADE_SKIP && !__any(dd < B.w)) return;
-                const float r = __builtin_amdgcn_rsqf(dd);
+                if (HVX_SHADE_SKIP && !__any((dd < B.w) & (ndd > 0.0f))) return;
+                r = __builtin_amdgcn_rsqf(dd);
                 s = dd * r;
                 L = mul3(d, r);
                 const f3 h = add3(V, L);
@@ -313,14 +320,15 @@ __device__ __forceinline__ void shade_one(const ShadeArgs& a, uint32_t idx, uint
                 // exact: L, H and N.H (max with 0 only differs in the sign of
                 // a zero, which no later term can observe)
                 const float dd = dot3(d, d);
-                if (HVX_SHADE_SKIP && !__any(dd < B.w)) return;
+                if (HVX_SHADE_SKIP && !__any((dd < B.w) & (ndd > 0.0f))) return;
                 s = sqrt_rn_normal(dd);
-                L = mul3(d, rcp_rn_normal(s));
+                r = rcp_rn_normal(s);
+                L = mul3(d, r);
                 const f3 h = add3(V, L);
                 Hh = mul3(h, rcp_rn_normal(sqrt_rn_normal(dot3(h, h))));
                 NoH = fmaxf(dot3(N, Hh), 0.0f);
             }
-            const float NoL = fmaxf(__builtin_fmaf(N.z, L.z, __builtin_fmaf(N.y, L.y, N.x * L.x)), 0.0f);
+            const float NoL = fmaxf(ndd * r, 0.0f);
             const float HoV = __builtin_fmaf(Hh.z, V.z, __builtin_fmaf(Hh.y, V.y, Hh.x * V.x));
             // fast: N.L and H.V fused (they enter only smooth factors), then
             // attenuation, D, G, Fresnel and the BRDF sum
@@ -333,12 +341,11 @@ __device__ __forceinline__ void shade_one(const ShadeArgs& a, uint32_t idx, uint
             // D * G_L * G_V / (4 NoV NoL + 1e-4) with one reciprocal of the
             // product of the three denominators (each bounded away from 0);
             // a^2 G_V / pi is a per-fragment constant
-            const float gden = __builtin_fmaf(NoL, omk, alphaRough);
-            const float sden = __builtin_fmaf(nov4, NoL, 0.0001f);
+            const float gsden = __builtin_fmaf(NoL, __builtin_fmaf(NoL, q2, q1), q0);
             const float x = 1.0f - HoV;
             const float x2 = x * x;
             const float p5 = (x2 * x2) * x;
-            const float DGr = (aGVpi * NoL) * rcp_fast(((den * den) * gden) * sden);
+            const float DGr = (aGVpi * NoL) * rcp_fast((den * den) * gsden);
             const float w = att * NoL;
             const float w1 = __builtin_fmaf(-w, p5, w);  // w (1 - p5)
             const float w2 = w * DGr;
