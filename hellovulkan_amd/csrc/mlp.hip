@@ -3,15 +3,19 @@
 // kernels and FP32 master weights (Adam).
 //
 // One training step over a batch of B samples (B a multiple of 256):
-//   pe            X0 = PE(d, lod)                        bf16 [B][128] (+ transpose);
+//   pe            X0 = PE(d, lod)                        bf16 [B][128];
 //                 once per training call when the call revisits its samples
-//   gemm FWD x3   H_l = relu(H_{l-1} W_l^T + b_l)        bf16 [B][64]  (+ transpose)
-//   out           y = H3 W4^T + b4, loss, dY, dZ3 = (dY W4) * [H3 > 0], dW4/db4 partials
-//   per layer l = 3, 2, 1:
-//     gemm PART   dW_l = dZ_l^T H_{l-1}, db_l = sum_b dZ_l   (K = batch, split into
-//                 128-sample slices over waves, reduced in slice order)
-//     gemm BWD    dZ_{l-1} = (dZ_l W_l) * [H_{l-1} > 0]   (l > 1)
-//   adam          FP32 master update and the BF16 copies of W1..W3 (and W2^T, W3^T)
+//   step          per block of 128 samples, everything in LDS: the three
+//                 layers H_l = relu(H_{l-1} W_l^T + b_l), the output layer
+//                 y = H3 W4^T + b4 with the loss, dZ3 = (dY W4) * [H3 > 0],
+//                 dZ_{l-1} = (dZ_l W_l) * [H_{l-1} > 0], and per slice of the
+//                 batch the gradient partials dW_l = dZ_l^T H_{l-1}, db_l, dW4, db4
+//   reduce        the slices' partials summed in slice order, with the Adam
+//                 update of the FP32 masters and of the BF16 copies of W1..W3
+//                 in the same launch
+// HVX_OPT_MLP_SEPARATE_LAUNCHES runs the same step as one launch per product
+// (gemm FWD x3, out, gemm PART and BWD per layer, reductions, adam), with the
+// activations and gradients in memory.
 // Every GEMM is C = A Bt^T with both operands row-major along K, so each MFMA
 // operand load is one contiguous 16-byte read; the epilogues also write the
 // transposed activation that the weight-gradient GEMMs read that way.
@@ -83,43 +87,36 @@ __global__ __launch_bounds__(256) void mlp_data_kernel(const float4* __restrict_
 }
 
 // ----------------------------------------------------------------- encoding
-// thread per (sample, input j, frequency k); rows >= n are the encoding of 0
-// One thread per sample: its 128 features (row of X, sixteen 16-byte
-// stores) and their transposed copies (XT, coalesced across the samples).
-__global__ __launch_bounds__(64) void mlp_pe_kernel(const float4* __restrict__ in, uint32_t n, uint32_t B,
-                                                    float lod_max, bf16* __restrict__ X, bf16* __restrict__ XT) {
-    const uint32_t b = blockIdx.x * 64 + threadIdx.x;
-    if (b >= B) return;
-    float xin[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (b < n) {
-        const float4 v = in[b];
-        xin[0] = v.x;
-        xin[1] = v.y;
-        xin[2] = v.z;
-        xin[3] = 2.0f * v.w / lod_max - 1.0f;
-    }
-    bf16x8* xrow = reinterpret_cast<bf16x8*>(X + (size_t)b * kIn);
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            // frequencies 4 g .. 4 g + 3 of input j, as mlp_sincos evaluates them
-            float sv[4], cv[4];
-            hvx::mlp_sincos_direct(xin[j], 4 * g, sv[0], cv[0]);
-            hvx::mlp_sincos_direct(xin[j], 4 * g + 1, sv[1], cv[1]);
-            hvx::mlp_sincos_double(sv[0], cv[0], sv[2], cv[2]);
-            hvx::mlp_sincos_double(sv[1], cv[1], sv[3], cv[3]);
-            bf16x8 pk;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                pk[2 * q] = (bf16)sv[q];
-                pk[2 * q + 1] = (bf16)cv[q];
-            }
-            xrow[4 * j + g] = pk;
-            const uint32_t c0 = 32 * j + 8 * g;
-#pragma unroll
-            for (int q = 0; q < 8; ++q) XT[(size_t)(c0 + q) * B + b] = pk[q];
+// Sixteen threads per sample, each one 16-byte store of its row of X (8 of the
+// 128 features), so a wave writes 1 KB in one piece; rows >= n are the
+// encoding of 0. XT (may be null): the transposed copy the weight-gradient
+// GEMM of the separate launches reads.
+__global__ __launch_bounds__(256) void mlp_pe_kernel(const float4* __restrict__ in, uint32_t n, uint32_t B,
+                                                     float lod_max, bf16* __restrict__ X, bf16* __restrict__ XT) {
+    const uint32_t j = threadIdx.x / 4 % 4, g = threadIdx.x % 4;
+    for (size_t b = (size_t)blockIdx.x * 16 + threadIdx.x / 16; b < B; b += (size_t)gridDim.x * 16) {
+        float x = 0.0f;
+        if (b < n) {
+            const float4 v = in[b];
+            x = j == 0 ? v.x : (j == 1 ? v.y : (j == 2 ? v.z : 2.0f * v.w / lod_max - 1.0f));
         }
+        // frequencies 4 g .. 4 g + 3 of input j, as mlp_sincos evaluates them
+        float sv[4], cv[4];
+        hvx::mlp_sincos_direct(x, (int)(4 * g), sv[0], cv[0]);
+        hvx::mlp_sincos_direct(x, (int)(4 * g + 1), sv[1], cv[1]);
+        hvx::mlp_sincos_double(sv[0], cv[0], sv[2], cv[2]);
+        hvx::mlp_sincos_double(sv[1], cv[1], sv[3], cv[3]);
+        bf16x8 pk;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            pk[2 * q] = (bf16)sv[q];
+            pk[2 * q + 1] = (bf16)cv[q];
+        }
+        reinterpret_cast<bf16x8*>(X)[b * (kIn / 8) + 4 * j + g] = pk;
+        if (XT)
+#pragma unroll
+            for (int q = 0; q < 8; ++q) XT[(size_t)(32 * j + 8 * g + q) * B + b] = pk[q];
+    }
 }
 
 // -------------------------------------------------------------------- GEMM
@@ -129,7 +126,6 @@ struct GemmArgs {
     const bf16* A;   // [M][Kd]
     const bf16* Bt;  // [Nc][Kd]
     uint32_t M, Nc, Kd, splitk;
-    uint32_t lda, ldb;  // row strides of A and Bt in elements (0: Kd)
     const float* bias;  // FWD: [Nc]
     const bf16* mask;   // BWD: [M][Nc], zero where <= 0
     bf16* C;            // FWD/BWD: [M][Nc]
@@ -146,12 +142,13 @@ __device__ __forceinline__ void gemm_abt_wave(const GemmArgs& g, uint32_t wave, 
     if (wave >= rts * cgs * g.splitk) return;  // uniform per wave; no barriers below
     const uint32_t slice = wave % g.splitk, t = wave / g.splitk, cg = t % cgs, rt = t / cgs;
     const uint32_t ks = g.Kd / 32;
-    const uint32_t kb = slice * ks / g.splitk, ke = (slice + 1) * ks / g.splitk;
+    // PART slices are whole blocks of the fused step's 128 samples
+    constexpr uint32_t unit = EPI == EPI_PART ? 4 : 1;
+    const uint32_t kb = slice * (ks / unit) / g.splitk * unit, ke = (slice + 1) * (ks / unit) / g.splitk * unit;
     const uint32_t i = lane & 15, gq = lane >> 4;
-    const size_t lda = g.lda ? g.lda : g.Kd, ldb = g.ldb ? g.ldb : g.Kd;
-    const bf16* ap = g.A + (size_t)(rt * 16 + i) * lda + 8 * gq;
-    const bf16* bp = g.Bt + (size_t)(cg * 64 + i) * ldb + 8 * gq;
-    const size_t bstep = (size_t)16 * ldb;
+    const bf16* ap = g.A + (size_t)(rt * 16 + i) * g.Kd + 8 * gq;
+    const bf16* bp = g.Bt + (size_t)(cg * 64 + i) * g.Kd + 8 * gq;
+    const size_t bstep = (size_t)16 * g.Kd;
     f32x4 acc[4];
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) acc[nb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -206,19 +203,6 @@ __device__ __forceinline__ void gemm_abt_wave(const GemmArgs& g, uint32_t wave, 
 template <int EPI>
 __global__ __launch_bounds__(256) void gemm_abt_kernel(GemmArgs g) {
     gemm_abt_wave<EPI>(g, blockIdx.x * 4 + (threadIdx.x >> 6), threadIdx.x & 63);
-}
-
-// The three weight-gradient GEMMs of a step in one launch: waves [0, w1)
-// compute g[0], [w1, w2) g[1], the rest g[2], each as gemm_abt_kernel does.
-struct GemmArgs3 {
-    GemmArgs g[3];
-    uint32_t w1, w2;
-};
-__global__ __launch_bounds__(256) void gemm_part3_kernel(GemmArgs3 a) {
-    const uint32_t wave = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (wave < a.w1) gemm_abt_wave<EPI_PART>(a.g[0], wave, lane);
-    else if (wave < a.w2) gemm_abt_wave<EPI_PART>(a.g[1], wave - a.w1, lane);
-    else gemm_abt_wave<EPI_PART>(a.g[2], wave - a.w2, lane);
 }
 
 // ------------------------------------------------------- output and loss
@@ -326,276 +310,464 @@ __global__ __launch_bounds__(64 * kOutRedGroups) void reduce_out_kernel(const fl
 }
 
 // ------------------------------------------------ fused per-sample step
-// The per-sample part of a training step for a block of kOutBlock samples
-// (eight waves, one 16-sample row tile each): the three forward layers, the
-// output layer with the loss and the block's output-layer partials, and the
-// two backward products dZ2 = (dZ3 W3) [H2 > 0], dZ1 = (dZ2 W2) [H1 > 0],
-// with the activations kept in LDS between them. Every product is the MFMA
-// sequence of gemm_abt_kernel over the same BF16 operands and the output
-// part is mlp_out_kernel's, so the results equal those separate launches
-// bit for bit; the activations and gradients the weight-gradient GEMMs read
-// (H_l, dZ_l and their transposes) are written as they write them.
-struct StepArgs {
-    const bf16* X;  // [B][kIn] encodings of the batch
-    const float* P;
-    const bf16 *W[3], *W2T, *W3T;
-    const float4* tgt;
-    uint32_t B;
-    float inv_norm;
-    bf16 *H[3], *HT[3];
-    bf16 *dZ[3], *dZT[3];  // dZ1, dZ2, dZ3 and their transposes
-    float* part;            // [B / kOutBlock][kOutPart]
+// A training step of a slice of the batch, in blocks of kOutBlock samples:
+// forward, output layer, backward and the slice's gradient partials, with
+// every activation and gradient in LDS (131 KB: one workgroup per CU). Every
+// product is the MFMA sequence of gemm_abt_wave over the same BF16 operands,
+// and the output part is mlp_out_kernel's, so the results equal those separate
+// launches bit for bit.
+//
+// 128 samples are 0.1 us of matrix work in a chain of eight dependent
+// products, so the time is latency and the 17 MB of partials. Every global
+// read (the block's encodings, the weights of all five products, one 16-unit
+// column per wave) is asked for at the start, and a stage is an LDS round trip
+// and a barrier. Wave w computes units 16 (w & 3) .. of rows 64 (w >> 2) ..;
+// the products and their derivatives have the same lanes, so the ReLU masks
+// are 16 bits of a register. The gradient GEMMs read the row-major activations
+// through transposing LDS reads (a second, transposed copy took two-byte
+// writes, 7,800 cycles for the encodings alone), and the partials are stored
+// past the L2, whose write-back at the end of the launch cost 2.4 us.
+//
+// A step of 32,768 samples: 53 us (step 29.6, gradient GEMMs over activations
+// in memory 14.3, reductions 5.6, Adam 4.8) -> 21.7 us (step 16.0, reductions
+// with Adam 5.6). Without the partials' stores the step is 12.7 us, without
+// its reads and dW4's serial sums too 9.9: the chain.
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+constexpr uint32_t kStepThreads = 512;
+
+// The step's weights as the matrix operands: fragment (16-row tile nb, 32-K
+// block s) of a product is 64 lanes x 8 values in one piece, so a wave's load
+// is eight whole lines (as rows of W it took half of sixteen: the loads of a
+// workgroup took 13,000 cycles, so 7,500).
+constexpr uint32_t kWs1 = 0, kWs2 = kH * kIn, kWs3 = kWs2 + kH * kH, kWs3T = kWs3 + kH * kH, kWs2T = kWs3T + kH * kH,
+                   kWsLen = kWs2T + kH * kH;
+__device__ __forceinline__ uint32_t operand_index(uint32_t row, uint32_t k, uint32_t K) {
+    return ((row / 16 * (K / 32) + k / 32) * 64 + (k % 32 / 8) * 16 + row % 16) * 8 + k % 8;
+}
+// BF16 copies of parameter i: the rows W1..W3 and the operands of the step
+struct WeightCopies {
+    bf16 *W1, *W2, *W3, *Ws;
 };
-constexpr int kHp = kH + 8;  // LDS row of 64 units (bf16), padded
-
-// C block (16 rows x 64 columns) of A Bt^T: row i of A at arow (this lane's
-// 8 of each 32 K), Bt row i at bt; gemm_abt_kernel's sequence of MFMAs
-template <int KD>
-__device__ __forceinline__ void step_tile(const bf16* arow, const bf16* bt, f32x4 acc[4]) {
-#pragma unroll
-    for (int nb = 0; nb < 4; ++nb) acc[nb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int s = 0; s < KD / 32; ++s) {
-        const bf16x8 a = *reinterpret_cast<const bf16x8*>(arow + 32 * s);
-#pragma unroll
-        for (int nb = 0; nb < 4; ++nb) {
-            const bf16x8 b = *reinterpret_cast<const bf16x8*>(bt + nb * 16 * KD + 32 * s);
-            acc[nb] = hvx::mfma16x16x32(a, b, acc[nb]);
-        }
+__device__ __forceinline__ void write_copies(const WeightCopies& c, uint32_t i, bf16 h) {
+    if (i - (uint32_t)hvx::kMlpW1 < (uint32_t)(kH * kIn)) {
+        const uint32_t j = i - hvx::kMlpW1;
+        c.W1[j] = h;
+        c.Ws[kWs1 + operand_index(j / kIn, j % kIn, kIn)] = h;
+    }
+    if (i - (uint32_t)hvx::kMlpW2 < (uint32_t)(kH * kH)) {
+        const uint32_t j = i - hvx::kMlpW2, o = j / kH, k = j % kH;
+        c.W2[j] = h;
+        c.Ws[kWs2 + operand_index(o, k, kH)] = h;
+        c.Ws[kWs2T + operand_index(k, o, kH)] = h;
+    }
+    if (i - (uint32_t)hvx::kMlpW3 < (uint32_t)(kH * kH)) {
+        const uint32_t j = i - hvx::kMlpW3, o = j / kH, k = j % kH;
+        c.W3[j] = h;
+        c.Ws[kWs3 + operand_index(o, k, kH)] = h;
+        c.Ws[kWs3T + operand_index(k, o, kH)] = h;
     }
 }
 
-// Epilogue of one C block (local rows lr0 .. lr0 + 15 of the block): FWD
-// (bias and ReLU) or BWD (zero where the mask activation is not positive),
-// rounded to BF16 into C, CT (global) and the LDS rows out
-template <bool FWD>
-__device__ __forceinline__ void step_store(const f32x4 acc[4], uint32_t b0, uint32_t lr0, uint32_t B, const float* bias,
-                                           const bf16 (*mask)[kHp], bf16* C, bf16* CT, bf16 (*out)[kHp]) {
-    const uint32_t lane = threadIdx.x & 63, i = lane & 15, gq = lane >> 4;
-#pragma unroll
-    for (int nb = 0; nb < 4; ++nb) {
-        const uint32_t col = nb * 16 + i;
-        bf16 ht[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const uint32_t lrow = lr0 + 4 * gq + r;
-            float v = acc[nb][r];
-            if (FWD) v = fmaxf(v + bias[col], 0.0f);
-            else if (!((float)mask[lrow][col] > 0.0f)) v = 0.0f;
-            const bf16 h = (bf16)v;
-            C[(size_t)(b0 + lrow) * kH + col] = h;
-            if (out) out[lrow][col] = h;
-            ht[r] = h;
-        }
-        typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-        *reinterpret_cast<bf16x4*>(CT + (size_t)col * B + b0 + lr0 + 4 * gq) = bf16x4{ht[0], ht[1], ht[2], ht[3]};
-    }
+// LDS matrices [sample][unit or feature] (and h3t [unit][sample]) without
+// padding: the 16-byte chunks of a row are exchanged by a pattern of the row's
+// low bits such that the sixteen rows of an operand read, the eight rows x two
+// chunks of a transposing read and the rows of a write meet all 64 banks once.
+struct StepShared {
+    __align__(16) bf16 x[kOutBlock * kIn];
+    __align__(16) bf16 h1[kOutBlock * kH], h2[kOutBlock * kH], h3[kOutBlock * kH], z3[kOutBlock * kH],
+        z2[kOutBlock * kH], h3t[kH * kOutBlock];
+    float dy[3][kOutBlock], loss[kOutBlock];
+    float bias[3][kH];
+};
+// element of chunk c of row r, W elements a row
+template <int W> __device__ __forceinline__ uint32_t chunk_at(uint32_t r, uint32_t c) {
+    static_assert(W == kH || W == kIn, "8 or 16 chunks");
+    const uint32_t x = W == kH ? (r >> 2 & 1) | (r & 2) | (r >> 1 & 4) : (r >> 2 & 1) | (r & 3) << 1 | (r & 8);
+    return r * W + ((c ^ x) << 3);
+}
+// chunk c of row r of h3t
+__device__ __forceinline__ uint32_t chunk_t(uint32_t r, uint32_t c) { return r * kOutBlock + ((c ^ (r & 15)) << 3); }
+
+// Row `row`'s 8 values from 32 s + 8 gq as an MFMA operand
+template <int W>
+__device__ __forceinline__ bf16x8 rows_operand(const bf16* m, uint32_t row, uint32_t s, uint32_t gq) {
+    return *reinterpret_cast<const bf16x8*>(m + chunk_at<W>(row, 4 * s + gq));
+}
+// Column 16 ct + i, rows 32 s + 8 gq .. + 7, as an MFMA operand: two
+// transposing reads (each takes 4 rows x 16 columns per 16 lanes, lane j
+// addressing 4 columns of row j / 4, and returns column j).
+template <int W>
+__device__ __forceinline__ bf16x8 cols_operand(const bf16* m, uint32_t s, uint32_t ct, uint32_t i, uint32_t gq) {
+    typedef __attribute__((address_space(3))) s16x4* lds;
+    const uint32_t r = 32 * s + 8 * gq + (i >> 2), c = 2 * ct + (i >> 1 & 1), e = 4 * (i & 1);
+    union {
+        s16x4 s[2];
+        bf16x8 v;
+    } u;
+    u.s[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds)(m + chunk_at<W>(r, c) + e));
+    u.s[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds)(m + chunk_at<W>(r + 4, c) + e));
+    return u.v;
 }
 
-constexpr uint32_t kStepWaves = 8;                           // waves per block
-constexpr uint32_t kStepTiles = kOutBlock / 16 / kStepWaves;  // 16-sample row tiles per wave
-static_assert(kStepTiles >= 1 && kStepTiles * 16 * kStepWaves == kOutBlock, "whole row tiles per wave");
-__global__ __launch_bounds__(64 * kStepWaves) void mlp_step_kernel(StepArgs g) {
-    __shared__ __align__(16) bf16 sH[3][kOutBlock][kHp];  // H1, H2, H3; H3's rows later hold dZ2
-    __shared__ __align__(16) bf16 sZ[kOutBlock][kHp];     // dZ3
-    __shared__ float sdY[kOutBlock][3];
-    __shared__ float sl[kOutBlock];
-    const uint32_t t = threadIdx.x, wave = t >> 6, lane = t & 63, i = lane & 15, gq = lane >> 4;
-    const uint32_t b0 = blockIdx.x * kOutBlock, B = g.B;
-    const int bias[3] = {hvx::kMlpB1, hvx::kMlpB2, hvx::kMlpB3};
-    // forward: each wave its own rows, its row tiles interleaved
+// Partial of dW += dZ^T H over the block, for the 16 units of tile ut and NT
+// tiles of 16 columns from tile c0: lane (g, i) holds unit 16 ut + i, columns
+// 4 g .. of each tile. rs: the unit's sum of dZ over this lane's samples (the bias).
+template <int NT, int W>
+__device__ __forceinline__ void step_partial(const bf16* z, const bf16* h, uint32_t ut, uint32_t c0, uint32_t i,
+                                             uint32_t gq, f32x4 (&acc)[NT], float& rs) {
+#pragma unroll
+    for (uint32_t s = 0; s < kOutBlock / 32; ++s) {
+        const bf16x8 zo = cols_operand<kH>(z, s, ut, i, gq);
+#pragma unroll
+        for (int n = 0; n < NT; ++n) acc[n] = hvx::mfma16x16x32(cols_operand<W>(h, s, c0 + n, i, gq), zo, acc[n]);
+        float t = 0.0f;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) t += (float)zo[q];
+        rs += t;
+    }
+}
+template <int NT>
+__device__ __forceinline__ void step_write_partial(float* part, uint32_t K, uint32_t ut, uint32_t c0, uint32_t i,
+                                                   uint32_t gq, const f32x4 (&acc)[NT], float rs) {
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+        __builtin_nontemporal_store(
+            acc[n], reinterpret_cast<f32x4*>(part + (size_t)(16 * ut + i) * K + 16 * (c0 + n) + 4 * gq));
+    rs += __shfl_xor(rs, 16, 64);
+    rs += __shfl_xor(rs, 32, 64);
+    if (c0 == 0 && gq == 0) part[(size_t)kH * K + 16 * ut + i] = rs;
+}
+
+// X: [blocks * kOutBlock][kIn] encodings; Ws: the weights in operand order;
+// slice q of the launch takes blocks q * blocks / slices ..; part: per layer,
+// then slice, [kH][K] and the bias gradient [kH]; opart: [blocks][kOutPart]
+constexpr uint32_t kLen1 = kH * kIn + kH, kLen23 = kH * kH + kH;  // a layer's partial
+__global__ __launch_bounds__(kStepThreads) void mlp_step_kernel(const bf16* __restrict__ X, const float* __restrict__ P,
+                                                                const bf16* __restrict__ Ws,
+                                                                const float4* __restrict__ tgt, uint32_t blocks,
+                                                                float inv_norm, float* __restrict__ part,
+                                                                float* __restrict__ opart) {
+    __shared__ StepShared sh;
+    const uint32_t t = threadIdx.x;
+    uint32_t lane = t & 63;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(t >> 6), nb = wave & 3, r0 = (wave >> 2) * 64;
+    const uint32_t ut = wave >> 1, ch = wave & 1;   // its tile of units and half of the columns in the partials
+    const uint32_t tg = wave >> 1;                  // output layer: unit group (as mlp_output's g)
+
+    // the encodings: wave w fetches rows 16 w ..
+    bf16x8 x[4];
+    float4 tv;
+    auto fetch = [&](uint32_t q) {
+        const bf16* xp = X + ((size_t)q * kOutBlock + 16 * wave) * kIn;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) x[s] = *reinterpret_cast<const bf16x8*>(xp + 4 * s * kIn + 8 * lane);
+        tv = tgt[(size_t)q * kOutBlock + (wave & 1) * 64 + lane];
+    };
+    const uint32_t q0 = blockIdx.x * blocks / gridDim.x, q1 = (blockIdx.x + 1) * blocks / gridDim.x;
+    fetch(q0);
+    // this wave's fragment s of a product's weights
+    auto weights = [&](uint32_t ofs, uint32_t frags, uint32_t s) {
+        return *reinterpret_cast<const bf16x8*>(Ws + ofs + (nb * frags + s) * 512 + 8 * lane);
+    };
+    bf16x8 w1[4], w2[2], w3[2], w3t[2], w2t[2];
+#pragma unroll
+    for (uint32_t s = 0; s < 4; ++s) w1[s] = weights(kWs1, 4, s);
+#pragma unroll
+    for (uint32_t s = 0; s < 2; ++s) {
+        w2[s] = weights(kWs2, 2, s);
+        w3[s] = weights(kWs3, 2, s);
+        w3t[s] = weights(kWs3T, 2, s);
+        w2t[s] = weights(kWs2T, 2, s);
+    }
+    const uint32_t bl = t / kH;  // threads 0 .. 191: the biases
+    const float bias = t < 3 * kH ? P[(bl == 0 ? hvx::kMlpB1 : (bl == 1 ? hvx::kMlpB2 : hvx::kMlpB3)) + t % kH] : 0.0f;
+    float w4[3][16], b4[3];  // output weights of the thread's 16 units (uniform over the wave)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        b4[c] = P[hvx::kMlpB4 + c];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) w4[c][j] = P[hvx::kMlpW4 + c * kH + 16 * (j >> 2) + 4 * tg + (j & 3)];
+    }
+    __builtin_amdgcn_sched_barrier(0);  // every read above is on its way before the first wait
+    if (t < 3 * kH) sh.bias[bl][t % kH] = bias;
+
+    const f32x4 zero{0.0f, 0.0f, 0.0f, 0.0f};
+    f32x4 p1[4] = {zero, zero, zero, zero}, p2[2] = {zero, zero}, p3[2] = {zero, zero};
+    float rs1 = 0.0f, rs2 = 0.0f, rs3 = 0.0f;
 #pragma unroll 1
-    for (int l = 0; l < 3; ++l) {
-        f32x4 acc[kStepTiles][4];
+    for (uint32_t q = q0; q < q1; ++q) {
+        if (q > q0) __syncthreads();  // the block before has been read
+        // the LDS addresses are made anew for every block: hoisted out of the
+        // loop they take more registers than there are
+        __asm__ volatile("" : "+v"(lane));
+        const uint32_t i = lane & 15, gq = lane >> 4, ts = (wave & 1) * 64 + lane;
+        const uint32_t un = 16 * nb + 4 * gq;  // this lane's four units in the forward and backward products
 #pragma unroll
-        for (uint32_t rt = 0; rt < kStepTiles; ++rt) {
-            const uint32_t lr0 = (wave * kStepTiles + rt) * 16;
-            if (l == 0)
-                step_tile<kIn>(g.X + (size_t)(b0 + lr0 + i) * kIn + 8 * gq, g.W[0] + (size_t)i * kIn + 8 * gq, acc[rt]);
-            else
-                step_tile<kH>(&sH[l - 1][lr0 + i][8 * gq], g.W[l] + (size_t)i * kH + 8 * gq, acc[rt]);
-        }
-#pragma unroll
-        for (uint32_t rt = 0; rt < kStepTiles; ++rt)
-            step_store<true>(acc[rt], b0, (wave * kStepTiles + rt) * 16, B, g.P + bias[l], nullptr, g.H[l], g.HT[l],
-                             sH[l]);
+        for (int s = 0; s < 4; ++s)
+            *reinterpret_cast<bf16x8*>(sh.x + chunk_at<kIn>(16 * wave + 4 * s + gq, i)) = x[s];
+        const float want[3] = {tv.x, tv.y, tv.z};
+        if (q + 1 < q1) fetch(q + 1);
         __syncthreads();
-    }
-    // output layer, loss, dZ3 (one thread per sample)
-    const float* W4 = g.P + hvx::kMlpW4;
-    const float* b4 = g.P + hvx::kMlpB4;
-    if (t < kOutBlock) {
-        float h[kH];
+        // 64 rows of a product: units un .. of row r0 + 16 rt + i
+        uint32_t m1 = 0, m2 = 0, m3 = 0;
+        auto put = [&](bf16x4 h, int rt, bf16* out) {
+            *reinterpret_cast<bf16x4*>(out + chunk_at<kH>(r0 + 16 * rt + i, un >> 3) + (un & 4)) = h;
+        };
+        auto relu = [&](const f32x4 (&acc)[4], int l, uint32_t& mask, bf16* out) {
+            const f32x4 b = *reinterpret_cast<const f32x4*>(&sh.bias[l][un]);
 #pragma unroll
-        for (int k = 0; k < kH; ++k) h[k] = (float)sH[2][t][k];
-        float y[3];
+            for (int rt = 0; rt < 4; ++rt) {
+                bf16x4 h;
 #pragma unroll
-        for (int c = 0; c < 3; ++c) y[c] = hvx::mlp_output(h, W4 + c * kH, b4[c]);
-        const float4 tv = g.tgt[b0 + t];
-        const float e0 = y[0] - tv.x, e1 = y[1] - tv.y, e2 = y[2] - tv.z;
-        sdY[t][0] = e0 * g.inv_norm;
-        sdY[t][1] = e1 * g.inv_norm;
-        sdY[t][2] = e2 * g.inv_norm;
-        sl[t] = (e0 * e0 + e1 * e1) + e2 * e2;
-#pragma unroll
-        for (int k8 = 0; k8 < kH / 8; ++k8) {
-            bf16x8 pk;
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                const int k = 8 * k8 + q;
-                const float dh = (sdY[t][0] * W4[k] + sdY[t][1] * W4[kH + k]) + sdY[t][2] * W4[2 * kH + k];
-                const bf16 v = (bf16)(h[k] > 0.0f ? dh : 0.0f);
-                pk[q] = v;
-                g.dZT[2][(size_t)k * B + b0 + t] = v;
-                sZ[t][k] = v;
+                for (int r = 0; r < 4; ++r) {
+                    h[r] = (bf16)fmaxf(acc[rt][r] + b[r], 0.0f);
+                    mask |= (float)h[r] > 0.0f ? 1u << (4 * rt + r) : 0u;
+                }
+                put(h, rt, out);
             }
-            reinterpret_cast<bf16x8*>(g.dZ[2] + (size_t)(b0 + t) * kH)[k8] = pk;
+        };
+        auto masked = [&](const f32x4 (&acc)[4], uint32_t mask, bf16* out) {
+#pragma unroll
+            for (int rt = 0; rt < 4; ++rt) {
+                bf16x4 h;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) h[r] = (bf16)(mask >> (4 * rt + r) & 1u ? acc[rt][r] : 0.0f);
+                put(h, rt, out);
+            }
+        };
+        auto product = [&](const bf16* in, const bf16x8 (&w)[2], f32x4 (&acc)[4]) {
+#pragma unroll
+            for (int rt = 0; rt < 4; ++rt) {
+                acc[rt] = zero;
+#pragma unroll
+                for (uint32_t s = 0; s < 2; ++s)
+                    acc[rt] = hvx::mfma16x16x32(w[s], rows_operand<kH>(in, r0 + 16 * rt + i, s, gq), acc[rt]);
+            }
+        };
+        f32x4 acc[4];
+#pragma unroll
+        for (int rt = 0; rt < 4; ++rt) {
+            acc[rt] = zero;
+#pragma unroll
+            for (uint32_t s = 0; s < 4; ++s)
+                acc[rt] = hvx::mfma16x16x32(w1[s], rows_operand<kIn>(sh.x, r0 + 16 * rt + i, s, gq), acc[rt]);
         }
-    }
-    __syncthreads();
-    float* pp = g.part + (size_t)blockIdx.x * kOutPart;
-    static_assert(64 * kStepWaves >= (uint32_t)kOutPart - 1, "one thread per output-layer partial");
-    if (t < 3 * kH) {
-        const uint32_t c = t / kH, k = t % kH;
-        float acc = 0.0f;
-        for (uint32_t j = 0; j < kOutBlock; ++j) acc += sdY[j][c] * (float)sH[2][j][k];
-        pp[t] = acc;
-    } else if (t < 3 * kH + 3) {
-        const uint32_t c = t - 3 * kH;
-        float acc = 0.0f;
-        for (uint32_t j = 0; j < kOutBlock; ++j) acc += sdY[j][c];
-        pp[t] = acc;
-    }
-    for (uint32_t hh = kOutBlock / 2; hh > 0; hh >>= 1) {
+        relu(acc, 0, m1, sh.h1);
         __syncthreads();
-        if (t < hh) sl[t] += sl[t + hh];
-    }
-    if (t == 0) pp[kOutPart - 1] = sl[0];
-    __syncthreads();  // H3 is read for the last time above
-    // dZ2 = (dZ3 W3) [H2 > 0] into H3's rows, then dZ1 = (dZ2 W2) [H1 > 0]
-    {
-        f32x4 acc[kStepTiles][4];
+        product(sh.h1, w2, acc);
+        relu(acc, 1, m2, sh.h2);
+        __syncthreads();
+        product(sh.h2, w3, acc);
+        relu(acc, 2, m3, sh.h3);
+        __syncthreads();
+        // output layer: a quarter of a sample's units per thread, in the order
+        // of mlp_output; the partial sums meet in z2. H3's transpose for dW4.
+        float(*py)[3][kOutBlock] = reinterpret_cast<float(*)[3][kOutBlock]>(sh.z2);
+        static_assert(sizeof(sh.z2) >= 4 * 3 * kOutBlock * sizeof(float), "partial sums fit");
+        float h3[16];
 #pragma unroll
-        for (uint32_t rt = 0; rt < kStepTiles; ++rt)
-            step_tile<kH>(&sZ[(wave * kStepTiles + rt) * 16 + i][8 * gq], g.W3T + (size_t)i * kH + 8 * gq, acc[rt]);
+        for (uint32_t j = 0; j < 4; ++j) {
+            const bf16x4 h = *reinterpret_cast<const bf16x4*>(sh.h3 + chunk_at<kH>(ts, 2 * j + (tg >> 1)) + 4 * (tg & 1));
 #pragma unroll
-        for (uint32_t rt = 0; rt < kStepTiles; ++rt)
-            step_store<false>(acc[rt], b0, (wave * kStepTiles + rt) * 16, B, nullptr, sH[1], g.dZ[1], g.dZT[1], sH[2]);
-    }
-    __syncthreads();
-    {
-        f32x4 acc[kStepTiles][4];
+            for (int r = 0; r < 4; ++r) h3[4 * j + r] = (float)h[r];
+        }
 #pragma unroll
-        for (uint32_t rt = 0; rt < kStepTiles; ++rt)
-            step_tile<kH>(&sH[2][(wave * kStepTiles + rt) * 16 + i][8 * gq], g.W2T + (size_t)i * kH + 8 * gq,
-                          acc[rt]);
+        for (uint32_t s = 0; s < 2; ++s)
+            *reinterpret_cast<bf16x8*>(sh.h3t + chunk_t(16 * ut + i, 4 * (2 * ch + s) + gq)) =
+                cols_operand<kH>(sh.h3, 2 * ch + s, ut, i, gq);
 #pragma unroll
-        for (uint32_t rt = 0; rt < kStepTiles; ++rt)
-            step_store<false>(acc[rt], b0, (wave * kStepTiles + rt) * 16, B, nullptr, sH[0], g.dZ[0], g.dZT[0],
-                              nullptr);
+        for (int c = 0; c < 3; ++c) {
+            float v = h3[0] * w4[c][0];
+#pragma unroll
+            for (int j = 1; j < 16; ++j) v = v + h3[j] * w4[c][j];
+            py[tg][c][ts] = v;
+        }
+        __syncthreads();
+        // the loss and dZ3
+        {
+            float e[3], dy[3];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                e[c] = ((py[0][c][ts] + py[1][c][ts]) + (py[2][c][ts] + py[3][c][ts])) + b4[c] - want[c];
+                dy[c] = e[c] * inv_norm;
+            }
+            if (tg == 0) {
+#pragma unroll
+                for (int c = 0; c < 3; ++c) sh.dy[c][ts] = dy[c];
+                sh.loss[ts] = (e[0] * e[0] + e[1] * e[1]) + e[2] * e[2];
+            }
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j) {
+                bf16x4 z;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int k = 4 * j + r;
+                    const float dh = (dy[0] * w4[0][k] + dy[1] * w4[1][k]) + dy[2] * w4[2][k];
+                    z[r] = (bf16)(h3[k] > 0.0f ? dh : 0.0f);
+                }
+                *reinterpret_cast<bf16x4*>(sh.z3 + chunk_at<kH>(ts, 2 * j + (tg >> 1)) + 4 * (tg & 1)) = z;
+            }
+        }
+        __syncthreads();
+        // dZ2, the partials of layer 3 and of the output layer
+        product(sh.z3, w3t, acc);
+        masked(acc, m2, sh.z2);
+        float* pp = opart + (size_t)q * kOutPart;
+        if (wave < 3) {  // dW4[wave][lane]: the samples in order
+            float sum = 0.0f;
+#pragma unroll 1
+            for (uint32_t c0 = 0; c0 < kOutBlock / 8; c0 += 4) {
+                bf16x8 h[4];
+                f32x4 d[8];
+#pragma unroll
+                for (uint32_t c = 0; c < 4; ++c) {
+                    h[c] = *reinterpret_cast<const bf16x8*>(sh.h3t + chunk_t(lane, c0 + c));
+                    d[2 * c] = *reinterpret_cast<const f32x4*>(&sh.dy[wave][8 * (c0 + c)]);
+                    d[2 * c + 1] = *reinterpret_cast<const f32x4*>(&sh.dy[wave][8 * (c0 + c) + 4]);
+                }
+#pragma unroll
+                for (uint32_t j = 0; j < 32; ++j) sum += d[j / 4][j % 4] * (float)h[j / 8][j % 8];
+            }
+            pp[wave * kH + lane] = sum;
+        } else if (wave == 3) {
+            if (lane < 3) {
+                float sum = 0.0f;
+#pragma unroll 8
+                for (uint32_t j = 0; j < kOutBlock; j += 4) {
+                    const f32x4 d = *reinterpret_cast<const f32x4*>(&sh.dy[lane][j]);
+                    sum += d[0];
+                    sum += d[1];
+                    sum += d[2];
+                    sum += d[3];
+                }
+                pp[3 * kH + lane] = sum;
+            }
+        } else if (wave == 4) {
+            float v = sh.loss[lane] + sh.loss[lane + 64];
+            for (int d = 32; d > 0; d >>= 1) v += __shfl_down(v, d, 64);
+            if (lane == 0) pp[kOutPart - 1] = v;
+        }
+        step_partial<2, kH>(sh.z3, sh.h2, ut, 2 * ch, i, gq, p3, rs3);
+        const bool last = q + 1 == q1;
+        const size_t sl = blockIdx.x, n = gridDim.x;
+        if (last) step_write_partial<2>(part + n * (kLen1 + kLen23) + sl * kLen23, kH, ut, 2 * ch, i, gq, p3, rs3);
+        __syncthreads();
+        // dZ1 (over dZ3) and the partials of layer 2
+        product(sh.z2, w2t, acc);
+        masked(acc, m1, sh.z3);
+        step_partial<2, kH>(sh.z2, sh.h1, ut, 2 * ch, i, gq, p2, rs2);
+        if (last) step_write_partial<2>(part + n * kLen1 + sl * kLen23, kH, ut, 2 * ch, i, gq, p2, rs2);
+        __syncthreads();
+        step_partial<4, kIn>(sh.z3, sh.x, ut, 4 * ch, i, gq, p1, rs1);
+        if (last) step_write_partial<4>(part + sl * kLen1, kIn, ut, 4 * ch, i, gq, p1, rs1);
     }
 }
 
-// out[i] = scale * sum_s part[s * stride + i] for many slices: a workgroup
-// takes 64 outputs and 16 slice ranges (one per wave), each summed in slice
-// order, then adds the 16 range sums in a fixed tree
+// Sum over the slices of part[s * stride + i] for i < len: a workgroup takes
+// 64 outputs and 16 slice ranges (one per wave), each summed in slice order,
+// then adds the 16 range sums in a fixed tree. True for the lane that then
+// holds output i's sum.
 constexpr uint32_t kRedGroups = 16;
-// out[i] = scale * (sum over slices of part[s * stride + i]) for i < len,
-// except that with `last` set element len - 1 goes to *last (times
-// last_scale) instead
-__device__ __forceinline__ void reduce_slices_block(const float* __restrict__ part, uint32_t slices, uint32_t stride,
-                                                    uint32_t len, float scale, float* __restrict__ out,
-                                                    uint32_t block, float* __restrict__ last = nullptr,
-                                                    float last_scale = 1.0f) {
+__device__ __forceinline__ bool reduce_slices_block(const float* __restrict__ part, uint32_t slices, uint32_t len,
+                                                    uint32_t i, float& sum) {
     __shared__ float sh[kRedGroups][64];
-    const uint32_t l = threadIdx.x & 63, gq = threadIdx.x >> 6, i = block * 64 + l;
+    const uint32_t l = threadIdx.x & 63, gq = threadIdx.x >> 6;
     float acc = 0.0f;
     if (i < len) {
         const uint32_t s0 = gq * slices / kRedGroups, s1 = (gq + 1) * slices / kRedGroups;
-#pragma unroll 8
-        for (uint32_t s = s0; s < s1; ++s) acc += part[(size_t)s * stride + i];
+#pragma unroll 16
+        for (uint32_t s = s0; s < s1; ++s) acc += part[(size_t)s * len + i];
     }
     sh[gq][l] = acc;
-    for (uint32_t h = kRedGroups / 2; h > 0; h >>= 1) {
-        __syncthreads();
-        if (gq < h) sh[gq][l] += sh[gq + h][l];
-    }
-    if (gq != 0 || i >= len) return;
-    if (last && i == len - 1) *last = sh[0][l] * last_scale;
-    else out[i] = sh[0][l] * scale;
+    __syncthreads();
+    if (gq != 0 || i >= len) return false;
+    float v[kRedGroups];
+#pragma unroll
+    for (uint32_t k = 0; k < kRedGroups; ++k) v[k] = sh[k][l];
+#pragma unroll
+    for (uint32_t h = kRedGroups / 2; h > 0; h >>= 1)
+#pragma unroll
+        for (uint32_t k = 0; k < h; ++k) v[k] += v[k + h];
+    sum = v[0];
+    return true;
 }
 __global__ __launch_bounds__(64 * kRedGroups) void reduce_slices_kernel(const float* __restrict__ part,
-                                                                         uint32_t slices, uint32_t stride,
-                                                                         uint32_t len, float scale,
+                                                                         uint32_t slices, uint32_t len,
                                                                          float* __restrict__ out) {
-    reduce_slices_block(part, slices, stride, len, scale, out, blockIdx.x);
+    const uint32_t i = blockIdx.x * 64 + (threadIdx.x & 63);
+    float sum;
+    if (reduce_slices_block(part, slices, len, i, sum)) out[i] = sum;
 }
+
+// Adam step of parameter i; an updated weight also refreshes its BF16 working
+// copies, so a step needs no cast launch.
+struct AdamArgs {
+    float *P, *m, *v;
+    float lr, bc1, bc2;
+    WeightCopies copies;
+};
+struct AdamState {
+    float p, m, v;
+};
+__device__ __forceinline__ AdamState adam_load(const AdamArgs& a, uint32_t i) { return {a.P[i], a.m[i], a.v[i]}; }
+__device__ __forceinline__ void adam_update(const AdamArgs& a, uint32_t i, const AdamState& s, float g) {
+    const float mi = 0.9f * s.m + 0.1f * g, vi = 0.999f * s.v + 0.001f * g * g;
+    a.m[i] = mi;
+    a.v[i] = vi;
+    const float p = s.p - a.lr * (mi / a.bc1) / (sqrtf(vi / a.bc2) + 1e-8f);
+    a.P[i] = p;
+    write_copies(a.copies, i, (bf16)p);
+}
+__global__ __launch_bounds__(256) void adam_kernel(AdamArgs a, const float* __restrict__ G, uint32_t n) {
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) adam_update(a, i, adam_load(a, i), G[i]);
+}
+
 // A step's reductions in one launch: segment k (blocks [b[k], b[k + 1]))
-// reduces len[k] outputs over slices[k] partials of stride[k] into out[k]
-// (scale 1): the three layers' weight gradients and the output layer's block
-// partials, whose last element (the loss, scaled by loss_scale) goes to
-// *loss when it is set (otherwise it is not written).
+// reduces len[k] outputs over slices[k] partials: the three layers' weight
+// and bias gradients and the output layer's block partials, whose last element
+// is the loss (scaled by loss_scale into *loss when it is set). The others
+// are gradients of the parameters from ofs[k] on: into G or, with ADAM,
+// straight into the parameters, which nothing else in this launch reads.
 struct ReduceStep {
     const float* part[4];
-    float* out[4];
-    uint32_t len[4], stride[4], slices[4], b[5];
-    float* loss;
+    uint32_t ofs[4], len[4], slices[4], b[5];
+    float *G, *loss;
     float loss_scale;
+    AdamArgs adam;
 };
-__global__ __launch_bounds__(64 * kRedGroups) void reduce_step_kernel(ReduceStep r) {
+template <bool ADAM> __global__ __launch_bounds__(64 * kRedGroups) void reduce_step_kernel(ReduceStep r) {
     const uint32_t blk = blockIdx.x;
     uint32_t k = 0;
     while (k < 3 && blk >= r.b[k + 1]) ++k;
-    const bool out_layer = k == 3;
-    // without a loss pointer the output layer's last element is not written
-    const uint32_t len = out_layer && !r.loss ? r.len[k] - 1 : r.len[k];
-    reduce_slices_block(r.part[k], r.slices[k], r.stride[k], len, 1.0f, r.out[k], blk - r.b[k],
-                        out_layer ? r.loss : nullptr, r.loss_scale);
-}
-
-
-// Adam step of every parameter; the updated weights also refresh their BF16
-// working copies (as mlp_cast_kernel does), so a step needs no cast launch.
-__global__ __launch_bounds__(256) void adam_kernel(float* __restrict__ P, const float* __restrict__ G,
-                                                   float* __restrict__ m, float* __restrict__ v, uint32_t n, float lr,
-                                                   float bc1, float bc2, bf16* __restrict__ W1, bf16* __restrict__ W2,
-                                                   bf16* __restrict__ W3, bf16* __restrict__ W2T,
-                                                   bf16* __restrict__ W3T) {
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const float g = G[i];
-    const float mi = 0.9f * m[i] + 0.1f * g, vi = 0.999f * v[i] + 0.001f * g * g;
-    m[i] = mi;
-    v[i] = vi;
-    const float p = P[i] - lr * (mi / bc1) / (sqrtf(vi / bc2) + 1e-8f);
-    P[i] = p;
-    const bf16 h = (bf16)p;
-    if (i - (uint32_t)hvx::kMlpW1 < (uint32_t)(kH * kIn)) W1[i - hvx::kMlpW1] = h;
-    if (i - (uint32_t)hvx::kMlpW2 < (uint32_t)(kH * kH)) {
-        const uint32_t j = i - hvx::kMlpW2;
-        W2[j] = h;
-        W2T[(j % kH) * kH + j / kH] = h;
-    }
-    if (i - (uint32_t)hvx::kMlpW3 < (uint32_t)(kH * kH)) {
-        const uint32_t j = i - hvx::kMlpW3;
-        W3[j] = h;
-        W3T[(j % kH) * kH + j / kH] = h;
+    const uint32_t i = (blk - r.b[k]) * 64 + (threadIdx.x & 63), len = r.len[k], at = r.ofs[k] + i;
+    const bool is_loss = k == 3 && i == len - 1;
+    // the state is on its way while the partials are summed
+    AdamState st{};
+    if (ADAM && threadIdx.x < 64 && i < len && !is_loss) st = adam_load(r.adam, at);
+    float sum;
+    if (!reduce_slices_block(r.part[k], r.slices[k], len, i, sum)) return;
+    if (is_loss) {
+        if (r.loss) *r.loss = sum * r.loss_scale;
+    } else if (ADAM) {
+        adam_update(r.adam, at, st, sum);
+    } else {
+        r.G[at] = sum;
     }
 }
 
-// BF16 working copies: W1, W2, W3 as [out][in]; W2^T, W3^T as [in][out]
-__global__ __launch_bounds__(256) void mlp_cast_kernel(const float* __restrict__ P, bf16* __restrict__ W1,
-                                                       bf16* __restrict__ W2, bf16* __restrict__ W3,
-                                                       bf16* __restrict__ W2T, bf16* __restrict__ W3T) {
+// The BF16 working copies of every weight
+__global__ __launch_bounds__(256) void mlp_cast_kernel(const float* __restrict__ P, WeightCopies c) {
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i < (uint32_t)(kH * kIn)) W1[i] = (bf16)P[hvx::kMlpW1 + i];
-    if (i < (uint32_t)(kH * kH)) {
-        const uint32_t o = i / kH, k = i % kH;
-        W2[i] = (bf16)P[hvx::kMlpW2 + i];
-        W3[i] = (bf16)P[hvx::kMlpW3 + i];
-        W2T[k * kH + o] = (bf16)P[hvx::kMlpW2 + i];
-        W3T[k * kH + o] = (bf16)P[hvx::kMlpW3 + i];
-    }
+    if (i < (uint32_t)hvx::kMlpParams) write_copies(c, i, (bf16)P[i]);
+}
+// W2^T and W3^T ([in][out]) for the separate launches' backward products
+__global__ __launch_bounds__(256) void mlp_transpose_kernel(const bf16* __restrict__ W2, const bf16* __restrict__ W3,
+                                                            bf16* __restrict__ W2T, bf16* __restrict__ W3T) {
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x, t = (i % kH) * kH + i / kH;
+    W2T[t] = W2[i];
+    W3T[t] = W3[i];
 }
 
 // Inference through the in-shading path (mlp_device.h): each workgroup
@@ -703,21 +875,23 @@ struct hvx_mlp {
     hvx_ctx* ctx = nullptr;
     float lod_max = 1.0f;
     float *P = nullptr, *G = nullptr, *m = nullptr, *v = nullptr;
-    bf16 *W1 = nullptr, *W2 = nullptr, *W3 = nullptr, *W2T = nullptr, *W3T = nullptr;
+    bf16 *W1 = nullptr, *W2 = nullptr, *W3 = nullptr, *Ws = nullptr;
     uint32_t cap = 0;  // batch capacity
-    bf16 *X0 = nullptr, *X0T = nullptr, *H[3] = {}, *HT[3] = {}, *dZa = nullptr, *dZaT = nullptr, *dZb = nullptr,
-         *dZbT = nullptr, *dZc = nullptr, *dZcT = nullptr;
+    bf16* X0 = nullptr;
     float *part = nullptr, *opart = nullptr;
-    uint32_t splitk = 1;
+    // HVX_OPT_MLP_SEPARATE_LAUNCHES: the activations and gradients in memory
+    uint32_t sep_cap = 0;
+    bf16 *W2T = nullptr, *W3T = nullptr;
+    bf16 *X0T = nullptr, *H[3] = {}, *HT[3] = {}, *dZa = nullptr, *dZaT = nullptr, *dZb = nullptr, *dZbT = nullptr;
     uint64_t steps_done = 0;
-    // a training call's inputs encoded once: [n][kIn] and [kIn][enc_cap]
-    bf16 *enc = nullptr, *encT = nullptr;
+    // a training call's inputs encoded once: [n][kIn]
+    bf16* enc = nullptr;
     size_t enc_cap = 0;
     // per-cell estimate from below of the network's output, from the last
     // hvx_mlp_cell_errors call (cell grid lo_face x lo_face x lo_bins)
     float4* cell_lo = nullptr;  // RGB and a pad per cell
     uint32_t lo_face = 0, lo_bins = 0;
-    std::vector<void*> batch_allocs;
+    std::vector<void*> batch_allocs, sep_allocs;
     std::vector<void*> allocs;
 };
 
@@ -749,27 +923,44 @@ template <class T> hipError_t dalloc(std::vector<void*>& list, T** p, size_t cou
     return e;
 }
 
+// slices of a batch's gradient partials (whole blocks of kOutBlock samples)
+uint32_t slices_of(uint32_t B) { return std::min(256u, B / kOutBlock); }
+
+void encode(const float4* in, uint32_t n, uint32_t B, float lod_max, bf16* X, bf16* XT, hipStream_t s) {
+    hipLaunchKernelGGL(mlp_pe_kernel, dim3(std::min((B + 15) / 16, 1u << 18)), dim3(256), 0, s, in, n, B, lod_max, X, XT);
+}
+
 hipError_t ensure_batch(hvx_mlp* M, uint32_t B) {
-    if (B <= M->cap) return hipSuccess;
+    const bool separate = M->ctx->mlp_separate != 0;
+    if (B <= M->cap && (!separate || B <= M->sep_cap)) return hipSuccess;
     hipError_t e = hipDeviceSynchronize();
     if (e != hipSuccess) return e;
-    for (void* p : M->batch_allocs) (void)hipFree(p);
-    M->batch_allocs.clear();
-    M->cap = 0;
-    auto& L = M->batch_allocs;
-    // weight gradients are [64][<=128] GEMMs over K = B: split K into slices
-    // of 128 samples (up to 256) so that the GEMM has 1-2 k waves
-    M->splitk = std::max(1u, std::min(256u, B / 128));
-    if ((e = dalloc(L, &M->X0, (size_t)B * kIn)) || (e = dalloc(L, &M->X0T, (size_t)B * kIn))) return e;
-    for (int l = 0; l < 3; ++l)
-        if ((e = dalloc(L, &M->H[l], (size_t)B * kH)) || (e = dalloc(L, &M->HT[l], (size_t)B * kH))) return e;
-    if ((e = dalloc(L, &M->dZa, (size_t)B * kH)) || (e = dalloc(L, &M->dZaT, (size_t)B * kH)) ||
-        (e = dalloc(L, &M->dZb, (size_t)B * kH)) || (e = dalloc(L, &M->dZbT, (size_t)B * kH)) ||
-        (e = dalloc(L, &M->dZc, (size_t)B * kH)) || (e = dalloc(L, &M->dZcT, (size_t)B * kH)) ||
-        (e = dalloc(L, &M->part, (size_t)M->splitk * ((kH * kIn + kH) + 2 * (kH * kH + kH)))) ||
-        (e = dalloc(L, &M->opart, (size_t)(B / kOutBlock) * kOutPart)))
-        return e;
-    M->cap = B;
+    if (B > M->cap) {
+        for (void* p : M->batch_allocs) (void)hipFree(p);
+        M->batch_allocs.clear();
+        M->cap = 0;
+        auto& L = M->batch_allocs;
+        if ((e = dalloc(L, &M->X0, (size_t)B * kIn)) ||
+            (e = dalloc(L, &M->part, (size_t)slices_of(B) * ((kH * kIn + kH) + 2 * (kH * kH + kH)))) ||
+            (e = dalloc(L, &M->opart, (size_t)(B / kOutBlock) * kOutPart)))
+            return e;
+        M->cap = B;
+    }
+    if (separate && B > M->sep_cap) {
+        for (void* p : M->sep_allocs) (void)hipFree(p);
+        M->sep_allocs.clear();
+        M->sep_cap = 0;
+        auto& L = M->sep_allocs;
+        if ((e = dalloc(L, &M->W2T, (size_t)kH * kH)) || (e = dalloc(L, &M->W3T, (size_t)kH * kH)) ||
+            (e = dalloc(L, &M->X0T, (size_t)B * kIn)))
+            return e;
+        for (int l = 0; l < 3; ++l)
+            if ((e = dalloc(L, &M->H[l], (size_t)B * kH)) || (e = dalloc(L, &M->HT[l], (size_t)B * kH))) return e;
+        if ((e = dalloc(L, &M->dZa, (size_t)B * kH)) || (e = dalloc(L, &M->dZaT, (size_t)B * kH)) ||
+            (e = dalloc(L, &M->dZb, (size_t)B * kH)) || (e = dalloc(L, &M->dZbT, (size_t)B * kH)))
+            return e;
+        M->sep_cap = B;
+    }
     return hipSuccess;
 }
 
@@ -778,14 +969,12 @@ template <int EPI> void gemm(const GemmArgs& g, hipStream_t s) {
     hipLaunchKernelGGL(gemm_abt_kernel<EPI>, dim3((waves + 3) / 4), dim3(256), 0, s, g);
 }
 
-// forward of B (padded) samples, n of them real; x0: their encoding, if
-// already made
-void forward(hvx_mlp* M, const float4* in, uint32_t n, uint32_t B, hipStream_t s, const bf16* x0 = nullptr) {
-    if (!x0)
-        hipLaunchKernelGGL(mlp_pe_kernel, dim3((B + 63) / 64), dim3(64), 0, s, in, n, B, M->lod_max, M->X0, M->X0T);
+// forward of B samples, as separate launches
+void forward(hvx_mlp* M, const float4* in, uint32_t B, hipStream_t s) {
+    encode(in, B, B, M->lod_max, M->X0, M->X0T, s);
     const bf16* Ws[3] = {M->W1, M->W2, M->W3};
     const int bias[3] = {hvx::kMlpB1, hvx::kMlpB2, hvx::kMlpB3};
-    const bf16* prev = x0 ? x0 : M->X0;
+    const bf16* prev = M->X0;
     for (int l = 0; l < 3; ++l) {
         GemmArgs g{};
         g.A = prev;
@@ -803,36 +992,28 @@ void forward(hvx_mlp* M, const float4* in, uint32_t n, uint32_t B, hipStream_t s
 }
 
 // gradient of the mean squared log-radiance error over B samples into G (and
-// the loss into *loss); x0 / x0t (row stride ldx): the samples' encoding, if
-// already made
-void gradient_fused(hvx_mlp* M, const float4* in, const float4* tgt, uint32_t B, float* G, float* loss,
-                    hipStream_t s, const bf16* x0, const bf16* x0t, uint32_t ldx);
-
-void gradient(hvx_mlp* M, const float4* in, const float4* tgt, uint32_t B, float* G, float* loss, hipStream_t s,
-              const bf16* x0 = nullptr, const bf16* x0t = nullptr, uint32_t ldx = 0) {
-    if (!M->ctx->mlp_separate) {
-        gradient_fused(M, in, tgt, B, G, loss, s, x0, x0t, ldx);
-        return;
-    }
-    forward(M, in, B, B, s, x0);
+// the loss into *loss) as separate launches
+void gradient_separate(hvx_mlp* M, const float4* in, const float4* tgt, uint32_t B, float* G, float* loss,
+                       hipStream_t s) {
+    forward(M, in, B, s);
     const uint32_t nblk = B / kOutBlock;
     hipLaunchKernelGGL(mlp_out_kernel<true>, dim3(nblk), dim3(kOutBlock), 0, s, M->H[2], M->P, tgt, B, B,
                        2.0f / (3.0f * (float)B), nullptr, M->dZa, M->dZaT, M->opart);
     hipLaunchKernelGGL(reduce_out_kernel, dim3((kOutPart + 63) / 64), dim3(64 * kOutRedGroups), 0, s, M->opart, nblk, G + hvx::kMlpW4,
                        1.0f / (3.0f * (float)B), loss);
     const int wofs[3] = {hvx::kMlpW1, hvx::kMlpW2, hvx::kMlpW3};
+    hipLaunchKernelGGL(mlp_transpose_kernel, dim3(kH * kH / 256), dim3(256), 0, s, M->W2, M->W3, M->W2T, M->W3T);
     const bf16* WT[3] = {nullptr, M->W2T, M->W3T};
     bf16 *dz = M->dZa, *dzT = M->dZaT, *nz = M->dZb, *nzT = M->dZbT;
     for (int l = 2; l >= 0; --l) {
         const uint32_t K = l == 0 ? kIn : kH;
         GemmArgs g{};
         g.A = dzT;
-        g.Bt = l == 0 ? (x0t ? x0t : M->X0T) : M->HT[l - 1];
-        g.ldb = l == 0 && x0t ? ldx : 0;
+        g.Bt = l == 0 ? M->X0T : M->HT[l - 1];
         g.M = kH;
         g.Nc = K;
         g.Kd = B;
-        g.splitk = M->splitk;
+        g.splitk = slices_of(B);
         g.part = M->part;
         g.pstride = kH * K + kH;
         g.colsum = 1;
@@ -842,7 +1023,7 @@ void gradient(hvx_mlp* M, const float4* in, const float4* tgt, uint32_t B, float
                           hvx::kMlpB3 == hvx::kMlpW3 + kH * kH,
                       "each layer's bias follows its weights");
         hipLaunchKernelGGL(reduce_slices_kernel, dim3((kH * K + kH + 63) / 64), dim3(64 * kRedGroups), 0, s,
-                           M->part, M->splitk, (uint32_t)(kH * K + kH), (uint32_t)(kH * K + kH), 1.0f, G + wofs[l]);
+                           M->part, slices_of(B), (uint32_t)(kH * K + kH), G + wofs[l]);
         if (l > 0) {
             GemmArgs d{};
             d.A = dz;
@@ -861,83 +1042,38 @@ void gradient(hvx_mlp* M, const float4* in, const float4* tgt, uint32_t B, float
     }
 }
 
-// The same gradient with the per-sample work in one launch (mlp_step_kernel),
-// then the three weight-gradient GEMMs and their reductions as in gradient().
-void gradient_fused(hvx_mlp* M, const float4* in, const float4* tgt, uint32_t B, float* G, float* loss,
-                    hipStream_t s, const bf16* x0, const bf16* x0t, uint32_t ldx) {
-    if (!x0)
-        hipLaunchKernelGGL(mlp_pe_kernel, dim3((B + 63) / 64), dim3(64), 0, s, in, B, B, M->lod_max, M->X0, M->X0T);
-    const uint32_t nblk = B / kOutBlock;
-    StepArgs a{};
-    a.X = x0 ? x0 : M->X0;
-    a.P = M->P;
-    a.W[0] = M->W1;
-    a.W[1] = M->W2;
-    a.W[2] = M->W3;
-    a.W2T = M->W2T;
-    a.W3T = M->W3T;
-    a.tgt = tgt;
-    a.B = B;
-    a.inv_norm = 2.0f / (3.0f * (float)B);
-    for (int l = 0; l < 3; ++l) {
-        a.H[l] = M->H[l];
-        a.HT[l] = M->HT[l];
-    }
-    a.dZ[0] = M->dZc;
-    a.dZT[0] = M->dZcT;
-    a.dZ[1] = M->dZb;
-    a.dZT[1] = M->dZbT;
-    a.dZ[2] = M->dZa;
-    a.dZT[2] = M->dZaT;
-    a.part = M->opart;
-    hipLaunchKernelGGL(mlp_step_kernel, dim3(nblk), dim3(64 * kStepWaves), 0, s, a);
-    // the three weight-gradient GEMMs in one launch, each into its own
-    // partials, then their reductions in one launch (the same per-wave and
-    // per-output work as separate launches)
-    const int wofs[3] = {hvx::kMlpW1, hvx::kMlpW2, hvx::kMlpW3};
-    GemmArgs3 g3{};
-    ReduceStep r3{};
+// The same gradient in two launches (and the encoding, if x0 does not hold
+// it): mlp_step_kernel and the reduction of its partials, into G or, with
+// adam set, straight into the parameters.
+void gradient_fused(hvx_mlp* M, const float4* in, const bf16* x0, const float4* tgt, uint32_t B, float* G,
+                    const AdamArgs* adam, float* loss, hipStream_t s) {
+    if (!x0) encode(in, B, B, M->lod_max, M->X0, nullptr, s);
+    const uint32_t blocks = B / kOutBlock, slices = slices_of(B);
+    const int wofs[4] = {hvx::kMlpW1, hvx::kMlpW2, hvx::kMlpW3, hvx::kMlpW4};
+    ReduceStep r{};
     float* part = M->part;
-    uint32_t waves = 0;
-    for (int l = 0; l < 3; ++l) {
-        const uint32_t K = l == 0 ? kIn : kH, len = kH * K + kH;
-        GemmArgs& g = g3.g[l];
-        g.A = a.dZT[l];
-        g.Bt = l == 0 ? (x0t ? x0t : M->X0T) : M->HT[l - 1];
-        g.ldb = l == 0 && x0t ? ldx : 0;
-        g.M = kH;
-        g.Nc = K;
-        g.Kd = B;
-        g.splitk = M->splitk;
-        g.part = part;
-        g.pstride = len;
-        g.colsum = 1;
-        r3.part[l] = part;
-        r3.out[l] = G + wofs[l];
-        r3.len[l] = r3.stride[l] = len;
-        r3.slices[l] = M->splitk;
-        r3.b[l + 1] = r3.b[l] + (len + 63) / 64;
-        part += (size_t)M->splitk * len;
-        const uint32_t w = (g.M / 16) * (g.Nc / 64) * g.splitk;
-        if (l == 0) g3.w1 = w;
-        else if (l == 1) g3.w2 = g3.w1 + w;
-        waves += w;
+    for (int l = 0; l < 4; ++l) {
+        const uint32_t len = l == 3 ? kOutPart : (l == 0 ? kLen1 : kLen23);
+        r.part[l] = l == 3 ? M->opart : part;
+        r.ofs[l] = wofs[l];
+        r.len[l] = len;
+        r.slices[l] = l == 3 ? blocks : slices;
+        r.b[l + 1] = r.b[l] + (len + 63) / 64;
+        if (l < 3) part += (size_t)slices * len;
     }
-    // the output layer: dW4, db4 and the loss from the step kernel's block partials
-    r3.part[3] = M->opart;
-    r3.out[3] = G + hvx::kMlpW4;
-    r3.len[3] = r3.stride[3] = kOutPart;
-    r3.slices[3] = nblk;
-    r3.b[4] = r3.b[3] + (kOutPart + 63) / 64;
-    r3.loss = loss;
-    r3.loss_scale = 1.0f / (3.0f * (float)B);
-    hipLaunchKernelGGL(gemm_part3_kernel, dim3((waves + 3) / 4), dim3(256), 0, s, g3);
-    hipLaunchKernelGGL(reduce_step_kernel, dim3(r3.b[4]), dim3(64 * kRedGroups), 0, s, r3);
+    r.loss = loss;
+    r.loss_scale = 1.0f / (3.0f * (float)B);
+    r.G = G;
+    if (adam) r.adam = *adam;
+    hipLaunchKernelGGL(mlp_step_kernel, dim3(slices), dim3(kStepThreads), 0, s, x0 ? x0 : M->X0, M->P, M->Ws,
+                       tgt, blocks, 2.0f / (3.0f * (float)B), M->part, M->opart);
+    if (adam) hipLaunchKernelGGL(reduce_step_kernel<true>, dim3(r.b[4]), dim3(64 * kRedGroups), 0, s, r);
+    else hipLaunchKernelGGL(reduce_step_kernel<false>, dim3(r.b[4]), dim3(64 * kRedGroups), 0, s, r);
 }
 
 void cast(hvx_mlp* M, hipStream_t s) {
-    hipLaunchKernelGGL(mlp_cast_kernel, dim3(kH * kIn / 256), dim3(256), 0, s, M->P, M->W1, M->W2, M->W3, M->W2T,
-                       M->W3T);
+    hipLaunchKernelGGL(mlp_cast_kernel, dim3((hvx::kMlpParams + 255) / 256), dim3(256), 0, s, M->P,
+                       WeightCopies{M->W1, M->W2, M->W3, M->Ws});
 }
 
 int bind(hvx_ctx* ctx) {
@@ -967,7 +1103,7 @@ int hvx_mlp_create(hvx_ctx* ctx, float lod_max, uint64_t seed, hvx_mlp** out) {
     if ((e = dalloc(L, &M->P, np)) || (e = dalloc(L, &M->G, np)) || (e = dalloc(L, &M->m, np)) ||
         (e = dalloc(L, &M->v, np)) || (e = dalloc(L, &M->W1, (size_t)kH * kIn)) ||
         (e = dalloc(L, &M->W2, (size_t)kH * kH)) || (e = dalloc(L, &M->W3, (size_t)kH * kH)) ||
-        (e = dalloc(L, &M->W2T, (size_t)kH * kH)) || (e = dalloc(L, &M->W3T, (size_t)kH * kH))) {
+        (e = dalloc(L, &M->Ws, (size_t)kWsLen))) {
         hvx_mlp_destroy(M);
         return mfail(ctx, HVX_ERR_HIP, "hvx_mlp_create: %s", hipGetErrorString(e));
     }
@@ -1008,9 +1144,9 @@ int hvx_mlp_destroy(hvx_mlp* M) {
     if (!M) return HVX_ERR_NULL;
     (void)hipDeviceSynchronize();
     for (void* p : M->batch_allocs) (void)hipFree(p);
+    for (void* p : M->sep_allocs) (void)hipFree(p);
     for (void* p : M->allocs) (void)hipFree(p);
     if (M->enc) (void)hipFree(M->enc);
-    if (M->encT) (void)hipFree(M->encT);
     if (M->cell_lo) (void)hipFree(M->cell_lo);
     delete M;
     return HVX_OK;
@@ -1055,8 +1191,9 @@ int hvx_mlp_gradient(hvx_mlp* M, const float* d_inputs, const float* d_targets, 
     if ((st = bind(M->ctx))) return st;
     hipError_t e = ensure_batch(M, batch);
     if (e != hipSuccess) return mfail(M->ctx, HVX_ERR_HIP, "hvx_mlp_gradient: %s", hipGetErrorString(e));
-    gradient(M, reinterpret_cast<const float4*>(d_inputs), reinterpret_cast<const float4*>(d_targets), batch, d_grads,
-             d_loss, (hipStream_t)stream);
+    const float4 *in = reinterpret_cast<const float4*>(d_inputs), *tg = reinterpret_cast<const float4*>(d_targets);
+    if (M->ctx->mlp_separate) gradient_separate(M, in, tg, batch, d_grads, d_loss, (hipStream_t)stream);
+    else gradient_fused(M, in, nullptr, tg, batch, d_grads, nullptr, d_loss, (hipStream_t)stream);
     e = hipGetLastError();
     return e == hipSuccess ? HVX_OK : mfail(M->ctx, HVX_ERR_HIP, "hvx_mlp_gradient: %s", hipGetErrorString(e));
 }
@@ -1074,43 +1211,40 @@ int hvx_mlp_train(hvx_mlp* M, const float* d_inputs, const float* d_targets, uin
     const uint32_t per_epoch = n / batch;
     const float4* in = reinterpret_cast<const float4*>(d_inputs);
     const float4* tg = reinterpret_cast<const float4*>(d_targets);
-    // Encode the call's samples once (2 x 256 B per sample) when they are
+    // Encode the call's samples once (256 B per sample) when they are
     // revisited, instead of once per step; without the memory, each step
-    // encodes its batch.
-    const size_t npad = ((size_t)per_epoch * batch + 255) / 256 * 256;
-    if (steps > per_epoch && M->enc_cap < npad) {
+    // encodes its batch (as the separate launches always do).
+    const bool separate = M->ctx->mlp_separate != 0;
+    const size_t npad = (size_t)per_epoch * batch;
+    const bool revisit = steps > per_epoch && !separate;
+    if (revisit && M->enc_cap < npad) {
         if (M->enc) (void)hipFree(M->enc);
-        if (M->encT) (void)hipFree(M->encT);
-        M->enc = M->encT = nullptr;
+        M->enc = nullptr;
         M->enc_cap = 0;
-        if (hipMalloc(reinterpret_cast<void**>(&M->enc), npad * kIn * sizeof(bf16)) == hipSuccess &&
-            hipMalloc(reinterpret_cast<void**>(&M->encT), npad * kIn * sizeof(bf16)) == hipSuccess) {
+        if (hipMalloc(reinterpret_cast<void**>(&M->enc), npad * kIn * sizeof(bf16)) == hipSuccess)
             M->enc_cap = npad;
-        } else {
-            if (M->enc) (void)hipFree(M->enc);
-            M->enc = nullptr;
-            (void)hipGetLastError();  // a failed allocation leaves the slower path, not an error
-        }
+        else
+            M->enc = nullptr, (void)hipGetLastError();  // a failed allocation leaves the slower path, not an error
     }
-    const bool pre = steps > per_epoch && M->enc_cap >= npad;
-    if (pre)
-        hipLaunchKernelGGL(mlp_pe_kernel, dim3((uint32_t)(npad / 64)), dim3(64), 0, s, in, per_epoch * batch,
-                           (uint32_t)npad, M->lod_max, M->enc, M->encT);
+    const bool pre = revisit && M->enc_cap >= npad;
+    if (pre) encode(in, (uint32_t)npad, (uint32_t)npad, M->lod_max, M->enc, nullptr, s);
     for (uint32_t k = 0; k < steps; ++k) {
         const size_t off = (size_t)(k % per_epoch) * batch;
-        if (pre)
-            gradient(M, in + off, tg + off, batch, M->G, d_loss_curve ? d_loss_curve + k : nullptr, s,
-                     M->enc + off * kIn, M->encT + off, (uint32_t)npad);
-        else
-            gradient(M, in + off, tg + off, batch, M->G, d_loss_curve ? d_loss_curve + k : nullptr, s);
+        float* loss = d_loss_curve ? d_loss_curve + k : nullptr;
         // cosine decay from lr to lr / 100 over the call
         const double ph = steps > 1 ? (double)k / (double)(steps - 1) : 0.0;
         const float lr_k = (float)(lr * (0.01 + 0.99 * 0.5 * (1.0 + std::cos(hvx::kMlpPi * ph))));
         ++M->steps_done;
         const float bc1 = (float)(1.0 - std::pow(0.9, (double)M->steps_done));
         const float bc2 = (float)(1.0 - std::pow(0.999, (double)M->steps_done));
-        hipLaunchKernelGGL(adam_kernel, dim3((hvx::kMlpParams + 255) / 256), dim3(256), 0, s, M->P, M->G, M->m, M->v,
-                           (uint32_t)hvx::kMlpParams, lr_k, bc1, bc2, M->W1, M->W2, M->W3, M->W2T, M->W3T);
+        AdamArgs ad{M->P, M->m, M->v, lr_k, bc1, bc2, {M->W1, M->W2, M->W3, M->Ws}};
+        if (separate) {
+            gradient_separate(M, in + off, tg + off, batch, M->G, loss, s);
+            hipLaunchKernelGGL(adam_kernel, dim3((hvx::kMlpParams + 255) / 256), dim3(256), 0, s, ad, M->G,
+                               (uint32_t)hvx::kMlpParams);
+        } else {
+            gradient_fused(M, in + off, pre ? M->enc + off * kIn : nullptr, tg + off, batch, nullptr, &ad, loss, s);
+        }
     }
     e = hipGetLastError();
     return e == hipSuccess ? HVX_OK : mfail(M->ctx, HVX_ERR_HIP, "hvx_mlp_train: %s", hipGetErrorString(e));
