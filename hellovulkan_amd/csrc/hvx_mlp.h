@@ -44,6 +44,9 @@ template <class T> HVX_MLP_HD inline T mlp_freq(int k) {
     return f;
 }
 
+HVX_MLP_HD inline uint32_t mlp_bits(float x) { return __builtin_bit_cast(uint32_t, x); }
+HVX_MLP_HD inline float mlp_float(uint32_t x) { return __builtin_bit_cast(float, x); }
+
 // sin and cos of f_k x for k = 0, 1 mod 4, as every kernel (and the
 // oracle's BF16 emulation) evaluates them: in FP32, each step an IEEE
 // operation or a fused multiply-add, so any IEEE target gives the same bits.
@@ -56,7 +59,9 @@ HVX_MLP_HD inline void mlp_sincos_direct(float x, int k, float& s, float& c) {
     const float m = ldexpf((k & 1) ? 0.70710678118654752f : 0.5f, k >> 1);  // 2^(k/2) / 2
     const float t = x * m;
     const float r = t - rintf(t);
-    const float q = rintf(4.0f * r);
+    // q = rint(4 r), |q| <= 2: the sum with 1.5 2^23 is rounded to an integer
+    // and ends in the low bits of q
+    const float z = fmaf(4.0f, r, 12582912.0f), q = z - 12582912.0f;
     const float f = fmaf(q, -0.25f, r);
     const float a = f * 6.28318530717958647692f;
     const float a2 = a * a;
@@ -68,13 +73,13 @@ HVX_MLP_HD inline void mlp_sincos_direct(float x, int k, float& s, float& c) {
     pc = fmaf(a2, pc, 4.1666666666666667e-2f);                             // 1/4!
     pc = fmaf(a2, pc, -0.5f);
     const float ca = fmaf(a2, pc, 1.0f);
-    // quadrant qi = q mod 4 (q in [-2, 2]): (s, c) = (sa, ca), (ca, -sa),
-    // (-sa, -ca), (-ca, sa) for qi = 0..3, as selects rather than a branch
-    // per quadrant (lanes of one wave hold different quadrants)
-    const uint32_t qi = (uint32_t)(int)q;
+    // quadrant qi = q mod 4: (s, c) = (sa, ca), (ca, -sa), (-sa, -ca), (-ca, sa)
+    // for qi = 0..3, as selects and sign bits rather than a branch per
+    // quadrant (lanes of one wave hold different quadrants)
+    const uint32_t qi = mlp_bits(z);
     const float s0 = (qi & 1u) ? ca : sa, c0 = (qi & 1u) ? sa : ca;
-    s = (qi & 2u) ? -s0 : s0;
-    c = ((qi + 1u) & 2u) ? -c0 : c0;
+    s = mlp_float(mlp_bits(s0) ^ (qi << 30 & 0x80000000u));
+    c = mlp_float(mlp_bits(c0) ^ ((qi + 1u) << 30 & 0x80000000u));
 }
 
 // Frequency k + 2 from frequency k (f_(k+2) = 2 f_k): sin 2u = 2 sin u cos u,

@@ -771,25 +771,37 @@ __global__ __launch_bounds__(256) void mlp_transpose_kernel(const bf16* __restri
 }
 
 // Inference through the in-shading path (mlp_device.h): each workgroup
-// stages the weights once, its four waves evaluate 16 samples per call.
-__global__ __launch_bounds__(256) void mlp_infer_kernel(MlpView v, const float4* __restrict__ in, uint32_t n,
-                                                        float* __restrict__ rgb) {
+// stages the weights once, its four waves evaluate kInferTiles x 16 samples
+// per call. Bound by its vector instructions, 1,090 per 32 samples (512 of
+// them the encoding): 2 million samples 549 -> 123 us, of which those are 110;
+// one tile per call reads the weights twice as often (165 against 151 us before
+// the encoding's quadrants became sign bits), three and four are no faster.
+// Four waves per SIMD asked for: without it the accumulators go through the
+// second register file (159 us).
+constexpr int kInferTiles = 2;
+constexpr uint32_t kInferStep = 64 * kInferTiles;  // samples per workgroup and step
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void mlp_infer_kernel(
+    MlpView v, const float4* __restrict__ in, uint32_t n, float* __restrict__ rgb) {
     __shared__ MlpLds L;
     mlp_stage(L, v);
     __syncthreads();
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
-    for (uint32_t base = blockIdx.x * 64; base < n; base += gridDim.x * 64) {
-        const uint32_t sidx = base + wave * 16 + i;
-        float x[4] = {0.0f, 0.0f, 1.0f, 0.0f};
-        if (sidx < n) {
-            const float4 q = in[sidx];
-            x[0] = q.x;
-            x[1] = q.y;
-            x[2] = q.z;
-            x[3] = q.w;
+    for (size_t base = (size_t)blockIdx.x * kInferStep; base < n; base += (size_t)gridDim.x * kInferStep) {
+        float x[kInferTiles][4], y[kInferTiles];
+        size_t at[kInferTiles];
+#pragma unroll
+        for (int t = 0; t < kInferTiles; ++t) {
+            at[t] = base + (wave * kInferTiles + t) * 16 + i;
+            const float4 q = at[t] < n ? in[at[t]] : make_float4(0.0f, 0.0f, 1.0f, 0.0f);
+            x[t][0] = q.x;
+            x[t][1] = q.y;
+            x[t][2] = q.z;
+            x[t][3] = q.w;
         }
-        const float y = mlp_forward_tile(L, x, v.lod_max);
-        if (g < 3 && sidx < n) rgb[(size_t)sidx * 3 + g] = y;
+        mlp_forward_tiles(L, x, v.lod_max, y);
+#pragma unroll
+        for (int t = 0; t < kInferTiles; ++t)
+            if (g < 3 && at[t] < n) rgb[at[t] * 3 + g] = y[t];
     }
 }
 
@@ -1251,10 +1263,10 @@ int hvx_mlp_train(hvx_mlp* M, const float* d_inputs, const float* d_targets, uin
 }
 
 // Workgroups of mlp_infer_kernel: each stages the weights (34 KB) once and
-// loops over 64-sample steps, so a few per CU suffice.
+// loops over kInferStep samples, so a few per CU suffice.
 static uint32_t infer_blocks(const hvx_mlp* M, uint32_t n) {
     const uint32_t cap = 4u * (uint32_t)std::max(M->ctx->num_cus, 1);
-    return std::max(1u, std::min(cap, (n + 63) / 64));
+    return std::max(1u, std::min(cap, n / kInferStep + (n % kInferStep != 0)));
 }
 
 int hvx_mlp_eval(hvx_mlp* M, const float* d_inputs, uint32_t n, float* d_rgb, void* stream) {
@@ -1311,8 +1323,8 @@ int hvx_mlp_cell_errors(hvx_mlp* M, const float* d_chain, uint32_t face, uint32_
     hipStream_t s = (hipStream_t)stream;
     hipLaunchKernelGGL(mask_points_kernel, dim3((unsigned)((npts + 255) / 256)), dim3(256), 0, s, mask_face, lod_bins,
                        M->lod_max, pts);
-    hipLaunchKernelGGL(mlp_infer_kernel, dim3(infer_blocks(M, npts)), dim3(256), 0, s,
-                       hvx::mlp_view(M), pts, (uint32_t)npts, rgb);
+    hipLaunchKernelGGL(mlp_infer_kernel, dim3(infer_blocks(M, npts)), dim3(256), 0, s, hvx::mlp_view(M), pts,
+                       (uint32_t)npts, rgb);
     hipLaunchKernelGGL(cell_error_kernel, dim3((cells + 255) / 256), dim3(256), 0, s, pts, rgb,
                        reinterpret_cast<const float4*>(d_chain), face, mips, cells, raw, M->cell_lo);
     hipLaunchKernelGGL(cell_margin_kernel, dim3((cells + 255) / 256), dim3(256), 0, s, raw, cells, d_err);
