@@ -251,6 +251,49 @@ HVX_HD float cosf_(float x) { return (float)cos_d((double)x); }
 HVX_HD float atan2f_(float y, float x) { return (float)atan2_d((double)y, (double)x); }
 HVX_HD float acosf_(float x) { return (float)acos_d((double)x); }
 
+// ------------------------------------------------- sums of equal terms
+// ((t + t) + t) + ... of n terms t, each addition rounded (0 for n = 0): the
+// value of the sequential loop from 0, to the bit. Where two additions stay in
+// one binade, later ones there add the same amount d: t rounded to the binade's
+// spacing, and where t lies halfway between two multiples of it the sum is even
+// after the first. d and the sums are multiples of that spacing, so k of those
+// steps are one exact fused multiply-add. About 20 operations per binade
+// (log2 n of them) in place of n additions.
+HVX_HD float repeat_sum(float t, uint32_t n) {
+    float a = 0.0f;
+    uint32_t i = 0;
+    if (n >= 16u)
+        for (; i < 16u; ++i) a = a + t;
+    while (i < n) {
+        const float b = a + t;
+        if (n - ++i < 6u) {
+            a = b;
+            continue;
+        }
+        const float c = b + t, e = c + t, d = e - c;
+        i += 2u;
+        a = e;
+        const uint32_t x = f2u(e) & 0x7f800000u;
+        // nothing is added any more, or the sum is infinite or NaN for good
+        if (d == 0.0f || x == 0x7f800000u) break;
+        if (x != (f2u(b) & 0x7f800000u) || x >= 0x7f000000u) continue;
+        // steps that stay below the binade's end, with one and 2^-18 of them
+        // to spare for the error of the quotient (2^-22 of it)
+        const float left = u2f(x + 0x00800000u) - __builtin_fabsf(e);
+#if defined(__HIP_DEVICE_COMPILE__)
+        const float steps = left * __builtin_amdgcn_rcpf(__builtin_fabsf(d));
+#else
+        const float steps = left / __builtin_fabsf(d);
+#endif
+        // (a subnormal d has no finite reciprocal: no steps, one addition after the other)
+        const uint32_t q = steps < 16777217.0f ? (uint32_t)steps : 0u, spare = 1u + (q >> 18);
+        const uint32_t k = q > spare ? q - spare : 0u, m = k < n - i ? k : n - i;
+        a = __builtin_fmaf((float)m, d, e);
+        i += m;
+    }
+    return a;
+}
+
 // ------------------------------------------------------------- Hammersley
 // PBR/Hammersley.glsl:4-19. Bit reversal, then float(bits) * 2^-32.
 HVX_HD uint32_t bitrev32(uint32_t b) {

@@ -387,19 +387,17 @@ __device__ __forceinline__ float4 specular_texel_value(const float4* __restrict_
         // cos(theta) = sqrt((1-y)/(1-y)) = 1 and sin(theta) = 0 for every
         // Hammersley sample, so each sample's half vector is normalize(N + (+-0))
         // and all n samples produce the same L, NoL and texel value. Evaluate it
-        // once and form the reference's sequential sums of the n identical terms.
+        // once and form the reference's sequential sums of the n identical terms
+        // (6 x 512^2 texels, 1,024 samples: 200 us one addition after the other, 73 so).
         const f3 Hh = ggx_world(fr, N, tab[0]);
         const f3 L = normalize3(sub3(mul3(Hh, 2.0f * dot3(V, Hh)), V));
         const float NoL = gmax(dot3(N, L), 0.0f);
         if (NoL > 0.0f) {
             const f3 c = sample_cube(cube, (int)S, L);
-            const float t0 = c.x * NoL, t1 = c.y * NoL, t2 = c.z * NoL;
-            for (uint32_t i = 0; i < n; ++i) {
-                acc0 = acc0 + t0;
-                acc1 = acc1 + t1;
-                acc2 = acc2 + t2;
-                wsum = wsum + NoL;
-            }
+            acc0 = repeat_sum(c.x * NoL, n);
+            acc1 = repeat_sum(c.y * NoL, n);
+            acc2 = repeat_sum(c.z * NoL, n);
+            wsum = repeat_sum(NoL, n);
         }
     } else {
         for (uint32_t i = 0; i < n; ++i) {
