@@ -106,6 +106,61 @@ __device__ __forceinline__ float div_by_normal(float a, float b, float y) {  // 
 }
 __device__ __forceinline__ float div_rn_normal(float a, float b) { return div_by_normal(a, b, rcp_rn_normal(b)); }
 
+// atan2f_ and acosf_ of hvx_math.h to the bit, for finite arguments (acosf_:
+// |x| < 1; others go to hvx_math.h). Those round a double whose error is a few
+// of its ulps to float, so any value within 2^-42 of it whose float is the same
+// at both ends of that range gives the same result. This one takes a single
+// quotient with an unscaled reciprocal, fused Horner steps and no terms below
+// 2^-46; about one argument in 10^5 lies too near the middle between two floats
+// and takes the functions themselves.
+__device__ __forceinline__ double atan2_near(double y, double x) {
+    const double ax = __builtin_fabs(x), ay = __builtin_fabs(y);
+    const double mn = __builtin_fmin(ax, ay), mx = __builtin_fmax(ax, ay);
+    // t = mn / mx, or (t sqrt3 - 1) / (t + sqrt3) past tan(pi / 12)
+    const bool far = mn > 0.2679491924311227 * mx;
+    const double num = far ? __builtin_fma(mn, kSqrt3, -mx) : mn, den = far ? __builtin_fma(mx, kSqrt3, mn) : mx;
+    double r = __builtin_amdgcn_rcp(den);
+    r = __builtin_fma(__builtin_fma(-den, r, 1.0), r, r);
+    r = __builtin_fma(__builtin_fma(-den, r, 1.0), r, r);
+    const double t = num * r, t2 = t * t;
+    double p = 1.0 / 21.0;
+    p = __builtin_fma(p, t2, -1.0 / 19.0);
+    p = __builtin_fma(p, t2, 1.0 / 17.0);
+    p = __builtin_fma(p, t2, -1.0 / 15.0);
+    p = __builtin_fma(p, t2, 1.0 / 13.0);
+    p = __builtin_fma(p, t2, -1.0 / 11.0);
+    p = __builtin_fma(p, t2, 1.0 / 9.0);
+    p = __builtin_fma(p, t2, -1.0 / 7.0);
+    p = __builtin_fma(p, t2, 1.0 / 5.0);
+    p = __builtin_fma(p, t2, -1.0 / 3.0);
+    double a = (far ? kPio6 : 0.0) + __builtin_fma(t * t2, p, t);
+    a = ay > ax ? kPio2 - a : a;
+    a = x < 0.0 ? kPiD - a : a;
+    return __builtin_copysign(a, y);
+}
+// a's float if every value within 2^-42 of it has the same
+__device__ __forceinline__ bool float_of_near(double a, float& f) {
+    f = (float)(a * (1.0 + 0x1p-42));
+    return f == (float)(a * (1.0 - 0x1p-42));
+}
+__device__ __forceinline__ float atan2f_rn(float y, float x) {
+    float f;
+    if (__builtin_expect(float_of_near(atan2_near((double)y, (double)x), f), 1)) return f;
+    return atan2f_(y, x);
+}
+__device__ __forceinline__ float acosf_rn(float x) {
+    // square root of z = (1 - x)(1 + x), at least 2^-24: two Newton steps from the hardware's estimate
+    const double z = (1.0 - (double)x) * (1.0 + (double)x), r = __builtin_amdgcn_rsq(z);
+    double g = z * r, h = 0.5 * r;
+    const double e = __builtin_fma(-h, g, 0.5);
+    g = __builtin_fma(g, e, g);
+    h = __builtin_fma(h, e, h);
+    g = __builtin_fma(g, __builtin_fma(-h, g, 0.5), g);
+    float f;
+    if (__builtin_expect(__builtin_fabsf(x) < 1.0f && float_of_near(atan2_near(g, (double)x), f), 1)) return f;
+    return acosf_(x);
+}
+
 // normalize3 of a vector whose squared length is a float in [2^-102, FLT_MAX]
 // (every near-unit vector): the same correctly rounded square root and
 // reciprocal, by the fast paths above, so the result is bit-identical.
@@ -326,8 +381,13 @@ __device__ __forceinline__ f3 cube_combine(const float4* __restrict__ level, int
 
 // ------------------------------------------------------------- 2D sampling
 __device__ __forceinline__ int wrap_rep(int i, int n) {
-    int r = i % n;
-    return r < 0 ? r + n : r;
+    // within one period of the image without a division (35 instructions)
+    int r = i < 0 ? i + n : (i >= n ? i - n : i);
+    if (__builtin_expect((uint32_t)r >= (uint32_t)n, 0)) {
+        r = i % n;
+        if (r < 0) r += n;
+    }
+    return r;
 }
 
 // Bilinear REPEAT sample of an RGBA32F image (returns RGB).
@@ -364,8 +424,9 @@ __device__ __forceinline__ float2 sample_2d_rg_repeat(const float2* __restrict__
 // IBL output-texel direction: texCoord = (x + .5)/D, uv = texCoord*2 - 1,
 // normalize(UVToXYZ(face, uv)), then y = -y.
 __device__ __forceinline__ f3 texel_dir(int face, int x, int y, int D) {
-    const float u = (((float)x + 0.5f) / (float)D) * 2.0f - 1.0f;
-    const float v = (((float)y + 0.5f) / (float)D) * 2.0f - 1.0f;
+    const float rd = rcp_rn_normal((float)D);
+    const float u = div_by_normal((float)x + 0.5f, (float)D, rd) * 2.0f - 1.0f;
+    const float v = div_by_normal((float)y + 0.5f, (float)D, rd) * 2.0f - 1.0f;
     f3 p;
     switch (face) {
         case 0: p = {1.0f, v, -u}; break;
@@ -375,7 +436,7 @@ __device__ __forceinline__ f3 texel_dir(int face, int x, int y, int D) {
         case 4: p = {u, v, 1.0f}; break;
         default: p = {-u, v, -1.0f}; break;
     }
-    f3 d = normalize3(p);
+    f3 d = normalize3_rn(p);  // squared length in [1, 3]
     d.y = -d.y;
     return d;
 }
