@@ -63,6 +63,23 @@ constexpr int kShadeWavesLearned = 4;
 namespace hvx {
 namespace {
 
+// n / W for a fixed W without a division: n < 2^31 times a 32-bit reciprocal
+// rounded up (m = floor(2^(31 + s) / W) + 1 with 2^s >= W: the error m W - 2^(31 + s)
+// is at most W, so below 2^31 it never reaches the next quotient).
+struct RowOf {
+    uint32_t m, shift;  // m = 0: n may be larger, divide
+    static RowOf make(uint64_t n_max, uint32_t W) {
+        uint32_t s = 0;
+        while ((1ull << s) < W) ++s;
+        if (n_max >= 1ull << 31 || s > 31) return {0, 0};
+        const unsigned __int128 m = ((unsigned __int128)1 << (31 + s)) / W + 1;
+        return m >> 32 ? RowOf{0, 0} : RowOf{(uint32_t)m, s};
+    }
+    __device__ __forceinline__ uint32_t of(uint32_t n, uint32_t W) const {
+        return m ? (uint32_t)(((uint64_t)n * m) >> 31 >> shift) : n / W;
+    }
+};
+
 struct ShadeArgs {
     const float* depth;
     const float* nrm[3];
@@ -101,6 +118,8 @@ struct ShadeArgs {
     // unbin_kernel moves to pixel order
     float* out_binned;
     uint32_t unbin_cap;  // floats of unbin_kernel's LDS tile image
+    RowOf row;
+    uint32_t order_cap;  // pixels of bin_kernel's LDS segment
     uint32_t rclasses;   // binning sub-key classes per slice: 2 splits by roughness, else 1
 };
 
@@ -116,14 +135,10 @@ constexpr float kRoughFastH = 0.7f;
 // distance dd >= it with a few ulp of error, still satisfies s * (1/r) >= 1.
 constexpr float kOutOfRangeMargin = 1.0f + 1.0f / 65536.0f;
 
-__global__ __launch_bounds__(256) void shade_light_prep_kernel(const hvx_light* __restrict__ lights, uint32_t n,
-                                                               float intensity, float4* __restrict__ lrec) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const hvx_light& l = lights[i];
-    lrec[2 * i] = make_float4(l.position[0], l.position[1], l.position[2], 1.0f / l.radius);
-    lrec[2 * i + 1] = make_float4(l.color[0] * intensity, l.color[1] * intensity, l.color[2] * intensity,
-                                  (l.radius * l.radius) * kOutOfRangeMargin);
+__device__ __forceinline__ void shade_light_prep(const hvx_light& l, float intensity, float4* __restrict__ lrec) {
+    lrec[0] = make_float4(l.position[0], l.position[1], l.position[2], 1.0f / l.radius);
+    lrec[1] = make_float4(l.color[0] * intensity, l.color[1] * intensity, l.color[2] * intensity,
+                          (l.radius * l.radius) * kOutOfRangeMargin);
 }
 
 __device__ __forceinline__ f3 sample_spec_lod(const ShadeArgs& a, f3 dir, float lod) {
@@ -150,13 +165,13 @@ __device__ __forceinline__ uint32_t tile_y(const ShadeArgs& a, uint32_t py) {
     const float tsy = a.scr_y / (float)a.Y;
     return min((uint32_t)(((float)py + 0.5f) / tsy), a.Y - 1);
 }
-__device__ __forceinline__ uint32_t slice_of(const ShadeArgs& a, uint32_t idx) {
-    const float z = a.depth[idx];
+__device__ __forceinline__ uint32_t slice_at(const ShadeArgs& a, float z) {
     const float lin = (a.nearv * a.farv) / (a.farv + z * (a.nearv - a.farv));
     const float zf = gmax(log2f_(lin) * a.scale + a.bias, 0.0f);
     const uint32_t zi = (uint32_t)zf;
     return zi >= a.Z ? a.Z - 1 : zi;
 }
+__device__ __forceinline__ uint32_t slice_of(const ShadeArgs& a, uint32_t idx) { return slice_at(a, a.depth[idx]); }
 __device__ __forceinline__ uint32_t cluster_of(const ShadeArgs& a, uint32_t idx) {
     return tile_x(a, idx % a.W) + tile_y(a, idx / a.W) * a.X + slice_of(a, idx) * a.X * a.Y;
 }
@@ -531,8 +546,7 @@ constexpr uint32_t kBinMaxZ = 1024;  // depth slices a tile's LDS histogram hold
 // tiles[X] = W), then the same for rows. One thread per pixel column or row;
 // tile_x is non-decreasing, so the thread of the first column of a tile
 // writes that tile's start (and the starts of any empty tiles before it).
-__global__ __launch_bounds__(256) void tile_bounds_kernel(ShadeArgs a) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void tile_bounds(const ShadeArgs& a, uint32_t i) {
     if (i >= a.W + a.H) return;
     const bool col = i < a.W;
     const uint32_t p = col ? i : i - a.W, n = col ? a.W : a.H, T = col ? a.X : a.Y;
@@ -543,6 +557,38 @@ __global__ __launch_bounds__(256) void tile_bounds_kernel(ShadeArgs a) {
     if (p == n - 1)
         for (uint32_t t = c + 1; t <= T; ++t) b[t] = n;
 }
+
+// What shading needs before its binning and its lights, in one launch: the
+// first bound_blocks workgroups the tile bounds, the others the light records.
+__global__ __launch_bounds__(256) void shade_prep_kernel(ShadeArgs a, uint32_t bound_blocks, uint32_t n_lights,
+                                                         float4* __restrict__ lrec) {
+    if (blockIdx.x < bound_blocks) {
+        tile_bounds(a, blockIdx.x * 256 + threadIdx.x);
+        return;
+    }
+    const uint32_t i = (blockIdx.x - bound_blocks) * 256 + threadIdx.x;
+    if (i < n_lights) shade_light_prep(a.lights[i], a.pc.light_intensity, lrec + 2 * (size_t)i);
+}
+
+// Pixels t, t + kBinThreads, ... of a tile w pixels wide, row by row: one
+// division, then steps of (dx, dy).
+struct TileWalk {
+    uint32_t x, y, dx, dy, w;
+    __device__ __forceinline__ TileWalk(uint32_t t, uint32_t width) : w(width) {
+        y = t / width;
+        x = t - y * width;
+        dy = kBinThreads / width;
+        dx = kBinThreads - dy * width;
+    }
+    __device__ __forceinline__ void next() {
+        x += dx;
+        y += dy;
+        if (x >= w) {
+            x -= w;
+            ++y;
+        }
+    }
+};
 
 // One workgroup per screen tile and RGB plane: moves the tile's segment of
 // the binned plane to pixel order through an LDS image of the tile, so that
@@ -564,13 +610,16 @@ __global__ __launch_bounds__(kBinThreads) void unbin_kernel(ShadeArgs a) {
             a.out[(size_t)c * nfrag + a.order[start + i]] = a.out_binned[(size_t)c * nfrag + start + i];
         return;
     }
+#pragma unroll 4
     for (uint32_t i = t; i < area; i += kBinThreads) {
-        const uint32_t idx = a.order[start + i];
-        s_img[(idx / a.W - y0) * w + (idx % a.W - x0)] = a.out_binned[(size_t)c * nfrag + start + i];
+        const uint32_t idx = a.order[start + i], v = idx - y0 * a.W, r = a.row.of(v, a.W);
+        s_img[r * w + (v - r * a.W - x0)] = a.out_binned[(size_t)c * nfrag + start + i];
     }
     __syncthreads();
-    for (uint32_t i = t; i < area; i += kBinThreads)
-        a.out[(size_t)c * nfrag + (y0 + i / w) * a.W + x0 + i % w] = s_img[i];
+    TileWalk p(t, w);
+#pragma unroll 4
+    for (uint32_t i = t; i < area; i += kBinThreads, p.next())
+        a.out[(size_t)c * nfrag + (y0 + p.y) * a.W + x0 + p.x] = s_img[i];
 }
 
 // Binning key of a fragment: its depth slice, then (rclasses = 2) whether it
@@ -582,39 +631,56 @@ __device__ __forceinline__ uint32_t bin_of(const ShadeArgs& a, uint32_t idx) {
 }
 
 // One workgroup per screen tile: counting sort of the tile's pixels by depth
-// slice into the tile's segment of the order. Tiles are laid out row band by
+// slice into the tile's segment of the order (one count per pixel, no division
+// per pixel: 1366x768 18.4 -> 14.0 us, 3840x2160 80 -> 64). Tiles are laid out row band by
 // row band, so tile (cx, cy) starts at y0 * W + (y1 - y0) * x0. Within a
 // slice the order is that of the LDS atomics (see the note on the fast
 // variant at the top of this file).
 __global__ __launch_bounds__(kBinThreads) void bin_kernel(ShadeArgs a) {
-    __shared__ uint32_t s_hist[kBinMaxZ];
+    extern __shared__ uint32_t s_order[];
+    __shared__ uint32_t s_hist[kBinMaxZ], s_next[kBinMaxZ];
     __shared__ uint32_t s_wave[kBinThreads / 64];
     const uint32_t cx = blockIdx.x % a.X, cy = blockIdx.x / a.X, t = threadIdx.x;
     const uint32_t x0 = a.tiles[cx], x1 = a.tiles[cx + 1];
     const uint32_t y0 = a.tiles[a.X + 1 + cy], y1 = a.tiles[a.X + 1 + cy + 1];
     const uint32_t w = x1 - x0, area = w * (y1 - y0);
     if (area == 0) return;  // uniform over the workgroup
-    const uint32_t start = y0 * a.W + (y1 - y0) * x0;
+    const uint32_t start = y0 * a.W + (y1 - y0) * x0, first = y0 * a.W + x0;
     for (uint32_t z = t; z < a.Z * a.rclasses; z += kBinThreads) s_hist[z] = 0;
     __syncthreads();
     const uint32_t nb = a.Z * a.rclasses;  // bins: (slice, roughness class)
-    // the bins of a thread's first kBinCache pixels stay in registers for
-    // the second pass (a 120 x 120 tile takes 15 rounds)
+    // a thread's first kBinCache pixels (a 120 x 120 tile takes 15 rounds) keep
+    // their bin and their rank in it, so they count once; their depths and
+    // roughnesses are all asked for before the first is waited for
     constexpr uint32_t kBinCache = 16;
-    uint32_t cache[kBinCache];
+    uint32_t bin[kBinCache], rank[kBinCache];
+    float dep[kBinCache], rgh[kBinCache];
+    TileWalk p(t, w);
+    const bool split = a.rclasses == 2;
 #pragma unroll
-    for (uint32_t k = 0; k < kBinCache; ++k) {
-        const uint32_t i = t + k * kBinThreads;
-        cache[k] = 0;
-        if (i < area) {
-            const uint32_t idx = (y0 + i / w) * a.W + x0 + i % w;
-            cache[k] = bin_of(a, idx);
-            atomicAdd(&s_hist[cache[k]], 1u);
+    for (uint32_t k = 0; k < kBinCache; ++k, p.next()) {
+        if (t + k * kBinThreads < area) {
+            dep[k] = a.depth[first + p.y * a.W + p.x];
+            rgh[k] = split ? a.rough[first + p.y * a.W + p.x] : 0.0f;
         }
     }
-    for (uint32_t i = t + kBinCache * kBinThreads; i < area; i += kBinThreads) {
-        const uint32_t idx = (y0 + i / w) * a.W + x0 + i % w;
-        atomicAdd(&s_hist[bin_of(a, idx)], 1u);
+#pragma unroll
+    for (uint32_t k = 0; k < kBinCache; ++k) {
+        if (t + k * kBinThreads < area) {
+            const uint32_t z = slice_at(a, dep[k]);
+            bin[k] = split ? 2 * z + (rgh[k] >= kRoughFastH ? 1u : 0u) : z;
+            rank[k] = atomicAdd(&s_hist[bin[k]], 1u);
+        }
+    }
+    // the pixels beyond count after those, and again when they are placed
+    const bool more = area > kBinCache * kBinThreads;  // uniform over the workgroup
+    if (more) {
+        __syncthreads();
+        if (t < nb) s_next[t] = s_hist[t];
+        __syncthreads();
+        TileWalk r = p;
+        for (uint32_t i = t + kBinCache * kBinThreads; i < area; i += kBinThreads, r.next())
+            atomicAdd(&s_hist[bin_of(a, first + r.y * a.W + r.x)], 1u);
     }
     __syncthreads();
     // exclusive scan of the Z <= kBinThreads slice counts: per wave, then
@@ -639,17 +705,26 @@ __global__ __launch_bounds__(kBinThreads) void bin_kernel(ShadeArgs a) {
         if (t < kBinThreads / 64) s_wave[t] = wi - wt;
     }
     __syncthreads();
-    if (t < nb) s_hist[t] = start + s_wave[wv] + inc - v;
+    if (t < nb) s_hist[t] = s_wave[wv] + inc - v;
     __syncthreads();
+    // the segment is put together in LDS where it fits and stored in one piece
+    const bool staged = area <= a.order_cap;
+    auto place = [&](uint32_t at, uint32_t idx) {
+        if (staged) s_order[at] = idx;
+        else a.order[start + at] = idx;
+    };
+    TileWalk q(t, w);
 #pragma unroll
-    for (uint32_t k = 0; k < kBinCache; ++k) {
-        const uint32_t i = t + k * kBinThreads;
-        if (i < area) a.order[atomicAdd(&s_hist[cache[k]], 1u)] = (y0 + i / w) * a.W + x0 + i % w;
-    }
-    for (uint32_t i = t + kBinCache * kBinThreads; i < area; i += kBinThreads) {
-        const uint32_t idx = (y0 + i / w) * a.W + x0 + i % w;
-        a.order[atomicAdd(&s_hist[bin_of(a, idx)], 1u)] = idx;
-    }
+    for (uint32_t k = 0; k < kBinCache; ++k, q.next())
+        if (t + k * kBinThreads < area) place(s_hist[bin[k]] + rank[k], first + q.y * a.W + q.x);
+    if (more)
+        for (uint32_t i = t + kBinCache * kBinThreads; i < area; i += kBinThreads, p.next()) {
+            const uint32_t idx = first + p.y * a.W + p.x, b = bin_of(a, idx);
+            place(s_hist[b] + atomicAdd(&s_next[b], 1u), idx);
+        }
+    if (!staged) return;
+    __syncthreads();
+    for (uint32_t i = t; i < area; i += kBinThreads) a.order[start + i] = s_order[i];
 }
 
 
@@ -885,13 +960,21 @@ hipError_t launch_shade(const hvx_frag_soa& fr, const hvx_camera_ubo& cam, const
         if (staged) {
             a.out_binned = reinterpret_cast<float*>(bin_scratch + F + a.X + a.Y + 2);
             a.unbin_cap = (uint32_t)(unbin_lds / sizeof(float));
+            // four-byte stores to 64 lines a wave bound the binning once the
+            // tiles fill the card (3840x2160, 576 tiles: 84 us scattered, 64
+            // in pieces); fewer tiles than CUs wait for their loads, and the
+            // pass through LDS only adds to that (1366x768, 144: 14.0, 16.8)
+            a.order_cap = (uint64_t)a.X * a.Y > 256 ? a.unbin_cap : 0;
         }
-        hipLaunchKernelGGL(tile_bounds_kernel, dim3((fr.width + fr.height + 255) / 256), dim3(256), 0, s, a);
-        hipLaunchKernelGGL(bin_kernel, dim3(a.X * a.Y), dim3(kBinThreads), 0, s, a);
+        a.row = RowOf::make(F, fr.width);
     }
-    if (!exact && n_lights > 0)
-        hipLaunchKernelGGL(shade_light_prep_kernel, dim3((n_lights + 255) / 256), dim3(256), 0, s, d_lights, n_lights,
-                           pc.light_intensity, light_scratch);
+    const uint32_t bound_blocks = binned ? (fr.width + fr.height + 255) / 256 : 0;
+    const uint32_t light_blocks = exact ? 0 : n_lights / 256 + (n_lights % 256 != 0);
+    if (bound_blocks + light_blocks > 0)
+        hipLaunchKernelGGL(shade_prep_kernel, dim3(bound_blocks + light_blocks), dim3(256), 0, s, a, bound_blocks,
+                           n_lights, light_scratch);
+    if (binned) hipLaunchKernelGGL(bin_kernel, dim3(a.X * a.Y), dim3(kBinThreads),
+                                   a.order_cap * sizeof(uint32_t), s, a);
     if (ev_begin) (void)hipEventRecord(ev_begin, s);
     if (exact) {
         if (learned) hipLaunchKernelGGL((shade_kernel<true, true>), grid, block, 0, s, a);
