@@ -162,7 +162,7 @@ hipError_t launch_gather_copy(const float* const* d_src, size_t floats, float* d
                               uint32_t n, hipStream_t s);
 // Bytes of the diffuse filter's staged footprints for a level-0 face of S
 // (0: not staged: S < 2, or more than kDiffuseStageMaxBytes).
-constexpr size_t kDiffuseStageMaxBytes = size_t(1) << 30;
+constexpr size_t kDiffuseStageMaxBytes = size_t(1) << 29;
 size_t diffuse_stage_size(uint32_t S);
 // d_stage: diffuse_stage_size(S) bytes of scratch, or nullptr (taps
 // gathered from the cube; the same results)

@@ -235,40 +235,45 @@ static_assert(kDThreads == 128 || kDThreads == 256, "lanes per workgroup: 128 or
 #define HVX_DIFFUSE_WAVES_PER_EU 4
 #endif
 
-// Staged footprints: for every bilinear footprint of level 0, first texel
-// (i0, j0) with -1 <= i0, j0 <= S - 1 on face f, one 64-byte entry at
-// (f (S+1) + j0 + 1) (S+1) + i0 + 1 holding the RGB of its four taps
-// exactly as sample_cube reads them (texels across an edge folded onto the
-// neighbouring face, a tap off both edges the mean of three texels):
-// (t00.rgb, t11.r) (t10.rgb, t11.g) (t01.rgb, t11.b), then 16 bytes of zeros.
-// A sample then reads one 128-byte line instead of two rows of texels (2.3
-// lines on average), and the bilinear sums are unchanged to the bit.
+// Staged footprints: a bilinear footprint of level 0 with first texel (i0, j0),
+// -1 <= i0, j0 <= S - 1, on face f is two columns of two texels, and four
+// neighbouring footprints of a row are five columns: one 128-byte line at
+// (f (S+1) + j0 + 1) stage_lines(S) + (i0 + 1) / 4 holds columns 4 k - 1 .. 4 k + 3
+// as (texel j0, texel j0 + 1) RGB RGB, 24 bytes each, exactly as sample_cube
+// reads the taps (texels across an edge folded onto the neighbouring face, a
+// tap off both edges the mean of three texels). A sample reads the 48 bytes from
+// column (i0 + 1) % 4 on: one line instead of two rows of texels (2.3 lines on
+// average), and the bilinear sums are unchanged to the bit. Twice the cube (202
+// MB at 1024^2), so it stays in the 256 MB of last-level cache: with an entry of
+// 64 bytes for every footprint (403 MB) 32^2 from 1024^2 took 1.77 ms, so 1.64 (12 GB of lines at 7.9 TB/s).
+__host__ __device__ inline uint32_t stage_lines(uint32_t S) { return (S + 4) / 4; }
 __global__ __launch_bounds__(256) void diffuse_stage_kernel(const float4* __restrict__ cube, uint32_t S,
-                                                           float4* __restrict__ quads) {
-    // lane g writes 16-byte part g % 4 of entry g / 4: a wave's stores are
-    // one contiguous kilobyte
-    const uint32_t Se = S + 1, per = Se * Se;
-    const uint32_t g = blockIdx.x * 256u + threadIdx.x, e = g / 4u, k = g % 4u;
-    if (e >= 6u * per) return;
-    float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);  // part 3: zeros (whole lines written)
-    if (k < 3u) {
-        // part k: tap k (t00, t10, t01) and channel k of t11
-        const uint32_t f = e / per, r = e % per;
-        const int j0 = (int)(r / Se) - 1, i0 = (int)(r % Se) - 1, Si = (int)S;
-        const int ti = i0 + (k == 1u ? 1 : 0), tj = j0 + (k == 2u ? 1 : 0);
-        f3 t, t11;
-        if (i0 >= 0 && j0 >= 0 && i0 + 1 < Si && j0 + 1 < Si) {
-            const float4 a = cube[((size_t)f * S + tj) * S + ti];
-            const float4 d = cube[((size_t)f * S + j0 + 1) * S + i0 + 1];
-            t = {a.x, a.y, a.z};
-            t11 = {d.x, d.y, d.z};
-        } else {
-            t = cube_texel_seamless(cube, Si, (int)f, ti, tj);
-            t11 = cube_texel_seamless(cube, Si, (int)f, i0 + 1, j0 + 1);
-        }
-        v = make_float4(t.x, t.y, t.z, k == 0u ? t11.x : (k == 1u ? t11.y : t11.z));
+                                                           float2* __restrict__ lines) {
+    // eight lanes per line: five write a column, the sixth the 8 bytes left over
+    const uint32_t L = stage_lines(S), rows = 6u * (S + 1);
+    const uint32_t l = blockIdx.x * 32u + threadIdx.x / 8u, k = threadIdx.x % 8u, r = blockIdx.y + gridDim.y * blockIdx.z;
+    if (l >= L || r >= rows || k > 5u) return;
+    float2* out = lines + ((size_t)r * L + l) * 16 + 3 * k;
+    if (k == 5u) {
+        *out = make_float2(0.0f, 0.0f);
+        return;
     }
-    quads[g] = v;
+    const uint32_t f = r / (S + 1);
+    const int Si = (int)S, i = (int)(4u * l + k) - 1, j = (int)(r - f * (S + 1)) - 1;
+    f3 a, b;
+    if (i > Si) {  // past the last footprint's second column: never read
+        a = b = make3(0.0f, 0.0f, 0.0f);
+    } else if (i >= 0 && i < Si && j >= 0 && j + 1 < Si) {
+        const float4 p = cube[((size_t)f * S + j) * S + i], q = cube[((size_t)f * S + j + 1) * S + i];
+        a = {p.x, p.y, p.z};
+        b = {q.x, q.y, q.z};
+    } else {
+        a = cube_texel_seamless(cube, Si, (int)f, i, j);
+        b = cube_texel_seamless(cube, Si, (int)f, i, j + 1);
+    }
+    out[0] = make_float2(a.x, a.y);
+    out[1] = make_float2(a.z, b.x);
+    out[2] = make_float2(b.y, b.z);
 }
 
 // One lane's sample of one round: direction, theta terms, taps and loads
@@ -286,7 +291,7 @@ struct DiffSample {
 // passed on through LDS) measured slower: 2.36 ms against 1.82.
 template <int TEX, int THREADS, bool STAGED>
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(HVX_DIFFUSE_WAVES_PER_EU, 8))) void
-diffuse_kernel(const float4* __restrict__ cube, uint32_t S, const float4* __restrict__ quads, float4* __restrict__ out,
+diffuse_kernel(const float4* __restrict__ cube, uint32_t S, const float* __restrict__ stage, float4* __restrict__ out,
                uint32_t Sd) {
     constexpr uint32_t SLOT = THREADS / TEX;  // samples per texel per round
     __shared__ float s_phi[kMaxPhi], s_theta[kMaxTheta];
@@ -344,9 +349,10 @@ diffuse_kernel(const float4* __restrict__ cube, uint32_t S, const float4* __rest
             // i0, j0 lie in [-1, S - 1] (the face coordinates are in [0, 1]);
             // the clamp only keeps the index inside the table
             const int i0 = min(max(p.taps.i0, -1), (int)S - 1), j0 = min(max(p.taps.j0, -1), (int)S - 1);
-            const uint32_t e = ((uint32_t)p.taps.face * (S + 1) + (uint32_t)(j0 + 1)) * (S + 1) + (uint32_t)(i0 + 1);
-#pragma unroll
-            for (int k = 0; k < 3; ++k) p.q[k] = quads[4 * (size_t)e + k];
+            const uint32_t r = (uint32_t)p.taps.face * (S + 1) + (uint32_t)(j0 + 1), e = (uint32_t)(i0 + 1);
+            // 24-byte steps: loads aligned to 8
+            const float* q = stage + ((size_t)r * stage_lines(S) + e / 4u) * 32 + 6u * (e % 4u);
+            __builtin_memcpy(p.q, q, 48);
         } else {
 #pragma unroll
             for (int k = 0; k < 4; ++k) p.q[k] = cube[p.taps.idx[k]];
@@ -361,9 +367,9 @@ diffuse_kernel(const float4* __restrict__ cube, uint32_t S, const float4* __rest
             // sample_cube's bilinear sum of the entry's taps
             const float4 q0 = p.q[0], q1 = p.q[1], q2 = p.q[2];
             const CubeTaps& t = p.taps;
-            c = {((t.w00 * q0.x + t.w10 * q1.x) + t.w01 * q2.x) + t.w11 * q0.w,
-                 ((t.w00 * q0.y + t.w10 * q1.y) + t.w01 * q2.y) + t.w11 * q1.w,
-                 ((t.w00 * q0.z + t.w10 * q1.z) + t.w01 * q2.z) + t.w11 * q2.w};
+            c = {((t.w00 * q0.x + t.w10 * q1.z) + t.w01 * q0.w) + t.w11 * q2.y,
+                 ((t.w00 * q0.y + t.w10 * q1.w) + t.w01 * q1.x) + t.w11 * q2.z,
+                 ((t.w00 * q0.z + t.w10 * q2.x) + t.w01 * q1.y) + t.w11 * q2.w};
         } else {
             c = cube_combine(cube, (int)S, p.L, p.taps, p.q);
         }
@@ -788,20 +794,21 @@ hipError_t launch_gather_copy(const float* const* d_src, size_t floats, float* d
 }
 
 size_t diffuse_stage_size(uint32_t S) {
-    const size_t b = (size_t)6 * (S + 1) * (S + 1) * 64;
+    const size_t b = (size_t)6 * (S + 1) * stage_lines(S) * 128;
     return b <= kDiffuseStageMaxBytes ? b : 0;
 }
 
 hipError_t launch_diffuse(const float* d_cube, uint32_t S, float* d_out, uint32_t Sd, float* d_stage, hipStream_t s) {
     const float4* cube = reinterpret_cast<const float4*>(d_cube);
-    float4* quads = diffuse_stage_size(S) ? reinterpret_cast<float4*>(d_stage) : nullptr;
+    float* stage = diffuse_stage_size(S) ? d_stage : nullptr;
     const uint32_t T = 6u * Sd * Sd;
     float4* out = reinterpret_cast<float4*>(d_out);
-    if (quads) {
-        const uint32_t parts = 4u * 6u * (S + 1) * (S + 1);  // 16-byte parts of the entries
-        hipLaunchKernelGGL(diffuse_stage_kernel, dim3((parts + 255) / 256), dim3(256), 0, s, cube, S, quads);
+    if (stage) {
+        const uint32_t rows = 6u * (S + 1), gy = std::min(rows, 32768u);
+        hipLaunchKernelGGL(diffuse_stage_kernel, dim3((stage_lines(S) + 31) / 32, gy, (rows + gy - 1) / gy), dim3(256), 0,
+                           s, cube, S, reinterpret_cast<float2*>(stage));
         hipLaunchKernelGGL((diffuse_kernel<kDTex, kDThreads, true>), dim3((T + kDTex - 1) / kDTex), dim3(kDThreads), 0,
-                           s, cube, S, quads, out, Sd);
+                           s, cube, S, stage, out, Sd);
     } else {
         hipLaunchKernelGGL((diffuse_kernel<kDTex, kDThreads, false>), dim3((T + kDTex - 1) / kDTex), dim3(kDThreads),
                            0, s, cube, S, nullptr, out, Sd);
