@@ -21,4 +21,9 @@ def test_rows_ending_anywhere_in_a_line(ctx, S):
     torch.cuda.synchronize()
     ids = np.arange(6 * Sd * Sd, dtype=np.uint32)
     ref = np.asarray(O.diffuse(cube, S, Sd, ids), np.float32).reshape(-1)
-    assert np.array_equal(out.cpu().numpy().view(np.uint32), ref.view(np.uint32))
+    got = out.cpu().numpy()
+    # the middle texels of the two Y faces look along the frame's up axis: their
+    # frame is 0 / 0, and a NaN's bits are nobody's
+    nan = np.isnan(ref)
+    assert np.array_equal(np.isnan(got), nan) and int(nan.sum()) <= 6
+    assert np.array_equal(got[~nan].view(np.uint32), ref[~nan].view(np.uint32))
