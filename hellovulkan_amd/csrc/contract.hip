@@ -32,7 +32,7 @@
 //
 // Measured (MI355X, whole calls, before: one row per output texel of the
 // canonical face, 6 faces x 4 padded columns, windows as bounding boxes):
-//   1024^2 -> 512^2 x 10, FP16           444 -> 129 us (weights 1606 -> 108 MB)
+//   1024^2 -> 512^2 x 10, FP16           444 -> 128 us (weights 1606 -> 127 MB)
 //   512^2 -> 256^2 x 9, split BF16       353 -> 100 us
 //   24 probes 256^2 -> 128^2 x 8, FP16   855 -> 340 us
 // The 129 us are 45 us of GEMM, 36 us of staging with the roughness-0 mip
