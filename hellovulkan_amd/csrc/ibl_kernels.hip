@@ -480,7 +480,7 @@ __global__ __launch_bounds__(256) void specular_delta_kernel(const float4* __res
 // addresser, at about a lane per cycle for gathers of lanes in different lines,
 // then VALU issue (236 instructions per 64 samples). So the two lanes of a pair
 // load the two texels of a footprint row together, one sample of the pair per
-// load (cube_taps / pair_taps): lanes side by side in one line are one access.
+// load (pair_exchange): lanes side by side in one line are one access.
 //   one run of all mips' tiles per XCD                   7.43 ms
 //   (two XCDs held the tiles of mip 2, which cost about
 //   twice those of mip 1; six waited for them)
@@ -488,6 +488,8 @@ __global__ __launch_bounds__(256) void specular_delta_kernel(const float4* __res
 //   lengths from bit patterns, faces by selects          4.33 ms (still the addresser)
 //   footprint rows loaded by lane pairs                  3.78 ms (addresser 88 -> 70 % busy)
 //   no length checks, 32-bit offsets                     3.71 ms (VALU 81 % busy)
+//   roughness 0 summed by binades                        3.60 ms
+//   pairs exchanged by selects that read across lanes    3.53 ms
 #ifndef HVX_SPEC_TPW
 #define HVX_SPEC_TPW 4
 #endif
@@ -520,10 +522,41 @@ struct SpecSample {
     f3 q[4];  // [2 r + s]: row r, column (lane & 1) of the footprint of the pair's sample s
 };
 
-// The value of the other lane of a pair (2k, 2k + 1).
-__device__ __forceinline__ int pair_swap(int v) { return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xf, 0xf, true); }
-__device__ __forceinline__ float pair_swap(float v) {
-    return __builtin_bit_cast(float, pair_swap(__builtin_bit_cast(int, v)));
+// Exchanges between the lanes of a pair (2k, 2k + 1): a = (even lane: its x,
+// odd lane: the even lane's y), b = (even lane: the odd lane's x, odd lane: its
+// y), three values at a time. Each is one select that reads one operand through
+// the lane crossing; the compiler writes the crossing and the select as two
+// instructions each (it forms the crossing select only for a condition that is
+// already in vcc). The leading no-op is the two wait states between a vector
+// write of an operand and its reading across lanes.
+__device__ __forceinline__ void pair_exchange(const float (&x)[3], const float (&y)[3], float (&a)[3], float (&b)[3]) {
+    __asm__ volatile("s_nop 1\n\t"
+            "s_mov_b32 vcc_lo, 0x55555555\n\t"
+            "s_mov_b32 vcc_hi, 0x55555555\n\t"
+            "v_cndmask_b32_dpp %0, %9, %6, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+            "v_cndmask_b32_dpp %1, %10, %7, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+            "v_cndmask_b32_dpp %2, %11, %8, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+            "s_not_b64 vcc, vcc\n\t"
+            "v_cndmask_b32_dpp %3, %6, %9, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+            "v_cndmask_b32_dpp %4, %7, %10, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+            "v_cndmask_b32_dpp %5, %8, %11, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf"
+            : "=&v"(a[0]), "=&v"(a[1]), "=&v"(a[2]), "=&v"(b[0]), "=&v"(b[1]), "=&v"(b[2])
+            : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(y[0]), "v"(y[1]), "v"(y[2])
+            : "vcc", "scc");
+}
+// The same for two pairs of texel indices.
+__device__ __forceinline__ void pair_exchange(const int (&x)[2], const int (&y)[2], int (&a)[2], int (&b)[2]) {
+    __asm__ volatile("s_nop 1\n\t"
+            "s_mov_b32 vcc_lo, 0x55555555\n\t"
+            "s_mov_b32 vcc_hi, 0x55555555\n\t"
+            "v_cndmask_b32_dpp %0, %6, %4, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+            "v_cndmask_b32_dpp %1, %7, %5, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+            "s_not_b64 vcc, vcc\n\t"
+            "v_cndmask_b32_dpp %2, %4, %6, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+            "v_cndmask_b32_dpp %3, %5, %7, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf"
+            : "=&v"(a[0]), "=&v"(a[1]), "=&v"(b[0]), "=&v"(b[1])
+            : "v"(x[0]), "v"(x[1]), "v"(y[0]), "v"(y[1])
+            : "vcc", "scc");
 }
 
 // Texel i of a cube level. WIDE false: the level is smaller than 4 GiB, so a
@@ -543,37 +576,32 @@ __device__ __forceinline__ void spec_begin(SpecSample& p, const float4* __restri
     p.L = normalize3_unit(sub3(mul3(Hh, 2.0f * dot3(N, Hh)), N));                              // V = N
     p.nol = gmax(dot3(N, p.L), 0.0f);
     p.taps = cube_taps<true>(S, p.L);
-    const bool odd = threadIdx.x & 1u;
+    // the first load takes the even lane's sample (even lane texel 0, odd lane
+    // texel 1 of the row), the second the odd lane's
+    const int (&id)[4] = p.taps.idx;
+    const int t0[2] = {id[0], id[2]}, t1[2] = {id[1], id[3]};
+    int first[2], second[2];
+    pair_exchange(t0, t1, first, second);
 #pragma unroll
     for (int r = 0; r < 2; ++r) {
-        const int i0 = p.taps.idx[2 * r], i1 = p.taps.idx[2 * r + 1];
-        const int s0 = pair_swap(i0), s1 = pair_swap(i1);
-        const int a0 = odd ? s1 : i0, a1 = odd ? i1 : s0;
-        const float4 v0 = cube_at<WIDE>(cube, a0), v1 = cube_at<WIDE>(cube, a1);
+        const float4 v0 = cube_at<WIDE>(cube, first[r]), v1 = cube_at<WIDE>(cube, second[r]);
         p.q[2 * r] = {v0.x, v0.y, v0.z};
         p.q[2 * r + 1] = {v1.x, v1.y, v1.z};
     }
 }
 
-// The two texels t0, t1 of this lane's sample: the even lane loaded texel 0 of
-// both samples (v0: the even lane's sample, v1: the odd one's), the odd lane
-// texel 1.
-__device__ __forceinline__ void pair_taps(float v0, float v1, bool odd, float& t0, float& t1) {
-    const float x0 = pair_swap(v0), x1 = pair_swap(v1);
-    t0 = odd ? x1 : v0;
-    t1 = odd ? v1 : x0;
-}
-
 // (c * NoL, NoL) of a sample that counts (NoL > 0); -0 in every term of one
 // that does not (a rejected or padding sample): x + (-0) == x for every x.
 __device__ __forceinline__ float4 spec_term(const SpecSample& p, bool live, const float4* __restrict__ cube, int S) {
-    const bool odd = threadIdx.x & 1u;
     float4 q[4];
 #pragma unroll
     for (int r = 0; r < 2; ++r) {
-        pair_taps(p.q[2 * r].x, p.q[2 * r + 1].x, odd, q[2 * r].x, q[2 * r + 1].x);
-        pair_taps(p.q[2 * r].y, p.q[2 * r + 1].y, odd, q[2 * r].y, q[2 * r + 1].y);
-        pair_taps(p.q[2 * r].z, p.q[2 * r + 1].z, odd, q[2 * r].z, q[2 * r + 1].z);
+        const f3 &u = p.q[2 * r], &v = p.q[2 * r + 1];
+        const float x[3] = {u.x, u.y, u.z}, y[3] = {v.x, v.y, v.z};
+        float t0[3], t1[3];
+        pair_exchange(x, y, t0, t1);
+        q[2 * r] = make_float4(t0[0], t0[1], t0[2], 0.0f);
+        q[2 * r + 1] = make_float4(t1[0], t1[1], t1[2], 0.0f);
     }
     if (!(live && p.nol > 0.0f)) return make_float4(-0.0f, -0.0f, -0.0f, -0.0f);
     const f3 c = cube_combine(cube, S, p.L, p.taps, q);
