@@ -27,6 +27,8 @@
 // inputs), they are only hoisted out of the per-texel loops.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "hvx_device.h"
 #include "hvx_internal.h"
 
@@ -212,20 +214,22 @@ __device__ __forceinline__ void wave_lds_sync() {
 // (diffuse_stage_kernel, one line per sample), a lane's loads are issued
 // one round ahead of their use, and the LDS rounds are double-buffered: the
 // gathers of round r+1 are in flight while round r is weighted, stored and
-// summed. 32^2 from 1024^2 (staging included): 1.79 ms with 8 texels per
-// 256-lane workgroup (staging 0.12 ms of it; 1.80 with 4 texels and the
-// staging's stores one entry per lane); 2.01 ms when only footprints inside a
-// face were staged (the others gathered per lane); gathered from the cube
-// (the path for stream capture before the context holds a staging buffer)
-// 2.66 ms with 4 texels (3.11 / 3.31 / 2.77 ms with 8 / 16 / 2, 3.02 with 4
-// per 128-lane workgroup); 3.54 ms with 16 texels and no loads ahead.
-// Staged loads two rounds ahead (79 VGPRs): no faster (1.81 ms).
+// summed. 32^2 from 1024^2 (staging included): 3.54 ms with 16 texels and no
+// loads ahead; gathered from the cube (the path for stream capture before the
+// context holds a staging buffer) 2.66 ms with 4 texels per 256-lane workgroup
+// (3.11 / 3.31 / 2.77 ms with 8 / 16 / 2); 1.77 ms with a staged 64-byte entry
+// per footprint and 8 texels; 1.64 with four footprints to a line; 1.58 with 4
+// texels. Small maps wait for their rounds, so they take fewer texels and more
+// samples a round (us with 1 / 2 / 4 texels per workgroup): 4^2 from 32^2 161 /
+// 205 / 223, 9^2 from 700^2 192 / 220 / 251, 16^2 from 128^2 184 / 207 / 242 but
+// from 1024^2 534 / 507 / 479, 24^2 from 64^2 362 / 249 / 272, 32^2 from 64^2
+// 597 / 427 / 349.
 constexpr int kMaxPhi = 512, kMaxTheta = 128;
 #ifndef HVX_DIFFUSE_TEX
-#define HVX_DIFFUSE_TEX 8
+#define HVX_DIFFUSE_TEX 4
 #endif
 constexpr int kDTex = HVX_DIFFUSE_TEX;  // texels per workgroup
-static_assert(kDTex == 2 || kDTex == 4 || kDTex == 8 || kDTex == 16, "texels per workgroup: 2, 4, 8 or 16");
+static_assert(kDTex == 1 || kDTex == 2 || kDTex == 4 || kDTex == 8 || kDTex == 16, "texels per workgroup: 1, 2, 4, 8 or 16");
 #ifndef HVX_DIFFUSE_THREADS
 #define HVX_DIFFUSE_THREADS 256
 #endif
@@ -835,8 +839,16 @@ hipError_t launch_diffuse(const float* d_cube, uint32_t S, float* d_out, uint32_
         const uint32_t rows = 6u * (S + 1), gy = std::min(rows, 32768u);
         hipLaunchKernelGGL(diffuse_stage_kernel, dim3((stage_lines(S) + 31) / 32, gy, (rows + gy - 1) / gy), dim3(256), 0,
                            s, cube, S, reinterpret_cast<float2*>(stage));
-        hipLaunchKernelGGL((diffuse_kernel<kDTex, kDThreads, true>), dim3((T + kDTex - 1) / kDTex), dim3(kDThreads), 0,
-                           s, cube, S, stage, out, Sd);
+        // few texels: fewer to a workgroup, for more workgroups and fewer
+        // rounds; large faces of medium maps stay with the fabric's best
+        auto run = [&](auto tex) {
+            constexpr int kTex = decltype(tex)::value;
+            hipLaunchKernelGGL((diffuse_kernel<kTex, kDThreads, true>), dim3((T + kTex - 1) / kTex), dim3(kDThreads), 0,
+                               s, cube, S, stage, out, Sd);
+        };
+        if (T <= 512) run(std::integral_constant<int, 1>());
+        else if (T <= 4096 && S <= 512) run(std::integral_constant<int, 2>());
+        else run(std::integral_constant<int, kDTex>());
     } else {
         hipLaunchKernelGGL((diffuse_kernel<kDTex, kDThreads, false>), dim3((T + kDTex - 1) / kDTex), dim3(kDThreads),
                            0, s, cube, S, nullptr, out, Sd);

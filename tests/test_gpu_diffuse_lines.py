@@ -27,3 +27,23 @@ def test_rows_ending_anywhere_in_a_line(ctx, S):
     nan = np.isnan(ref)
     assert np.array_equal(np.isnan(got), nan) and int(nan.sum()) <= 6
     assert np.array_equal(got[~nan].view(np.uint32), ref[~nan].view(np.uint32))
+
+
+@pytest.mark.parametrize("S,Sd", [(30, 9), (30, 10), (24, 26), (20, 27), (520, 10)])
+def test_texels_per_workgroup(ctx, S, Sd):
+    """Output maps on both sides of the sizes where a workgroup takes another
+    number of texels, whole and with a last workgroup that is not full."""
+    import torch
+    cube = np.random.default_rng(S + Sd).uniform(0, 40, 6 * S * S * 4).astype(np.float32)
+    out = torch.full((6 * Sd * Sd * 4 + 16,), -1.0, dtype=torch.float32, device="cuda")
+    ctx.filter(abi.FILTER_DIFFUSE, to_dev(cube), S, out, Sd, 1, 0)
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    assert np.all(got[6 * Sd * Sd * 4:] == -1.0)
+    ids = np.unique(np.concatenate([np.arange(40), np.random.default_rng(1).integers(0, 6 * Sd * Sd, 300),
+                                    np.arange(6 * Sd * Sd - 40, 6 * Sd * Sd)])).astype(np.uint32)
+    ref = np.asarray(O.diffuse(cube, S, Sd, ids), np.float32)
+    sub = got[:6 * Sd * Sd * 4].reshape(-1, 4)[ids]
+    nan = np.isnan(ref)
+    assert np.array_equal(np.isnan(sub), nan)
+    assert np.array_equal(sub[~nan].view(np.uint32), ref[~nan].view(np.uint32))
