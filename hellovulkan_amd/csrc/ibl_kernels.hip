@@ -497,13 +497,22 @@ __global__ __launch_bounds__(256) void specular_delta_kernel(const float4* __res
 #ifndef HVX_SPEC_TPW
 #define HVX_SPEC_TPW 4
 #endif
-constexpr int kSpecTPW = HVX_SPEC_TPW;                   // texels per wave: 4, 8 or 16
-constexpr int kSpecSPR = 64 / kSpecTPW;                  // samples per texel per round
-constexpr int kSpecTW = kSpecTPW >= 8 ? 8 : 4;           // tile width (texels)
-constexpr int kSpecRPW = kSpecTPW / kSpecTW;             // texel rows per wave
-constexpr int kSpecTH = 4 * kSpecRPW;                    // tile height: four waves
-constexpr int kSpecRow = 4 * kSpecSPR + 4;               // floats per texel row of the LDS buffer (padded)
+constexpr int kSpecTPW = HVX_SPEC_TPW;  // texels per wave: 4, 8 or 16
 static_assert(kSpecTPW == 4 || kSpecTPW == 8 || kSpecTPW == 16, "HVX_SPEC_TPW is 4, 8 or 16");
+template <int TPW> struct SpecShape {
+    static constexpr int kSPR = 64 / TPW;                         // samples per texel per round
+    static constexpr int kTW = TPW >= 8 ? 8 : (TPW >= 4 ? 4 : 1);  // tile width (texels)
+    static constexpr int kRPW = TPW / kTW;                        // texel rows per wave
+    static constexpr int kTH = 4 * kRPW;                          // tile height: four waves
+    static constexpr int kRow = 4 * kSPR + 4;                     // floats per texel row of the LDS buffer (padded)
+};
+// Small maps wait for their rounds (a texel's 1,024 samples are 64 of them with
+// four texels to a wave) with most of the card idle: with at most kSpecFewTiles
+// tiles a wave takes one texel and 64 samples a round. us of the whole call with
+// four / one: 16^2 x 4 and 256 samples (36 tiles) 44 / 27, 40^2 x 5 and 1,024 (234)
+// 94 / 55, 64^2 x 6 and 512 (516) 79 / 71, 90^2 x 4 and 700 (1,134) 326 / 272,
+// 128^2 x 6 and 1,024 (2,046) 244 / 259.
+constexpr uint32_t kSpecFewTiles = 1536;
 
 struct SpecSplitArgs {
     const float4* cube;
@@ -612,16 +621,17 @@ __device__ __forceinline__ float4 spec_term(const SpecSample& p, bool live, cons
     return make_float4(c.x * p.nol, c.y * p.nol, c.z * p.nol, p.nol);
 }
 
-// Tiles of one mip of size Sm: kSpecTW x kSpecTH texels, taken face by face in
+// Tiles of one mip of size Sm: kTW x kTH texels, taken face by face in
 // supertiles of 16 x 16 tiles (row-major supertiles, row-major tiles in each;
 // the last column and row of supertiles are as wide and high as is left).
 struct SpecTileGeom {
     uint32_t tiles_x, tiles_y, per_face;
 };
-__host__ __device__ inline SpecTileGeom spec_tile_geom(uint32_t Sm) {
+template <int TPW> __host__ __device__ inline SpecTileGeom spec_tile_geom(uint32_t Sm) {
+    constexpr uint32_t kTW = SpecShape<TPW>::kTW, kTH = SpecShape<TPW>::kTH;
     SpecTileGeom g;
-    g.tiles_x = (Sm + kSpecTW - 1) / kSpecTW;
-    g.tiles_y = (Sm + kSpecTH - 1) / kSpecTH;
+    g.tiles_x = (Sm + kTW - 1) / kTW;
+    g.tiles_y = (Sm + kTH - 1) / kTH;
     g.per_face = g.tiles_x * g.tiles_y;
     return g;
 }
@@ -640,37 +650,39 @@ __host__ __device__ inline void spec_tile_at(const SpecTileGeom& g, uint32_t k, 
 // One tile of the sample-split specular loop (four waves, each independent):
 // texels of face `face` of a mip of size Sm whose directions lie on a D x D
 // grid, out_level that mip's texels, tab its n tangent-space samples, s_buf
-// the workgroup's [4][2][kSpecTPW][kSpecRow] summation buffer.
-template <bool WIDE>
+// the workgroup's [4][2][TPW][kRow] summation buffer.
+template <bool WIDE, int TPW>
 __device__ __forceinline__ void specular_split_tile(const float4* __restrict__ cube, int S,
                                                     float4* __restrict__ out_level, uint32_t Sm, uint32_t D,
                                                     const float4* __restrict__ tab, uint32_t n, uint32_t face,
                                                     uint32_t tx, uint32_t ty, float* s_buf) {
+    using Sh = SpecShape<TPW>;
+    constexpr int kSPR = Sh::kSPR, kTW = Sh::kTW, kRPW = Sh::kRPW, kTH = Sh::kTH, kRow = Sh::kRow;
     const uint32_t wave = threadIdx.x / 64u, lane = threadIdx.x % 64u;
     // evaluating lane: texel t of the wave, sample slot s
-    const uint32_t t = lane / kSpecSPR, s = lane % kSpecSPR;
-    const uint32_t x = min(tx * kSpecTW + t % kSpecTW, Sm - 1),
-                   y = min(ty * kSpecTH + wave * kSpecRPW + t / kSpecTW, Sm - 1);
+    const uint32_t t = lane / kSPR, s = lane % kSPR;
+    const uint32_t x = min(tx * kTW + t % kTW, Sm - 1),
+                   y = min(ty * kTH + wave * kRPW + t / kTW, Sm - 1);
     const f3 N = texel_dir((int)face, (int)x, (int)y, (int)D);
     const Frame fr = ggx_frame(N);
     // summing lane: texel st of the wave, term sc (R, G, B, NoL)
-    const bool summer = lane < 4u * kSpecTPW;
+    const bool summer = lane < 4u * TPW;
     const uint32_t st = lane / 4u, sc = lane % 4u;
     float acc = 0.0f;
-    constexpr uint32_t kHalf = kSpecTPW * kSpecRow;  // floats between the two buffers
-    float* const wbuf = s_buf + wave * 2u * kHalf + t * kSpecRow + 4u * s;
-    const float* const rbuf = s_buf + wave * 2u * kHalf + st * kSpecRow + sc;
+    constexpr uint32_t kHalf = (uint32_t)TPW * kRow;  // floats between the two buffers
+    float* const wbuf = s_buf + wave * 2u * kHalf + t * kRow + 4u * s;
+    const float* const rbuf = s_buf + wave * 2u * kHalf + st * kRow + sc;
     // rounds in pairs (A: even, B: odd); sample i of round r is r * SPR + s,
     // table entries are fetched two rounds ahead and tap loads one round
     // ahead of their use
-    const uint32_t rounds = (n + kSpecSPR - 1) / kSpecSPR;
-    auto tab_at = [&](uint32_t r) { return tab[min(r * kSpecSPR + s, n - 1)]; };
+    const uint32_t rounds = (n + kSPR - 1) / kSPR;
+    auto tab_at = [&](uint32_t r) { return tab[min(r * kSPR + s, n - 1)]; };
     auto sum_round = [&](uint32_t parity, float4 term) {
         *reinterpret_cast<float4*>(wbuf + parity * kHalf) = term;
         wave_lds_sync();
         if (summer) {
 #pragma unroll
-            for (int q = 0; q < kSpecSPR; ++q) acc = acc + rbuf[parity * kHalf + 4 * q];
+            for (int q = 0; q < kSPR; ++q) acc = acc + rbuf[parity * kHalf + 4 * q];
         }
     };
     SpecSample A, B;
@@ -680,13 +692,13 @@ __device__ __forceinline__ void specular_split_tile(const float4* __restrict__ c
     for (uint32_t r = 0; r < rounds; r += 2) {
         spec_begin<WIDE>(B, cube, S, fr, N, hB);
         hB = tab_at(r + 3);
-        sum_round(0, spec_term(A, r * kSpecSPR + s < n, cube, S));
+        sum_round(0, spec_term(A, r * kSPR + s < n, cube, S));
         spec_begin<WIDE>(A, cube, S, fr, N, hA);
         hA = tab_at(r + 4);
-        sum_round(1, spec_term(B, (r + 1) * kSpecSPR + s < n, cube, S));
+        sum_round(1, spec_term(B, (r + 1) * kSPR + s < n, cube, S));
     }
     const float wsum = __shfl(acc, (int)((lane & ~3u) | 3u));
-    const uint32_t xs = tx * kSpecTW + st % kSpecTW, ys = ty * kSpecTH + wave * kSpecRPW + st / kSpecTW;
+    const uint32_t xs = tx * kTW + st % kTW, ys = ty * kTH + wave * kRPW + st / kTW;
     if (summer && xs < Sm && ys < Sm) {
         float* o = reinterpret_cast<float*>(out_level + (face * Sm + ys) * Sm + xs);
         o[sc] = sc == 3u ? 1.0f : acc / wsum;
@@ -699,10 +711,10 @@ __device__ __forceinline__ void specular_split_tile(const float4* __restrict__ c
 #ifndef HVX_SPEC_WAVES_PER_EU
 #define HVX_SPEC_WAVES_PER_EU 4
 #endif
-template <bool WIDE>
+template <bool WIDE, int TPW>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HVX_SPEC_WAVES_PER_EU, 8))) void
 specular_split_kernel(SpecSplitArgs a) {
-    __shared__ __align__(16) float s_buf[4][2][kSpecTPW][kSpecRow];
+    __shared__ __align__(16) float s_buf[4][2][TPW][SpecShape<TPW>::kRow];
     // XCD x (workgroups b with b % 8 = x) works through run x of every mip's
     // tiles in turn: a mip's tiles cost about the same, but those of different
     // mips up to several times each other (wider lobes miss the L2 more)
@@ -710,12 +722,12 @@ specular_split_kernel(SpecSplitArgs a) {
     uint32_t m = 1;
     while (k >= a.run_begin[m + 1]) ++m;
     const uint32_t Sm = max(a.So >> m, 1u);
-    const SpecTileGeom g = spec_tile_geom(Sm);
+    const SpecTileGeom g = spec_tile_geom<TPW>(Sm);
     const uint32_t tile = x * (a.run_begin[m + 1] - a.run_begin[m]) + k - a.run_begin[m];
     if (tile >= 6u * g.per_face) return;  // the last run may be short
     uint32_t face, tx, ty;
     spec_tile_at(g, tile, face, tx, ty);
-    specular_split_tile<WIDE>(a.cube, (int)a.S, a.out + cube_level_offset_floats(a.So, m) / 4, Sm, a.emulate ? a.So : Sm,
+    specular_split_tile<WIDE, TPW>(a.cube, (int)a.S, a.out + cube_level_offset_floats(a.So, m) / 4, Sm, a.emulate ? a.So : Sm,
                         a.table + (size_t)m * a.n, a.n, face, tx, ty, &s_buf[0][0][0][0]);
 }
 
@@ -731,7 +743,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HVX_SPEC_WA
 probe_batch_kernel(const ProbeJob* __restrict__ jobs, const ProbeItem* __restrict__ items,
                    const uint32_t* __restrict__ xcd_begin, const float4* __restrict__ tables,
                    uint32_t* __restrict__ queues) {
-    __shared__ __align__(16) float s_buf[4][2][kSpecTPW][kSpecRow];
+    __shared__ __align__(16) float s_buf[4][2][kSpecTPW][SpecShape<kSpecTPW>::kRow];
     __shared__ uint32_t s_item;
     const uint32_t x = blockIdx.x % 8u;
     const uint32_t begin = xcd_begin[x], end = xcd_begin[x + 1];
@@ -754,14 +766,14 @@ probe_batch_kernel(const ProbeJob* __restrict__ jobs, const ProbeItem* __restric
                 out[local] = specular_texel_value(j.cube, j.S, tab, j.n, true, (int)face, (int)tx, (int)ty, (int)Sm);
             }
         } else {
-            const SpecTileGeom g = spec_tile_geom(Sm);
+            const SpecTileGeom g = spec_tile_geom<kSpecTPW>(Sm);
             for (uint32_t k = it.first; k < it.first + it.count; ++k) {
                 uint32_t face, tx, ty;
                 spec_tile_at(g, k, face, tx, ty);
                 if (j.S > kNarrowFace)
-                    specular_split_tile<true>(j.cube, (int)j.S, out, Sm, Sm, tab, j.n, face, tx, ty, &s_buf[0][0][0][0]);
+                    specular_split_tile<true, kSpecTPW>(j.cube, (int)j.S, out, Sm, Sm, tab, j.n, face, tx, ty, &s_buf[0][0][0][0]);
                 else
-                    specular_split_tile<false>(j.cube, (int)j.S, out, Sm, Sm, tab, j.n, face, tx, ty, &s_buf[0][0][0][0]);
+                    specular_split_tile<false, kSpecTPW>(j.cube, (int)j.S, out, Sm, Sm, tab, j.n, face, tx, ty, &s_buf[0][0][0][0]);
             }
         }
     }
@@ -876,13 +888,22 @@ hipError_t launch_specular(const float* d_cube, uint32_t S, float* d_out, uint32
         a.n = n;
         a.emulate = emulate_static_viewport ? 1u : 0u;
         a.table = ggx_table;
-        uint32_t t = 0;
-        for (uint32_t m = 1; m <= (uint32_t)kMaxMips; ++m) {
-            a.run_begin[m] = t;
-            if (m < mips) t += (6u * spec_tile_geom(std::max(So >> m, 1u)).per_face + 7) / 8;
-        }
-        hipLaunchKernelGGL(S > kNarrowFace ? specular_split_kernel<true> : specular_split_kernel<false>, dim3(t * 8),
-                           dim3(256), 0, s, a);
+        auto run = [&](auto wide, auto tpw) {
+            constexpr int kTPW = decltype(tpw)::value;
+            uint32_t t = 0;
+            for (uint32_t m = 1; m <= (uint32_t)kMaxMips; ++m) {
+                a.run_begin[m] = t;
+                if (m < mips) t += (6u * spec_tile_geom<kTPW>(std::max(So >> m, 1u)).per_face + 7) / 8;
+            }
+            hipLaunchKernelGGL((specular_split_kernel<decltype(wide)::value, kTPW>), dim3(t * 8), dim3(256), 0, s, a);
+        };
+        uint32_t tiles = 0;
+        for (uint32_t m = 1; m < mips && tiles <= kSpecFewTiles; ++m)
+            tiles += 6u * spec_tile_geom<kSpecTPW>(std::max(So >> m, 1u)).per_face;
+        const std::integral_constant<int, kSpecTPW> many;
+        const std::integral_constant<int, 1> one;
+        if (S > kNarrowFace) tiles <= kSpecFewTiles ? run(std::true_type(), one) : run(std::true_type(), many);
+        else tiles <= kSpecFewTiles ? run(std::false_type(), one) : run(std::false_type(), many);
     }
     return hipGetLastError();
 }
@@ -908,7 +929,7 @@ void make_probe_items(const ProbeJob* jobs, uint32_t n_probes, uint32_t texels, 
                       uint32_t xcd_begin[9]) {
     items.clear();
     std::vector<double> cost;
-    const uint32_t per_item = std::max(texels / (uint32_t)(kSpecTW * kSpecTH), 1u);
+    const uint32_t per_item = std::max(texels / (uint32_t)(SpecShape<kSpecTPW>::kTW * SpecShape<kSpecTPW>::kTH), 1u);
     for (uint32_t p = 0; p < n_probes; ++p) {
         const ProbeJob& j = jobs[p];
         for (uint32_t m = 0; m < j.mips; ++m) {
@@ -922,11 +943,11 @@ void make_probe_items(const ProbeJob* jobs, uint32_t n_probes, uint32_t texels, 
                 }
                 continue;
             }
-            const SpecTileGeom g = spec_tile_geom(Sm);
+            const SpecTileGeom g = spec_tile_geom<kSpecTPW>(Sm);
             for (uint32_t k = 0; k < 6u * g.per_face; k += per_item) {
                 const uint32_t c = std::min(per_item, 6u * g.per_face - k);
                 items.push_back({p, m, k, c});
-                cost.push_back((double)c * kSpecTW * kSpecTH * j.n * 216.0);
+                cost.push_back((double)c * SpecShape<kSpecTPW>::kTW * SpecShape<kSpecTPW>::kTH * j.n * 216.0);
             }
         }
     }
