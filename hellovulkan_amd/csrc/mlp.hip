@@ -142,9 +142,7 @@ __device__ __forceinline__ void gemm_abt_wave(const GemmArgs& g, uint32_t wave, 
     if (wave >= rts * cgs * g.splitk) return;  // uniform per wave; no barriers below
     const uint32_t slice = wave % g.splitk, t = wave / g.splitk, cg = t % cgs, rt = t / cgs;
     const uint32_t ks = g.Kd / 32;
-    // PART slices are whole blocks of the fused step's 128 samples
-    constexpr uint32_t unit = EPI == EPI_PART ? 4 : 1;
-    const uint32_t kb = slice * (ks / unit) / g.splitk * unit, ke = (slice + 1) * (ks / unit) / g.splitk * unit;
+    const uint32_t kb = slice * ks / g.splitk, ke = (slice + 1) * ks / g.splitk;
     const uint32_t i = lane & 15, gq = lane >> 4;
     const bf16* ap = g.A + (size_t)(rt * 16 + i) * g.Kd + 8 * gq;
     const bf16* bp = g.Bt + (size_t)(cg * 64 + i) * g.Kd + 8 * gq;
@@ -310,7 +308,7 @@ __global__ __launch_bounds__(64 * kOutRedGroups) void reduce_out_kernel(const fl
 }
 
 // ------------------------------------------------ fused per-sample step
-// A training step of a slice of the batch, in blocks of kOutBlock samples:
+// A training step of a slice of the batch, by blocks of kOutBlock samples:
 // forward, output layer, backward and the slice's gradient partials, with
 // every activation and gradient in LDS (131 KB: one workgroup per CU). Every
 // product is the MFMA sequence of gemm_abt_wave over the same BF16 operands,
@@ -413,11 +411,11 @@ __device__ __forceinline__ bf16x8 cols_operand(const bf16* m, uint32_t s, uint32
 // Partial of dW += dZ^T H over the block, for the 16 units of tile ut and NT
 // tiles of 16 columns from tile c0: lane (g, i) holds unit 16 ut + i, columns
 // 4 g .. of each tile. rs: the unit's sum of dZ over this lane's samples (the bias).
+// [lo, hi): the block's steps of 32 samples that are the slice's.
 template <int NT, int W>
 __device__ __forceinline__ void step_partial(const bf16* z, const bf16* h, uint32_t ut, uint32_t c0, uint32_t i,
-                                             uint32_t gq, f32x4 (&acc)[NT], float& rs) {
-#pragma unroll
-    for (uint32_t s = 0; s < kOutBlock / 32; ++s) {
+                                             uint32_t gq, uint32_t lo, uint32_t hi, f32x4 (&acc)[NT], float& rs) {
+    auto step = [&](uint32_t s) {
         const bf16x8 zo = cols_operand<kH>(z, s, ut, i, gq);
 #pragma unroll
         for (int n = 0; n < NT; ++n) acc[n] = hvx::mfma16x16x32(cols_operand<W>(h, s, c0 + n, i, gq), zo, acc[n]);
@@ -425,6 +423,13 @@ __device__ __forceinline__ void step_partial(const bf16* z, const bf16* h, uint3
 #pragma unroll
         for (int q = 0; q < 8; ++q) t += (float)zo[q];
         rs += t;
+    };
+    if (hi - lo == kOutBlock / 32) {
+#pragma unroll
+        for (uint32_t s = 0; s < kOutBlock / 32; ++s) step(s);
+    } else {
+#pragma unroll 1
+        for (uint32_t s = lo; s < hi; ++s) step(s);
     }
 }
 template <int NT>
@@ -440,9 +445,14 @@ __device__ __forceinline__ void step_write_partial(float* part, uint32_t K, uint
 }
 
 // X: [blocks * kOutBlock][kIn] encodings; Ws: the weights in operand order;
-// slice q of the launch takes blocks q * blocks / slices ..; part: per layer,
-// then slice, [kH][K] and the bias gradient [kH]; opart: [blocks][kOutPart]
+// slice q of the launch sums steps of 32 samples from q * steps / slices on
+// (gemm_abt_wave's slices); a block that two slices share is evaluated for
+// both, and its output-layer partials are those of the slice with its first
+// step. part: per layer, then slice, [kH][K] and the bias gradient [kH]; opart:
+// [blocks][kOutPart]
 constexpr uint32_t kLen1 = kH * kIn + kH, kLen23 = kH * kH + kH;  // a layer's partial
+// WHOLE: every slice is whole blocks.
+template <bool WHOLE>
 __global__ __launch_bounds__(kStepThreads) void mlp_step_kernel(const bf16* __restrict__ X, const float* __restrict__ P,
                                                                 const bf16* __restrict__ Ws,
                                                                 const float4* __restrict__ tgt, uint32_t blocks,
@@ -464,7 +474,19 @@ __global__ __launch_bounds__(kStepThreads) void mlp_step_kernel(const bf16* __re
         for (int s = 0; s < 4; ++s) x[s] = *reinterpret_cast<const bf16x8*>(xp + 4 * s * kIn + 8 * lane);
         tv = tgt[(size_t)q * kOutBlock + (wave & 1) * 64 + lane];
     };
-    const uint32_t q0 = blockIdx.x * blocks / gridDim.x, q1 = (blockIdx.x + 1) * blocks / gridDim.x;
+    constexpr uint32_t kSteps = kOutBlock / 32;
+    const uint32_t k0 = blockIdx.x * (blocks * kSteps) / gridDim.x, k1 = (blockIdx.x + 1) * (blocks * kSteps) / gridDim.x;
+    const uint32_t q0 = k0 / kSteps, q1 = (k1 + kSteps - 1) / kSteps;
+    if (!WHOLE && k0 == k1) {  // a slice of no steps (uniform over the workgroup)
+        const f32x4 none[4] = {};
+        const f32x4 none2[2] = {};
+        const size_t sl = blockIdx.x, n = gridDim.x;
+        const uint32_t i = lane & 15, gq = lane >> 4;
+        step_write_partial<2>(part + n * (kLen1 + kLen23) + sl * kLen23, kH, ut, 2 * ch, i, gq, none2, 0.0f);
+        step_write_partial<2>(part + n * kLen1 + sl * kLen23, kH, ut, 2 * ch, i, gq, none2, 0.0f);
+        step_write_partial<4>(part + sl * kLen1, kIn, ut, 4 * ch, i, gq, none, 0.0f);
+        return;
+    }
     fetch(q0);
     // this wave's fragment s of a product's weights
     auto weights = [&](uint32_t ofs, uint32_t frags, uint32_t s) {
@@ -614,7 +636,11 @@ __global__ __launch_bounds__(kStepThreads) void mlp_step_kernel(const bf16* __re
         product(sh.z3, w3t, acc);
         masked(acc, m2, sh.z2);
         float* pp = opart + (size_t)q * kOutPart;
-        if (wave < 3) {  // dW4[wave][lane]: the samples in order
+        const uint32_t lo = WHOLE ? 0 : max(k0, kSteps * q) - kSteps * q,
+                       hi = WHOLE ? kSteps : min(k1 - kSteps * q, kSteps);
+        if (!WHOLE && kSteps * q < k0) {
+            // the slice before has written them
+        } else if (wave < 3) {  // dW4[wave][lane]: the samples in order
             float sum = 0.0f;
 #pragma unroll 1
             for (uint32_t c0 = 0; c0 < kOutBlock / 8; c0 += 4) {
@@ -648,7 +674,7 @@ __global__ __launch_bounds__(kStepThreads) void mlp_step_kernel(const bf16* __re
             for (int d = 32; d > 0; d >>= 1) v += __shfl_down(v, d, 64);
             if (lane == 0) pp[kOutPart - 1] = v;
         }
-        step_partial<2, kH>(sh.z3, sh.h2, ut, 2 * ch, i, gq, p3, rs3);
+        step_partial<2, kH>(sh.z3, sh.h2, ut, 2 * ch, i, gq, lo, hi, p3, rs3);
         const bool last = q + 1 == q1;
         const size_t sl = blockIdx.x, n = gridDim.x;
         if (last) step_write_partial<2>(part + n * (kLen1 + kLen23) + sl * kLen23, kH, ut, 2 * ch, i, gq, p3, rs3);
@@ -656,10 +682,10 @@ __global__ __launch_bounds__(kStepThreads) void mlp_step_kernel(const bf16* __re
         // dZ1 (over dZ3) and the partials of layer 2
         product(sh.z2, w2t, acc);
         masked(acc, m1, sh.z3);
-        step_partial<2, kH>(sh.z2, sh.h1, ut, 2 * ch, i, gq, p2, rs2);
+        step_partial<2, kH>(sh.z2, sh.h1, ut, 2 * ch, i, gq, lo, hi, p2, rs2);
         if (last) step_write_partial<2>(part + n * kLen1 + sl * kLen23, kH, ut, 2 * ch, i, gq, p2, rs2);
         __syncthreads();
-        step_partial<4, kIn>(sh.z3, sh.x, ut, 4 * ch, i, gq, p1, rs1);
+        step_partial<4, kIn>(sh.z3, sh.x, ut, 4 * ch, i, gq, lo, hi, p1, rs1);
         if (last) step_write_partial<4>(part + sl * kLen1, kIn, ut, 4 * ch, i, gq, p1, rs1);
     }
 }
@@ -891,6 +917,7 @@ struct hvx_mlp {
     uint32_t cap = 0;  // batch capacity
     bf16* X0 = nullptr;
     float *part = nullptr, *opart = nullptr;
+    uint32_t splitk = 1;
     // HVX_OPT_MLP_SEPARATE_LAUNCHES: the activations and gradients in memory
     uint32_t sep_cap = 0;
     bf16 *W2T = nullptr, *W3T = nullptr;
@@ -935,9 +962,6 @@ template <class T> hipError_t dalloc(std::vector<void*>& list, T** p, size_t cou
     return e;
 }
 
-// slices of a batch's gradient partials (whole blocks of kOutBlock samples)
-uint32_t slices_of(uint32_t B) { return std::min(256u, B / kOutBlock); }
-
 void encode(const float4* in, uint32_t n, uint32_t B, float lod_max, bf16* X, bf16* XT, hipStream_t s) {
     hipLaunchKernelGGL(mlp_pe_kernel, dim3(std::min((B + 15) / 16, 1u << 18)), dim3(256), 0, s, in, n, B, lod_max, X, XT);
 }
@@ -952,8 +976,11 @@ hipError_t ensure_batch(hvx_mlp* M, uint32_t B) {
         M->batch_allocs.clear();
         M->cap = 0;
         auto& L = M->batch_allocs;
+        // weight gradients are summed in slices of 128 samples of the largest
+        // batch, up to 256 of them
+        M->splitk = std::max(1u, std::min(256u, B / kOutBlock));
         if ((e = dalloc(L, &M->X0, (size_t)B * kIn)) ||
-            (e = dalloc(L, &M->part, (size_t)slices_of(B) * ((kH * kIn + kH) + 2 * (kH * kH + kH)))) ||
+            (e = dalloc(L, &M->part, (size_t)M->splitk * (kLen1 + 2 * kLen23))) ||
             (e = dalloc(L, &M->opart, (size_t)(B / kOutBlock) * kOutPart)))
             return e;
         M->cap = B;
@@ -1025,7 +1052,7 @@ void gradient_separate(hvx_mlp* M, const float4* in, const float4* tgt, uint32_t
         g.M = kH;
         g.Nc = K;
         g.Kd = B;
-        g.splitk = slices_of(B);
+        g.splitk = M->splitk;
         g.part = M->part;
         g.pstride = kH * K + kH;
         g.colsum = 1;
@@ -1035,7 +1062,7 @@ void gradient_separate(hvx_mlp* M, const float4* in, const float4* tgt, uint32_t
                           hvx::kMlpB3 == hvx::kMlpW3 + kH * kH,
                       "each layer's bias follows its weights");
         hipLaunchKernelGGL(reduce_slices_kernel, dim3((kH * K + kH + 63) / 64), dim3(64 * kRedGroups), 0, s,
-                           M->part, slices_of(B), (uint32_t)(kH * K + kH), G + wofs[l]);
+                           M->part, M->splitk, (uint32_t)(kH * K + kH), G + wofs[l]);
         if (l > 0) {
             GemmArgs d{};
             d.A = dz;
@@ -1060,7 +1087,7 @@ void gradient_separate(hvx_mlp* M, const float4* in, const float4* tgt, uint32_t
 void gradient_fused(hvx_mlp* M, const float4* in, const bf16* x0, const float4* tgt, uint32_t B, float* G,
                     const AdamArgs* adam, float* loss, hipStream_t s) {
     if (!x0) encode(in, B, B, M->lod_max, M->X0, nullptr, s);
-    const uint32_t blocks = B / kOutBlock, slices = slices_of(B);
+    const uint32_t blocks = B / kOutBlock, slices = M->splitk;
     const int wofs[4] = {hvx::kMlpW1, hvx::kMlpW2, hvx::kMlpW3, hvx::kMlpW4};
     ReduceStep r{};
     float* part = M->part;
@@ -1077,7 +1104,7 @@ void gradient_fused(hvx_mlp* M, const float4* in, const bf16* x0, const float4* 
     r.loss_scale = 1.0f / (3.0f * (float)B);
     r.G = G;
     if (adam) r.adam = *adam;
-    hipLaunchKernelGGL(mlp_step_kernel, dim3(slices), dim3(kStepThreads), 0, s, x0 ? x0 : M->X0, M->P, M->Ws,
+    hipLaunchKernelGGL(blocks % slices == 0 ? mlp_step_kernel<true> : mlp_step_kernel<false>, dim3(slices), dim3(kStepThreads), 0, s, x0 ? x0 : M->X0, M->P, M->Ws,
                        tgt, blocks, 2.0f / (3.0f * (float)B), M->part, M->opart);
     if (adam) hipLaunchKernelGGL(reduce_step_kernel<true>, dim3(r.b[4]), dim3(64 * kRedGroups), 0, s, r);
     else hipLaunchKernelGGL(reduce_step_kernel<false>, dim3(r.b[4]), dim3(64 * kRedGroups), 0, s, r);

@@ -1,6 +1,6 @@
 """The training step's block kernel at the sizes where its slices change: one
-block per slice up to 32,768 samples, then whole blocks shared out over 256
-slices (258 blocks: two slices of two; 516; 2 x 256). Gradient, loss and
+block per slice up to 32,768 samples, then 256 slices of any number of steps of 32
+(33,024: four or five, across blocks; 66,048; 2 x 256 blocks). Gradient, loss and
 parameters after steps equal the separate launches bit for bit (both sum the
 same products over the same slices in the same order)."""
 import numpy as np
