@@ -507,12 +507,18 @@ template <int TPW> struct SpecShape {
     static constexpr int kRow = 4 * kSPR + 4;                     // floats per texel row of the LDS buffer (padded)
 };
 // Small maps wait for their rounds (a texel's 1,024 samples are 64 of them with
-// four texels to a wave) with most of the card idle: with at most kSpecFewTiles
-// tiles a wave takes one texel and 64 samples a round. us of the whole call with
-// four / one: 16^2 x 4 and 256 samples (36 tiles) 44 / 27, 40^2 x 5 and 1,024 (234)
-// 94 / 55, 64^2 x 6 and 512 (516) 79 / 71, 90^2 x 4 and 700 (1,134) 326 / 272,
-// 128^2 x 6 and 1,024 (2,046) 244 / 259.
-constexpr uint32_t kSpecFewTiles = 1536;
+// four texels to a wave) with most of the card idle: there a wave takes one
+// texel and 64 samples a round. What is left of a round's gain past the starts
+// of four times the waves grows with the samples and falls with the tiles. us
+// of the whole call with four / one:
+//   16^2 x 4 and 256 samples (36 tiles) 44 / 27, 64^2 x 2 (384): 16 samples
+//   13.2 / 17.3, 64: 22.5 / 23.6, 1,024: 102 / 98, 64^2 x 7 (522): 64 samples
+//   21.3 / 23.8, 1,024: 107 / 89, 80^2 x 2 (600): 64 samples 24.1 / 27.5, 256:
+//   53 / 49, 90^2 x 4 from 1000^2 (1,134): 128 samples 78 / 68, 1,024: 463 / 375,
+//   100^2 x 7 (1,398): 128 samples 38 / 43, 1,024: 188 / 169, but 110^2 x 3
+//   (1,470) 244 / 259, 128^2 x 2 (1,536): 64 samples 33 / 46, 1,024: 275 / 305
+constexpr uint32_t kSpecFewTiles = 1500;
+inline bool spec_few(uint32_t tiles, uint32_t n) { return tiles <= kSpecFewTiles && 9ull * n >= tiles; }
 
 struct SpecSplitArgs {
     const float4* cube;
@@ -902,8 +908,9 @@ hipError_t launch_specular(const float* d_cube, uint32_t S, float* d_out, uint32
             tiles += 6u * spec_tile_geom<kSpecTPW>(std::max(So >> m, 1u)).per_face;
         const std::integral_constant<int, kSpecTPW> many;
         const std::integral_constant<int, 1> one;
-        if (S > kNarrowFace) tiles <= kSpecFewTiles ? run(std::true_type(), one) : run(std::true_type(), many);
-        else tiles <= kSpecFewTiles ? run(std::false_type(), one) : run(std::false_type(), many);
+        const bool few = spec_few(tiles, n);
+        if (S > kNarrowFace) few ? run(std::true_type(), one) : run(std::true_type(), many);
+        else few ? run(std::false_type(), one) : run(std::false_type(), many);
     }
     return hipGetLastError();
 }
