@@ -15,6 +15,7 @@
 
 #include "hvx_device.h"
 #include "hvx_internal.h"
+#include "spec_tiles.h"
 
 static_assert(sizeof(hvx_probe) == 32 && sizeof(hvx_view) == 232 && sizeof(hvx_batch_tuning) == 24,
               "batch descriptor layouts are part of the ABI");
@@ -74,6 +75,7 @@ struct hvx_batch {
     DevBuf<hvx::ProbeItem> d_items;
     DevBuf<uint32_t> d_xcd_begin;  // [9]: item runs of the per-XCD probe queues
     uint32_t n_items = 0;
+    bool wide = false, one = false;  // probe_batch_kernel's variant
     std::vector<ViewScratch> vscratch;
     DevBuf<hvx::CullBatchView> d_views;
     hvx::CullBatchTotals totals{};
@@ -111,7 +113,9 @@ bool misaligned(const void* p, size_t a) { return (reinterpret_cast<uintptr_t>(p
 int upload_items(hvx_batch* b) {
     std::vector<hvx::ProbeItem> items;
     uint32_t xcd_begin[9];
-    hvx::make_probe_items(b->jobs.data(), (uint32_t)b->jobs.size(), b->tuning.probe_tile, items, xcd_begin);
+    b->one = hvx::make_probe_items(b->jobs.data(), (uint32_t)b->jobs.size(), b->tuning.probe_tile,
+                                   (uint32_t)b->ctx->num_cus * b->tuning.probe_wgs_per_cu, items, xcd_begin);
+    b->wide = std::any_of(b->jobs.begin(), b->jobs.end(), [](const hvx::ProbeJob& j) { return j.S > hvx::kNarrowFace; });
     hipError_t e;
     if (b->d_items.n < items.size() && (e = b->d_items.alloc(items.size())) != hipSuccess)
         return bhip(b, e, "batch item allocation");
@@ -201,7 +205,8 @@ hipError_t run_probes(hvx_batch* b, hipStream_t s) {
     if (!b->classes.empty()) return run_contract(b, s);
     if (b->n_items == 0) return hipSuccess;
     return hvx::launch_probe_batch(b->d_jobs.p, b->d_items.p, b->d_xcd_begin.p, b->d_tables.p,
-                                   (uint32_t)b->ctx->num_cus * b->tuning.probe_wgs_per_cu, b->d_queues.p, s);
+                                   (uint32_t)b->ctx->num_cus * b->tuning.probe_wgs_per_cu, b->wide, b->one,
+                                   b->d_queues.p, s);
 }
 
 hipError_t run_culls(hvx_batch* b, hipStream_t s) {
@@ -402,7 +407,8 @@ int hvx_batch_set_tuning(hvx_batch* b, const hvx_batch_tuning* t) {
     int st;
     if ((st = check_tuning(b, *t))) return st;
     (void)hipDeviceSynchronize();  // the device tables may be in use
-    const bool items = t->probe_tile != b->tuning.probe_tile, views = t->cull_shape != b->tuning.cull_shape;
+    const bool items = t->probe_tile != b->tuning.probe_tile || t->probe_wgs_per_cu != b->tuning.probe_wgs_per_cu,
+               views = t->cull_shape != b->tuning.cull_shape;
     b->tuning = *t;
     if ((items && (st = upload_items(b))) || (views && (st = upload_views(b)))) return st;
     b->graph_stale = true;

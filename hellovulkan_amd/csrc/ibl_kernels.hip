@@ -31,6 +31,7 @@
 
 #include "hvx_device.h"
 #include "hvx_internal.h"
+#include "spec_tiles.h"
 
 namespace hvx {
 namespace {
@@ -494,32 +495,6 @@ __global__ __launch_bounds__(256) void specular_delta_kernel(const float4* __res
 //   no length checks, 32-bit offsets                     3.71 ms (VALU 81 % busy)
 //   roughness 0 summed by binades                        3.60 ms
 //   pairs exchanged by selects that read across lanes    3.53 ms
-#ifndef HVX_SPEC_TPW
-#define HVX_SPEC_TPW 4
-#endif
-constexpr int kSpecTPW = HVX_SPEC_TPW;  // texels per wave: 4, 8 or 16
-static_assert(kSpecTPW == 4 || kSpecTPW == 8 || kSpecTPW == 16, "HVX_SPEC_TPW is 4, 8 or 16");
-template <int TPW> struct SpecShape {
-    static constexpr int kSPR = 64 / TPW;                         // samples per texel per round
-    static constexpr int kTW = TPW >= 8 ? 8 : (TPW >= 4 ? 4 : 1);  // tile width (texels)
-    static constexpr int kRPW = TPW / kTW;                        // texel rows per wave
-    static constexpr int kTH = 4 * kRPW;                          // tile height: four waves
-    static constexpr int kRow = 4 * kSPR + 4;                     // floats per texel row of the LDS buffer (padded)
-};
-// Small maps wait for their rounds (a texel's 1,024 samples are 64 of them with
-// four texels to a wave) with most of the card idle: there a wave takes one
-// texel and 64 samples a round. What is left of a round's gain past the starts
-// of four times the waves grows with the samples and falls with the tiles. us
-// of the whole call with four / one:
-//   16^2 x 4 and 256 samples (36 tiles) 44 / 27, 64^2 x 2 (384): 16 samples
-//   13.2 / 17.3, 64: 22.5 / 23.6, 1,024: 102 / 98, 64^2 x 7 (522): 64 samples
-//   21.3 / 23.8, 1,024: 107 / 89, 80^2 x 2 (600): 64 samples 24.1 / 27.5, 256:
-//   53 / 49, 90^2 x 4 from 1000^2 (1,134): 128 samples 78 / 68, 1,024: 463 / 375,
-//   100^2 x 7 (1,398): 128 samples 38 / 43, 1,024: 188 / 169, but 110^2 x 3
-//   (1,470) 244 / 259, 128^2 x 2 (1,536): 64 samples 33 / 46, 1,024: 275 / 305
-constexpr uint32_t kSpecFewTiles = 1500;
-inline bool spec_few(uint32_t tiles, uint32_t n) { return tiles <= kSpecFewTiles && 9ull * n >= tiles; }
-
 struct SpecSplitArgs {
     const float4* cube;
     uint32_t S;
@@ -578,9 +553,8 @@ __device__ __forceinline__ void pair_exchange(const int (&x)[2], const int (&y)[
             : "vcc", "scc");
 }
 
-// Texel i of a cube level. WIDE false: the level is smaller than 4 GiB, so a
-// 32-bit byte offset from the uniform base will do.
-constexpr uint32_t kNarrowFace = 6688;  // largest face of such a level
+// Texel i of a cube level. WIDE false: the level is smaller than 4 GiB (faces up
+// to kNarrowFace), so a 32-bit byte offset from the uniform base will do.
 template <bool WIDE>
 __device__ __forceinline__ float4 cube_at(const float4* __restrict__ cube, int i) {
     if constexpr (WIDE) return cube[i];
@@ -625,32 +599,6 @@ __device__ __forceinline__ float4 spec_term(const SpecSample& p, bool live, cons
     if (!(live && p.nol > 0.0f)) return make_float4(-0.0f, -0.0f, -0.0f, -0.0f);
     const f3 c = cube_combine(cube, S, p.L, p.taps, q);
     return make_float4(c.x * p.nol, c.y * p.nol, c.z * p.nol, p.nol);
-}
-
-// Tiles of one mip of size Sm: kTW x kTH texels, taken face by face in
-// supertiles of 16 x 16 tiles (row-major supertiles, row-major tiles in each;
-// the last column and row of supertiles are as wide and high as is left).
-struct SpecTileGeom {
-    uint32_t tiles_x, tiles_y, per_face;
-};
-template <int TPW> __host__ __device__ inline SpecTileGeom spec_tile_geom(uint32_t Sm) {
-    constexpr uint32_t kTW = SpecShape<TPW>::kTW, kTH = SpecShape<TPW>::kTH;
-    SpecTileGeom g;
-    g.tiles_x = (Sm + kTW - 1) / kTW;
-    g.tiles_y = (Sm + kTH - 1) / kTH;
-    g.per_face = g.tiles_x * g.tiles_y;
-    return g;
-}
-// Tile index (< 6 per_face) -> (face, tx, ty).
-__host__ __device__ inline void spec_tile_at(const SpecTileGeom& g, uint32_t k, uint32_t& face, uint32_t& tx,
-                                             uint32_t& ty) {
-    face = k / g.per_face;
-    const uint32_t kk = k % g.per_face, row = kk / (16u * g.tiles_x), kr = kk % (16u * g.tiles_x);
-    const uint32_t high = g.tiles_y - 16u * row < 16u ? g.tiles_y - 16u * row : 16u;
-    const uint32_t col = kr / (16u * high), kc = kr % (16u * high);
-    const uint32_t wide = g.tiles_x - 16u * col < 16u ? g.tiles_x - 16u * col : 16u;
-    tx = 16u * col + kc % wide;
-    ty = 16u * row + kc / wide;
 }
 
 // One tile of the sample-split specular loop (four waves, each independent):
@@ -739,17 +687,16 @@ specular_split_kernel(SpecSplitArgs a) {
 
 // ------------------------------------------------- batched probe prefilter
 // Persistent: the workgroups on XCD x (workgroup b runs on XCD b % 8) pull
-// items from queue x, which serves the contiguous run [xcd_begin[x],
-// xcd_begin[x+1]) of the item list; the host orders items by probe, mip and
-// tile and cuts the runs at equal estimated cost, so each XCD works through
-// neighbouring tiles of a few probes and shares their texels in its L2.
+// items from queue x, which serves the run [xcd_begin[x], xcd_begin[x+1]) of
+// the item list (make_probe_items: XCD x's share of every mip of every probe).
 // Items of mip 0 are texel ranges (lane per texel, as specular_delta_kernel);
 // other items are runs of tiles (specular_split_tile).
+template <bool WIDE, int TPW>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HVX_SPEC_WAVES_PER_EU, 8))) void
 probe_batch_kernel(const ProbeJob* __restrict__ jobs, const ProbeItem* __restrict__ items,
                    const uint32_t* __restrict__ xcd_begin, const float4* __restrict__ tables,
                    uint32_t* __restrict__ queues) {
-    __shared__ __align__(16) float s_buf[4][2][kSpecTPW][SpecShape<kSpecTPW>::kRow];
+    __shared__ __align__(16) float s_buf[4][2][TPW][SpecShape<TPW>::kRow];
     __shared__ uint32_t s_item;
     const uint32_t x = blockIdx.x % 8u;
     const uint32_t begin = xcd_begin[x], end = xcd_begin[x + 1];
@@ -772,14 +719,11 @@ probe_batch_kernel(const ProbeJob* __restrict__ jobs, const ProbeItem* __restric
                 out[local] = specular_texel_value(j.cube, j.S, tab, j.n, true, (int)face, (int)tx, (int)ty, (int)Sm);
             }
         } else {
-            const SpecTileGeom g = spec_tile_geom<kSpecTPW>(Sm);
+            const SpecTileGeom g = spec_tile_geom<TPW>(Sm);
             for (uint32_t k = it.first; k < it.first + it.count; ++k) {
                 uint32_t face, tx, ty;
                 spec_tile_at(g, k, face, tx, ty);
-                if (j.S > kNarrowFace)
-                    specular_split_tile<true, kSpecTPW>(j.cube, (int)j.S, out, Sm, Sm, tab, j.n, face, tx, ty, &s_buf[0][0][0][0]);
-                else
-                    specular_split_tile<false, kSpecTPW>(j.cube, (int)j.S, out, Sm, Sm, tab, j.n, face, tx, ty, &s_buf[0][0][0][0]);
+                specular_split_tile<WIDE, TPW>(j.cube, (int)j.S, out, Sm, Sm, tab, j.n, face, tx, ty, &s_buf[0][0][0][0]);
             }
         }
     }
@@ -921,54 +865,13 @@ hipError_t launch_ggx_tables(uint32_t mips, uint32_t n, float4* table, hipStream
 }
 
 hipError_t launch_probe_batch(const ProbeJob* d_jobs, const ProbeItem* d_items, const uint32_t* d_xcd_begin,
-                              const float4* d_tables, uint32_t persistent_wgs, uint32_t* d_queues, hipStream_t s) {
+                              const float4* d_tables, uint32_t persistent_wgs, bool wide, bool one, uint32_t* d_queues,
+                              hipStream_t s) {
     const uint32_t grid = std::max((persistent_wgs + 7) / 8, 1u) * 8;  // every XCD gets workgroups
-    hipLaunchKernelGGL(probe_batch_kernel, dim3(grid), dim3(256), 0, s, d_jobs, d_items, d_xcd_begin, d_tables,
-                       d_queues);
+    const auto kernel = wide ? (one ? probe_batch_kernel<true, 1> : probe_batch_kernel<true, kSpecTPW>)
+                             : (one ? probe_batch_kernel<false, 1> : probe_batch_kernel<false, kSpecTPW>);
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, s, d_jobs, d_items, d_xcd_begin, d_tables, d_queues);
     return hipGetLastError();
-}
-
-// Batch work items (probe, mip, range) for the probes of `jobs`, in probe,
-// mip, tile order: mip 0 as ranges of `texels` texels, other mips as runs of
-// about texels / 16 tiles; xcd_begin[0..8] cuts the
-// list into eight runs of equal estimated cost.
-void make_probe_items(const ProbeJob* jobs, uint32_t n_probes, uint32_t texels, std::vector<ProbeItem>& items,
-                      uint32_t xcd_begin[9]) {
-    items.clear();
-    std::vector<double> cost;
-    const uint32_t per_item = std::max(texels / (uint32_t)(SpecShape<kSpecTPW>::kTW * SpecShape<kSpecTPW>::kTH), 1u);
-    for (uint32_t p = 0; p < n_probes; ++p) {
-        const ProbeJob& j = jobs[p];
-        for (uint32_t m = 0; m < j.mips; ++m) {
-            const uint32_t Sm = std::max(j.So >> m, 1u);
-            if (m == 0) {
-                const uint32_t T = 6u * Sm * Sm;
-                for (uint32_t f = 0; f < T; f += texels) {
-                    const uint32_t c = std::min(texels, T - f);
-                    items.push_back({p, 0, f, c});
-                    cost.push_back((double)c * (200.0 + 4.0 * j.n));  // one sample and n sums per texel
-                }
-                continue;
-            }
-            const SpecTileGeom g = spec_tile_geom<kSpecTPW>(Sm);
-            for (uint32_t k = 0; k < 6u * g.per_face; k += per_item) {
-                const uint32_t c = std::min(per_item, 6u * g.per_face - k);
-                items.push_back({p, m, k, c});
-                cost.push_back((double)c * SpecShape<kSpecTPW>::kTW * SpecShape<kSpecTPW>::kTH * j.n * 216.0);
-            }
-        }
-    }
-    double total = 0.0;
-    for (double c : cost) total += c;
-    uint32_t x = 1;
-    double run = 0.0;
-    xcd_begin[0] = 0;
-    for (uint32_t i = 0; i < (uint32_t)items.size() && x < 8; ++i) {
-        run += cost[i];
-        while (x < 8 && run >= total * x / 8.0) xcd_begin[x++] = i + 1;
-    }
-    while (x < 8) xcd_begin[x++] = (uint32_t)items.size();
-    xcd_begin[8] = (uint32_t)items.size();
 }
 
 }  // namespace hvx

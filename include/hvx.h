@@ -518,7 +518,7 @@ typedef struct hvx_view {
 
 /* Tile shapes of the batched kernels. hvx_batch_autotune fills the timings. */
 typedef struct hvx_batch_tuning {
-    uint32_t probe_tile;        /* output texels per probe work item, 32..8192 */
+    uint32_t probe_tile;        /* output texels per probe work item at most, 32..8192 */
     uint32_t probe_wgs_per_cu;  /* persistent probe workgroups per CU, 1..16 */
     uint32_t cull_shape;        /* cluster block: 0 = 4x4x1, 1 = 8x4x1, 2 = 4x4x2, 3 = 2x2x4 */
     uint32_t cull_wgs_per_cu;   /* persistent culling workgroups per CU, 1..16 */
