@@ -126,6 +126,7 @@ struct GemmArgs {
     const bf16* A;   // [M][Kd]
     const bf16* Bt;  // [Nc][Kd]
     uint32_t M, Nc, Kd, splitk;
+    uint32_t ldb;       // elements between the rows of Bt
     const float* bias;  // FWD: [Nc]
     const bf16* mask;   // BWD: [M][Nc], zero where <= 0
     bf16* C;            // FWD/BWD: [M][Nc]
@@ -145,8 +146,8 @@ __device__ __forceinline__ void gemm_abt_wave(const GemmArgs& g, uint32_t wave, 
     const uint32_t kb = slice * ks / g.splitk, ke = (slice + 1) * ks / g.splitk;
     const uint32_t i = lane & 15, gq = lane >> 4;
     const bf16* ap = g.A + (size_t)(rt * 16 + i) * g.Kd + 8 * gq;
-    const bf16* bp = g.Bt + (size_t)(cg * 64 + i) * g.Kd + 8 * gq;
-    const size_t bstep = (size_t)16 * g.Kd;
+    const bf16* bp = g.Bt + (size_t)(cg * 64 + i) * g.ldb + 8 * gq;
+    const size_t bstep = (size_t)16 * g.ldb;
     f32x4 acc[4];
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) acc[nb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -343,9 +344,10 @@ constexpr uint32_t kWs1 = 0, kWs2 = kH * kIn, kWs3 = kWs2 + kH * kH, kWs3T = kWs
 __device__ __forceinline__ uint32_t operand_index(uint32_t row, uint32_t k, uint32_t K) {
     return ((row / 16 * (K / 32) + k / 32) * 64 + (k % 32 / 8) * 16 + row % 16) * 8 + k % 8;
 }
-// BF16 copies of parameter i: the rows W1..W3 and the operands of the step
+// BF16 copies of parameter i: the rows W1..W3, the operands of the step and, if
+// set, the transposes of W2 and W3 ([in][out]) for the separate launches
 struct WeightCopies {
-    bf16 *W1, *W2, *W3, *Ws;
+    bf16 *W1, *W2, *W3, *Ws, *W2T, *W3T;
 };
 __device__ __forceinline__ void write_copies(const WeightCopies& c, uint32_t i, bf16 h) {
     if (i - (uint32_t)hvx::kMlpW1 < (uint32_t)(kH * kIn)) {
@@ -358,12 +360,14 @@ __device__ __forceinline__ void write_copies(const WeightCopies& c, uint32_t i, 
         c.W2[j] = h;
         c.Ws[kWs2 + operand_index(o, k, kH)] = h;
         c.Ws[kWs2T + operand_index(k, o, kH)] = h;
+        if (c.W2T) c.W2T[k * kH + o] = h;
     }
     if (i - (uint32_t)hvx::kMlpW3 < (uint32_t)(kH * kH)) {
         const uint32_t j = i - hvx::kMlpW3, o = j / kH, k = j % kH;
         c.W3[j] = h;
         c.Ws[kWs3 + operand_index(o, k, kH)] = h;
         c.Ws[kWs3T + operand_index(k, o, kH)] = h;
+        if (c.W3T) c.W3T[k * kH + o] = h;
     }
 }
 
@@ -788,14 +792,6 @@ __global__ __launch_bounds__(256) void mlp_cast_kernel(const float* __restrict__
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;
     if (i < (uint32_t)hvx::kMlpParams) write_copies(c, i, (bf16)P[i]);
 }
-// W2^T and W3^T ([in][out]) for the separate launches' backward products
-__global__ __launch_bounds__(256) void mlp_transpose_kernel(const bf16* __restrict__ W2, const bf16* __restrict__ W3,
-                                                            bf16* __restrict__ W2T, bf16* __restrict__ W3T) {
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x, t = (i % kH) * kH + i / kH;
-    W2T[t] = W2[i];
-    W3T[t] = W3[i];
-}
-
 // Inference through the in-shading path (mlp_device.h): each workgroup
 // stages the weights once, its four waves evaluate kInferTiles x 16 samples
 // per call. Bound by its vector instructions, 1,090 per 32 samples (512 of
@@ -914,18 +910,20 @@ struct hvx_mlp {
     float lod_max = 1.0f;
     float *P = nullptr, *G = nullptr, *m = nullptr, *v = nullptr;
     bf16 *W1 = nullptr, *W2 = nullptr, *W3 = nullptr, *Ws = nullptr;
+    bf16 *W2T = nullptr, *W3T = nullptr;
+    bool transposes = false;  // W2T and W3T hold the weights: only the separate launches keep them so
     uint32_t cap = 0;  // batch capacity
     bf16* X0 = nullptr;
     float *part = nullptr, *opart = nullptr;
     uint32_t splitk = 1;
     // HVX_OPT_MLP_SEPARATE_LAUNCHES: the activations and gradients in memory
     uint32_t sep_cap = 0;
-    bf16 *W2T = nullptr, *W3T = nullptr;
     bf16 *X0T = nullptr, *H[3] = {}, *HT[3] = {}, *dZa = nullptr, *dZaT = nullptr, *dZb = nullptr, *dZbT = nullptr;
     uint64_t steps_done = 0;
-    // a training call's inputs encoded once: [n][kIn]
-    bf16* enc = nullptr;
-    size_t enc_cap = 0;
+    // a training call's inputs encoded once: [n][kIn] and, for the separate
+    // launches, transposed [kIn][n]
+    bf16 *enc = nullptr, *encT = nullptr;
+    size_t enc_cap = 0, encT_cap = 0;
     // per-cell estimate from below of the network's output, from the last
     // hvx_mlp_cell_errors call (cell grid lo_face x lo_face x lo_bins)
     float4* cell_lo = nullptr;  // RGB and a pad per cell
@@ -990,9 +988,7 @@ hipError_t ensure_batch(hvx_mlp* M, uint32_t B) {
         M->sep_allocs.clear();
         M->sep_cap = 0;
         auto& L = M->sep_allocs;
-        if ((e = dalloc(L, &M->W2T, (size_t)kH * kH)) || (e = dalloc(L, &M->W3T, (size_t)kH * kH)) ||
-            (e = dalloc(L, &M->X0T, (size_t)B * kIn)))
-            return e;
+        if ((e = dalloc(L, &M->X0T, (size_t)B * kIn))) return e;
         for (int l = 0; l < 3; ++l)
             if ((e = dalloc(L, &M->H[l], (size_t)B * kH)) || (e = dalloc(L, &M->HT[l], (size_t)B * kH))) return e;
         if ((e = dalloc(L, &M->dZa, (size_t)B * kH)) || (e = dalloc(L, &M->dZaT, (size_t)B * kH)) ||
@@ -1008,19 +1004,34 @@ template <int EPI> void gemm(const GemmArgs& g, hipStream_t s) {
     hipLaunchKernelGGL(gemm_abt_kernel<EPI>, dim3((waves + 3) / 4), dim3(256), 0, s, g);
 }
 
+void cast(hvx_mlp* M, hipStream_t s) {
+    hipLaunchKernelGGL(mlp_cast_kernel, dim3((hvx::kMlpParams + 255) / 256), dim3(256), 0, s, M->P,
+                       WeightCopies{M->W1, M->W2, M->W3, M->Ws, M->W2T, M->W3T});
+    M->transposes = true;
+}
+
+// A batch's encodings: rows X, columns XT (ld elements apart); null: to be made.
+struct Encoded {
+    const bf16 *X, *XT;
+    uint32_t ld;
+};
+
 // forward of B samples, as separate launches
-void forward(hvx_mlp* M, const float4* in, uint32_t B, hipStream_t s) {
-    encode(in, B, B, M->lod_max, M->X0, M->X0T, s);
+void forward(hvx_mlp* M, const float4* in, Encoded& x, uint32_t B, hipStream_t s) {
+    if (!x.X) {
+        encode(in, B, B, M->lod_max, M->X0, M->X0T, s);
+        x = Encoded{M->X0, M->X0T, B};
+    }
     const bf16* Ws[3] = {M->W1, M->W2, M->W3};
     const int bias[3] = {hvx::kMlpB1, hvx::kMlpB2, hvx::kMlpB3};
-    const bf16* prev = M->X0;
+    const bf16* prev = x.X;
     for (int l = 0; l < 3; ++l) {
         GemmArgs g{};
         g.A = prev;
         g.Bt = Ws[l];
         g.M = B;
         g.Nc = kH;
-        g.Kd = l == 0 ? kIn : kH;
+        g.Kd = g.ldb = l == 0 ? kIn : kH;
         g.splitk = 1;
         g.bias = M->P + bias[l];
         g.C = M->H[l];
@@ -1032,26 +1043,27 @@ void forward(hvx_mlp* M, const float4* in, uint32_t B, hipStream_t s) {
 
 // gradient of the mean squared log-radiance error over B samples into G (and
 // the loss into *loss) as separate launches
-void gradient_separate(hvx_mlp* M, const float4* in, const float4* tgt, uint32_t B, float* G, float* loss,
+void gradient_separate(hvx_mlp* M, const float4* in, Encoded x, const float4* tgt, uint32_t B, float* G, float* loss,
                        hipStream_t s) {
-    forward(M, in, B, s);
+    if (!M->transposes) cast(M, s);
+    forward(M, in, x, B, s);
     const uint32_t nblk = B / kOutBlock;
     hipLaunchKernelGGL(mlp_out_kernel<true>, dim3(nblk), dim3(kOutBlock), 0, s, M->H[2], M->P, tgt, B, B,
                        2.0f / (3.0f * (float)B), nullptr, M->dZa, M->dZaT, M->opart);
     hipLaunchKernelGGL(reduce_out_kernel, dim3((kOutPart + 63) / 64), dim3(64 * kOutRedGroups), 0, s, M->opart, nblk, G + hvx::kMlpW4,
                        1.0f / (3.0f * (float)B), loss);
     const int wofs[3] = {hvx::kMlpW1, hvx::kMlpW2, hvx::kMlpW3};
-    hipLaunchKernelGGL(mlp_transpose_kernel, dim3(kH * kH / 256), dim3(256), 0, s, M->W2, M->W3, M->W2T, M->W3T);
     const bf16* WT[3] = {nullptr, M->W2T, M->W3T};
     bf16 *dz = M->dZa, *dzT = M->dZaT, *nz = M->dZb, *nzT = M->dZbT;
     for (int l = 2; l >= 0; --l) {
         const uint32_t K = l == 0 ? kIn : kH;
         GemmArgs g{};
         g.A = dzT;
-        g.Bt = l == 0 ? M->X0T : M->HT[l - 1];
+        g.Bt = l == 0 ? x.XT : M->HT[l - 1];
         g.M = kH;
         g.Nc = K;
         g.Kd = B;
+        g.ldb = l == 0 ? x.ld : B;
         g.splitk = M->splitk;
         g.part = M->part;
         g.pstride = kH * K + kH;
@@ -1069,7 +1081,7 @@ void gradient_separate(hvx_mlp* M, const float4* in, const float4* tgt, uint32_t
             d.Bt = WT[l];
             d.M = B;
             d.Nc = kH;
-            d.Kd = kH;
+            d.Kd = d.ldb = kH;
             d.splitk = 1;
             d.mask = M->H[l - 1];
             d.C = nz;
@@ -1110,11 +1122,6 @@ void gradient_fused(hvx_mlp* M, const float4* in, const bf16* x0, const float4* 
     else hipLaunchKernelGGL(reduce_step_kernel<false>, dim3(r.b[4]), dim3(64 * kRedGroups), 0, s, r);
 }
 
-void cast(hvx_mlp* M, hipStream_t s) {
-    hipLaunchKernelGGL(mlp_cast_kernel, dim3((hvx::kMlpParams + 255) / 256), dim3(256), 0, s, M->P,
-                       WeightCopies{M->W1, M->W2, M->W3, M->Ws});
-}
-
 int bind(hvx_ctx* ctx) {
     int cur = -1;
     if (hipGetDevice(&cur) != hipSuccess || (cur != ctx->device && hipSetDevice(ctx->device) != hipSuccess))
@@ -1142,7 +1149,8 @@ int hvx_mlp_create(hvx_ctx* ctx, float lod_max, uint64_t seed, hvx_mlp** out) {
     if ((e = dalloc(L, &M->P, np)) || (e = dalloc(L, &M->G, np)) || (e = dalloc(L, &M->m, np)) ||
         (e = dalloc(L, &M->v, np)) || (e = dalloc(L, &M->W1, (size_t)kH * kIn)) ||
         (e = dalloc(L, &M->W2, (size_t)kH * kH)) || (e = dalloc(L, &M->W3, (size_t)kH * kH)) ||
-        (e = dalloc(L, &M->Ws, (size_t)kWsLen))) {
+        (e = dalloc(L, &M->Ws, (size_t)kWsLen)) || (e = dalloc(L, &M->W2T, (size_t)kH * kH)) ||
+        (e = dalloc(L, &M->W3T, (size_t)kH * kH))) {
         hvx_mlp_destroy(M);
         return mfail(ctx, HVX_ERR_HIP, "hvx_mlp_create: %s", hipGetErrorString(e));
     }
@@ -1186,6 +1194,7 @@ int hvx_mlp_destroy(hvx_mlp* M) {
     for (void* p : M->sep_allocs) (void)hipFree(p);
     for (void* p : M->allocs) (void)hipFree(p);
     if (M->enc) (void)hipFree(M->enc);
+    if (M->encT) (void)hipFree(M->encT);
     if (M->cell_lo) (void)hipFree(M->cell_lo);
     delete M;
     return HVX_OK;
@@ -1231,7 +1240,7 @@ int hvx_mlp_gradient(hvx_mlp* M, const float* d_inputs, const float* d_targets, 
     hipError_t e = ensure_batch(M, batch);
     if (e != hipSuccess) return mfail(M->ctx, HVX_ERR_HIP, "hvx_mlp_gradient: %s", hipGetErrorString(e));
     const float4 *in = reinterpret_cast<const float4*>(d_inputs), *tg = reinterpret_cast<const float4*>(d_targets);
-    if (M->ctx->mlp_separate) gradient_separate(M, in, tg, batch, d_grads, d_loss, (hipStream_t)stream);
+    if (M->ctx->mlp_separate) gradient_separate(M, in, Encoded{}, tg, batch, d_grads, d_loss, (hipStream_t)stream);
     else gradient_fused(M, in, nullptr, tg, batch, d_grads, nullptr, d_loss, (hipStream_t)stream);
     e = hipGetLastError();
     return e == hipSuccess ? HVX_OK : mfail(M->ctx, HVX_ERR_HIP, "hvx_mlp_gradient: %s", hipGetErrorString(e));
@@ -1250,23 +1259,28 @@ int hvx_mlp_train(hvx_mlp* M, const float* d_inputs, const float* d_targets, uin
     const uint32_t per_epoch = n / batch;
     const float4* in = reinterpret_cast<const float4*>(d_inputs);
     const float4* tg = reinterpret_cast<const float4*>(d_targets);
-    // Encode the call's samples once (256 B per sample) when they are
-    // revisited, instead of once per step; without the memory, each step
-    // encodes its batch (as the separate launches always do).
+    // Encode the call's samples once (256 B per sample, the separate launches'
+    // transposed copy as much again) when they are revisited, instead of once
+    // per step; without the memory, each step encodes its batch.
     const bool separate = M->ctx->mlp_separate != 0;
     const size_t npad = (size_t)per_epoch * batch;
-    const bool revisit = steps > per_epoch && !separate;
-    if (revisit && M->enc_cap < npad) {
-        if (M->enc) (void)hipFree(M->enc);
-        M->enc = nullptr;
-        M->enc_cap = 0;
-        if (hipMalloc(reinterpret_cast<void**>(&M->enc), npad * kIn * sizeof(bf16)) == hipSuccess)
-            M->enc_cap = npad;
-        else
-            M->enc = nullptr, (void)hipGetLastError();  // a failed allocation leaves the slower path, not an error
-    }
-    const bool pre = revisit && M->enc_cap >= npad;
-    if (pre) encode(in, (uint32_t)npad, (uint32_t)npad, M->lod_max, M->enc, nullptr, s);
+    const bool revisit = steps > per_epoch;
+    auto hold = [&](bf16*& p, size_t& cap) {
+        if (cap >= npad) return true;
+        if (p) (void)hipFree(p);
+        p = nullptr;
+        cap = 0;
+        if (hipMalloc(reinterpret_cast<void**>(&p), npad * kIn * sizeof(bf16)) == hipSuccess) {
+            cap = npad;
+            return true;
+        }
+        p = nullptr;
+        (void)hipGetLastError();  // a failed allocation leaves the slower path, not an error
+        return false;
+    };
+    const bool pre = revisit && hold(M->enc, M->enc_cap) && (!separate || hold(M->encT, M->encT_cap));
+    if (pre) encode(in, (uint32_t)npad, (uint32_t)npad, M->lod_max, M->enc, separate ? M->encT : nullptr, s);
+    if (!separate) M->transposes = false;
     for (uint32_t k = 0; k < steps; ++k) {
         const size_t off = (size_t)(k % per_epoch) * batch;
         float* loss = d_loss_curve ? d_loss_curve + k : nullptr;
@@ -1276,9 +1290,12 @@ int hvx_mlp_train(hvx_mlp* M, const float* d_inputs, const float* d_targets, uin
         ++M->steps_done;
         const float bc1 = (float)(1.0 - std::pow(0.9, (double)M->steps_done));
         const float bc2 = (float)(1.0 - std::pow(0.999, (double)M->steps_done));
-        AdamArgs ad{M->P, M->m, M->v, lr_k, bc1, bc2, {M->W1, M->W2, M->W3, M->Ws}};
+        AdamArgs ad{M->P, M->m, M->v, lr_k, bc1, bc2, {M->W1, M->W2, M->W3, M->Ws, nullptr, nullptr}};
         if (separate) {
-            gradient_separate(M, in + off, tg + off, batch, M->G, loss, s);
+            ad.copies.W2T = M->W2T;
+            ad.copies.W3T = M->W3T;
+            const Encoded x = pre ? Encoded{M->enc + off * kIn, M->encT + off, (uint32_t)npad} : Encoded{};
+            gradient_separate(M, in + off, x, tg + off, batch, M->G, loss, s);
             hipLaunchKernelGGL(adam_kernel, dim3((hvx::kMlpParams + 255) / 256), dim3(256), 0, s, ad, M->G,
                                (uint32_t)hvx::kMlpParams);
         } else {
