@@ -221,10 +221,13 @@ __device__ __forceinline__ void wave_lds_sync() {
 // (3.11 / 3.31 / 2.77 ms with 8 / 16 / 2); 1.77 ms with a staged 64-byte entry
 // per footprint and 8 texels; 1.64 with four footprints to a line; 1.58 with 4
 // texels. Small maps wait for their rounds, so they take fewer texels and more
-// samples a round (us with 1 / 2 / 4 texels per workgroup): 4^2 from 32^2 161 /
-// 205 / 223, 9^2 from 700^2 192 / 220 / 251, 16^2 from 128^2 184 / 207 / 242 but
-// from 1024^2 534 / 507 / 479, 24^2 from 64^2 362 / 249 / 272, 32^2 from 64^2
-// 597 / 427 / 349.
+// samples a round (us with 1 / 2 / 4 texels per workgroup): 4^2 from 32^2 159 /
+// 196 / 221, 16^2 from 128^2 183 / 207 / 240 and 18^2 198 / 214 / 243, but 20^2 (2,400
+// workgroups of one texel do not fit the card at once) 327 / 228 / 256; from larger
+// faces the fabric sets in earlier: 12^2 from 256^2 177 / 209 / 232 and from 512^2
+// 292 / 228 / 240, 16^2 from 1024^2 535 / 502 / 477; 10^2 from 512^2 184 / 216 / 239
+// and from 1024^2 289 / 276 / 299; 24^2 from 64^2 363 / 249 / 270, from 512^2 802 /
+// 790 / 826 (18^2: 506 / 489 / 439), 32^2 from 64^2 589 / 426 / 348.
 constexpr int kMaxPhi = 512, kMaxTheta = 128;
 #ifndef HVX_DIFFUSE_TEX
 #define HVX_DIFFUSE_TEX 4
@@ -802,13 +805,15 @@ hipError_t launch_diffuse(const float* d_cube, uint32_t S, float* d_out, uint32_
         hipLaunchKernelGGL(diffuse_stage_kernel, dim3((stage_lines(S) + 31) / 32, gy, (rows + gy - 1) / gy), dim3(256), 0,
                            s, cube, S, reinterpret_cast<float2*>(stage));
         // few texels: fewer to a workgroup, for more workgroups and fewer
-        // rounds; large faces of medium maps stay with the fabric's best
+        // rounds, as long as they are all in flight (eight per CU) and, past
+        // 640, the face is small for the texels; large faces of medium maps
+        // stay with the fabric's best
         auto run = [&](auto tex) {
             constexpr int kTex = decltype(tex)::value;
             hipLaunchKernelGGL((diffuse_kernel<kTex, kDThreads, true>), dim3((T + kTex - 1) / kTex), dim3(kDThreads), 0,
                                s, cube, S, stage, out, Sd);
         };
-        if (T <= 512) run(std::integral_constant<int, 1>());
+        if (T <= 640 || (T <= 2048 && T * S <= (1u << 18))) run(std::integral_constant<int, 1>());
         else if (T <= 4096 && S <= 512) run(std::integral_constant<int, 2>());
         else run(std::integral_constant<int, kDTex>());
     } else {
