@@ -476,8 +476,8 @@ int shade_impl(hvx_ctx* ctx, const hvx_frag_soa* fr, const hvx_camera_ubo* cam, 
     }
     e = hvx::launch_shade(*fr, *cam, *ubo, *pc, d_lights, n_lights, d_cells, d_indices, *ibl, d_rgb,
                           ctx->shade_exact != 0, static_cast<float4*>(ctx->shade_lights),
-                          binned ? static_cast<uint32_t*>(ctx->shade_bins) : nullptr, learned, (hipStream_t)stream,
-                          ev0, ev1);
+                          binned ? static_cast<uint32_t*>(ctx->shade_bins) : nullptr, learned, ctx->num_cus,
+                          (hipStream_t)stream, ev0, ev1);
     return e == hipSuccess ? HVX_OK : hip_fail(ctx, e, "shading launch");
 }
 }  // namespace

@@ -143,7 +143,7 @@ hipError_t launch_shade(const hvx_frag_soa& fr, const hvx_camera_ubo& cam, const
                         const hvx_pbr_pc& pc, const hvx_light* d_lights, uint32_t n_lights,
                         const hvx_light_cell* d_cells, const uint32_t* d_indices, const hvx_ibl_maps& ibl,
                         float* d_rgb, bool exact, float4* light_scratch, uint32_t* bin_scratch,
-                        const LearnedShade* learned, hipStream_t s, hipEvent_t ev_begin = nullptr,
+                        const LearnedShade* learned, int num_cus, hipStream_t s, hipEvent_t ev_begin = nullptr,
                         hipEvent_t ev_end = nullptr);
 // Whether shading bins fragments by cluster for this grid, and the scratch
 // it needs for that (the fragment order and the tile bounds).

@@ -924,7 +924,7 @@ hipError_t launch_shade(const hvx_frag_soa& fr, const hvx_camera_ubo& cam, const
                         const hvx_pbr_pc& pc, const hvx_light* d_lights, uint32_t n_lights,
                         const hvx_light_cell* d_cells, const uint32_t* d_indices, const hvx_ibl_maps& ibl,
                         float* d_rgb, bool exact, float4* light_scratch, uint32_t* bin_scratch,
-                        const LearnedShade* learned, hipStream_t s, hipEvent_t ev_begin, hipEvent_t ev_end) {
+                        const LearnedShade* learned, int num_cus, hipStream_t s, hipEvent_t ev_begin, hipEvent_t ev_end) {
     ShadeArgs a{};
     a.depth = fr.depth;
     for (int c = 0; c < 3; ++c) {
@@ -985,7 +985,7 @@ hipError_t launch_shade(const hvx_frag_soa& fr, const hvx_camera_ubo& cam, const
             // tiles fill the card (3840x2160, 576 tiles: 84 us scattered, 64
             // in pieces); fewer tiles than CUs wait for their loads, and the
             // pass through LDS only adds to that (1366x768, 144: 14.0, 16.8)
-            a.order_cap = (uint64_t)a.X * a.Y > 256 ? a.unbin_cap : 0;
+            a.order_cap = (uint64_t)a.X * a.Y > (uint64_t)num_cus ? a.unbin_cap : 0;
         }
         a.row = RowOf::make(F, fr.width);
     }
