@@ -2025,7 +2025,7 @@ int hvx_ibl_contract_plan_reserve(hvx_contract_plan* P, uint32_t max_probes) {
     if (max_probes == 0 || max_probes > kMaxProbes)
         return pfail(P->ctx, HVX_ERR_INVALID_ARG, "max_probes must be in [1, %u]", kMaxProbes);
     if (max_probes <= P->mcap) return HVX_OK;
-    const uint32_t copies = multi_copies(P->scratch_bytes, max_probes);
+    uint32_t copies = multi_copies(P->scratch_bytes, max_probes);
     if (copies <= P->mcopies) {
         P->mcap = max_probes;
         return HVX_OK;
@@ -2034,13 +2034,17 @@ int hvx_ibl_contract_plan_reserve(hvx_contract_plan* P, uint32_t max_probes) {
     if (P->mscratch) (void)hipFree(P->mscratch);
     P->mscratch = nullptr;
     P->mcap = P->mcopies = 0;
-    const size_t bytes = P->scratch_bytes * copies;
+    // where the memory is short, fewer copies and more passes
     hipError_t e;
-    if ((e = hipMalloc(reinterpret_cast<void**>(&P->mscratch), bytes)) != hipSuccess ||
-        (e = hipMemset(P->mscratch, 0, bytes)) != hipSuccess) {
+    while ((e = hipMalloc(reinterpret_cast<void**>(&P->mscratch), P->scratch_bytes * copies)) != hipSuccess && copies > 1) {
+        (void)hipGetLastError();
+        copies = (copies + 1) / 2;
+    }
+    if (e != hipSuccess || (e = hipMemset(P->mscratch, 0, P->scratch_bytes * copies)) != hipSuccess) {
         if (P->mscratch) (void)hipFree(P->mscratch);
         P->mscratch = nullptr;
-        return pfail(P->ctx, HVX_ERR_HIP, "multi-probe scratch (%zu bytes): %s", bytes, hipGetErrorString(e));
+        return pfail(P->ctx, HVX_ERR_HIP, "multi-probe scratch (%zu bytes): %s", P->scratch_bytes * copies,
+                     hipGetErrorString(e));
     }
     P->mcap = max_probes;
     P->mcopies = copies;
