@@ -486,7 +486,7 @@ struct StageItem {
     uint64_t lo_off;         // split: offset of the lo parts (16-byte units; planes: in the texel's own record)
 };
 struct StageTable {
-    StageItem it[kMaxJobs];
+    StageItem it[kMaxJobs + 2];  // and the roughness-0 mip, and stage_rest's first
     uint32_t n, blocks;
     const uint32_t* map;  // source_table
 };
@@ -705,6 +705,13 @@ struct GemmArgs {
     uint32_t nitems;
     const half8* R[kMaxJobs];
     uint64_t r_lo[kMaxJobs];
+    // gemm_direct: ulist as the levels count their units, stage_kernel's
+    // scales, source_table, the levels
+    const uint32_t* raw_ulist;
+    const float* sc;
+    const uint32_t* map;
+    uint64_t level_off[kMaxJobs];
+    uint32_t log2_S[kMaxJobs];
 };
 static_assert(sizeof(StageTable) < 4000 && sizeof(MapTable) < 4000 && sizeof(GemmArgs) < 4000,
               "launch tables must fit the kernel argument space");
@@ -812,9 +819,85 @@ __device__ __forceinline__ void gemm_item(const GemmArgs& A, const Block& B, con
     }
 }
 
+// The same products (and sums, to the bit) with the B operand staged from the
+// level by the workgroup that multiplies it, for levels that one block of rows
+// sums: their staged units would be written to memory (2,304 bytes each) to be
+// read once. With many probes of small outputs that was most of the call:
+// 1,024 probes 32^2 -> 16^2 x 5 take 465 us so, 825 staged. A wave loads one image
+// of eight units' texels at a time, as stage_tile does (a thread per (unit, image)
+// instead, loads of 64 lines each: 591). level: the probe's; sU: the slice's units
+// as the level counts them; sc: 1 / the levels' scale.
+__device__ __forceinline__ void gemm_direct(const GemmArgs& A, const Block& B, const Item& I,
+                                            const float4* __restrict__ level, uint32_t ls, float sc,
+                                            half8 (*sB)[kGroup * 4 * kColsPad], const uint32_t* sU,
+                                            const uint32_t* sMap, f32x4 (&acc)[2][kNt]) {
+    constexpr uint32_t kWaveImages = kImages / 4;
+    static_assert(kGroup * 4 == 16 && kWaveImages % 4 == 0, "two halves of eight units; whole words of the map");
+    const uint32_t t = threadIdx.x, lane = t & 63, wave = t >> 6, i = lane & 15, g = lane >> 4;
+    const uint32_t nrt = B.nrt, rt0 = 2 * wave, n = I.n, S = 1u << ls;
+    const bool live = rt0 < nrt, has1 = rt0 + 1 < nrt;  // uniform per wave
+    const half8* w0 = A.W + B.woff + ((size_t)I.s0 * nrt + (live ? rt0 : 0)) * 64 + lane;
+    const half8* w1 = has1 ? w0 + 64 : w0;
+    const size_t wstep = (size_t)nrt * 64;
+    auto stage = [&](uint32_t s, uint32_t buf) {
+#pragma unroll
+        for (uint32_t h = 0; h < 2; ++h) {
+            const uint32_t u = 8 * h + lane / 8, k8 = sU[s * 4 + u] * 8 + lane % 8;
+            const uint32_t x = k8 & (S - 1), y = k8 >> ls & (S - 1), f = k8 >> (2 * ls);
+            uint32_t m[kWaveImages / 4];
+            float4 v[kWaveImages];
+#pragma unroll
+            for (uint32_t k = 0; k < kWaveImages / 4; ++k) m[k] = sMap[(f * kImages + wave * kWaveImages) / 4 + k];
+#pragma unroll
+            for (uint32_t k = 0; k < kWaveImages; ++k) {
+                const uint32_t b = m[k / 4] >> (8 * (k % 4));
+                uint32_t a = b & 8u ? y : x, c = b & 8u ? x : y;
+                a = b & 16u ? S - 1 - a : a;
+                c = b & 32u ? S - 1 - c : c;
+                v[k] = level[((b & 7u) * S + c) * S + a];
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < kWaveImages; ++k) {
+                const LevelTexel<false> T{v[k], sc};
+                _Float16* o = reinterpret_cast<_Float16*>(&sB[buf][u * kColsPad + 3 * (wave * kWaveImages + k)]) + lane % 8;
+                o[0] = T.hi(0);
+                o[8] = T.hi(1);
+                o[16] = T.hi(2);
+            }
+        }
+    };
+    stage(0, 0);
+    __syncthreads();
+    const uint32_t groups = (n + kGroup - 1) / kGroup;
+    for (uint32_t gi = 0; gi < groups; ++gi) {
+        const uint32_t s = gi * kGroup;
+        half8 x[kGroup][2];
+#pragma unroll
+        for (uint32_t k = 0; k < kGroup; ++k) {
+            const size_t o = (size_t)(s + k < n ? s + k : n - 1) * wstep;
+            x[k][0] = w0[o];
+            x[k][1] = w1[o];
+        }
+        if (gi + 1 < groups) stage(s + kGroup, (gi & 1) ^ 1);  // its readers passed the previous barrier
+        const half8* sb = sB[gi & 1];
+#pragma unroll
+        for (uint32_t k = 0; k < kGroup; ++k)
+            if (live && s + k < n) {
+#pragma unroll
+                for (uint32_t nt = 0; nt < kNt; ++nt) {
+                    const half8 b = sb[(k * 4 + g) * kColsPad + nt * 16 + i];
+                    acc[0][nt] = hvx::mfma16x16x32(x[k][0], b, acc[0][nt]);
+                    acc[1][nt] = hvx::mfma16x16x32(x[k][1], b, acc[1][nt]);
+                }
+            }
+        __syncthreads();
+    }
+}
+
+template <bool DIRECT>
 __global__ __launch_bounds__(256, 2) void contract_gemm_kernel(Probes Q, GemmArgs A) {
-    __shared__ half8 sB[2][kGroup * 4 * kCols];
-    __shared__ uint32_t sU[(kMaxSlice + kGroup) * 4];
+    __shared__ half8 sB[2][kGroup * 4 * (DIRECT ? kColsPad : kCols)];
+    __shared__ uint32_t sU[(kMaxSlice + kGroup) * 4], sMap[DIRECT ? 6 * kImages / 4 : 1];
     // hardware workgroup b runs on XCD b % 8: each XCD takes one run of the
     // items, whose neighbours share staged units, and of an item's probes,
     // which share its weights
@@ -825,17 +908,24 @@ __global__ __launch_bounds__(256, 2) void contract_gemm_kernel(Probes Q, GemmArg
     const Item I = A.items[item];
     const Block B = A.blocks[I.block];
     const uint32_t left = B.nunits - I.s0 * 4;  // units from the slice's first on (its last step may be short of four)
+    const uint32_t* ulist = DIRECT ? A.raw_ulist : A.ulist;
     for (uint32_t k = t; k < (kMaxSlice + kGroup) * 4; k += 256)
-        sU[k] = A.ulist[B.unit0 + I.s0 * 4 + min(k, min(I.n * 4, left) - 1)];
+        sU[k] = ulist[B.unit0 + I.s0 * 4 + min(k, min(I.n * 4, left) - 1)];
+    if (DIRECT && t < 6 * kImages / 4) sMap[t] = A.map[t];
     __syncthreads();
-    const half8* R = scr(Q, A.R[B.src], pr);
     f32x4 acc[2][kNt];
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
         for (uint32_t nt = 0; nt < kNt; ++nt) acc[h][nt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    if (B.split) gemm_item<true>(A, B, I, R, sB, sU, acc);
-    else gemm_item<false>(A, B, I, R, sB, sU, acc);
+    if constexpr (DIRECT) {
+        gemm_direct(A, B, I, probe_chain(Q, pr) + A.level_off[B.src], A.log2_S[B.src], 1.0f / scr(Q, A.sc, pr)[6], sB,
+                    sU, sMap, acc);
+    } else {
+        const half8* R = scr(Q, A.R[B.src], pr);
+        if (B.split) gemm_item<true>(A, B, I, R, sB, sU, acc);
+        else gemm_item<false>(A, B, I, R, sB, sU, acc);
+    }
     const uint32_t lane = t & 63, i = lane & 15, g = lane >> 4, rt0 = 2 * (t >> 6);
     float* p = scr(Q, A.part, pr) + (size_t)I.slot * kBlockRows * kCols;
 #pragma unroll
@@ -1374,10 +1464,10 @@ struct hvx_contract_plan {
     float* sc = nullptr;
     uint32_t min_level = 0;  // deepest input chain level read
     uint32_t scale_level = ~0u;  // finest staged level: its maxima bound every staged value
-    StageTable stage{};
+    StageTable stage{}, stage_rest{};  // stage_rest: for gemm_direct
     MapTable maps{};
     GemmArgs gemm{};
-    uint32_t items = 0;
+    uint32_t items = 0, direct_units = 0;  // direct_units: of the levels, if gemm_direct can take them
     uint32_t dense_rows = 0, near_rows = 0;  // rows [0, dense_rows) whole and far, then the near ones
     const Job* d_jobs = nullptr;
     const Row* d_rows = nullptr;
@@ -1549,7 +1639,7 @@ hipError_t build_plan(hvx_contract_plan* P, int ctype, bool split) {
     for (Job& J : jobs)
         if (J.piece != PIECE_WHOLE) J.zmap = d_zmaps + (size_t)J.zmap / sizeof(float4);
     // unit lists: the blocks' units with weight, as indices into the source's staged units
-    std::vector<uint32_t> ulist;
+    std::vector<uint32_t> ulist, raw_ulist;  // raw: as the level or plane counts them
     Tables first;
     const size_t fj = first.add(jobs), fr = first.add(rows), fb = first.add(blocks);
     Scratch first_mem;
@@ -1585,7 +1675,7 @@ hipError_t build_plan(hvx_contract_plan* P, int ctype, bool split) {
             Block& B = blocks[S.block0 + b];
             B.unit0 = (uint32_t)ulist.size();
             for (uint32_t u : S.units)
-                if (flags[(size_t)b * S.raw + u]) ulist.push_back(index[u]);
+                if (flags[(size_t)b * S.raw + u]) ulist.push_back(index[u]), raw_ulist.push_back(u);
             B.nunits = (uint32_t)ulist.size() - B.unit0;
             B.nsteps = (B.nunits + 3) / 4;
         }
@@ -1679,7 +1769,7 @@ hipError_t build_plan(hvx_contract_plan* P, int ctype, bool split) {
     // pages touched here are not first touched by a call
     if ((e = hipMemset(P->scratch, 0, P->scratch_bytes)) != hipSuccess) return e;
     Tables tab;
-    const size_t tj = tab.add(jobs), tr = tab.add(rows), tb = tab.add(blocks), ti = tab.add(items), tu = tab.add(ulist);
+    const size_t tj = tab.add(jobs), tr = tab.add(rows), tb = tab.add(blocks), ti = tab.add(items), tu = tab.add(ulist), traw = tab.add(raw_ulist);
     for (SourcePlan& S : src) {
         S.units_off = tab.add(S.units);
         S.need_off = tab.add(S.need);
@@ -1773,8 +1863,14 @@ hipError_t build_plan(hvx_contract_plan* P, int ctype, bool split) {
             I.dst = R;
             I.lo_off = lo;
             stage_item(I, tiles);
+            A.level_off[s] = I.level_off;
+            A.log2_S[s] = ilog2(I.S);
+            P->direct_units += nu;
         }
     }
+    A.map = ST.map;
+    A.sc = P->sc;
+    A.raw_ulist = reinterpret_cast<const uint32_t*>(d_tab + traw);
     if (delta_mip != ~0u) {
         StageItem I{};
         I.kind = STAGE_DELTA;
@@ -1782,8 +1878,31 @@ hipError_t build_plan(hvx_contract_plan* P, int ctype, bool split) {
         I.level_off = hvx::cube_level_offset_floats(P->So, delta_mip) / 4;
         stage_item(I, (6 * I.S * I.S + 255) / 256);
     }
+    // gemm_direct takes plans of levels that one block of rows sums each (mixed
+    // with others, its slower slices left some XCDs waiting). What is left to
+    // stage: an item of no texels, whose workgroup writes the scales, and the
+    // roughness-0 mip
+    for (const SourcePlan& S : src)
+        if (S.nblocks != 1 || S.split || S.G.pad) P->direct_units = 0;
+    StageTable& SR = P->stage_rest;
+    SR.it[SR.n++] = StageItem{.kind = STAGE_PLANE};
+    SR.blocks = 1;
+    SR.map = ST.map;
+    if (delta_mip != ~0u) {
+        SR.it[SR.n] = ST.it[ST.n - 1];
+        SR.it[SR.n++].block_begin = SR.blocks;
+        SR.blocks += ST.blocks - ST.it[ST.n - 1].block_begin;
+    }
     return hipSuccess;
 }
+
+// From this many units over all probes on, plans that it can take go through
+// gemm_direct; below, the latency of its staging counts. us staged / direct: 24
+// probes 16^2 -> 16^2 x 5 (4,608 units) 22.8 / 22.9, 64 31.1 / 26.5, 1,024 242 / 159;
+// 64 probes 8^2 -> 8^2 x 4 (3,072) 25.7 / 28.0, 256 37.1 / 30.5; 24 probes 32^2 ->
+// 16^2 x 5 (23,040) 31.9 / 24.5; 64^2 -> 32^2 x 6, 2 (6,144) 30.3 / 30.6, 8 42.1 /
+// 37.4, 24 77.6 / 69.7, 256 876 / 585.
+constexpr uint64_t kDirectUnits = 8192;
 
 // The launches of a filter call over n probes (grid dimension y, z for the
 // face maxima, interleaved for the GEMM: probe). delta_chain (single probe,
@@ -1806,14 +1925,16 @@ int launch_call(hvx_contract_plan* P, const Probes& Q, uint32_t n, uint32_t chai
         hipLaunchKernelGGL(facemax_kernel, dim3(nb, 6, n), dim3(256), 0, s, Q,
                            hvx::cube_level_offset_floats(P->S, P->scale_level) / 4, Sl, P->fmax);
     }
-    if (P->stage.blocks)
-        hipLaunchKernelGGL(stage_kernel, dim3(P->stage.blocks, n), dim3(256), 0, s, Q, P->stage, P->fmax, nb, P->sc,
+    const bool direct = n * (uint64_t)P->direct_units >= kDirectUnits;
+    const StageTable& stage = direct ? P->stage_rest : P->stage;
+    if (stage.blocks)
+        hipLaunchKernelGGL(stage_kernel, dim3(stage.blocks, n), dim3(256), 0, s, Q, stage, P->fmax, nb, P->sc,
                            delta_chain, P->S);
     if (P->maps.blocks)
         hipLaunchKernelGGL(plane_map_kernel, dim3(P->maps.blocks, n), dim3(256), 0, s, Q, P->maps);
     if (P->items) {
-        hipLaunchKernelGGL(contract_gemm_kernel, dim3((P->items * n + kXcds - 1) / kXcds * kXcds), dim3(256), 0,
-                           s, Q, P->gemm);
+        hipLaunchKernelGGL(direct ? contract_gemm_kernel<true> : contract_gemm_kernel<false>,
+                           dim3((P->items * n + kXcds - 1) / kXcds * kXcds), dim3(256), 0, s, Q, P->gemm);
         hipLaunchKernelGGL(epilogue_kernel<false>, dim3((P->dense_rows * kImages + 255) / 256, n), dim3(256), 0, s, Q,
                            P->d_jobs, P->d_rows, P->gemm.blocks, P->gemm.part, P->rowscale, P->invZ, P->sc, 0u,
                            P->dense_rows);
