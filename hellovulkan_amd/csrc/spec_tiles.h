@@ -31,12 +31,12 @@ template <int TPW> struct SpecShape {
 // texel and 64 samples a round. What is left of a round's gain past the starts
 // of four times the waves grows with the samples and falls with the tiles. us
 // of the whole call with four / one:
-//   16^2 x 4 and 256 samples (36 tiles) 44 / 27, 64^2 x 2 (384): 16 samples
-//   13.2 / 17.3, 64: 22.5 / 23.6, 1,024: 102 / 98, 64^2 x 7 (522): 64 samples
-//   21.3 / 23.8, 1,024: 107 / 89, 80^2 x 2 (600): 64 samples 24.1 / 27.5, 256:
-//   53 / 49, 90^2 x 4 from 1000^2 (1,134): 128 samples 78 / 68, 1,024: 463 / 375,
-//   100^2 x 7 (1,398): 128 samples 38 / 43, 1,024: 188 / 169, but 110^2 x 3
-//   (1,470) 244 / 259, 128^2 x 2 (1,536): 64 samples 33 / 46, 1,024: 275 / 305
+//   16^2 x 2 (24 tiles) and 256 samples 67 / 34, 64^2 x 2 (384): 16 samples 13.0 /
+//   17.2, 64: 19.3 / 20.3, 1,024: 102 / 98, 64^2 x 7 (522): 64 samples 18.2 / 20.4,
+//   1,024: 107 / 89, 80^2 x 2 (600): 64 samples 20.7 / 24.0, 256: 51 / 47, 90^2 x 4
+//   from 1000^2 (1,134): 128 samples 74 / 65, 1,024: 462 / 375, 100^2 x 7 (1,398):
+//   128 samples 35 / 40, 1,024: 187 / 170, but 110^2 x 3 (1,470) 243 / 259, 128^2 x 2
+//   (1,536): 64 samples 29 / 43, 1,024: 275 / 305
 constexpr uint32_t kSpecFewTiles = 1500;
 inline bool spec_few(uint32_t tiles, uint32_t n) { return tiles <= kSpecFewTiles && 9ull * n >= tiles; }
 
