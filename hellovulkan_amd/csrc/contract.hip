@@ -35,9 +35,9 @@
 //   1024^2 -> 512^2 x 10, FP16           444 -> 128 us (weights 1606 -> 127 MB)
 //   512^2 -> 256^2 x 9, split BF16       353 -> 100 us
 //   24 probes 256^2 -> 128^2 x 8, FP16   855 -> 340 us
-// The 129 us are 45 us of GEMM, 36 us of staging with the roughness-0 mip
-// (100 MB of level 0 read, 25 MB written), 22 us for the near rows' epilogue
-// and 22 us for the four small launches.
+// The 128 us are 45 us of GEMM, 35 us of staging with the roughness-0 mip (100
+// MB of level 0 read, 25 MB written), 23 us of the near rows' epilogue and 22 us
+// of face maxima, plane maps and the other rows' epilogue.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -415,7 +415,7 @@ __global__ __launch_bounds__(256) void row_scale_kernel(const Job* __restrict__ 
 }
 
 // ------------------------------------------------------ per-call staging
-// A filter call is at most seven launches: face maxima, staging (with the
+// A filter call is at most six launches: face maxima, staging (with the
 // roughness-0 mip), the maps of the staged planes, the GEMM over every weight
 // matrix, the epilogue of the whole and far rows, that of the near rows.
 
@@ -723,9 +723,10 @@ constexpr uint32_t kMaxSlice = 64;    // K steps of an item, at most
 constexpr uint32_t kXcds = 8;
 constexpr uint32_t kNt = kCols / 16;  // MFMA column tiles
 
-// Bound by what reaches the CUs: at 512^2 x 10 about 110 MB of weights and
-// 125 MB of staged units (each read by the blocks whose windows hold it) in
-// 45 us, while its MFMAs need 6 us and its LDS reads 7 us.
+// Bound by what reaches the CUs: at 512^2 x 10 127 MB of weights and 125 MB of
+// staged units (each read by the blocks whose windows hold it) in 45 us, 190 MB
+// of it past the L2, while its MFMAs (36 GFLOP with the padding of rows) need 14
+// us and its LDS reads 7 us.
 // One workgroup per (item, probe): four waves of two 16-row tiles each over
 // the item's K steps, all 144 columns, so a wave's 18 accumulators reuse each
 // weight fragment nine times and each B fragment twice. The B operand of a
@@ -1716,8 +1717,9 @@ hipError_t build_plan(hvx_contract_plan* P, int ctype, bool split) {
     // slice costs its 74 KB of partial sums, written and read once: 24 probes
     // 256^2 -> 128^2 x 8 took 384 us with slices of at least 16 steps, 361 us
     // with 24, 349 us with 32, 347 us with 40 (one probe 512^2 -> 256^2 x 9 in
-    // split BF16 100 us up to 32, 103 us with 40); the 512^2 x 10 chain 139 us
-    // with 541 slices, in two rounds, 129 us with 440 in one.
+    // split BF16 100 us up to 32, 103 us with 40; each timed before the kernels
+    // around the GEMM had their present form); the 512^2 x 10 chain 10 us more
+    // with 541 slices, in two rounds, than with 440 in one.
     uint64_t wunits = 0;
     const uint32_t slots = 2u * (uint32_t)std::max(P->ctx->num_cus, 1);
     auto slices = [&](const Block& B, uint32_t len) {
@@ -1949,9 +1951,9 @@ int launch_call(hvx_contract_plan* P, const Probes& Q, uint32_t n, uint32_t chai
 
 // Copies of the per-call scratch that a multi-probe call over n probes runs
 // in: all of them up to 16 GiB, then the call is cut. Cutting it further, so
-// that what one launch stages stays in the caches for the next, does not pay:
-// 24 probes 256^2 -> 128^2 x 8 take 519 us at once, 563 us cut at 512 MiB,
-// 660 us at 128 MiB.
+// that what one launch stages stays in the caches for the next, mostly does not
+// pay: 24 probes 256^2 -> 128^2 x 8 take 341 us at once, 374 cut at 192 MiB, 425
+// at 96 MiB; 256 probes 64^2 -> 64^2 x 7 1,316 us, 1,170 cut at 256 MiB, 1,644 at 64.
 constexpr size_t kMultiBytes = 16ull << 30;
 uint32_t multi_copies(size_t scratch_bytes, uint32_t n) {
     const size_t fit = kMultiBytes / std::max<size_t>(scratch_bytes, 1);

@@ -25,7 +25,7 @@ struct hvx_ctx {
     size_t light_vs_bytes = 0;
     void* ggx_table = nullptr;    // float4 [mips * samples]: tangent-space GGX H
     size_t ggx_table_bytes = 0;
-    void* diffuse_stage = nullptr; // the diffuse filter's staged footprints (64 B each)
+    void* diffuse_stage = nullptr; // the diffuse filter's staged footprints (four to 128 B)
     size_t diffuse_stage_bytes = 0;
     void* shade_lights = nullptr; // float4 [2 * lights]: compact shading light table
     size_t shade_lights_bytes = 0;
@@ -161,7 +161,7 @@ hipError_t launch_cube_mips(float* d_chain, uint32_t S, uint32_t levels, hipStre
 hipError_t launch_gather_copy(const float* const* d_src, size_t floats, float* d_dst, size_t dst_stride_floats,
                               uint32_t n, hipStream_t s);
 // Bytes of the diffuse filter's staged footprints for a level-0 face of S
-// (0: not staged: S < 2, or more than kDiffuseStageMaxBytes).
+// (0: not staged, more than kDiffuseStageMaxBytes).
 constexpr size_t kDiffuseStageMaxBytes = size_t(1) << 29;
 size_t diffuse_stage_size(uint32_t S);
 // d_stage: diffuse_stage_size(S) bytes of scratch, or nullptr (taps

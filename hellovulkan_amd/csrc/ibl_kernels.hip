@@ -4,10 +4,10 @@
 //   BRDFLUT.comp:26-71             -> brdf_lut_kernel (workgroup per LUT row;
 //                                     the row's GGX half-vectors staged in LDS)
 //   Equirect2Cube.frag:87-107      -> equirect_kernel (lane per cube texel)
-//   VulkanImage::GenerateMipmap    -> mip_kernel (2x2 box, lane per texel)
-//   CubeFilterDiffuse.frag:35-136  -> diffuse_stage_kernel (each bilinear
-//                                     footprint's texels in one 64-byte
-//                                     entry) and diffuse_kernel (32 lanes per
+//   VulkanImage::GenerateMipmap    -> mip_kernel (2x2 boxes, five levels a launch)
+//   CubeFilterDiffuse.frag:35-136  -> diffuse_stage_kernel (four bilinear
+//                                     footprints to a 128-byte line) and
+//                                     diffuse_kernel (64 to 256 lanes per
 //                                     output texel evaluate samples, loads one
 //                                     round ahead; one lane per texel and
 //                                     channel sums them in order; the
@@ -253,7 +253,8 @@ static_assert(kDThreads == 128 || kDThreads == 256, "lanes per workgroup: 128 or
 // column (i0 + 1) % 4 on: one line instead of two rows of texels (2.3 lines on
 // average), and the bilinear sums are unchanged to the bit. Twice the cube (202
 // MB at 1024^2), so it stays in the 256 MB of last-level cache: with an entry of
-// 64 bytes for every footprint (403 MB) 32^2 from 1024^2 took 1.77 ms, so 1.64 (12 GB of lines at 7.9 TB/s).
+// 64 bytes for every footprint (403 MB) 32^2 from 1024^2 took 1.77 ms, so 1.64 (with
+// 4 texels to a workgroup 11 GB of lines at 7.2 TB/s).
 __host__ __device__ inline uint32_t stage_lines(uint32_t S) { return (S + 4) / 4; }
 __global__ __launch_bounds__(256) void diffuse_stage_kernel(const float4* __restrict__ cube, uint32_t S,
                                                            float2* __restrict__ lines) {
@@ -293,10 +294,11 @@ struct DiffSample {
     float4 q[4];
 };
 
-// STAGED: the samples read staged footprints (three 16-byte loads from one
-// line); otherwise their four taps from the cube. Four lanes loading one
-// entry together (16 lines per load instruction instead of 64, the parts
-// passed on through LDS) measured slower: 2.36 ms against 1.82.
+// STAGED: the samples read staged footprints (48 bytes of one line, aligned to
+// 8); otherwise their four taps from the cube. Four lanes loading one footprint
+// together (16 lines per load instruction instead of 64, the parts passed on
+// through LDS) measured slower while each had an entry of 64 bytes: 2.36 ms
+// against 1.82.
 template <int TEX, int THREADS, bool STAGED>
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(HVX_DIFFUSE_WAVES_PER_EU, 8))) void
 diffuse_kernel(const float4* __restrict__ cube, uint32_t S, const float* __restrict__ stage, float4* __restrict__ out,

@@ -343,9 +343,9 @@ int hvx_ibl_cube_mips(hvx_ctx* ctx, float* d_cube_chain, uint32_t face_size,
  * running Shaders/IBL/CubeFilterDiffuse.frag:35-136 and
  * CubeFilterSpecular.frag:34-146. opts may be NULL.
  * Context scratch: the specular filter's sample table (16 B per mip and
- * sample); the diffuse filter's staged footprints, 64 B for each bilinear
- * footprint (6 (face_size+1)^2 entries, 403 MB at 1024^2; none when that
- * exceeds 1 GiB). Under stream capture, when the context holds no staging
+ * sample); the diffuse filter's staged footprints, 128 B for four bilinear
+ * footprints of a row (6 (face_size+1) ceil((face_size+1)/4) lines, 202 MB at
+ * 1024^2; none when that exceeds 512 MiB). Under stream capture, when the context holds no staging
  * buffer that large yet, the diffuse filter reads the taps from d_cube
  * instead and allocates nothing (the same results, bit for bit). */
 int hvx_ibl_filter(hvx_ctx* ctx, int type, const float* d_cube,
@@ -419,8 +419,12 @@ int hvx_ibl_contract_hot_info(hvx_contract_plan* plan, float* threshold, uint32_
  * (inputs as for hvx_ibl_filter_contract). Each probe's result equals the
  * single-probe call's bit for bit. The plan must first reserve per-probe
  * scratch for at least n probes (hvx_ibl_contract_plan_reserve, which
- * allocates; n <= 4096); the call itself allocates nothing. No reference
- * counterpart (batches many ResourcesIBL specular prefilters). */
+ * allocates; n <= 4096); the call itself allocates nothing. A probe's scratch
+ * is 15 MB at 256^2 -> 128^2 x 8, 50 MB at 1024^2 -> 512^2 x 10, 280 MB at
+ * 2048^2 -> 2048^2 x 12; at most 16 GiB of it are kept (at least four probes'),
+ * less where the memory is short, and a call over more probes than that takes
+ * several passes. No reference counterpart (batches many ResourcesIBL specular
+ * prefilters). */
 int hvx_ibl_contract_plan_reserve(hvx_contract_plan* plan, uint32_t max_probes);
 int hvx_ibl_filter_contract_multi(hvx_contract_plan* plan, uint32_t n, const float* const* d_chains,
                                   uint32_t chain_levels, float* const* d_outs, void* stream);
@@ -452,8 +456,9 @@ int hvx_mlp_gradient(hvx_mlp* mlp, const float* d_inputs, const float* d_targets
 /* `steps` Adam steps over consecutive batches of the n samples (cosine
  * learning-rate decay from lr to lr/100); d_loss_curve (nullable) receives
  * each step's loss. A call that revisits its samples (steps > n / batch)
- * encodes them once into network-owned memory (512 B per sample, kept for
- * later calls); without that memory each step encodes its batch. */
+ * encodes them once into network-owned memory (256 B per sample, twice that
+ * with HVX_OPT_MLP_SEPARATE_LAUNCHES; kept for later calls); without that
+ * memory each step encodes its batch. */
 int hvx_mlp_train(hvx_mlp* mlp, const float* d_inputs, const float* d_targets, uint32_t n, uint32_t batch,
                   uint32_t steps, float lr, float* d_loss_curve, void* stream);
 /* Radiance (RGB, n x 3 floats) predicted at n inputs (dir.xyz, lod), by the
@@ -466,7 +471,7 @@ int hvx_mlp_eval(hvx_mlp* mlp, const float* d_inputs, uint32_t n, float* d_rgb, 
  * network against the chain's textureLod value at the cell's 75 test points
  * (a 5 x 5 grid over the texel, corners included, at both bin ends and its
  * middle): a margin over the measured error, since the error between test
- * points is not measured. It also keeps, with the network, half the
+ * points is not measured. It also keeps, with the network, the
  * smallest output the network gave in each cell, which hvx_cf_shade_learned
  * uses on the same cell grid to skip the network where even that output
  * could not be used. A set-up call: it allocates and synchronises the
