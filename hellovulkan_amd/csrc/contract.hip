@@ -717,7 +717,8 @@ static_assert(sizeof(StageTable) < 4000 && sizeof(MapTable) < 4000 && sizeof(Gem
               "launch tables must fit the kernel argument space");
 
 constexpr uint32_t kGroup = 4;        // K steps staged per barrier (half as many split-BF16 ones)
-constexpr uint32_t kMinSlice = 8;     // and at least
+constexpr uint32_t kDGroup = 2;       // K steps per barrier in gemm_direct: there 4 hold up short slices
+constexpr uint32_t kMinSlice = 8;     // K steps of an item, at least
 constexpr uint32_t kGoodSlice = 32;   // and at least in plans that fill the chip
 constexpr uint32_t kMaxSlice = 64;    // K steps of an item, at most
 constexpr uint32_t kXcds = 8;
@@ -824,16 +825,18 @@ __device__ __forceinline__ void gemm_item(const GemmArgs& A, const Block& B, con
 // level by the workgroup that multiplies it, for levels that one block of rows
 // sums: their staged units would be written to memory (2,304 bytes each) to be
 // read once. With many probes of small outputs that was most of the call:
-// 1,024 probes 32^2 -> 16^2 x 5 take 465 us so, 825 staged. A wave loads one image
+// 1,024 probes 32^2 -> 16^2 x 5 take 423 us so, 825 staged. A wave loads one image
 // of eight units' texels at a time, as stage_tile does (a thread per (unit, image)
-// instead, loads of 64 lines each: 591). level: the probe's; sU: the slice's units
-// as the level counts them; sc: 1 / the levels' scale.
+// instead, loads of 64 lines each: 591). Two K steps per barrier: four hold up the
+// short slices of small outputs (1,024 probes 16^2 -> 8^2 x 4 128 us against 117;
+// 256 probes 64^2 -> 32^2 x 6, whose slices are long, 587 against 647). level: the
+// probe's; sU: the slice's units as the level counts them; sc: 1 / the levels' scale.
 __device__ __forceinline__ void gemm_direct(const GemmArgs& A, const Block& B, const Item& I,
                                             const float4* __restrict__ level, uint32_t ls, float sc,
-                                            half8 (*sB)[kGroup * 4 * kColsPad], const uint32_t* sU,
+                                            half8 (*sB)[kDGroup * 4 * kColsPad], const uint32_t* sU,
                                             const uint32_t* sMap, f32x4 (&acc)[2][kNt]) {
     constexpr uint32_t kWaveImages = kImages / 4;
-    static_assert(kGroup * 4 == 16 && kWaveImages % 4 == 0, "two halves of eight units; whole words of the map");
+    static_assert(kDGroup % 2 == 0 && kWaveImages % 4 == 0, "whole eights of units, whole words of the map");
     const uint32_t t = threadIdx.x, lane = t & 63, wave = t >> 6, i = lane & 15, g = lane >> 4;
     const uint32_t nrt = B.nrt, rt0 = 2 * wave, n = I.n, S = 1u << ls;
     const bool live = rt0 < nrt, has1 = rt0 + 1 < nrt;  // uniform per wave
@@ -842,7 +845,7 @@ __device__ __forceinline__ void gemm_direct(const GemmArgs& A, const Block& B, c
     const size_t wstep = (size_t)nrt * 64;
     auto stage = [&](uint32_t s, uint32_t buf) {
 #pragma unroll
-        for (uint32_t h = 0; h < 2; ++h) {
+        for (uint32_t h = 0; h < kDGroup / 2; ++h) {
             const uint32_t u = 8 * h + lane / 8, k8 = sU[s * 4 + u] * 8 + lane % 8;
             const uint32_t x = k8 & (S - 1), y = k8 >> ls & (S - 1), f = k8 >> (2 * ls);
             uint32_t m[kWaveImages / 4];
@@ -869,20 +872,20 @@ __device__ __forceinline__ void gemm_direct(const GemmArgs& A, const Block& B, c
     };
     stage(0, 0);
     __syncthreads();
-    const uint32_t groups = (n + kGroup - 1) / kGroup;
+    const uint32_t groups = (n + kDGroup - 1) / kDGroup;
     for (uint32_t gi = 0; gi < groups; ++gi) {
-        const uint32_t s = gi * kGroup;
-        half8 x[kGroup][2];
+        const uint32_t s = gi * kDGroup;
+        half8 x[kDGroup][2];
 #pragma unroll
-        for (uint32_t k = 0; k < kGroup; ++k) {
+        for (uint32_t k = 0; k < kDGroup; ++k) {
             const size_t o = (size_t)(s + k < n ? s + k : n - 1) * wstep;
             x[k][0] = w0[o];
             x[k][1] = w1[o];
         }
-        if (gi + 1 < groups) stage(s + kGroup, (gi & 1) ^ 1);  // its readers passed the previous barrier
+        if (gi + 1 < groups) stage(s + kDGroup, (gi & 1) ^ 1);  // its readers passed the previous barrier
         const half8* sb = sB[gi & 1];
 #pragma unroll
-        for (uint32_t k = 0; k < kGroup; ++k)
+        for (uint32_t k = 0; k < kDGroup; ++k)
             if (live && s + k < n) {
 #pragma unroll
                 for (uint32_t nt = 0; nt < kNt; ++nt) {
@@ -897,7 +900,7 @@ __device__ __forceinline__ void gemm_direct(const GemmArgs& A, const Block& B, c
 
 template <bool DIRECT>
 __global__ __launch_bounds__(256, 2) void contract_gemm_kernel(Probes Q, GemmArgs A) {
-    __shared__ half8 sB[2][kGroup * 4 * (DIRECT ? kColsPad : kCols)];
+    __shared__ half8 sB[2][DIRECT ? kDGroup * 4 * kColsPad : kGroup * 4 * kCols];
     __shared__ uint32_t sU[(kMaxSlice + kGroup) * 4], sMap[DIRECT ? 6 * kImages / 4 : 1];
     // hardware workgroup b runs on XCD b % 8: each XCD takes one run of the
     // items, whose neighbours share staged units, and of an item's probes,
@@ -1899,11 +1902,10 @@ hipError_t build_plan(hvx_contract_plan* P, int ctype, bool split) {
 }
 
 // From this many units over all probes on, plans that it can take go through
-// gemm_direct; below, the latency of its staging counts. us staged / direct: 24
-// probes 16^2 -> 16^2 x 5 (4,608 units) 22.8 / 22.9, 64 31.1 / 26.5, 1,024 242 / 159;
-// 64 probes 8^2 -> 8^2 x 4 (3,072) 25.7 / 28.0, 256 37.1 / 30.5; 24 probes 32^2 ->
-// 16^2 x 5 (23,040) 31.9 / 24.5; 64^2 -> 32^2 x 6, 2 (6,144) 30.3 / 30.6, 8 42.1 /
-// 37.4, 24 77.6 / 69.7, 256 876 / 585.
+// gemm_direct; below, the latency of its staging counts. us staged / direct: 64
+// probes 16^2 -> 16^2 x 5 31.1 / 26.3, 1,024 242 / 145; 64 probes 8^2 -> 8^2 x 4
+// (3,072 units) 25.7 / 28.0, 256 37.1 / 28.5; 24 probes 32^2 -> 16^2 x 5 31.9 / 24;
+// 8 probes 64^2 -> 32^2 x 6 42 / 37, 24 78 / 69, 256 876 / 647.
 constexpr uint64_t kDirectUnits = 8192;
 
 // The launches of a filter call over n probes (grid dimension y, z for the
